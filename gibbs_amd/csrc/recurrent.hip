@@ -6,8 +6,8 @@
 // A step's rows are a ragged batch: request r brings rows cu[r] .. cu[r+1]-1 and keeps its state in
 // slot[r] of the arena.  Every kernel treats a token the same way wherever its step was cut: the
 // recurrences here walk a request's rows in order with a fixed order of additions per token, so a prompt
-// in one step, in portions or token by token gives the same bits (the rules in chunks that long portions take, and the
-// one-kernel step of a decoded token, agree with these walks to rounding).
+// in one step, in portions or token by token gives the same bits, and 32-bit runs take these walks alone (the rules in chunks that
+// long portions take in bfloat16, and the one-kernel step of a decoded token, agree with them to rounding).
 #include "common.h"
 #include "lane8.h"
 

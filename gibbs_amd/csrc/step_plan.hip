@@ -1031,8 +1031,9 @@ struct DeltaBody : Body {
     const int act = g2.w ? 1 : 0;
     void* y = e.take((long)N * H * V * e.esize);
     // Requests at the head of the batch that bring one row each (row n is request n's) have a kernel of their own; the others prepare their
-    // rows and run in chunks where one of them brings a long portion, else they walk.
-    const bool steps = gibbs_delta_step_takes(D, V) && slot_stride % 4 == 0 && ((uintptr_t)rule_state % 16) == 0;
+    // rows and run in chunks where one of them brings a long portion, else they walk.  32-bit runs walk all of them: there a request's results
+    // do not depend, to the bit, on how it is cut or on what else is in the step.
+    const bool steps = e.bf16_run && gibbs_delta_step_takes(D, V) && slot_stride % 4 == 0 && ((uintptr_t)rule_state % 16) == 0;
     const int lead = !steps ? 0 : (e.rows_are_requests() ? N : a.lead_single), rest = N - lead, reqs = a.n_req - lead;
     if (lead > 0)
       RUN(e, gibbs_delta_step(qkv, C, raw + (long)off_b * e.esize, raw + (long)off_a * e.esize, in.O, e.p.dtype, a_channel, dt_bias, a_log, gate, ld_gate, act,
@@ -1048,7 +1049,7 @@ struct DeltaBody : Body {
                               a_channel ? a_channel + (long)lead * H * D : nullptr, dt_bias, a_log, beta, decay, rest, G, H, D, q_scale, unit_eps, a.stream));
       // (the rules address rows by cu, which counts the step's)
       float *b0 = beta - (long)lead * H, *d0 = decay - (long)lead * H * wide, *o0 = o - (long)lead * H * V;
-      if (a.max_q >= DELTA_CHUNKED_ROWS && C % 4 == 0 && gibbs_delta_chunks_take(D, V)) {
+      if (e.bf16_run && a.max_q >= DELTA_CHUNKED_ROWS && C % 4 == 0 && gibbs_delta_chunks_take(D, V)) {
         float* work = (float*)e.take(gibbs_delta_chunks_workspace(rest, reqs, H, D, V) * 4);
         RUN(e, gibbs_delta_chunks(qkv, qkv + (long)G * D, C, qkv + 2L * G * D, C, b0, d0, channel, rule_state, slot_stride, a.cu + lead, a.slot + lead, o0,
                                   work, rest, reqs, H, G, D, V, a.stream));
@@ -1113,8 +1114,9 @@ struct TimeMixBody : Body {
     e.give(t);
     void* y = e.take((long)N * C * e.esize);
     // Requests at the head of the batch that bring one row each (row n is request n's) take the row kernel; the others run in chunks where one
-    // of them brings a long portion, else they walk, with kernels for the decays and the gated norm around the walk.
-    const bool fits = 3 * apart < (1L << 31);
+    // of them brings a long portion, else they walk, with kernels for the decays and the gated norm around the walk (32-bit runs always:
+    // see DeltaBody).
+    const bool fits = e.bf16_run && 3 * apart < (1L << 31);
     const int lead = !(fits && gibbs_decayed_outer_rows_take(D)) ? 0 : (e.rows_are_requests() ? N : a.lead_single);
     const int rest = N - lead, reqs = a.n_req - lead;
     if (lead > 0)

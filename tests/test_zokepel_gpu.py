@@ -149,6 +149,19 @@ def test_cutting_changes_no_bit_in_32_bit(dirs, name):
         assert np.abs(cut[("r", p)] - whole[("r", p)]).max() <= 2e-6 * np.abs(whole[("r", p)]).max(), p
 
 
+@pytest.mark.parametrize("name", ["Q", "S"])
+def test_long_portions_and_what_shares_their_step_change_no_bit_in_32_bit(dirs, name):
+    """The same where portions are long enough for the rules in chunks of a bfloat16 run, and a decoded token, a short and a long portion share a step."""
+    d = dirs[name]
+    ids, other = ZH.tokens(21, 230, vocab_of(d)), ZH.tokens(22, 180, vocab_of(d))
+    whole = run_steps(make_engine(d, "float32"), [([("r", ids, list(range(230)))], [])])
+    steps = [([("r", ids[:30], list(range(30))), ("o", other[:140], [])], []), ([("r", ids[30:31], [0]), ("o", other[140:150], [])], []),
+             ([("o", other[150:151], []), ("r", ids[31:180], list(range(149)))], []), ([("r", ids[180:], list(range(50)))], [])]
+    cut = run_steps(make_engine(d, "float32"), steps)
+    for p in range(230):
+        assert np.array_equal(cut[("r", p)], whole[("r", p)]), (p, np.abs(cut[("r", p)] - whole[("r", p)]).max())
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", NAMES)
 def test_mixed_batches_with_pages_and_slots_used_again(dirs, name, dtype):
