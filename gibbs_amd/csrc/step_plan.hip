@@ -49,8 +49,8 @@ constexpr int SKINNY_ROWS_F32_OUT = 48;   // the same for float32 output (the he
 constexpr int ACT_CLAMPED = 4;            // the gated feed-forward's clamped activation (activation.h: ACT_CLAMPED_SWISH)
 constexpr int SSD_CHUNKED_ROWS = 256;     // rows of one request from which the state-space rule runs in chunks
 constexpr int GATED_CHUNKED_ROWS = 96;    // rows of a request from which the gated outer-product rule runs in chunks
-// rows of a request from which the gated delta rule runs in chunks (one request of 64 tokens, 16 heads of 128 x 128: walk 32 us, chunks 27 to 33;
-// 96 tokens 39 to 44 and 33 to 38)
+// rows of a request from which the gated delta rule runs in chunks (one request, 16 heads of 128 x 128, a decay per head and per channel, us:
+// 64 tokens walk 26 and 29, chunks 27 and 37; 96 tokens 36 and 41, 31 and 41; 128 tokens 47 and 53, 31 and 41)
 constexpr int DELTA_CHUNKED_ROWS = 96;
 // rows of a request from which the decayed outer-product rule runs in chunks: the line of the gated rules, whose chunk kernels it shares
 // (2,048 tokens, 32 heads of 64: walk with its decays and its norm 979 us, chunks 118)
