@@ -428,6 +428,26 @@ def test_delta_rule_in_chunks_is_as_exact_as_the_walk(D, per_channel, kind):
         assert mine <= 1.25 * walk, errors
 
 
+@pytest.mark.parametrize("lens,H", [([1100, 70], 64), ([64 * 65536 + 1], 1)])
+def test_delta_rule_in_chunks_of_long_prompts(lens, H):
+    """More chunks than the workspace holds at once, two requests across its border, and more than a launch's second dimension could be: the
+    workspace stays below 256 MB, and what comes out is the walk's to rounding (32 of 2^-24, as above)."""
+    from gibbs_amd import ops
+    from gibbs_amd.ops.lib import library
+    assert all(library().gibbs_delta_chunks_workspace(rows, 3, 16, 128, 128) * 4 <= 2 ** 28 for rows in (100, 16384, 2 ** 30))
+    n, D = sum(lens), 16
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rnd = lambda *shape: torch.randn(shape, generator=g, device="cuda")
+    q, k = (torch.nn.functional.normalize(rnd(n, H, D), dim=-1).reshape(n, -1) for _ in range(2))
+    v, beta, decay, start = rnd(n, H * D), torch.rand((n, H), generator=g, device="cuda"), 1 - 0.1 * torch.rand((n, H), generator=g, device="cuda"), rnd(len(lens), H, D, D)
+    cu, slot = (torch.tensor(x, dtype=torch.int32, device="cuda") for x in (np.concatenate([[0], np.cumsum(lens)]), range(len(lens))))
+    states = [start.clone(), start.clone()]
+    walk, mine = (ops.delta_rule(q, k, v, beta, decay, s, cu, slot, H, H, chunks=c) for s, c in zip(states, (False, True)))
+    for got, want in [(mine, walk)] + list(zip(states[1], states[0])):
+        assert (got - want).norm() <= 32 * 2.0 ** -24 * want.norm()
+    assert (mine - walk)[-64:].norm() <= 32 * 2.0 ** -24 * walk[-64:].norm()
+
+
 def test_decayed_outer_rule_two_requests_side_by_side():
     from gibbs_amd import ops
     rng = np.random.default_rng(3)
