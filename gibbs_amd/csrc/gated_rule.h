@@ -212,7 +212,7 @@ int launch_rule_rows(const RuleArgs& a, int n_req, hipStream_t stream) {
 //   s in the first half of t's segment, t in the second   both about the border between the halves
 //   both in the same half (8 tokens)   about the half's middle: a factor may grow over at most four tokens, and log2 f is kept
 //   above -28 here (f at least 3.7e-9: what is left of the state then is below the rounding of what is added), 2^112
-// so nothing overflows that is used.  Logarithms are to base 2: the vector unit's own exponential, logarithm and reciprocal
+// so nothing overflows that is used (RULE_BONUS has no such bound: `bonus_scores`).  Logarithms are to base 2: the vector unit's own exponential, logarithm and reciprocal
 // (one unit in the last place) are what the many factors cost.  The order of additions differs from the walk's: results
 // agree to rounding.
 constexpr int CHUNK = 64, SEG = 16, CT = 512, CWAVES = CT / WAVE, MAX_VT = 2;
@@ -220,6 +220,7 @@ constexpr float LOG2E = 1.44269504088896340736f;
 __device__ __forceinline__ float exp2_of(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float rcp_of(float x) { return __builtin_amdgcn_rcpf(x); }
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
+typedef __attribute__((__vector_size__(4 * sizeof(double)))) double doublex4;
 struct ChunkedArgs {
   RuleArgs r;
   float* u;                   // [places, H, D, V]: U, then the state in front of each chunk
@@ -248,10 +249,11 @@ __device__ __forceinline__ float log2_sigmoid(float x) {
   return fmaf(fminf(x, 0.f), LOG2E, -tail);
 }
 // q (optional), k and b of the chunk's tokens into LDS rows of `lq` floats (channels from D to Dp and tokens beyond the end:
-// q = k = 0, no decay), and the segments' sums tot [4][lq].  RULE_BONUS with q: se, the sums in front of each token, for its read-out.
+// q = k = 0, no decay), and the segments' sums tot [4][lq].  RULE_BONUS: instead of b the sums behind each token in its segment, and with q none,
+// but this thread's 16 exponents in `own` (its only turn: a thread for each channel of each segment).
 template <typename T, bool Q, int RULE>
-__device__ __forceinline__ void chunk_gates(const ChunkedArgs& ca, int h, int t0, int rows, int Dp, int lq, float* sq, float* sk, float* sb, float* se,
-                                            float* tot) {
+__device__ __forceinline__ void chunk_gates(const ChunkedArgs& ca, int h, int t0, int rows, int Dp, int lq, float* sq, float* sk, float* sb,
+                                            float (&own)[RULE == RULE_BONUS ? SEG : 1], float* tot) {
   const RuleArgs& a = ca.r;
   const int C = a.H * a.D, span = 1 << ca.d_shift;
   for (int idx = threadIdx.x; idx < (CHUNK / SEG) * span; idx += CT) {
@@ -286,18 +288,26 @@ __device__ __forceinline__ void chunk_gates(const ChunkedArgs& ca, int h, int t0
       } else {
         k = to_float(z[t]);
         if constexpr (RULE == RULE_LINEAR) lf = fmaxf(log2_sigmoid(zf[t] + bias) * a.inv_tau, -28.0f);
-        else lf = fmaxf(-LOG2E * expf(zf[t] + bias), -28.0f);
+        else lf = -LOG2E * expf(zf[t] + bias);
       }
-      if constexpr (Q && RULE == RULE_BONUS) se[row * lq + i] = run;
+      if constexpr (RULE == RULE_BONUS) own[t] = in ? lf : 0.f;
       run += in ? lf : 0.f;
       sk[row * lq + i] = in ? k : 0.f;
-      sb[row * lq + i] = run;
+      if constexpr (RULE != RULE_BONUS) sb[row * lq + i] = run;
       if constexpr (Q) {
         const float y = to_float(q[t]);
         sq[row * lq + i] = !in ? 0.f : (RULE == RULE_COMPLEMENT ? y * rcp_of(1.0f + exp2_of(-y * LOG2E)) : RULE == RULE_LINEAR ? y * a.q_scale : y);
       }
     }
     tot[seg * lq + i] = run;
+    if constexpr (!Q && RULE == RULE_BONUS) {
+      float behind = 0.f;
+#pragma unroll
+      for (int t = SEG - 1; t >= 0; --t) {
+        sb[(seg * SEG + t) * lq + i] = behind;
+        behind += own[t];
+      }
+    }
   }
 }
 template <typename T>
@@ -323,6 +333,9 @@ __device__ __forceinline__ void chunk_values(const ChunkedArgs& ca, int h, int t
   }
 }
 
+// The partial sums that a piece of the state is taken in: RULE_BONUS four, which brings its error below the walk's.
+template <int RULE>
+constexpr int SUMS = RULE == RULE_BONUS ? 4 : 1;
 template <typename T, int RULE>
 __global__ __launch_bounds__(CT) void gated_rule_chunk_state_kernel(ChunkedArgs ca) {
   extern __shared__ float lds[];
@@ -335,17 +348,18 @@ __global__ __launch_bounds__(CT) void gated_rule_chunk_state_kernel(ChunkedArgs 
   int t0, rows;
   if (!chunk_of(ca, blockIdx.x, &t0, &rows)) return;
   const int h = blockIdx.y;
-  chunk_gates<T, false, RULE>(ca, h, t0, rows, Dp, lq, nullptr, sk, sb, nullptr, tot);
+  float own[RULE == RULE_BONUS ? SEG : 1];
+  chunk_gates<T, false, RULE>(ca, h, t0, rows, Dp, lq, nullptr, sk, sb, own, tot);
   chunk_values<T>(ca, h, t0, rows, Vp, lv, sv);
   __syncthreads();
   // k_s times the decay from behind s to the chunk's end
   for (int idx = threadIdx.x; idx < (CHUNK / SEG) << ca.d_shift; idx += CT) {
     const int seg = idx >> ca.d_shift, i = idx & ((1 << ca.d_shift) - 1);
     if (i >= Dp) continue;
-    float rest = tot[seg * lq + i];
+    float rest = RULE == RULE_BONUS ? 0.f : tot[seg * lq + i];
     for (int m = seg + 1; m < CHUNK / SEG; ++m) rest += tot[m * lq + i];
 #pragma unroll
-    for (int t = seg * SEG; t < seg * SEG + SEG; ++t) sk[t * lq + i] *= exp2_of(rest - sb[t * lq + i]);
+    for (int t = seg * SEG; t < seg * SEG + SEG; ++t) sk[t * lq + i] *= exp2_of(RULE == RULE_BONUS ? rest + sb[t * lq + i] : rest - sb[t * lq + i]);
   }
   if (threadIdx.x < a.D) {
     const int i = threadIdx.x;
@@ -356,7 +370,7 @@ __global__ __launch_bounds__(CT) void gated_rule_chunk_state_kernel(ChunkedArgs 
   float* u = ca.u + ((size_t)blockIdx.x * a.H + h) * a.D * a.V;
   for (int n0 = wave * 16; n0 < Vp; n0 += CWAVES * 16) {
     for (int m0 = 0; m0 < Dp; m0 += 64) {           // four channel tiles at a time
-      floatx4 acc[4] = {};
+      floatx4 acc[4][SUMS<RULE>] = {};
       for (int s0 = 0; s0 < CHUNK; s0 += 16) {
         float vb[4];
 #pragma unroll
@@ -366,7 +380,8 @@ __global__ __launch_bounds__(CT) void gated_rule_chunk_state_kernel(ChunkedArgs 
           if (m0 + m * 16 >= Dp) break;
 #pragma unroll
           for (int j = 0; j < 4; ++j)
-            acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(sk[(s0 + g * 4 + j) * lq + m0 + m * 16 + lr], vb[j], acc[m], 0, 0, 0);
+            acc[m][j % SUMS<RULE>] =
+                __builtin_amdgcn_mfma_f32_16x16x4f32(sk[(s0 + g * 4 + j) * lq + m0 + m * 16 + lr], vb[j], acc[m][j % SUMS<RULE>], 0, 0, 0);
         }
       }
       const int col = n0 + lr;
@@ -375,7 +390,9 @@ __global__ __launch_bounds__(CT) void gated_rule_chunk_state_kernel(ChunkedArgs 
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int row = m0 + m * 16 + g * 4 + i;
-          if (row < a.D && col < a.V) u[(size_t)row * a.V + col] = acc[m][i];
+          float sum = acc[m][0][i];
+          if constexpr (SUMS<RULE> > 1) sum = (acc[m][0][i] + acc[m][1][i]) + (acc[m][2][i] + acc[m][3][i]);
+          if (row < a.D && col < a.V) u[(size_t)row * a.V + col] = sum;
         }
     }
   }
@@ -415,6 +432,112 @@ __global__ __launch_bounds__(256) void gated_rule_chunk_scan_kernel(ChunkedArgs 
   *state = S;
 }
 
+// The scores of RULE_BONUS: token t reads what s < t wrote, decayed by the tokens between them, and its own write through the bonus.  The
+// exponents of a factor are summed from the border out and never a difference of sums: a gentle decay behind a hard one keeps its digits, and
+// nothing grows, so there is no bound on a decay.  The border of two tokens of a segment is the middle of the smallest 2 span tokens
+// that hold both: a pass for each span, two at a time.  Summed in 64 bits.  Leaves q times the decays from the chunk's start.
+__device__ __forceinline__ void bonus_scores(const ChunkedArgs& ca, int h, int segs, int Dp, int lq, const float (&own)[SEG], float* sq, float* sk, float* f0,
+                                             float* f1, const float* tot, float* sA) {
+  constexpr int la = CHUNK + 4;
+  const RuleArgs& a = ca.r;
+  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE, lr = lane % 16, g = lane / 16;
+  const int seg = tid >> ca.d_shift, i = tid & ((1 << ca.d_shift) - 1);
+  const bool mine = seg < CHUNK / SEG && i < Dp;
+  for (int idx = tid; idx < CHUNK * la; idx += CT) sA[idx] = 0.f;
+#pragma unroll
+  for (int pass = 0; pass < 2; ++pass) {
+    if (mine) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int span = 1 << (2 * pass + k);
+        float* f = (k ? f1 : f0) + seg * SEG * lq + i;
+        float run = 0.f;
+#pragma unroll
+        for (int t = 0; t < SEG; ++t) {
+          if (t % span == 0) run = 0.f;
+          if (t & span) {
+            f[t * lq] = exp2_of(run);
+            run += own[t];
+          }
+        }
+#pragma unroll
+        for (int t = SEG - 1; t >= 0; --t) {
+          if (t % span == span - 1) run = 0.f;
+          if (!(t & span)) {
+            f[t * lq] = exp2_of(run);
+            run += own[t];
+          }
+        }
+      }
+    }
+    __syncthreads();
+    const int I = wave % 4, span = 1 << (2 * pass + wave / 4);
+    if (I < segs) {
+      const float *q = sq + (I * SEG + lr) * lq, *k = sk + (I * SEG + lr) * lq, *f = (wave / 4 ? f1 : f0) + (I * SEG + lr) * lq;
+      doublex4 sum = {};
+      for (int c0 = 4 * g; c0 < Dp; c0 += 16)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          sum = __builtin_amdgcn_mfma_f64_16x16x4f64((double)(q[c0 + j] * f[c0 + j]), (double)(k[c0 + j] * f[c0 + j]), sum, 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int t = g + 4 * j;      // (as a 64-bit product leaves it)
+        if ((t & span) && t / span == lr / span + 1) sA[(I * SEG + t) * la + I * SEG + lr] = (float)sum[j];
+      }
+    }
+    if (pass == 0) {      // a token with itself: eight threads a token
+      const int t = tid / 8;
+      double score = 0.0;
+      for (int c = tid % 8; c < a.D; c += 8) score += (double)sq[t * lq + c] * (double)a.bonus[h * a.D + c] * (double)sk[t * lq + c];
+#pragma unroll
+      for (int o = 1; o < 8; o *= 2) score += __shfl_xor(score, o, WAVE);
+      if (tid % 8 == 0) sA[t * la + t] = (float)score;
+    }
+    __syncthreads();
+  }
+  // between segments q times the decays in front of it in its segment, k times those behind it in its own
+  if (mine) {
+    float run = 0.f;
+#pragma unroll
+    for (int t = 0; t < SEG; ++t) {
+      const int at = (seg * SEG + t) * lq + i;
+      f0[at] = sq[at] * exp2_of(run);
+      run += own[t];
+    }
+    run = 0.f;
+#pragma unroll
+    for (int t = SEG - 1; t >= 0; --t) {
+      const int at = (seg * SEG + t) * lq + i;
+      f1[at] = sk[at] * exp2_of(run);
+      run += own[t];
+    }
+    // (and for what the state in front of the chunk gives)
+    run = 0.f;
+    for (int m = 0; m < seg; ++m) run += tot[m * lq + i];
+#pragma unroll
+    for (int t = 0; t < SEG; ++t) {
+      sq[(seg * SEG + t) * lq + i] *= exp2_of(run);
+      run += own[t];
+    }
+  }
+  __syncthreads();
+  for (int p = wave; p < 6; p += CWAVES) {      // pairs of segments
+    const int to = p < 1 ? 1 : (p < 3 ? 2 : 3), from = p < 1 ? 0 : (p < 3 ? p - 1 : p - 3);
+    if (to >= segs) continue;
+    const float *q = f0 + (to * SEG + lr) * lq, *k = f1 + (from * SEG + lr) * lq;
+    doublex4 sum = {};
+    for (int c0 = 4 * g; c0 < Dp; c0 += 16)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float between = 0.f;
+        for (int m = from + 1; m < to; ++m) between += tot[m * lq + c0 + j];
+        sum = __builtin_amdgcn_mfma_f64_16x16x4f64((double)q[c0 + j], (double)(k[c0 + j] * exp2_of(between)), sum, 0, 0, 0);
+      }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sA[(to * SEG + g + 4 * j) * la + from * SEG + lr] = (float)sum[j];
+  }
+}
+
 enum { PASS_EARLIER = 0, PASS_HALF = 1, PASS_BORDER = 2 };
 template <typename T, int RULE>
 __global__ __launch_bounds__(CT) void gated_rule_chunk_out_kernel(ChunkedArgs ca) {
@@ -429,23 +552,25 @@ __global__ __launch_bounds__(CT) void gated_rule_chunk_out_kernel(ChunkedArgs ca
   float* sA = sv + CHUNK * lv;            // [CHUNK][la]
   float* tot = sA + CHUNK * la;           // [4][lq]
   float* red = tot + 4 * lq;              // [CWAVES][CHUNK]
-  float* se = RULE == RULE_BONUS ? red + CWAVES * CHUNK : sb;      // [CHUNK][lq]: what has decayed when a token is read out
+  float* sf = RULE == RULE_BONUS ? red + CWAVES * CHUNK : sb;      // [CHUNK][lq]: the other of two passes' factors
   int t0, rows;
   if (!chunk_of(ca, blockIdx.x, &t0, &rows)) return;
   const int h = blockIdx.y;
-  chunk_gates<T, true, RULE>(ca, h, t0, rows, Dp, lq, sq, sk, sb, se, tot);
+  float own[RULE == RULE_BONUS ? SEG : 1];
+  chunk_gates<T, true, RULE>(ca, h, t0, rows, Dp, lq, sq, sk, sb, own, tot);
   chunk_values<T>(ca, h, t0, rows, Vp, lv, sv);
   __syncthreads();
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, lr = lane % 16, g = lane / 16;
   const int segs = (rows + SEG - 1) / SEG;
+  if constexpr (RULE == RULE_BONUS) bonus_scores(ca, h, segs, Dp, lq, own, sq, sk, sb, sf, tot, sA);
   // the scores' tiles: six of pairs of segments, and two passes for each segment with itself
-  for (int p = wave; p < 14; p += CWAVES) {
+  for (int p = wave; RULE != RULE_BONUS && p < 14; p += CWAVES) {
     const int kind = p < 6 ? PASS_EARLIER : (p < 10 ? PASS_HALF : PASS_BORDER);
     const int I = kind == PASS_EARLIER ? (p < 1 ? 1 : (p < 3 ? 2 : 3)) : (p - 6) % 4;
     const int J = kind == PASS_EARLIER ? (p < 1 ? 0 : (p < 3 ? p - 1 : p - 3)) : I;
     if (I >= segs) continue;
     const float* qr = sq + (I * SEG + lr) * lq;
-    const float* bq = se + (I * SEG + lr) * lq;
+    const float* bq = sb + (I * SEG + lr) * lq;
     const float* kr = sk + (J * SEG + lr) * lq;
     const float* bk = sb + (J * SEG + lr) * lq;
     const float* ref = kind == PASS_EARLIER ? tot + J * lq : sb + (I * SEG + (kind == PASS_BORDER ? 7 : (lr < 8 ? 3 : 11))) * lq;
@@ -474,29 +599,29 @@ __global__ __launch_bounds__(CT) void gated_rule_chunk_out_kernel(ChunkedArgs ca
       float* dst = sA + (I * SEG + t) * la + J * SEG + lr;
       if (kind == PASS_EARLIER) *dst = acc[i];
       else if (kind == PASS_BORDER) { if (t >= 8 && lr < 8) *dst = acc[i]; }
-      else if (!(t >= 8 && lr < 8) && (RULE != RULE_BONUS || lr != t)) *dst = (t / 8 == lr / 8 && lr <= t) ? acc[i] : 0.f;
+      else if (!(t >= 8 && lr < 8)) *dst = (t / 8 == lr / 8 && lr <= t) ? acc[i] : 0.f;
     }
-  }
-  if constexpr (RULE == RULE_BONUS) {      // a token with itself: eight threads a token
-    const int t = threadIdx.x / 8;
-    float own = 0.f;
-    for (int i = threadIdx.x % 8; i < a.D; i += 8) own = fmaf(sq[t * lq + i] * a.bonus[h * a.D + i], sk[t * lq + i], own);
-    own = group_sum<8>(own);
-    if (threadIdx.x % 8 == 0) sA[t * la + t] = own;
   }
   __syncthreads();
   // q_t times the decay from the chunk's start to t
-  for (int idx = threadIdx.x; idx < (CHUNK / SEG) << ca.d_shift; idx += CT) {
+  for (int idx = threadIdx.x; RULE != RULE_BONUS && idx < (CHUNK / SEG) << ca.d_shift; idx += CT) {
     const int seg = idx >> ca.d_shift, i = idx & ((1 << ca.d_shift) - 1);
     if (i >= Dp) continue;
     float before = 0.f;
     for (int m = 0; m < seg; ++m) before += tot[m * lq + i];
 #pragma unroll
-    for (int t = seg * SEG; t < seg * SEG + SEG; ++t) sq[t * lq + i] *= exp2_of(before + se[t * lq + i]);
+    for (int t = seg * SEG; t < seg * SEG + SEG; ++t) sq[t * lq + i] *= exp2_of(before + sb[t * lq + i]);
   }
   __syncthreads();
   const float* s0 = ca.u + ((size_t)blockIdx.x * a.H + h) * a.D * a.V;
   floatx4 acc[MAX_VT][CHUNK / SEG] = {};
+  // sum += 16 tokens' or channels' products (RULE_BONUS: summed by themselves, which brings its error to the walk's)
+  auto add = [](floatx4& sum, const float (&x)[4], const float (&y)[4]) {
+    floatx4 part = RULE == RULE_BONUS ? floatx4{} : sum;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) part = __builtin_amdgcn_mfma_f32_16x16x4f32(x[j], y[j], part, 0, 0, 0);
+    sum = RULE == RULE_BONUS ? sum + part : part;
+  };
 #pragma unroll
   for (int v = 0; v < MAX_VT; ++v) {
     const int n0 = (wave + v * CWAVES) * 16, col = n0 + lr;
@@ -510,8 +635,7 @@ __global__ __launch_bounds__(CT) void gated_rule_chunk_out_kernel(ChunkedArgs ca
         if (I < c / SEG || I >= segs) continue;
         const float4 a4 = *(const float4*)(sA + (I * SEG + lr) * la + c + g * 4);
         const float av[4] = {a4.x, a4.y, a4.z, a4.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[v][I] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j], vb[j], acc[v][I], 0, 0, 0);
+        add(acc[v][I], av, vb);
       }
     }
 #pragma unroll 2
@@ -526,8 +650,7 @@ __global__ __launch_bounds__(CT) void gated_rule_chunk_out_kernel(ChunkedArgs ca
       for (int I = 0; I < CHUNK / SEG; ++I) {
         const float4 q4 = *(const float4*)(sq + (I * SEG + lr) * lq + c + g * 4);
         const float qv[4] = {q4.x, q4.y, q4.z, q4.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[v][I] = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[j], sb4[j], acc[v][I], 0, 0, 0);
+        add(acc[v][I], qv, sb4);
       }
     }
   }

@@ -52,8 +52,8 @@ constexpr int GATED_CHUNKED_ROWS = 96;    // rows of a request from which the ga
 // rows of a request from which the gated delta rule runs in chunks (one request, 16 heads of 128 x 128, a decay per head and per channel, us:
 // 64 tokens walk 26 and 29, chunks 27 and 37; 96 tokens 36 and 41, 31 and 41; 128 tokens 47 and 53, 31 and 41)
 constexpr int DELTA_CHUNKED_ROWS = 96;
-// rows of a request from which the decayed outer-product rule runs in chunks: the line of the gated rules, whose chunk kernels it shares
-// (2,048 tokens, 32 heads of 64: walk with its decays and its norm 979 us, chunks 118)
+// rows of a request from which the decayed outer-product rule runs in chunks (one request, 16 and 32 heads of 64, the walk with its decays and its
+// norm, us: 48 tokens walk 23 and 25, chunks 31; 64 tokens 29, 33 and 34; 96 tokens 39, 33 and 34; 128 tokens 49 and 50, 33 and 34)
 constexpr int TIME_MIX_CHUNKED_ROWS = 96;
 constexpr int WALKED_ROWS = 24;           // rows of a request from which gated linear attention and the matrix memory run in chunks
 constexpr int MATRIX_SLICE_PAGES = 510;   // page ids of a key slice that the decode attention's matrix-core walk keeps in LDS
