@@ -50,6 +50,33 @@ __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
+__device__ __forceinline__ bool finite(float x) { return x * 0.f == 0.f; }
+// For an operand of a product whose other operand has zeros above a diagonal (lane (g, c) of a wave: rows 4 g .. 4 g + 3 of column c of a 16 x
+// 16 tile): what is not finite is taken out of it, since 0 times that would reach the rows in front of it too.  Returned is what
+// to add to the product: NaN in the rows from the first such one of its column on, else 0.
+template <typename F4>
+__device__ __forceinline__ F4 nan_behind(F4& x, int g) {
+  F4 add = {0.f, 0.f, 0.f, 0.f};
+  if (__builtin_amdgcn_ballot_w64(!finite(x[0] * 0.f + x[1] * 0.f + x[2] * 0.f + x[3] * 0.f)) != 0) {
+    float run = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      run += x[i] * 0.f;
+      add[i] = run;
+      if (!finite(x[i])) x[i] = 0.f;
+    }
+    float before = 0.f;
+#pragma unroll
+    for (int o = 1; o < 4; ++o) {
+      const float y = __shfl_up(run, 16 * o, WAVE);
+      if (g >= o) before += y;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) add[i] += before;
+  }
+  return add;
+}
+
 // Rotation factors of this lane's 8 elements at position `pos` (the same for every head).
 struct Rot8 {
   float c[EPL], s[EPL];

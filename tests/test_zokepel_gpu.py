@@ -428,6 +428,36 @@ def test_delta_rule_in_chunks_is_as_exact_as_the_walk(D, per_channel, kind):
         assert mine <= 1.25 * walk, errors
 
 
+@pytest.mark.parametrize("what", ["q", "k", "v", "beta", "decay"])
+@pytest.mark.parametrize("per_channel", [False, True])
+def test_delta_rule_in_chunks_keeps_a_value_that_is_not_finite_behind_it(per_channel, what):
+    """The read-outs in front of such a value are what they are without it, to the bit, and another request's too; from it on what the walk leaves not
+    finite is not finite here either, and the rest (a column of v, a row of q) agrees with the walk to rounding, the state likewise."""
+    from gibbs_amd import ops
+    rng = np.random.default_rng(5)
+    n, H, D, V, lens = 200, 2, 48, 32, [150, 50]
+    q, k = rng.normal(size=(n, H, D)), rng.normal(size=(n, H, D))
+    q, k = q / np.linalg.norm(q, axis=-1, keepdims=True), k / np.linalg.norm(k, axis=-1, keepdims=True)
+    values = {"q": q, "k": k, "v": rng.normal(size=(n, H, V)), "beta": rng.uniform(0, 1, size=(n, H)),
+              "decay": rng.uniform(0.8, 1, size=(n, H, D) if per_channel else (n, H))}
+    start = torch.tensor(rng.normal(size=(2, H, D, V)), dtype=torch.float32, device="cuda")
+    cu, slot = (torch.tensor(x, dtype=torch.int32, device="cuda") for x in ([0, 150, 200], [1, 0]))
+    def run(x, chunks):
+        dev = {name: torch.tensor(a.reshape(n, -1), dtype=torch.float32, device="cuda") for name, a in x.items()}
+        state = start.clone()
+        return ops.delta_rule(*(dev[name] for name in ("q", "k", "v", "beta", "decay")), state, cu, slot, H, H, chunks=chunks).reshape(n, H, V), state
+    clean, _ = run(values, True)
+    for t, bad in ((7, np.nan), (77, np.inf), (64, -np.inf), (149, np.nan)):
+        x = {name: a.copy() for name, a in values.items()}
+        x[what][(t, 1) + (3,) * (x[what].ndim - 2)] = bad
+        (got, mine), (want, state) = run(x, True), run(x, False)
+        assert torch.equal(got[:t], clean[:t]) and torch.equal(got[:, 0], clean[:, 0]) and torch.equal(got[150:], clean[150:]), (t, bad)
+        assert not want[t, 1].isfinite().all()
+        for a, b in ((got, want), (mine, state)):
+            assert torch.equal(a.isfinite(), b.isfinite()), (t, bad)
+            assert (a - b)[b.isfinite()].norm() <= 32 * 2.0 ** -24 * b[b.isfinite()].norm()
+
+
 @pytest.mark.parametrize("lens,H", [([1100, 70], 64), ([64 * 65536 + 1], 1)])
 def test_delta_rule_in_chunks_of_long_prompts(lens, H):
     """More chunks than the workspace holds at once, two requests across its border, and more than a launch's second dimension could be: the
