@@ -310,10 +310,12 @@ __device__ __forceinline__ void chunk_gates(const ChunkedArgs& ca, int h, int t0
     }
   }
 }
+// The chunk's values into LDS; false: one that this thread has brought is not finite.
 template <typename T>
-__device__ __forceinline__ void chunk_values(const ChunkedArgs& ca, int h, int t0, int rows, int Vp, int lv, float* sv) {
+__device__ __forceinline__ bool chunk_values(const ChunkedArgs& ca, int h, int t0, int rows, int Vp, int lv, float* sv) {
   const RuleArgs& a = ca.r;
   const T* at = (const T*)a.raw + (size_t)t0 * a.ld + a.off_v + h * a.V;
+  float probe = 0.f;
   if (ca.v8) {
     const int span = 1 << ca.v_shift;
 #pragma unroll 2
@@ -322,15 +324,20 @@ __device__ __forceinline__ void chunk_values(const ChunkedArgs& ca, int h, int t
       if (j >= Vp) continue;
       float f[8] = {};
       if (t < rows && j < a.V) load_eight(at + (size_t)t * a.ld + j, f);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) probe = fmaf(f[e], 0.f, probe);
       *(float4*)(sv + t * lv + j) = make_float4(f[0], f[1], f[2], f[3]);
       *(float4*)(sv + t * lv + j + 4) = make_float4(f[4], f[5], f[6], f[7]);
     }
-    return;
+    return finite(probe);
   }
   for (int idx = threadIdx.x; idx < CHUNK * Vp; idx += CT) {
     const int t = idx / Vp, j = idx % Vp;
-    sv[t * lv + j] = (t < rows && j < a.V) ? to_float(at[(size_t)t * a.ld + j]) : 0.f;
+    const float f = (t < rows && j < a.V) ? to_float(at[(size_t)t * a.ld + j]) : 0.f;
+    probe = fmaf(f, 0.f, probe);
+    sv[t * lv + j] = f;
   }
+  return finite(probe);
 }
 
 // The partial sums that a piece of the state is taken in: RULE_BONUS four, which brings its error below the walk's.
@@ -558,10 +565,31 @@ __global__ __launch_bounds__(CT) void gated_rule_chunk_out_kernel(ChunkedArgs ca
   const int h = blockIdx.y;
   float own[RULE == RULE_BONUS ? SEG : 1];
   chunk_gates<T, true, RULE>(ca, h, t0, rows, Dp, lq, sq, sk, sb, own, tot);
-  chunk_values<T>(ca, h, t0, rows, Vp, lv, sv);
-  __syncthreads();
+  const bool clean = chunk_values<T>(ca, h, t0, rows, Vp, lv, sv);
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, lr = lane % 16, g = lane / 16;
   const int segs = (rows + SEG - 1) / SEG;
+  // A value that is not finite would meet the zeros above the scores' diagonal, and reach the tokens in front of it: it is taken out, and the
+  // read-outs of its column are made NaN from its token on.
+  const bool wave_clean = __builtin_amdgcn_ballot_w64(!clean) == 0;
+  if (lane == 0) red[wave] = wave_clean ? 0.f : 1.f;
+  __syncthreads();
+  bool unclean = false;
+#pragma unroll
+  for (int w = 0; w < CWAVES; ++w) unclean |= red[w] != 0.f;
+  int first_bad[MAX_VT];
+  if (unclean) {
+#pragma unroll
+    for (int v = 0; v < MAX_VT; ++v) {
+      const int col = (wave + v * CWAVES) * 16 + lr;
+      first_bad[v] = CHUNK;
+      for (int t = CHUNK - 1; t >= 0 && col < Vp; --t)
+        if (!finite(sv[t * lv + col])) first_bad[v] = t;
+    }
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < CHUNK * lv; idx += CT)
+      if (idx % lv < Vp && !finite(sv[idx])) sv[idx] = 0.f;
+    __syncthreads();
+  }
   if constexpr (RULE == RULE_BONUS) bonus_scores(ca, h, segs, Dp, lq, own, sq, sk, sb, sf, tot, sA);
   // the scores' tiles: six of pairs of segments, and two passes for each segment with itself
   for (int p = wave; RULE != RULE_BONUS && p < 14; p += CWAVES) {
@@ -653,6 +681,15 @@ __global__ __launch_bounds__(CT) void gated_rule_chunk_out_kernel(ChunkedArgs ca
         add(acc[v][I], qv, sb4);
       }
     }
+  }
+  if (unclean) {
+#pragma unroll
+    for (int v = 0; v < MAX_VT; ++v)
+#pragma unroll
+      for (int I = 0; I < CHUNK / SEG; ++I)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (I * SEG + g * 4 + i >= first_bad[v]) acc[v][I][i] = __builtin_nanf("");
   }
   // the heads' norm over V: a row's squares over the 16 columns of a tile, then over the waves (in order)
 #pragma unroll
