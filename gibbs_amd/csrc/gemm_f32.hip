@@ -267,17 +267,19 @@ struct F32Variant {
   int features, rows;
   float alone, loaded;
   void (*launch)(const float*, const float*, float*, int, int, int, long, long, long, bool, hipStream_t);
+  bool split;      // k cut over the waves, and rows along the grid's second dimension
 };
 const F32Variant F32_VARIANTS[] = {
-    {128, 128, 83.f, 78.f, launch_tile<4, 4>}, {64, 96, 39.f, 32.f, launch_tile<2, 3>},  {64, 64, 28.f, 21.f, launch_tile<2, 2>},
-    {32, 64, 19.4f, 12.2f, launch_tile<1, 2>}, {32, 32, 10.f, 9.6f, launch_split<2, 2>}, {16, 32, 6.1f, 6.f, launch_split<1, 2>},
-    {16, 16, 5.f, 4.2f, launch_split<1, 1>}};
+    {128, 128, 83.f, 78.f, launch_tile<4, 4>, false}, {64, 96, 39.f, 32.f, launch_tile<2, 3>, false}, {64, 64, 28.f, 21.f, launch_tile<2, 2>, false},
+    {32, 64, 19.4f, 12.2f, launch_tile<1, 2>, false}, {32, 32, 10.f, 9.6f, launch_split<2, 2>, true}, {16, 32, 6.1f, 6.f, launch_split<1, 2>, true},
+    {16, 16, 5.f, 4.2f, launch_split<1, 1>, true}};
 
 bool launch_f32(const float* A, const float* W, float* C, int N, int O, int I, long lda, long ldw, long ldc, hipStream_t stream) {
   if (I % 4 || lda % 4 || ldw % 4 || (uintptr_t)A % 16 || (uintptr_t)W % 16) return false;
   const F32Variant* best = nullptr;
   float least = 0.f;
   for (const F32Variant& v : F32_VARIANTS) {
+    if (v.split && ceil_div(N, v.rows) > 65535) continue;
     const long tiles = (long)ceil_div(N, v.rows) * ceil_div(O, v.features);
     const float cost = fmaxf(v.alone, (float)((tiles + 255) / 256) * v.loaded);
     if (!best || cost < least) {

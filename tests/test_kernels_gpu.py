@@ -90,6 +90,15 @@ def test_gemm_f32_tiles_and_stretches(shape):
             assert torch.equal(ops.gemm_f32(a[:m].contiguous(), w), out[:m]), (shape, m)
 
 
+def test_gemm_f32_as_many_rows_as_the_plain_kernel_takes():
+    """4,194,240 rows, which is where the plain kernel's grid ends, of few features: the tiles that cut k over their waves have no grid for them."""
+    from gibbs_amd import ops
+    n, o, i = 65535 * 64, 5, 4
+    a, w = rnd(n, i), rnd(o, i, seed=1)
+    out, want, scale = ops.gemm_f32(a, w), a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
+    assert ((out.double() - want).abs() <= i * 2.0 ** -24 * scale).all()
+
+
 @pytest.mark.parametrize("out_dtype", DT)
 @pytest.mark.parametrize("shape", [(1, 64, 32), (5, 331, 112), (130, 200, 72), (257, 129, 1000), (300, 512, 2048),
                                    (2048, 6144, 192), (1024, 12288, 64), (768, 16384, 320)])   # the 256 x 256 kernel: both tile orders
