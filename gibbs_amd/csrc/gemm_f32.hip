@@ -259,8 +259,10 @@ void launch_split(const float* A, const float* W, float* C, int N, int O, int I,
 }
 
 // The variants, and which one takes a shape.  A compute unit works through ceil(tiles / 256) tiles; one tile alone takes `alone`, one among
-// others on the same unit `loaded` (us at an inner size of 1,024, of which both are multiples; measured), so the least of max(alone, rounds *
-// loaded) is taken.  Features x rows of a tile; the last three cut k over their waves and serve few rows.  (1,194 rows, us, with the vector
+// others on the same unit `loaded` (us at an inner size of 1,024; measured), so the least of max(alone, rounds * loaded) is taken.  Both grow with
+// the inner size alike, but for inner sizes under 512, where one wave of a split tile's eight walks all of k: alone it then takes twice
+// its share, among others 1.25 times (inner size 508, us, without and with that: 45 rows x 4,096 features 11.0 / 7.5, 300 x 1,024 12.9 / 10.8, 300 x
+// 256 7.1 / 5.4).  Features x rows of a tile; the last three cut k over their waves and serve few rows.  (1,194 rows, us, with the vector
 // unit's kernel before / now: 9,216 x 1,024 360 / 250, 1,024 x 4,608 640 / 162, 1,024 x 1,024 147 / 39, 3,072 x 1,024 174 / 88;
 // 8 rows: 9,216 x 1,024 85 / 15, 1,024 x 4,608 250 / 16.)
 struct F32Variant {
@@ -281,7 +283,8 @@ bool launch_f32(const float* A, const float* W, float* C, int N, int O, int I, l
   for (const F32Variant& v : F32_VARIANTS) {
     if (v.split && ceil_div(N, v.rows) > 65535) continue;
     const long tiles = (long)ceil_div(N, v.rows) * ceil_div(O, v.features);
-    const float cost = fmaxf(v.alone, (float)((tiles + 255) / 256) * v.loaded);
+    const bool one_wave = v.split && f32_segments(I) == 1;
+    const float cost = fmaxf(v.alone * (one_wave ? 2.f : 1.f), (float)((tiles + 255) / 256) * v.loaded * (one_wave ? 1.25f : 1.f));
     if (!best || cost < least) {
       best = &v;
       least = cost;
