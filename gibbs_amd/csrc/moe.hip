@@ -22,7 +22,9 @@
 // that are not 16-byte aligned; on the matrix cores for aligned bfloat16, float32 accumulators, the activation in
 // float32: tiles of 16 pairs for steps of few pairs (the experts' matrices are streamed once, a workgroup's four
 // waves split k, operands straight from memory: rows of h and of every W are contiguous along k), tiles of 128
-// pairs beyond (128 pairs x 128 or 256 rows of W through LDS in tiles of 32 along k, double-buffered).
+// pairs beyond (inner sizes of whole tiles of 64 k: 128 pairs x 256 rows of W loaded straight into LDS, three tiles deep, a workgroup a
+// compute unit that goes from item to item; others: 128 pairs x 128 or 256 rows of W through registers into LDS in tiles of 32 k,
+// double-buffered).
 #include "common.h"
 #include "activation.h"
 #include <algorithm>
@@ -568,7 +570,7 @@ int launch_tiled_as(const bf16* X, long ldx, int top, const int* sorted_pair, co
 // 400; 830 TFLOP/s); 1,400 pairs of 8 experts, width 2,048, 512 features 41 and 20 (70 and 23).  Slower: a workgroup an item (122 us
 // in the first of these), tiles of 32 k with two workgroups a compute unit (133: requests of 64 bytes), 128 rows of W (148), and an
 // XCD's units on neighbouring items (129; 127 against 149 at a width of 2,112, but 750 against 654 at 4,096).
-constexpr int ASYNC_BK = 64, ASYNC_BN = 256, ASYNC_STAGES = 3;
+constexpr int ASYNC_BK = 64, ASYNC_BN = 256, ASYNC_STAGES = 3, ASYNC_UNITS = 256;   // (units: one workgroup a compute unit)
 // v <- activate(w * v): the activation is chosen once, not for each of the 16
 __device__ __forceinline__ void activate_all(floatx16& v, float w, int act) {
   auto all = [&](auto f) {
@@ -734,7 +736,7 @@ __global__ __launch_bounds__(512) void moe_gemm_async_kernel(const bf16* __restr
 template <bool GLU>
 int launch_async(const bf16* X, long ldx, int top, const int* sorted_pair, const int* tile_expert, int tiles, const bf16* wa, const bf16* wb,
                  long stride, bf16* Y, long ldy, int O, int I, int act, const float* in_weight, hipStream_t stream) {
-  constexpr int LDS = ASYNC_STAGES * (TBM + ASYNC_BN) * ASYNC_BK * (int)sizeof(bf16), UNITS = 256;   // one workgroup a compute unit
+  constexpr int LDS = ASYNC_STAGES * (TBM + ASYNC_BN) * ASYNC_BK * (int)sizeof(bf16);
   static bool prepared = false;    // (one flag per instantiation)
   if (!prepared) {
     hipError_t e = hipFuncSetAttribute((const void*)moe_gemm_async_kernel<GLU>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
@@ -743,16 +745,25 @@ int launch_async(const bf16* X, long ldx, int top, const int* sorted_pair, const
   }
   const int columns = ceil_div(O, GLU ? ASYNC_BN / 2 : ASYNC_BN);
   GIBBS_REQUIRE((long)columns * tiles < (1L << 30), "moe_gemm: %d columns of %d tiles", columns, tiles);
-  moe_gemm_async_kernel<GLU><<<std::min(UNITS, columns * tiles), 512, LDS, stream>>>(X, ldx, top, sorted_pair, tile_expert, wa, wb, stride, Y, ldy, O, I,
+  moe_gemm_async_kernel<GLU><<<std::min(ASYNC_UNITS, columns * tiles), 512, LDS, stream>>>(X, ldx, top, sorted_pair, tile_expert, wa, wb, stride, Y, ldy, O, I,
                                                                                     act, in_weight, columns, columns * tiles);
   return 0;
 }
 template <bool GLU>
 int launch_tiled(const bf16* X, long ldx, int top, const int* sorted_pair, const int* tile_expert, int tiles, const bf16* wa, const bf16* wb,
                  long stride, bf16* Y, long ldy, int O, int I, int act, const float* in_weight, hipStream_t stream) {
-  // (128 rows of W and 4 waves for the inner sizes that are left)
-  if (I % ASYNC_BK == 0 && I >= 2 * ASYNC_BK)
+  // Short inner sizes of one matrix stay with the kernel whose workgroups are many where the other's second or third round of items would be
+  // the last and leave three eighths of the units idle or more (8,320 pairs of 16 experts, us, here and there: 1,024 features, inner size 128
+  // 14.5 and 17.1, 256 19.3 and 21.5, 512 28.2 and 27.1; 2,048 features, 128 23.6 and 26.3).
+  const long items = (long)ceil_div(O, GLU ? ASYNC_BN / 2 : ASYNC_BN) * tiles, last = items % ASYNC_UNITS;
+  const bool idle = !GLU && I < 512 && items > ASYNC_UNITS && items <= 3 * ASYNC_UNITS && last > 0 && last <= ASYNC_UNITS * 5 / 8;
+  if (I % ASYNC_BK == 0 && I >= 2 * ASYNC_BK && !idle)
     return launch_async<GLU>(X, ldx, top, sorted_pair, tile_expert, tiles, wa, wb, stride, Y, ldy, O, I, act, in_weight, stream);
+  // what is left: wide results with a long inner size 256 rows of W a workgroup and 8 waves (the tile of X is read by half as many
+  // workgroups: 8,320 pairs, 2,048 features, inner size 2,056 gated 264 us, with 128 rows 306); otherwise 128 rows and 4 waves, which leaves
+  // more workgroups to spread
+  if (I > 1024 && O >= 512)
+    return launch_tiled_as<GLU, 32, 256, 8>(X, ldx, top, sorted_pair, tile_expert, tiles, wa, wb, stride, Y, ldy, O, I, act, in_weight, stream);
   return launch_tiled_as<GLU, 32, 128, 4>(X, ldx, top, sorted_pair, tile_expert, tiles, wa, wb, stride, Y, ldy, O, I, act, in_weight, stream);
 }
 

@@ -399,6 +399,14 @@ def test_many_pairs_products_at_the_edges_of_their_tiles(O, I, pad, gated):
     assert (got[rest] == 7.0).all() and (got[:, O:] == 7.0).all()
 
 
+@pytest.mark.parametrize("O,I,pad", [(520, 1032, 3), (513, 2056, 0), (500, 1032, 0), (6144, 128, 0), (6144, 256, 4)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_many_pairs_products_by_the_kernel_through_registers(O, I, pad, gated):
+    """The same for inner sizes that are no whole tiles of 64 k, with 256 and with 128 rows of W, and for short ones whose items leave the last round
+    of compute units part empty."""
+    test_many_pairs_products_at_the_edges_of_their_tiles(O, I, pad, gated)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("shared", ["gated", "plain", "none"])
 def test_experts_sum_inside_the_sublayer_boundary(dtype, shared):
