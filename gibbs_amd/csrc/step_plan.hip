@@ -29,6 +29,7 @@
 // was given back can be handed out again at once.
 #include "common.h"
 #include "step_plan_api.h"
+#include <algorithm>
 #include <map>
 #include <memory>
 #include <vector>
@@ -49,12 +50,7 @@ constexpr int SKINNY_ROWS_F32_OUT = 48;   // the same for float32 output (the he
 constexpr int ACT_CLAMPED = 4;            // the gated feed-forward's clamped activation (activation.h: ACT_CLAMPED_SWISH)
 constexpr int SSD_CHUNKED_ROWS = 256;     // rows of one request from which the state-space rule runs in chunks
 constexpr int GATED_CHUNKED_ROWS = 96;    // rows of a request from which the gated outer-product rule runs in chunks
-// rows of a request from which the gated delta rule runs in chunks (one request, 16 heads of 128 x 128, a decay per head and per channel, us:
-// 64 tokens walk 26 and 29, chunks 27 and 37; 96 tokens 36 and 41, 31 and 41; 128 tokens 47 and 53, 31 and 41)
-constexpr int DELTA_CHUNKED_ROWS = 96;
-// rows of a request from which the decayed outer-product rule runs in chunks (one request, 16 and 32 heads of 64, the walk with its decays and its
-// norm, us: 48 tokens walk 23 and 25, chunks 31; 64 tokens 29, 33 and 34; 96 tokens 39, 33 and 34; 128 tokens 49 and 50, 33 and 34)
-constexpr int TIME_MIX_CHUNKED_ROWS = 96;
+constexpr int RULE_CHUNKED_ROWS = 96;     // rows of a request from which the delta rule and time mixing may run in chunks (chunked_rule_pays)
 constexpr int WALKED_ROWS = 24;           // rows of a request from which gated linear attention and the matrix memory run in chunks
 constexpr int MATRIX_SLICE_PAGES = 510;   // page ids of a key slice that the decode attention's matrix-core walk keeps in LDS
 
@@ -119,6 +115,32 @@ int prefill_heads(int rows, int reqs, int nh, int nkv, int hd, int max_seq, int 
 
 // Which product runs y = x W^T, and in how many float32 partial sums it leaves its result.
 enum { LIN_F32, LIN_PLAIN, LIN_SKINNY, LIN_LIBRARY, LIN_TILED };
+// Whether the gated delta rule or time mixing over `rows` rows of `reqs` requests, the longest of max_q rows, runs in chunks or walks: the
+// lesser of two estimated times (us).  The walk: its longest request's chain, which others on the chip slow down (`load`: a fourth of the
+// columns of all states at which it takes twice as long), or the work of all rows once the chip is full.  The chunks: a start, and a share
+// for every chunk of a head; a request's last chunk costs a whole one, and each workgroup looks its chunk up among the requests.  So one long
+// portion runs in chunks and many short ones beside it walk.  Measured (walk / chunks; requests x rows):
+//   delta rule, 16 heads of 128 x 128: 1 x 96 36 / 30, 1 x 2,048 684 / 172, 4 x 512 202 / 111, 16 x 256 317 / 263, 1 x 2,048 + 30 x 30 949 / 291, 1 x 512 +
+//     63 x 2 1,202 / 464, 16 x 96 139 / 130, 1 x 100 + 63 x 20 325 / 455, 1 x 96 + 62 x 2 114 / 426, 64 x 100 657 / 792, 128 x 128 2,166 / 3,042
+//     (a decay per channel: 1 x 64 29 / 37, 1 x 96 41 / 41, 1 x 128 53 / 41);
+//   delta rule, 32 heads of 64 x 64: 1 x 96 27 / 23, 4 x 512 138 / 113, 16 x 96 52 / 131, 1 x 100 + 63 x 20 120 / 489, 64 x 100 214 / 974;
+//   time mixing, 32 heads of 64, the walk with its decays and its norm: 1 x 64 33 / 34, 1 x 96 42 / 34, 1 x 2,048 983 / 138, 4 x 512 285 / 139, 1 x 200 +
+//     7 x 30 122 / 74, 4 x 96 49 / 68, 1 x 100 + 63 x 20 245 / 484, 64 x 100 446 / 852.
+struct RuleCosts {
+  float token, token_128;   // the walk: a token of the chain at heads of no and, more, of 128 key channels
+  float area;               // the walk: a row of a head with a state of 128 x 128
+  float load;
+  float start, piece_128;   // the chunks: a chunk of a head of 128 key channels
+  float search;             // the chunks: requests at which a chunk takes twice as long
+};
+constexpr RuleCosts DELTA_COSTS{0.21f, 0.12f, 5.5e-3f, 8192.f, 15.f, 0.14f, 64.f}, TIME_MIX_COSTS{0.48f, 0.f, 1e-2f, 16384.f, 24.f, 0.2f, 192.f};
+bool chunked_rule_pays(const RuleCosts& c, int rows, int reqs, int max_q, int H, int D, int V) {
+  if (max_q < RULE_CHUNKED_ROWS) return false;
+  const float part = D / 128.f, busy = (float)(reqs - 1) * H * (V / 4) / c.load;
+  const float chain = max_q * (c.token + c.token_128 * part) * (1.f + busy), all = c.area * part * (V / 128.f) * rows * H;
+  return c.start + c.piece_128 * part * H * (rows / 64.f + reqs) * (1.f + reqs / c.search) < std::max(chain, all);
+}
+
 struct LinearChoice {
   int kernel, splits;
 };
@@ -1031,7 +1053,7 @@ struct DeltaBody : Body {
     const int act = g2.w ? 1 : 0;
     void* y = e.take((long)N * H * V * e.esize);
     // Requests at the head of the batch that bring one row each (row n is request n's) have a kernel of their own; the others prepare their
-    // rows and run in chunks where one of them brings a long portion, else they walk.  32-bit runs walk all of them: there a request's results
+    // rows and run in chunks where that is the faster form, else they walk.  32-bit runs walk all of them: there a request's results
     // do not depend, to the bit, on how it is cut or on what else is in the step.
     const bool steps = e.bf16_run && gibbs_delta_step_takes(D, V) && slot_stride % 4 == 0 && ((uintptr_t)rule_state % 16) == 0;
     const int lead = !steps ? 0 : (e.rows_are_requests() ? N : a.lead_single), rest = N - lead, reqs = a.n_req - lead;
@@ -1049,7 +1071,7 @@ struct DeltaBody : Body {
                               a_channel ? a_channel + (long)lead * H * D : nullptr, dt_bias, a_log, beta, decay, rest, G, H, D, q_scale, unit_eps, a.stream));
       // (the rules address rows by cu, which counts the step's)
       float *b0 = beta - (long)lead * H, *d0 = decay - (long)lead * H * wide, *o0 = o - (long)lead * H * V;
-      if (e.bf16_run && a.max_q >= DELTA_CHUNKED_ROWS && C % 4 == 0 && gibbs_delta_chunks_take(D, V)) {
+      if (e.bf16_run && chunked_rule_pays(DELTA_COSTS, rest, reqs, a.max_q, H, D, V) && C % 4 == 0 && gibbs_delta_chunks_take(D, V)) {
         float* work = (float*)e.take(gibbs_delta_chunks_workspace(rest, reqs, H, D, V) * 4);
         RUN(e, gibbs_delta_chunks(qkv, qkv + (long)G * D, C, qkv + 2L * G * D, C, b0, d0, channel, rule_state, slot_stride, a.cu + lead, a.slot + lead, o0,
                                   work, rest, reqs, H, G, D, V, a.stream));
@@ -1113,8 +1135,8 @@ struct TimeMixBody : Body {
     float* w = (float*)e.linear(t, w2, N, true, false, false, nullptr);
     e.give(t);
     void* y = e.take((long)N * C * e.esize);
-    // Requests at the head of the batch that bring one row each (row n is request n's) take the row kernel; the others run in chunks where one
-    // of them brings a long portion, else they walk, with kernels for the decays and the gated norm around the walk (32-bit runs always:
+    // Requests at the head of the batch that bring one row each (row n is request n's) take the row kernel; the others run in chunks where
+    // that is the faster form, else they walk, with kernels for the decays and the gated norm around the walk (32-bit runs always:
     // see DeltaBody).
     const bool fits = e.bf16_run && 3 * apart < (1L << 31);
     const int lead = !(fits && gibbs_decayed_outer_rows_take(D)) ? 0 : (e.rows_are_requests() ? N : a.lead_single);
@@ -1122,7 +1144,7 @@ struct TimeMixBody : Body {
     if (lead > 0)
       RUN(e, gibbs_decayed_outer_rows(r, C, (int)apart, (int)(2 * apart), (int)(3 * apart), w, w0, bonus, gain, eps, rule_state, slot_stride, nullptr, a.slot,
                                       y, e.p.dtype, lead, H, D, a.stream));
-    if (rest > 0 && a.max_q >= TIME_MIX_CHUNKED_ROWS && fits && gibbs_decayed_outer_chunks_take(D)) {
+    if (rest > 0 && fits && chunked_rule_pays(TIME_MIX_COSTS, rest, reqs, a.max_q, H, D, D) && gibbs_decayed_outer_chunks_take(D)) {
       float* work = (float*)e.take(gibbs_decayed_outer_chunks_workspace(rest, reqs, H, D) * 4);
       RUN(e, gibbs_decayed_outer_chunks(r, C, (int)apart, (int)(2 * apart), (int)(3 * apart), w + (long)lead * C, w0, bonus, gain, eps, rule_state,
                                         slot_stride, a.cu + lead, a.slot + lead, y, work, e.p.dtype, rest, reqs, H, D, a.stream));
@@ -2560,6 +2582,9 @@ GIBBS_EXPORT int gibbs_rule_prefill_splits(long n_tiles, int nh, int max_seq, in
 GIBBS_EXPORT long gibbs_rule_prefill_tiles(int rows, int reqs) { return prefill_tiles(rows, reqs); }
 GIBBS_EXPORT int gibbs_rule_prefill_heads(int rows, int reqs, int nh, int nkv, int hd, int max_seq, int n_splits) {
   return prefill_heads(rows, reqs, nh, nkv, hd, max_seq, n_splits);
+}
+GIBBS_EXPORT int gibbs_rule_chunked(int time_mix, int rows, int reqs, int max_q, int H, int D, int V) {
+  return chunked_rule_pays(time_mix ? TIME_MIX_COSTS : DELTA_COSTS, rows, reqs, max_q, H, D, V);
 }
 GIBBS_EXPORT int gibbs_rule_fused_rows(void) { return FUSED_ROWS; }
 

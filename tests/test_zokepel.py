@@ -141,3 +141,18 @@ def test_plain_conv_and_feed_forward():
     assert np.allclose(big[0, 0], 1.5 * Z.sigmoid(1.702 * 1.5) * 2.5)
     assert np.allclose(big[0, 1], -20 * Z.sigmoid(1.702 * -20) * (-0.5))    # the gate is clamped from above only
     assert math.isclose(Z.sinusoid([3], 4)[0, 1], math.cos(3.0), rel_tol=1e-6) and Z.sinusoid([0], 6)[0].tolist() == [0, 1, 0, 1, 0, 1]
+
+
+# rows of each request: what the two forms took, walk and chunks (us), with a decay per head
+@pytest.mark.parametrize("time_mix,H,D,longest,others,each,walk,chunks", [
+    (0, 16, 128, 96, 0, 0, 36, 30), (0, 16, 128, 2048, 0, 0, 684, 172), (0, 16, 128, 200, 7, 30, 145, 55), (0, 16, 128, 2048, 30, 30, 949, 291),
+    (0, 16, 128, 512, 63, 2, 1202, 464), (0, 16, 128, 100, 63, 20, 325, 455), (0, 16, 128, 96, 62, 2, 114, 426), (0, 16, 128, 100, 63, 100, 657, 792),
+    (0, 16, 128, 128, 127, 128, 2166, 3042), (0, 32, 64, 96, 0, 0, 27, 23), (0, 32, 64, 512, 3, 512, 138, 113), (0, 32, 64, 96, 15, 96, 52, 131),
+    (0, 32, 64, 100, 63, 20, 120, 489), (0, 32, 64, 100, 63, 100, 214, 974), (0, 8, 64, 100, 63, 20, 48, 104), (0, 8, 64, 512, 63, 2, 217, 107),
+    (1, 32, 64, 96, 0, 0, 42, 34), (1, 32, 64, 512, 3, 512, 285, 139), (1, 32, 64, 200, 7, 30, 122, 74), (1, 32, 64, 96, 3, 96, 49, 68),
+    (1, 32, 64, 100, 63, 20, 245, 484), (1, 32, 64, 96, 62, 2, 78, 406), (1, 32, 64, 2048, 30, 30, 1046, 317), (1, 16, 64, 100, 63, 100, 218, 424),
+    (0, 16, 128, 64, 0, 0, 26, 27), (1, 32, 64, 64, 0, 0, 33, 34)])
+def test_a_step_of_many_short_portions_beside_a_long_one_walks(time_mix, H, D, longest, others, each, walk, chunks):
+    """The rule between the recurrences' two forms takes the faster one of measured steps."""
+    from gibbs_amd.ops.lib import library
+    assert library().gibbs_rule_chunked(time_mix, longest + others * each, 1 + others, max(longest, each), H, D, D) == (chunks < walk)
