@@ -118,7 +118,7 @@ def test_changing_portions_down_to_two_tokens(dirs, name, dtype):
 
 @pytest.mark.parametrize("name", NAMES)
 def test_cutting_changes_nothing_in_32_bit(dirs, name):
-    """Products add in ascending k and the attention takes keys in blocks aligned to absolute positions, so 32-bit
+    """Products add in one order of k and the attention takes keys in blocks aligned to absolute positions, so 32-bit
     logits do not depend on how the prompt was cut or on what else was in the batch, beyond rounding."""
     d = dirs[name]
     ids = RH.tokens(5, 77, vocab_of(d))

@@ -128,7 +128,7 @@ def test_changing_portions_down_to_two_tokens(dirs, name, dtype):
 
 @pytest.mark.parametrize("name", NAMES)
 def test_cutting_and_batching_change_nothing_in_32_bit(dirs, name):
-    """Products add in ascending k, the attention takes keys in blocks aligned to absolute positions, and an expert's
+    """Products add in one order of k, the attention takes keys in blocks aligned to absolute positions, and an expert's
     result for a row does not depend on which other rows the expert serves: 32-bit logits do not depend on how the prompt
     was cut or on what else was in the batch, beyond rounding."""
     d = dirs[name]
