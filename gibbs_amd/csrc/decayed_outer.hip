@@ -22,7 +22,7 @@ RuleArgs outer_rule(const void* rows, long ld, int off_k, int off_v, int off_g, 
 }
 int check(const char* what, const RuleArgs& a, int dtype, int n_req) {
   GIBBS_REQUIRE(a.raw && a.z && a.bias && a.bonus && a.gain && a.state && a.slot && a.out, "%s: null operand", what);
-  GIBBS_REQUIRE(n_req > 0 && n_req <= 65535 && a.H > 0 && a.H <= 65535 && a.D > 0 && a.ld >= (long)a.H * a.D && a.off_k >= 0 && a.off_v >= 0 && a.off_g >= 0 &&
+  GIBBS_REQUIRE(n_req > 0 && a.H > 0 && a.H <= 65535 && a.D > 0 && a.ld >= (long)a.H * a.D && a.off_k >= 0 && a.off_v >= 0 && a.off_g >= 0 &&
                     a.slot_stride >= (long)a.H * a.D * a.D, "%s: requests=%d heads=%d D=%d", what, n_req, a.H, a.D);
   GIBBS_REQUIRE(dtype == GIBBS_F32 || dtype == GIBBS_BF16, "%s: unknown dtype %d", what, dtype);
   return 0;
@@ -55,7 +55,7 @@ GIBBS_EXPORT int gibbs_decayed_outer_chunks(const void* rows, long ld, int off_k
                                             hipStream_t stream) {
   const RuleArgs a = outer_rule(rows, ld, off_k, off_v, off_g, z, bias, bonus, gain, eps, state, slot_stride, cu, slot, out, H, D);
   if (check("decayed_outer_chunks", a, dtype, n_req)) return 1;
-  GIBBS_REQUIRE(cu && workspace && n_rows > 0 && gibbs_decayed_outer_chunks_take(D), "decayed_outer_chunks: rows=%d, heads of %d", n_rows, D);
+  GIBBS_REQUIRE(cu && workspace && n_rows > 0 && n_req <= 65535 && gibbs_decayed_outer_chunks_take(D), "decayed_outer_chunks: rows=%d requests=%d, heads of %d", n_rows, n_req, D);
   const int places = ceil_div(n_rows, CHUNK) + n_req;      // (more than the requests' chunks can be)
   if (dtype == GIBBS_F32 ? launch_chunks<float, RULE_BONUS>(a, workspace, places, n_req, stream) : launch_chunks<bf16, RULE_BONUS>(a, workspace, places, n_req, stream)) return 1;
   GIBBS_LAUNCH_STATUS("decayed_outer_chunks");

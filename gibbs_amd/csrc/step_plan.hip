@@ -135,7 +135,7 @@ struct RuleCosts {
 };
 constexpr RuleCosts DELTA_COSTS{0.21f, 0.12f, 5.5e-3f, 8192.f, 15.f, 0.14f, 64.f}, TIME_MIX_COSTS{0.48f, 0.f, 1e-2f, 16384.f, 24.f, 0.2f, 192.f};
 bool chunked_rule_pays(const RuleCosts& c, int rows, int reqs, int max_q, int H, int D, int V) {
-  if (max_q < RULE_CHUNKED_ROWS) return false;
+  if (max_q < RULE_CHUNKED_ROWS || reqs > 65535) return false;      // (the chunks' launches have a dimension for the requests)
   const float part = D / 128.f, busy = (float)(reqs - 1) * H * (V / 4) / c.load;
   const float chain = max_q * (c.token + c.token_128 * part) * (1.f + busy), all = c.area * part * (V / 128.f) * rows * H;
   return c.start + c.piece_128 * part * H * (rows / 64.f + reqs) * (1.f + reqs / c.search) < std::max(chain, all);

@@ -665,6 +665,24 @@ def test_decayed_outer_rule_with_norm_and_gate(lens, H, D, shift, dtype, how):
     assert np.array_equal(after[others], start[others])
 
 
+def test_decayed_outer_rows_of_as_many_requests_as_the_walk_takes():
+    """65,537 requests of one token in one call: the last ones' read-outs and states are those of a call of their own, to the bit; a step that long
+    never takes the rules in chunks, whose launches have a dimension for the requests."""
+    from gibbs_amd.ops.lib import call, library, ptr, stream
+    assert not any(library().gibbs_rule_chunked(t, 65536 + 2000, 65536, 2000, 1, 16, 16) for t in (0, 1))
+    n, D, last = 65537, 4, 5
+    g = torch.Generator(device="cuda").manual_seed(0)
+    rows, z, bias, bonus, gain = (torch.randn(s, generator=g, device="cuda") for s in ((4, n, D), (n, D), D, D, D))
+    start, slot = torch.randn((n, 1, D, D), generator=g, device="cuda"), torch.arange(n, dtype=torch.int32, device="cuda")
+    results = []
+    for first in (0, n - last):
+        state, out = start.clone(), torch.zeros((n, D), device="cuda")
+        call("gibbs_decayed_outer_rows", ptr(rows[0, first:]), D, n * D, 2 * n * D, 3 * n * D, ptr(z[first:]), ptr(bias), ptr(bonus), ptr(gain), 1e-6, ptr(state),
+             state.stride(0), None, ptr(slot[first:]), ptr(out[first:]), 0, n - first, 1, D, stream())
+        results.append((out[-last:], state[-last:]))
+    assert all(torch.equal(a, b) and a.isfinite().all() and (a != 0).any() for a, b in zip(*results))
+
+
 @pytest.mark.parametrize("kind", sorted(DECAYS))
 @pytest.mark.parametrize("D", [24, 64, 96])
 def test_decayed_outer_rule_in_chunks_is_as_exact_as_the_walk(D, kind):
