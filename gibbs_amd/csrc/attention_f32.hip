@@ -63,18 +63,30 @@ __global__ __launch_bounds__(THREADS) void attention_f32_kernel(const float* __r
   __shared__ __attribute__((aligned(16))) float sK[KEYS][LD];
   __shared__ __attribute__((aligned(16))) float sV[KEYS][LD];
 
-  int tile = blockIdx.x, r = 0, qlen = 0;
-  for (; r < a.n_req; ++r) {
-    qlen = a.cu[r + 1] - a.cu[r];
-    const int t = (qlen + ROWS - 1) / ROWS;
-    if (tile < t) {
-      tile = t - 1 - tile;  // a request's last rows see the most keys: those workgroups start first
+  const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+  // Which request and which of its tiles: 64 requests at a time, a lane each (one after the other, each a wait for memory, 256 requests of one
+  // token and 16 heads of 64 took 160 us behind 10 keys; 69 now)
+  int tile = blockIdx.x, r = -1, qlen = 0;
+  for (int base = 0; base < a.n_req; base += WAVE) {
+    const int i = min(base + lane, a.n_req - 1);
+    const int len = base + lane < a.n_req ? a.cu[i + 1] - a.cu[i] : 0;
+    int upto = (len + ROWS - 1) / ROWS;      // tiles of these requests up to this one
+#pragma unroll
+    for (int d = 1; d < WAVE; d *= 2) {
+      const int before = __shfl_up(upto, d, WAVE);
+      if (lane >= d) upto += before;
+    }
+    const unsigned long long behind = __builtin_amdgcn_ballot_w64(tile < upto);
+    if (behind) {
+      const int l = __builtin_ctzll(behind);
+      r = base + l;
+      qlen = __builtin_amdgcn_readlane(len, l);
+      tile = __builtin_amdgcn_readlane(upto, l) - 1 - tile;  // a request's last rows see the most keys: those workgroups start first
       break;
     }
-    tile -= t;
+    tile -= __builtin_amdgcn_readlane(upto, WAVE - 1);
   }
-  if (r >= a.n_req) return;
-  const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+  if (r < 0) return;
   const int lr = lane % 16, g = lane / 16;
   const int head = blockIdx.y, kvh = head / (a.nh / a.nkv);
   const int n0 = a.cu[r] + tile * ROWS, p0 = a.ctx[r] + tile * ROWS;

@@ -516,6 +516,29 @@ def test_attention_float32_portions(nh, nkv, hd, page, extra):
         assert (want - got)[want.isfinite()].abs().max() <= 1e-4 * max(1.0, float(want[want.isfinite()].abs().max()))
 
 
+def test_attention_float32_many_requests():
+    """150 requests of 1 to 130 rows in one call: each one's rows are those of a call of its own, to the bit (the workgroups find their request among
+    64 at a time)."""
+    from gibbs_amd.ops.lib import call, ptr, stream
+    nh, nkv, hd, page, R = 2, 1, 16, 16, 150
+    q_lens = [1 + (i * 37) % 130 if i % 3 else 1 for i in range(R)]
+    ctx = [(i * 53) % 90 for i in range(R)]
+    kp, vp, table, _, _ = paged_setup(torch.float32, nkv, hd, page, [c + ql for c, ql in zip(ctx, q_lens)], 2200, seed=5)
+    cu = np.concatenate([[0], np.cumsum(q_lens)])
+    n = int(cu[-1])
+    q = rnd(n, nh * hd, dtype=torch.float32, seed=6)
+    cud, ctxd = i32(cu), i32(ctx)
+    def run(first, count):
+        out = torch.zeros((n, nh * hd), device="cuda")
+        call("gibbs_attention_f32", ptr(q), ptr(kp), ptr(vp), ptr(out), ptr(cud[first:]), ptr(ctxd[first:]), ptr(table[first:]), count, table.shape[1], page, kp.shape[0],
+             int(cu[first + count] - cu[first]), nh, nkv, hd, nh * hd, nh * hd, 0.25, 0, None, None, 0, None, 0, 0.0, stream())
+        return out
+    whole = run(0, R)
+    for r in range(R):
+        assert torch.equal(run(r, 1)[cu[r]:cu[r + 1]], whole[cu[r]:cu[r + 1]]), r
+    assert whole.isfinite().all() and (whole.abs().sum(1) > 0).all()
+
+
 def test_prefill_splits_choice():
     from gibbs_amd.ops import prefill_splits
     assert prefill_splits(32, 32, 2048) == 1                 # a whole 2,048-token prompt fills the chip
