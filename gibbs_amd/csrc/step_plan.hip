@@ -141,6 +141,18 @@ bool chunked_rule_pays(const RuleCosts& c, int rows, int reqs, int max_q, int H,
   return c.start + c.piece_128 * part * H * (rows / 64.f + reqs) * (1.f + reqs / c.search) < std::max(chain, all);
 }
 
+// Whether requests of one row each, `rows` of them, take the kernels that do a decoded token's rule with all around it, a workgroup a head; else
+// their rows are prepared, walk and are normed by kernels of their own.  Heads of few values leave most of such a workgroup idle, and many of them
+// make many.  Measured (three kernels / one, us; requests x heads):
+//   delta rule: 64 x 8 of 16 x 16 18 / 9, 256 x 8 19 / 22, 1,000 x 8 20 / 69; 256 x 8 of 32 x 32 17 / 18, 512 x 8 18 / 31; 512 x 8 of 48 x 48 39 / 32; 8 x 16 of
+//     128 x 128 23 / 10;
+//   time mixing: 32 x 8 of 8 16 / 12, 64 x 8 15 / 24; 64 x 8 of 16 16 / 16, 256 x 8 16 / 57; 64 x 8 of 32 15 / 12, 128 x 8 16 / 22; 8 x 32 of 64 16 / 6,
+//     256 x 32 142 / 148, 1,000 x 32 854 / 636.
+bool token_kernel_pays(bool time_mix, int rows, int H, int D, int V) {
+  const long heads = (long)rows * H;
+  return time_mix ? D >= 64 || heads <= std::min(32 * D, 640) : D * V >= 48 * 48 || heads <= 2048;
+}
+
 struct LinearChoice {
   int kernel, splits;
 };
@@ -1052,11 +1064,12 @@ struct DeltaBody : Body {
     const long ld_gate = gate2 ? (long)H * V : in.O;
     const int act = g2.w ? 1 : 0;
     void* y = e.take((long)N * H * V * e.esize);
-    // Requests at the head of the batch that bring one row each (row n is request n's) have a kernel of their own; the others prepare their
-    // rows and run in chunks where that is the faster form, else they walk.  32-bit runs walk all of them: there a request's results
+    // Requests at the head of the batch that bring one row each (row n is request n's) have a kernel of their own where that pays; the others prepare
+    // their rows and run in chunks where that is the faster form, else they walk.  32-bit runs walk all of them: there a request's results
     // do not depend, to the bit, on how it is cut or on what else is in the step.
     const bool steps = e.bf16_run && gibbs_delta_step_takes(D, V) && slot_stride % 4 == 0 && ((uintptr_t)rule_state % 16) == 0;
-    const int lead = !steps ? 0 : (e.rows_are_requests() ? N : a.lead_single), rest = N - lead, reqs = a.n_req - lead;
+    const int single = !steps ? 0 : (e.rows_are_requests() ? N : a.lead_single), lead = token_kernel_pays(false, single, H, D, V) ? single : 0;
+    const int rest = N - lead, reqs = a.n_req - lead;
     if (lead > 0)
       RUN(e, gibbs_delta_step(qkv, C, raw + (long)off_b * e.esize, raw + (long)off_a * e.esize, in.O, e.p.dtype, a_channel, dt_bias, a_log, gate, ld_gate, act,
                               gain, eps, rule_state, slot_stride, a.slot, y, lead, G, H, D, V, q_scale, unit_eps, a.stream));
@@ -1139,7 +1152,8 @@ struct TimeMixBody : Body {
     // that is the faster form, else they walk, with kernels for the decays and the gated norm around the walk (32-bit runs always:
     // see DeltaBody).
     const bool fits = e.bf16_run && 3 * apart < (1L << 31);
-    const int lead = !(fits && gibbs_decayed_outer_rows_take(D)) ? 0 : (e.rows_are_requests() ? N : a.lead_single);
+    const int single = !(fits && gibbs_decayed_outer_rows_take(D)) ? 0 : (e.rows_are_requests() ? N : a.lead_single);
+    const int lead = token_kernel_pays(true, single, H, D, D) ? single : 0;
     const int rest = N - lead, reqs = a.n_req - lead;
     if (lead > 0)
       RUN(e, gibbs_decayed_outer_rows(r, C, (int)apart, (int)(2 * apart), (int)(3 * apart), w, w0, bonus, gain, eps, rule_state, slot_stride, nullptr, a.slot,
@@ -2586,6 +2600,7 @@ GIBBS_EXPORT int gibbs_rule_prefill_heads(int rows, int reqs, int nh, int nkv, i
 GIBBS_EXPORT int gibbs_rule_chunked(int time_mix, int rows, int reqs, int max_q, int H, int D, int V) {
   return chunked_rule_pays(time_mix ? TIME_MIX_COSTS : DELTA_COSTS, rows, reqs, max_q, H, D, V);
 }
+GIBBS_EXPORT int gibbs_rule_token_kernel(int time_mix, int rows, int H, int D, int V) { return token_kernel_pays(time_mix, rows, H, D, V); }
 GIBBS_EXPORT int gibbs_rule_fused_rows(void) { return FUSED_ROWS; }
 
 GIBBS_EXPORT int gibbs_linear_splits(int dtype, int n, int O, int I, long ldx, const void* x, const void* w, int out_f32,

@@ -211,6 +211,7 @@ _VALUE_SIGNATURES = {
     "gibbs_rule_prefill_tiles": ([c_int, c_int], c_long),
     "gibbs_rule_prefill_heads": ([c_int, c_int, c_int, c_int, c_int, c_int, c_int], c_int),
     "gibbs_rule_chunked": ([c_int] * 7, c_int),
+    "gibbs_rule_token_kernel": ([c_int] * 5, c_int),
     "gibbs_rule_fused_rows": ([], c_int),
     "gibbs_linear_splits": ([c_int, c_int, c_int, c_int, c_long, c_void_p, c_void_p, c_int, c_int, c_int], c_int),
     "gibbs_skinny_residual_workspace": ([c_int, c_int, c_int], c_long),

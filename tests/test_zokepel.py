@@ -156,3 +156,14 @@ def test_a_step_of_many_short_portions_beside_a_long_one_walks(time_mix, H, D, l
     """The rule between the recurrences' two forms takes the faster one of measured steps."""
     from gibbs_amd.ops.lib import library
     assert library().gibbs_rule_chunked(time_mix, longest + others * each, 1 + others, max(longest, each), H, D, D) == (chunks < walk)
+
+
+@pytest.mark.parametrize("time_mix,rows,H,D,three,one", [
+    (0, 64, 8, 16, 18.4, 8.6), (0, 512, 8, 16, 18.6, 38.1), (0, 1000, 8, 16, 20.2, 69.0), (0, 64, 8, 32, 17.1, 7.2), (0, 512, 8, 32, 18.4, 31.0),
+    (0, 512, 8, 48, 38.8, 32.5), (0, 1000, 8, 48, 78.5, 58.2), (0, 8, 16, 128, 23.2, 9.9),
+    (1, 32, 8, 8, 15.6, 12.4), (1, 64, 8, 8, 15.4, 23.7), (1, 1000, 8, 8, 17.4, 349.0), (1, 128, 8, 16, 15.5, 29.7), (1, 64, 8, 32, 15.3, 12.0),
+    (1, 128, 8, 32, 15.7, 22.5), (1, 64, 8, 48, 15.6, 10.4), (1, 256, 8, 48, 26.1, 36.5), (1, 8, 32, 64, 16.1, 6.2), (1, 1000, 32, 64, 853.8, 635.8)])
+def test_decoded_tokens_of_many_small_heads_keep_the_three_kernels(time_mix, rows, H, D, three, one):
+    """The rule between one kernel around a decoded token's state and the three that it stands for takes the faster way of measured steps."""
+    from gibbs_amd.ops.lib import library
+    assert library().gibbs_rule_token_kernel(time_mix, rows, H, D, D) == (one < three)
