@@ -1,28 +1,94 @@
-// True 32-bit matrix product for the float32 path:  C[n, o] = sum_k A[n, k] * W[o, k], on the matrix cores' own 32-bit
-// instruction (v_mfma_f32_16x16x4_f32: 32-bit operands, products and sums, 256 flop a cycle and compute unit as on the
-// vector units, but without a vector instruction and two LDS reads for every product).
+// True 32-bit matrix product for the float32 path:  C[n, o] = sum_k A[n, k] * W[o, k], on the matrix cores' bfloat16
+// instruction.  A float32 is exactly the sum of three bfloat16 (8 + 8 + 8 bits: high = round(x), middle = round(x - high),
+// low = x - high - middle, all differences exact), and a product of two such sums is nine products, of which the six down to
+// 2^-18 of the whole are taken: what is left out is below 2^-26 of it, a fourth of a float32 product's own rounding.  Six
+// products at 16 times the rate of v_mfma_f32_16x16x4_f32, and 6 additions to a float32 sum for 32 k where that instruction
+// makes 8.
 //
 // The order of a sum.  k is cut into f32_segments(I) stretches of f32_segment(I) values; inside one the sum runs through
-// blocks of 16 k in ascending order, in each of which step j takes the four k that are j modulo 4; the stretches' sums are
-// added in ascending order.  Both kernels below keep to this whatever tile an element falls in, so a row's result does not
-// depend on how many other rows the call holds, and the stretches may be given to different waves.
+// blocks of 32 k in ascending order, the six products of a block smallest first; the stretches' sums are added in ascending
+// order.  Both kernels below keep to this whatever tile an element falls in, so a row's result does not depend on how many
+// other rows the call holds, and the stretches may be given to different waves.
+//
+// Values without three such parts.  An infinity or a NaN, and what rounds up to infinity, leaves NaN in its parts, and below
+// 2^-110 the low part is lost to bfloat16's smallest value; results that are not finite or closer to 0 than 2^-100 are therefore
+// taken again in plain float32 (`again`), from the operands as they are.
 //
 // The plain kernel (vector units, ascending k) takes what these refuse: rows that are no whole number of 16 bytes, and
 // bfloat16 operands (float32 accumulation) of any size and stride.
 #include "common.h"
+#include <utility>
 
 namespace {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int F32_BK = 32;          // k of a tile in LDS
-constexpr int F32_SEGMENTS = 8;     // stretches of k with a sum of their own, for inner sizes of 512 and more
-__host__ __device__ inline int f32_segments(int I) { return I >= 512 ? F32_SEGMENTS : 1; }
+constexpr int F32_BK = 32;          // k of a tile in LDS, and of a product
+constexpr int F32_SEGMENTS = 8;     // stretches of k with a sum of their own, of 32 k and more
+__host__ __device__ inline int f32_segments(int I) { return I >= F32_SEGMENTS * F32_BK ? F32_SEGMENTS : (I + F32_BK - 1) / F32_BK; }
 __host__ __device__ inline int f32_segment(int I) {
   const int n = f32_segments(I);
   return ((I + n - 1) / n + F32_BK - 1) / F32_BK * F32_BK;
 }
 
-__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+// Calls f with the integral constants 0 .. N - 1 (a loop this long the compiler leaves rolled)
+template <typename F, int... M>
+__device__ __forceinline__ void each(F&& f, std::integer_sequence<int, M...>) { (f(std::integral_constant<int, M>{}), ...); }
+template <int N, typename F>
+__device__ __forceinline__ void each(F&& f) { each(f, std::make_integer_sequence<int, N>{}); }
+
+__device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+
+// Two values to bfloat16 (rounded)
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ bf16x2 round2(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  return __builtin_convertvector((f32x2){a, b}, bf16x2);
+}
+__device__ __forceinline__ void take_off(float& a, float& b, bf16x2 u) {
+  const uint32_t w = __builtin_bit_cast(uint32_t, u);
+  a -= __uint_as_float(w << 16);
+  b -= __uint_as_float(w & 0xffff0000u);
+}
+// Eight values x = p[0] + p[1] + p[2], highest first.  What is left of a value is its dot product with (-1, 0) or (0, -1): one
+// instruction where take_off has two, and exact like it.  (The tiles' kernel, whose vector instructions stand between products, was
+// slower with it.  As constants that the compiler knows, it writes them as -1 for both halves.)
+__device__ __forceinline__ void split8(f32x4 x, f32x4 y, bf16x8* p) {
+  float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+  uint32_t one = 0xbf80u, two = 0xbf800000u;
+  asm volatile("" : "+v"(one), "+v"(two));
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    bf16x2 u[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      u[i] = round2(v[2 * i], v[2 * i + 1]);
+      if (q < 2) {
+        v[2 * i] = __builtin_amdgcn_fdot2_f32_bf16(u[i], __builtin_bit_cast(bf16x2, one), v[2 * i], false);
+        v[2 * i + 1] = __builtin_amdgcn_fdot2_f32_bf16(u[i], __builtin_bit_cast(bf16x2, two), v[2 * i + 1], false);
+      }
+    }
+    p[q] = __builtin_shufflevector(__builtin_shufflevector(u[0], u[1], 0, 1, 2, 3), __builtin_shufflevector(u[2], u[3], 0, 1, 2, 3), 0, 1, 2, 3, 4, 5, 6, 7);
+  }
+}
+// The six products of a block, smallest first: (part of the first operand, part of the second)
+constexpr int F32_PRODUCTS = 6;
+__device__ constexpr int F32_PART[F32_PRODUCTS][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+
+__device__ __forceinline__ bool wants_again(float x) { return !(fabsf(x) <= 3.4028234e38f) || (x != 0.f && fabsf(x) < 0x1p-100f); }
+// One element in plain float32 (a sum that is NaN stays NaN).
+__device__ __forceinline__ float again(const float* a, const float* w, int I) {
+  float sum = 0.f;
+  for (int k = 0; k < I; k += 4) {
+    const f32x4 x = *(const f32x4*)(a + k), y = *(const f32x4*)(w + k);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sum = fmaf(x[j], y[j], sum);
+    if (sum != sum) break;
+  }
+  return sum;
+}
 
 // Four neighbouring features of one row: lane (g, c) of a product holds features 4 g .. 4 g + 3 of row c.
 __device__ __forceinline__ void store_f32x4(float* C, long ldc, int row, int col, int N, int O, bool wide, f32x4 v) {
@@ -36,78 +102,131 @@ __device__ __forceinline__ void store_f32x4(float* C, long ldc, int row, int col
       if (col + i < O) p[i] = v[i];
   }
 }
+__device__ __forceinline__ bool wants_again(f32x4 v) { return wants_again(v[0]) || wants_again(v[1]) || wants_again(v[2]) || wants_again(v[3]); }
+// The four again, those that want it (few calls ever have one).
+__device__ __forceinline__ f32x4 again4(const float* A, const float* W, int I, long lda, long ldw, int row, int col, int N, int O, f32x4 v) {
+  if (row < N) {
+#pragma unroll 1
+    for (int i = 0; i < 4; ++i) {
+      const float x = i == 0 ? v[0] : (i == 1 ? v[1] : (i == 2 ? v[2] : v[3]));
+      if (col + i >= O || !wants_again(x)) continue;
+      const float y = again(A + (size_t)row * lda, W + (size_t)(col + i) * ldw, I);
+      v[0] = i == 0 ? y : v[0];
+      v[1] = i == 1 ? y : v[1];
+      v[2] = i == 2 ? y : v[2];
+      v[3] = i == 3 ? y : v[3];
+    }
+  }
+  return v;
+}
 
-// Tiles of 32 FO features x 32 FN rows, four waves of 16 FO x 16 FN; both operands through LDS in stretches of 32 k, the next
-// stretch on its way through registers meanwhile, one barrier a stretch.  A row of 32 k lies 36 words apart, so the 16 rows of
-// an operand read (16 bytes a lane) start in 16 different fours of the 64 banks.  Bound by the matrix cores: a wave's
-// FO x FN x 8 instructions of 32 cycles stand against 2 (FO + FN) reads of LDS.
+// Tiles of 16 FO WO features x 16 FN WN rows, WO x WN waves of 16 FO x 16 FN.  Both operands are split on their way through registers into
+// LDS, in stretches of 32 k; one barrier a stretch.  A part's row of 32 k is 64 bytes, and its 16-byte pieces are exchanged by the
+// row, so that the 16 rows of an operand read (16 bytes a lane) lie in 16 different fours of the 64 banks.
+// A wave issues in order, and a product keeps the matrix cores busy for 16 cycles, so everything else stands between the products in
+// the order written here: the operands' reads a group of products ahead, and the 30 instructions that split and place four values of
+// the stretch after the next.  Three stretches in LDS let the reads for the first products of a stretch stand in front of its barrier.
 // Workgroup ids go round the 8 chips' L2 caches; the remapping gives each of them whole panels of features, whose rows of W
 // then come from memory once.
-template <int FO, int FN>
-__global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W,
+template <int WO, int WN, int FO, int FN, int OCC>
+__global__ __launch_bounds__(64 * WO * WN, OCC) void gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                             float* __restrict__ C, int N, int O, int I, long lda, long ldw,
                                                             long ldc, int row_tiles, int tiles, int wide) {
-  constexpr int BO = 32 * FO, BN = 32 * FN, LD = F32_BK + 4;
-  __shared__ __attribute__((aligned(16))) float s_w[2][BO][LD], s_x[2][BN][LD];
+  constexpr int T = 64 * WO * WN, BO = 16 * FO * WO, BN = 16 * FN * WN, ROWS = T / 8, NW = BO / ROWS, NX = BN / ROWS, NP = NW + NX;
+  constexpr int PART = (BO + BN) * F32_BK, BUF = 3 * PART;      // a part of both operands (W's rows first), a stretch
+  static_assert(NW * ROWS == BO && NX * ROWS == BN && ROWS % 16 == 0, "whole passes, a thread's rows in the same order");
+  __shared__ __attribute__((aligned(16))) __bf16 s_p[3 * BUF];
   const int per = (tiles + 7) / 8, tile = (blockIdx.x % 8) * per + blockIdx.x / 8;
   if (tile >= tiles) return;
   const int o0 = tile / row_tiles * BO, n0 = tile % row_tiles * BN;
   const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, g = lane / 16, c = lane % 16;
-  const int wo = wave / 2 * 16 * FO, wn = wave % 2 * 16 * FN;
-  const int r0 = threadIdx.x / 8, quad = threadIdx.x % 8 * 4;      // this thread's row (of 32 at a time) and four k of a stretch
-  const float* wp[FO];
-  const float* xp[FN];
+  const int wo = wave / WN * 16 * FO, wn = wave % WN * 16 * FN;
+  const int r0 = threadIdx.x / 8, quad = threadIdx.x % 8 * 4;      // this thread's row (of ROWS at a time) and four k of a stretch
+  const int at = r0 * F32_BK + ((quad / 8) ^ (r0 / 4 % 4)) * 8 + quad % 8, from = c * F32_BK + (g ^ (c / 4)) * 8;
+  const float* src[NP];
 #pragma unroll
-  for (int i = 0; i < FO; ++i) wp[i] = W + (size_t)min(o0 + r0 + 32 * i, O - 1) * ldw + quad;
+  for (int i = 0; i < NP; ++i)
+    src[i] = i < NW ? W + (size_t)min(o0 + r0 + ROWS * i, O - 1) * ldw : A + (size_t)min(n0 + r0 + ROWS * (i - NW), N - 1) * lda;
+  f32x4 raw[NP];
+  bf16x2 part[3][2];
+  // (k beyond I: the last four k again, made zero where they are taken up.  No branch may stand there: with one, every wait became a
+  // wait for all loads, and the kernel took 1.3 to 1.8 times as long)
+  auto ask = [&](int i, int k0) { raw[i] = *(const f32x4*)(src[i] + min(k0 + quad, I - 4)); };
+  // a thread's work on four values in eight steps of a few instructions
+  constexpr int STEPS = 8;
+  auto step = [&](auto index, int buf, int k0, int next) __attribute__((always_inline)) {
+    constexpr int i = index.value / STEPS, s = index.value % STEPS;
+    f32x4& x = raw[i];
+    if constexpr (s == 0 && i >= NW) {      // (of A alone: beyond I both operands hold values of the rows' ends)
+      const uint32_t keep = (uint32_t)((k0 + quad - I) >> 31);
+      x = __builtin_bit_cast(f32x4, __builtin_bit_cast(u32x4, x) & keep);
+    }
+    if constexpr (s == 0 || s == 3 || s == 6) {
+      part[s / 3][0] = round2(x[0], x[1]);
+      part[s / 3][1] = round2(x[2], x[3]);
+    }
+    if constexpr (s == 1 || s == 4) {
+      float x0 = x[0], x1 = x[1];
+      take_off(x0, x1, part[s / 3][0]);
+      x[0] = x0;
+      x[1] = x1;
+    }
+    if constexpr (s == 2 || s == 5) {
+      float x2 = x[2], x3 = x[3];
+      take_off(x2, x3, part[s / 3][1]);
+      x[2] = x2;
+      x[3] = x3;
+    }
+    if constexpr (s == 6) ask(i, next);
+    if constexpr (s == 7) {
 #pragma unroll
-  for (int i = 0; i < FN; ++i) xp[i] = A + (size_t)min(n0 + r0 + 32 * i, N - 1) * lda + quad;
-  f32x4 rw[FO], rx[FN];
-  // (k beyond I: the last four k again, made zero where the operands are taken up, so that no branch stands between a load
-  // and its use; whole stretches of 32 need no such thing, but the one asked for behind the last is that too)
-  bool in = true;
-  auto ask = [&](int k0) {
-    in = k0 + quad < I;
-    const int k = in ? k0 : I - 4 - quad;
-#pragma unroll
-    for (int i = 0; i < FO; ++i) rw[i] = *(const f32x4*)(wp[i] + k);
-#pragma unroll
-    for (int i = 0; i < FN; ++i) rx[i] = *(const f32x4*)(xp[i] + k);
+      for (int q = 0; q < 3; ++q) *(u32x2*)&s_p[buf + q * PART + ROWS * i * F32_BK + at] = u32x2{__builtin_bit_cast(uint32_t, part[q][0]), __builtin_bit_cast(uint32_t, part[q][1])};
+    }
   };
-  auto put = [&](int b) {
-#pragma unroll
-    for (int i = 0; i < FO; ++i) *(f32x4*)&s_w[b][r0 + 32 * i][quad] = in ? rw[i] : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < FN; ++i) *(f32x4*)&s_x[b][r0 + 32 * i][quad] = in ? rx[i] : f32x4{0.f, 0.f, 0.f, 0.f};
-  };
+  auto read = [&](int buf, int q, int row) { return *(const bf16x8*)&s_p[buf + q * PART + row * F32_BK + from]; };
   f32x4 total[FO][FN] = {};
   const int segment = f32_segment(I);
-  int b = 0;
-  ask(0);
-  put(0);
+  bf16x8 fw[3][FO], fx[3][FN], ahead[FN];      // `ahead`: the next stretch's high parts of A
+#pragma unroll
+  for (int i = 0; i < NP; ++i) ask(i, 0);
+  each<NP * STEPS>([&](auto x) __attribute__((always_inline)) { step(x, 0, 0, F32_BK); });
+  each<NP * STEPS>([&](auto x) __attribute__((always_inline)) { step(x, BUF, F32_BK, 2 * F32_BK); });
   __syncthreads();
+#pragma unroll
+  for (int i = 0; i < FO; ++i) fw[2][i] = read(0, 2, wo + 16 * i);
+#pragma unroll
+  for (int i = 0; i < FN; ++i) fx[0][i] = read(0, 0, BO + wn + 16 * i);
+  int now = 0, then = BUF, free = 2 * BUF;      // the stretch at hand, the next one, and the one that is filled
   for (int begin = 0; begin < I; begin += segment) {
     const int end = min(begin + segment, I);
     f32x4 acc[FO][FN] = {};
-    for (int k0 = begin; k0 < end; k0 += F32_BK, b ^= 1) {
-      ask(k0 + F32_BK);
-      __builtin_amdgcn_sched_barrier(0);     // (the compiler would move the loads down to where they are used)
+    for (int k0 = begin; k0 < end; k0 += F32_BK) {
+      constexpr int G = FO * FN, M = G * F32_PRODUCTS, S = NP * STEPS, R = FO + FN;
+      __builtin_amdgcn_sched_barrier(0);
+      each<M>([&](auto index) __attribute__((always_inline)) {
+        constexpr int m = index.value, p = m / G, t = m % G, i = t / FN, h = t % FN, r0 = t * R / G, s0 = m * S / M;
+        acc[i][h] = mfma_bf16(fw[F32_PART[p][0]][i], fx[F32_PART[p][1]][h], acc[i][h]);
+        // operands of the products after this group: high W, low A; middle W, A; the next stretch's low W, high A
+        if constexpr (p == 0 || p == 1 || p == F32_PRODUCTS - 1)
+          each<(t + 1) * R / G - r0>([&](auto j) __attribute__((always_inline)) {
+            constexpr int r = r0 + j.value, n = r - FO;
+            constexpr int qw = p == 0 ? 0 : (p == 1 ? 1 : 2), qx = p == 0 ? 2 : (p == 1 ? 1 : 0);
+            const int buf = p == F32_PRODUCTS - 1 ? then : now;
+            if constexpr (r < FO) fw[qw][r] = read(buf, qw, wo + 16 * r);
+            else (p == F32_PRODUCTS - 1 ? ahead[n] : fx[qx][n]) = read(buf, qx, BO + wn + 16 * n);
+          });
+        each<(m + 1) * S / M - s0>([&](auto j) __attribute__((always_inline)) {
+          step(std::integral_constant<int, s0 + j.value>{}, free, k0 + 2 * F32_BK, k0 + 3 * F32_BK);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+      });
 #pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        f32x4 fw[FO], fx[FN];
-#pragma unroll
-        for (int i = 0; i < FO; ++i) fw[i] = *(const f32x4*)&s_w[b][wo + 16 * i + c][16 * half + 4 * g];
-#pragma unroll
-        for (int i = 0; i < FN; ++i) fx[i] = *(const f32x4*)&s_x[b][wn + 16 * i + c][16 * half + 4 * g];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int i = 0; i < FO; ++i)
-#pragma unroll
-            for (int h = 0; h < FN; ++h) acc[i][h] = mfma_f32(fw[i][j], fx[h][j], acc[i][h]);
-      }
-      __builtin_amdgcn_sched_barrier(0);     // (nor may what becomes of them be moved up, in front of the products)
-      put(b ^ 1);
+      for (int i = 0; i < FN; ++i) fx[0][i] = ahead[i];
       __syncthreads();
+      const int last = now;
+      now = then;
+      then = free;
+      free = last;
     }
 #pragma unroll
     for (int i = 0; i < FO; ++i)
@@ -117,19 +236,24 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(const float* __re
 #pragma unroll
   for (int i = 0; i < FO; ++i)
 #pragma unroll
-    for (int h = 0; h < FN; ++h) store_f32x4(C, ldc, n0 + wn + 16 * h + c, o0 + wo + 16 * i + 4 * g, N, O, wide, total[i][h]);
+    for (int h = 0; h < FN; ++h) {
+      const int row = n0 + wn + 16 * h + c, col = o0 + wo + 16 * i + 4 * g;
+      if (__builtin_expect(wants_again(total[i][h]), 0)) total[i][h] = again4(A, W, I, lda, ldw, row, col, N, O, total[i][h]);
+      store_f32x4(C, ldc, row, col, N, O, wide, total[i][h]);
+    }
 }
 
 // Few rows or few tiles: a workgroup takes 16 FO features x 16 FN rows and its eight waves a stretch of k each, straight from
-// memory into the operands' registers (no barrier before the sums meet in LDS).  Bound by the stream of W (one row group) or
-// by what comes through L2.  The loads of the next 64 k are on their way while the present ones are used.
+// memory into the operands' registers, where they are split (no barrier before the sums meet in LDS).  Bound by the stream of
+// W (one row group) or by what comes through L2.  Four blocks of 32 k are on their way, and a block is split as soon as it is there (8 rows
+// x 1,024 features, inner size 1,024: 5.6 us; 6.3 where the first use waited for all loads).
 template <int FO, int FN>
 __global__ __launch_bounds__(512) void gemm_f32_split_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                              float* __restrict__ C, int N, int O, int I, long lda, long ldw,
                                                              long ldc, int wide) {
-  constexpr int DEEP = 2;           // stretches of 32 k a batch of loads holds
+  constexpr int SETS = 4;
   __shared__ __attribute__((aligned(16))) f32x4 s_sum[F32_SEGMENTS][FO * FN][WAVE];
-  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, g = lane / 16, c = lane % 16;
+  const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), g = lane / 16, c = lane % 16;
   const int o0 = blockIdx.x * 16 * FO, n0 = blockIdx.y * 16 * FN;
   const int segments = f32_segments(I), segment = f32_segment(I);
   const int first = wave * segment, last = wave < segments ? min(first + segment, I) : 0;
@@ -139,54 +263,57 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(const float* __rest
   for (int i = 0; i < FO; ++i) wp[i] = W + (size_t)min(o0 + 16 * i + c, O - 1) * ldw;
 #pragma unroll
   for (int i = 0; i < FN; ++i) xp[i] = A + (size_t)min(n0 + 16 * i + c, N - 1) * lda;
-  f32x4 fw[2][DEEP][2][FO], fx[2][DEEP][2][FN];
-  // (k beyond the matrix: its last four again; what lies beyond the wave's stretch is made zero when it is used)
+  f32x4 fw[SETS][2][FO], fx[SETS][2][FN];
+  // (k beyond the matrix: its last four again, and A's made zero when they are used)
   auto ask = [&](int set, int k0) {
 #pragma unroll
-    for (int d = 0; d < DEEP; ++d)
+    for (int half = 0; half < 2; ++half) {
+      const int k = min(k0 + 8 * g + 4 * half, I - 4);
 #pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        const int k = min(k0 + 32 * d + 16 * half + 4 * g, I - 4);
+      for (int i = 0; i < FO; ++i) fw[set][half][i] = *(const f32x4*)(wp[i] + k);
 #pragma unroll
-        for (int i = 0; i < FO; ++i) fw[set][d][half][i] = *(const f32x4*)(wp[i] + k);
-#pragma unroll
-        for (int i = 0; i < FN; ++i) fx[set][d][half][i] = *(const f32x4*)(xp[i] + k);
-      }
+      for (int i = 0; i < FN; ++i) fx[set][half][i] = *(const f32x4*)(xp[i] + k);
+    }
   };
   f32x4 acc[FO][FN] = {};
   auto use = [&](int set, int k0) {
-    if (k0 + 32 * DEEP > last) {
 #pragma unroll
-      for (int d = 0; d < DEEP; ++d)
+    for (int half = 0; half < 2; ++half) {
+      const uint32_t keep = (uint32_t)((k0 + 8 * g + 4 * half - I) >> 31);
 #pragma unroll
-        for (int half = 0; half < 2; ++half)
-          if (k0 + 32 * d + 16 * half + 4 * g >= last) {
+      for (int i = 0; i < FN; ++i) fx[set][half][i] = __builtin_bit_cast(f32x4, __builtin_bit_cast(u32x4, fx[set][half][i]) & keep);
+    }
+    bf16x8 pw[FO][3], px[FN][3];
 #pragma unroll
-            for (int i = 0; i < FO; ++i) fw[set][d][half][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < FO; ++i) split8(fw[set][0][i], fw[set][1][i], pw[i]);
 #pragma unroll
-            for (int i = 0; i < FN; ++i) fx[set][d][half][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-          }
+    for (int i = 0; i < FN; ++i) split8(fx[set][0][i], fx[set][1][i], px[i]);
+#pragma unroll
+    for (int p = 0; p < F32_PRODUCTS; ++p)
+#pragma unroll
+      for (int i = 0; i < FO; ++i)
+#pragma unroll
+        for (int h = 0; h < FN; ++h) acc[i][h] = mfma_bf16(pw[i][F32_PART[p][0]], px[h][F32_PART[p][1]], acc[i][h]);
+  };
+  // (the first loads stand behind no branch, or the first block's use would wait for all of them: blocks behind a wave's last are that one again)
+  if (first < last) {
+    const int end = (last - first + 31) / 32 * 32 + first - 32;      // the wave's last block
+#pragma unroll
+    for (int s = 0; s < SETS; ++s) ask(s, min(first + 32 * s, end));
+    int k0 = first;
+    for (; k0 + 32 * (2 * SETS - 1) <= end; k0 += 32 * SETS) {
+#pragma unroll
+      for (int s = 0; s < SETS; ++s) {
+        __builtin_amdgcn_sched_barrier(0);
+        use(s, k0 + 32 * s);
+        ask(s, k0 + 32 * (s + SETS));
+      }
     }
 #pragma unroll
-    for (int d = 0; d < DEEP; ++d)
-#pragma unroll
-      for (int half = 0; half < 2; ++half)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int i = 0; i < FO; ++i)
-#pragma unroll
-            for (int h = 0; h < FN; ++h) acc[i][h] = mfma_f32(fw[set][d][half][i][j], fx[set][d][half][h][j], acc[i][h]);
-  };
-  if (first < last) {
-    ask(0, first);
-    for (int k0 = first; k0 < last; k0 += 64 * DEEP) {
-      if (k0 + 32 * DEEP < last) ask(1, k0 + 32 * DEEP);
+    for (int s = 0; s < 2 * SETS - 1; ++s) {
       __builtin_amdgcn_sched_barrier(0);
-      use(0, k0);
-      if (k0 + 64 * DEEP < last) ask(0, k0 + 64 * DEEP);
-      __builtin_amdgcn_sched_barrier(0);
-      if (k0 + 32 * DEEP < last) use(1, k0 + 32 * DEEP);
+      if (k0 + 32 * s <= end) use(s % SETS, k0 + 32 * s);
+      if (s < SETS - 1 && k0 + 32 * (s + SETS) <= end) ask(s, k0 + 32 * (s + SETS));
     }
   }
 #pragma unroll
@@ -197,7 +324,9 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(const float* __rest
   for (int t = wave; t < FO * FN; t += F32_SEGMENTS) {
     f32x4 total = {0.f, 0.f, 0.f, 0.f};
     for (int s = 0; s < segments; ++s) total += s_sum[s][t][lane];
-    store_f32x4(C, ldc, n0 + 16 * (t % FN) + c, o0 + 16 * (t / FN) + 4 * g, N, O, wide, total);
+    const int row = n0 + 16 * (t % FN) + c, col = o0 + 16 * (t / FN) + 4 * g;
+    if (__builtin_expect(wants_again(total), 0)) total = again4(A, W, I, lda, ldw, row, col, N, O, total);
+    store_f32x4(C, ldc, row, col, N, O, wide, total);
   }
 }
 
@@ -248,10 +377,10 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const T* __restrict__ A
     }
   }
 }
-template <int FO, int FN>
+template <int WO, int WN, int FO, int FN, int OCC>
 void launch_tile(const float* A, const float* W, float* C, int N, int O, int I, long lda, long ldw, long ldc, bool wide, hipStream_t stream) {
-  const int row_tiles = ceil_div(N, 32 * FN), tiles = row_tiles * ceil_div(O, 32 * FO);
-  gemm_f32_tile_kernel<FO, FN><<<(tiles + 7) / 8 * 8, 256, 0, stream>>>(A, W, C, N, O, I, lda, ldw, ldc, row_tiles, tiles, wide);
+  const int row_tiles = ceil_div(N, 16 * FN * WN), tiles = row_tiles * ceil_div(O, 16 * FO * WO);
+  gemm_f32_tile_kernel<WO, WN, FO, FN, OCC><<<(tiles + 7) / 8 * 8, 64 * WO * WN, 0, stream>>>(A, W, C, N, O, I, lda, ldw, ldc, row_tiles, tiles, wide);
 }
 template <int FO, int FN>
 void launch_split(const float* A, const float* W, float* C, int N, int O, int I, long lda, long ldw, long ldc, bool wide, hipStream_t stream) {
@@ -259,12 +388,12 @@ void launch_split(const float* A, const float* W, float* C, int N, int O, int I,
 }
 
 // The variants, and which one takes a shape.  A compute unit works through ceil(tiles / 256) tiles; one tile alone takes `alone`, one among
-// others on the same unit `loaded` (us at an inner size of 1,024; measured), so the least of max(alone, rounds * loaded) is taken.  Both grow with
-// the inner size alike, but for inner sizes under 512, where one wave of a split tile's eight walks all of k: alone it then takes twice
-// its share, among others 1.25 times (inner size 508, us, without and with that: 45 rows x 4,096 features 11.0 / 7.5, 300 x 1,024 12.9 / 10.8, 300 x
-// 256 7.1 / 5.4).  Features x rows of a tile; the last three cut k over their waves and serve few rows.  (1,194 rows, us, with the vector
-// unit's kernel before / now: 9,216 x 1,024 360 / 250, 1,024 x 4,608 640 / 162, 1,024 x 1,024 147 / 39, 3,072 x 1,024 174 / 88;
-// 8 rows: 9,216 x 1,024 85 / 15, 1,024 x 4,608 250 / 16.)
+// others on the same unit `loaded` (us at an inner size of 1,024; measured), so the least of max(alone, rounds * loaded) is taken; both grow with
+// the inner size alike.  Features x rows of a tile; the last three cut k over their waves and serve few rows.
+// (1,194 rows, us, on the matrix cores' 32-bit instruction / in three parts: 9,216 features x 1,024 227 / 156, 1,024 x 4,608 154 / 123, 1,024 x
+// 1,024 38 / 34, 3,072 x 1,024 84 / 50; 333 rows: 9,216 x 1,024 82 / 49; 8 rows: 9,216 x 1,024 11.8 / 12.1, 1,024 x 4,608 15.0 / 15.9, 1,024 x 1,024 5.3 / 5.6
+// before the kernels' arguments came in registers, which gives that back: a decoded token of the 350M shape takes as long as it did.
+// Error against 64 bits, relative, the same two: inner size 1,024 2.1e-7 / 1.6e-7, 4,608 4.3e-7 / 3.7e-7.)
 struct F32Variant {
   int features, rows;
   float alone, loaded;
@@ -272,9 +401,9 @@ struct F32Variant {
   bool split;      // k cut over the waves, and rows along the grid's second dimension
 };
 const F32Variant F32_VARIANTS[] = {
-    {128, 128, 83.f, 78.f, launch_tile<4, 4>, false}, {64, 96, 39.f, 32.f, launch_tile<2, 3>, false}, {64, 64, 28.f, 21.f, launch_tile<2, 2>, false},
-    {32, 64, 19.4f, 12.2f, launch_tile<1, 2>, false}, {32, 32, 10.f, 9.6f, launch_split<2, 2>, true}, {16, 32, 6.1f, 6.f, launch_split<1, 2>, true},
-    {16, 16, 5.f, 4.2f, launch_split<1, 1>, true}};
+    {128, 128, 41.f, 49.f, launch_tile<2, 4, 4, 2, 2>, false}, {128, 64, 31.f, 34.f, launch_tile<4, 2, 2, 2, 2>, false},
+    {64, 64, 26.f, 18.f, launch_tile<2, 2, 2, 2, 2>, false}, {32, 64, 20.f, 13.5f, launch_tile<2, 2, 1, 2, 3>, false},
+    {32, 32, 10.f, 9.6f, launch_split<2, 2>, true}, {16, 32, 7.f, 7.f, launch_split<1, 2>, true}, {16, 16, 6.f, 4.2f, launch_split<1, 1>, true}};
 
 bool launch_f32(const float* A, const float* W, float* C, int N, int O, int I, long lda, long ldw, long ldc, hipStream_t stream) {
   if (I % 4 || lda % 4 || ldw % 4 || (uintptr_t)A % 16 || (uintptr_t)W % 16) return false;
@@ -283,8 +412,7 @@ bool launch_f32(const float* A, const float* W, float* C, int N, int O, int I, l
   for (const F32Variant& v : F32_VARIANTS) {
     if (v.split && ceil_div(N, v.rows) > 65535) continue;
     const long tiles = (long)ceil_div(N, v.rows) * ceil_div(O, v.features);
-    const bool one_wave = v.split && f32_segments(I) == 1;
-    const float cost = fmaxf(v.alone * (one_wave ? 2.f : 1.f), (float)((tiles + 255) / 256) * v.loaded * (one_wave ? 1.25f : 1.f));
+    const float cost = fmaxf(v.alone, (float)((tiles + 255) / 256) * v.loaded);
     if (!best || cost < least) {
       best = &v;
       least = cost;

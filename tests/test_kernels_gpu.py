@@ -90,6 +90,29 @@ def test_gemm_f32_tiles_and_stretches(shape):
             assert torch.equal(ops.gemm_f32(a[:m].contiguous(), w), out[:m]), (shape, m)
 
 
+@pytest.mark.parametrize("shape", [(5, 96, 512), (40, 1000, 516), (200, 2112, 100), (700, 2112, 512)])
+def test_gemm_f32_values_without_three_bfloat16_parts(shape):
+    """Infinities, NaN, values that round up to infinity and values whose low parts bfloat16 does not hold come out as in plain float32: which
+    results are infinite or NaN is the inputs' affair, and the others keep the error of a sum in 32 bits (of results that float32 holds
+    with fewer digits: 2^-149 a product)."""
+    from gibbs_amd import ops
+    n, o, i = shape
+    w = rnd(o, i, seed=1)
+    for size in (1e-36, 1e-30, 1e-20, 1.0, 1e15):
+        a = rnd(n, i) * size
+        want, scale = a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
+        assert ((ops.gemm_f32(a, w).double() - want).abs() <= i * (2.0 ** -24 * scale + 2.0 ** -149)).all(), (shape, size)
+    a = rnd(n, i)
+    a[0, 7], a[2, 9], a[3, i - 1], a[n - 1, 0] = float("inf"), float("nan"), 3.4e38, -float("inf")
+    w[o // 2, 5] = float("inf")
+    w[o - 1, i - 1] = 0.0            # (0 times an infinity or times what rounds up to one)
+    got, want = ops.gemm_f32(a, w), a.double() @ w.double().t()
+    assert torch.equal(got.isnan(), want.isnan())
+    big = want.abs() > 3.5e38
+    assert torch.equal(got[big], want[big].float())
+    assert got[~big & ~want.isnan() & (want.abs() < 3.3e38)].isfinite().all()
+
+
 def test_gemm_f32_as_many_rows_as_the_plain_kernel_takes():
     """4,194,240 rows, which is where the plain kernel's grid ends, of few features: the tiles that cut k over their waves have no grid for them."""
     from gibbs_amd import ops
