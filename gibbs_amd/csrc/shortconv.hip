@@ -12,6 +12,7 @@
 // thread can see a half-updated state.  Tap sums run in ascending j in every case, so a
 // row's value does not depend on how the sequence was cut into steps.
 #include "common.h"
+#include <type_traits>
 
 namespace {
 constexpr int TL = 32;  // rows per tile; K - 1 <= TL so that only tile 0 needs history
@@ -68,13 +69,14 @@ __global__ __launch_bounds__(256) void shortconv_kernel(
     }
   }
 }
-// The same for bfloat16 with 8 channels (16 bytes) per thread and the window kept in registers:
+// The same with 16 bytes of channels (8 bfloat16, 4 float32) per thread and the window kept in registers:
 // a prompt portion is a pass over 3 + 1 values per (row, channel), bound by memory traffic.
 // K is a template parameter (2..4, what LFM2 checkpoints use); other lengths take the kernel above.
+// (float32, 1,194 rows of 1,024 channels: 31.7 us a channel a thread, K loads and products a row; 5.0 us so.)
 constexpr int TLV = 8;   // rows per tile (>= K - 1)
 constexpr int RU = 4;    // rows whose loads are in flight together
 
-__device__ __forceinline__ void unpack8(const uint4& raw, float* f) {
+__device__ __forceinline__ void unpack16(const uint4& raw, float (&f)[8]) {
   const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -82,12 +84,29 @@ __device__ __forceinline__ void unpack8(const uint4& raw, float* f) {
     f[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
   }
 }
+__device__ __forceinline__ void unpack16(const uint4& raw, float (&f)[4]) {
+  f[0] = __uint_as_float(raw.x);
+  f[1] = __uint_as_float(raw.y);
+  f[2] = __uint_as_float(raw.z);
+  f[3] = __uint_as_float(raw.w);
+}
+__device__ __forceinline__ uint4 pack16(const float (&f)[8]) {
+  uint32_t w[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    w[i] = (uint32_t)__builtin_bit_cast(unsigned short, (bf16)f[2 * i]) | ((uint32_t)__builtin_bit_cast(unsigned short, (bf16)f[2 * i + 1]) << 16);
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+__device__ __forceinline__ uint4 pack16(const float (&f)[4]) {
+  return make_uint4(__float_as_uint(f[0]), __float_as_uint(f[1]), __float_as_uint(f[2]), __float_as_uint(f[3]));
+}
 
-template <int K>
-__global__ __launch_bounds__(64) void shortconv_bf16x8_kernel(
-    const bf16* __restrict__ bcx, const float* __restrict__ taps, const float* __restrict__ bias,
+template <typename T, int K>
+__global__ __launch_bounds__(64) void shortconv_vec_kernel(
+    const T* __restrict__ bcx, const float* __restrict__ taps, const float* __restrict__ bias,
     float* __restrict__ state, long slot_stride, const int* __restrict__ cu, const int* __restrict__ ctx,
-    const int* __restrict__ slot, bf16* __restrict__ y, int n_req, int C, int lead_single) {
+    const int* __restrict__ slot, T* __restrict__ y, int n_req, int C, int lead_single) {
+  constexpr int V = 16 / sizeof(T);
   // (the first lead_single requests bring one row each: tile i is request i, and there is no walk)
   int tile = blockIdx.y, r = tile, q = 1;
   if (tile < lead_single) {
@@ -102,14 +121,14 @@ __global__ __launch_bounds__(64) void shortconv_bf16x8_kernel(
     }
   }
   if (r >= n_req) return;
-  const int c0 = (blockIdx.x * blockDim.x + threadIdx.x) * 8;
+  const int c0 = (blockIdx.x * blockDim.x + threadIdx.x) * V;
   if (c0 >= C) return;
   const int row0 = cu[r], before = ctx[r];
   float* st = state + (size_t)slot[r] * slot_stride;
   const size_t ld = (size_t)3 * C;
-  float w[8][K], b[8];
+  float w[V][K], b[V];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < V; ++i) {
     b[i] = bias ? bias[c0 + i] : 0.f;
 #pragma unroll
     for (int j = 0; j < K; ++j) w[i][j] = taps[(size_t)(c0 + i) * K + j];
@@ -117,20 +136,20 @@ __global__ __launch_bounds__(64) void shortconv_bf16x8_kernel(
   // B * x of row tp of this step's chunk (tp may be negative: the request's state, or zero before its start)
   auto bx_at = [&](int tp, float* out) {
     if (tp >= 0) {
-      const bf16* row = bcx + (size_t)(row0 + tp) * ld + c0;
-      float bv[8], xv[8];
-      unpack8(*(const uint4*)row, bv);
-      unpack8(*(const uint4*)(row + 2 * C), xv);
+      const T* row = bcx + (size_t)(row0 + tp) * ld + c0;
+      float bv[V], xv[V];
+      unpack16(*(const uint4*)row, bv);
+      unpack16(*(const uint4*)(row + 2 * C), xv);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) out[i] = bv[i] * xv[i];
+      for (int i = 0; i < V; ++i) out[i] = bv[i] * xv[i];
     } else {
       const bool have = before + tp >= 0;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) out[i] = have ? st[(size_t)(K - 1 + tp) * C + c0 + i] : 0.f;
+      for (int i = 0; i < V; ++i) out[i] = have ? st[(size_t)(K - 1 + tp) * C + c0 + i] : 0.f;
     }
   };
   const int t0 = tile * TLV, t_end = min(q, t0 + TLV);
-  float win[K][8];  // win[j]: B * x of row t - (K-1) + j
+  float win[K][V];  // win[j]: B * x of row t - (K-1) + j
 #pragma unroll
   for (int j = 0; j < K - 1; ++j) bx_at(t0 - (K - 1) + j, win[j + 1]);
   for (int tg = t0; tg < t_end; tg += RU) {
@@ -140,7 +159,7 @@ __global__ __launch_bounds__(64) void shortconv_bf16x8_kernel(
     for (int u = 0; u < RU; ++u) {
       rb[u] = rx[u] = rc[u] = make_uint4(0, 0, 0, 0);
       if (tg + u < t_end) {
-        const bf16* row = bcx + (size_t)(row0 + tg + u) * ld + c0;
+        const T* row = bcx + (size_t)(row0 + tg + u) * ld + c0;
         rb[u] = *(const uint4*)row;
         rc[u] = *(const uint4*)(row + C);
         rx[u] = *(const uint4*)(row + 2 * C);
@@ -153,34 +172,32 @@ __global__ __launch_bounds__(64) void shortconv_bf16x8_kernel(
 #pragma unroll
       for (int j = 0; j < K - 1; ++j)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) win[j][i] = win[j + 1][i];
-      float bv[8], xv[8], cg[8];
-      unpack8(rb[u], bv);
-      unpack8(rx[u], xv);
-      unpack8(rc[u], cg);
+        for (int i = 0; i < V; ++i) win[j][i] = win[j + 1][i];
+      float bv[V], xv[V], cg[V];
+      unpack16(rb[u], bv);
+      unpack16(rx[u], xv);
+      unpack16(rc[u], cg);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) win[K - 1][i] = bv[i] * xv[i];
-      uint32_t ow[4];
+      for (int i = 0; i < V; ++i) win[K - 1][i] = bv[i] * xv[i];
+      float yv[V];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < V; ++i) {
         float acc = 0.f;
 #pragma unroll
         for (int j = 0; j < K; ++j) acc = fmaf(w[i][j], win[j][i], acc);
         acc += b[i];
-        const uint32_t bits = (uint32_t)__builtin_bit_cast(unsigned short, (bf16)(cg[i] * acc));
-        if (i % 2 == 0) ow[i / 2] = bits;
-        else ow[i / 2] |= bits << 16;
+        yv[i] = cg[i] * acc;
       }
-      *(uint4*)(y + (size_t)(row0 + t) * C + c0) = make_uint4(ow[0], ow[1], ow[2], ow[3]);
+      *(uint4*)(y + (size_t)(row0 + t) * C + c0) = pack16(yv);
     }
   }
   if (tile == 0) {
     // new[s] = window[q + s] reads old[q + s] (an index above s), so ascending s is safe
     for (int s2 = 0; s2 < K - 1; ++s2) {
-      float v[8];
+      float v[V];
       bx_at(q - (K - 1) + s2, v);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) st[(size_t)s2 * C + c0 + i] = v[i];
+      for (int i = 0; i < V; ++i) st[(size_t)s2 * C + c0 + i] = v[i];
     }
   }
 }
@@ -200,21 +217,27 @@ GIBBS_EXPORT int gibbs_shortconv(const void* bcx, const float* taps, const float
   auto tiles = [&](int per) { return lead_single + (rest_req > 0 ? ceil_div(rest_rows, per) + rest_req : 0); };
   dim3 grid(ceil_div(C, 256), tiles(TL));
   GIBBS_REQUIRE(grid.y <= 65535, "shortconv: too many row tiles (%d)", (int)grid.y);
-  if (dtype == GIBBS_F32)
+  GIBBS_REQUIRE(dtype == GIBBS_F32 || dtype == GIBBS_BF16, "shortconv: unknown dtype %d", dtype);
+  const int vec = dtype == GIBBS_F32 ? 4 : 8;
+  if (C % vec == 0 && K <= 4 && ((uintptr_t)bcx % 16) == 0 && ((uintptr_t)y % 16) == 0 && (dtype == GIBBS_BF16 || tiles(TLV) <= 65535)) {
+    GIBBS_REQUIRE(tiles(TLV) <= 65535, "shortconv: too many row tiles (%d)", (int)tiles(TLV));
+    const dim3 vgrid(ceil_div(C, vec * 64), tiles(TLV));
+    auto launch = [&](auto type, auto length) {
+      typedef decltype(type) T;
+      shortconv_vec_kernel<T, decltype(length)::value><<<vgrid, 64, 0, stream>>>((const T*)bcx, taps, bias, state, slot_stride, cu, ctx, slot, (T*)y, n_req, C, lead_single);
+    };
+    auto by_length = [&](auto type) {
+      if (K == 2) launch(type, std::integral_constant<int, 2>{});
+      else if (K == 3) launch(type, std::integral_constant<int, 3>{});
+      else launch(type, std::integral_constant<int, 4>{});
+    };
+    if (dtype == GIBBS_F32) by_length(float{});
+    else by_length(bf16{});
+  } else if (dtype == GIBBS_F32)
     shortconv_kernel<float><<<grid, 256, 0, stream>>>((const float*)bcx, taps, bias, state, slot_stride, cu, ctx,
                                                       slot, (float*)y, n_req, C, K, lead_single);
-  else if (dtype == GIBBS_BF16 && C % 8 == 0 && K >= 2 && K <= 4 && ((uintptr_t)bcx % 16) == 0 && ((uintptr_t)y % 16) == 0) {
-    dim3 vgrid(ceil_div(C, 8 * 64), tiles(TLV));
-    GIBBS_REQUIRE(vgrid.y <= 65535, "shortconv: too many row tiles (%d)", (int)vgrid.y);
-    const bf16* in = (const bf16*)bcx;
-    bf16* out = (bf16*)y;
-    if (K == 2) shortconv_bf16x8_kernel<2><<<vgrid, 64, 0, stream>>>(in, taps, bias, state, slot_stride, cu, ctx, slot, out, n_req, C, lead_single);
-    else if (K == 3) shortconv_bf16x8_kernel<3><<<vgrid, 64, 0, stream>>>(in, taps, bias, state, slot_stride, cu, ctx, slot, out, n_req, C, lead_single);
-    else shortconv_bf16x8_kernel<4><<<vgrid, 64, 0, stream>>>(in, taps, bias, state, slot_stride, cu, ctx, slot, out, n_req, C, lead_single);
-  } else if (dtype == GIBBS_BF16)
+  else
     shortconv_kernel<bf16><<<grid, 256, 0, stream>>>((const bf16*)bcx, taps, bias, state, slot_stride, cu, ctx,
                                                      slot, (bf16*)y, n_req, C, K, lead_single);
-  else
-    return gibbs_fail("shortconv: unknown dtype %d", dtype);
   GIBBS_LAUNCH_STATUS("shortconv");
 }
