@@ -207,6 +207,10 @@ int gibbs_group_rmsnorm(float* x, const void* delta, int parts, long part_stride
 int gibbs_gated_group_norm(const float* in, const float* skip, long ld_skip, const float* skip_w, int skip_len, const void* gate,
                            long ld_gate, const float* gain, float eps, int groups, void* y, int dtype, int n, int C,
                            hipStream_t stream);
+int gibbs_delta_conv_takes(const void* in, long ld, int dtype, const float* state, long slot_stride, const float* out, int n_rows, int C, int K, int D);
+int gibbs_delta_conv(const void* in, long ld, int dtype, const float* taps, float* state, long slot_stride, const int* row_req, const int* cu,
+                     const int* slot, float* out, int n_rows, int n_req, int C, int K, int single_rows, int first, int G, int D, float q_scale,
+                     float unit_eps, hipStream_t stream);
 int gibbs_delta_prep(float* q, float* k, long ldqk, const void* beta_raw, const void* a_head, long ld_raw, int dtype,
                      const float* a_channel, const float* dt_bias, const float* a_log, float* beta, float* decay, int n_rows,
                      int G, int H, int D, float q_scale, float unit_eps, hipStream_t stream);

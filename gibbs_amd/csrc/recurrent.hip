@@ -10,6 +10,7 @@
 // long portions take in bfloat16, and the one-kernel step of a decoded token, agree with them to rounding).
 #include "common.h"
 #include "lane8.h"
+#include <type_traits>
 
 namespace {
 __device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + expf(-z)); }
@@ -49,63 +50,113 @@ __global__ void causal_conv_silu_kernel(const T* __restrict__ in, long ld, const
   out[(size_t)n * ld_out + c] = from_float<TO>(acc);
 }
 
-// The same for bfloat16 inputs whose channels come in whole groups of 8: a thread takes 8 neighbouring channels of a row with
-// 16-byte loads.  A workgroup is 64 lanes of channels by CONV_ROWS rows; the taps of its 512 channels, one contiguous stretch of
-// the [C, K] table, come into LDS once (each thread's 8 K taps a word further along, so that the lanes read different banks)
-// instead of as 8 K scattered words per thread.  Sums in ascending j, as above.
-constexpr int CONV_ROWS = 4, CONV_LANES = 64;
-template <typename TO>
+// The same for bfloat16 inputs whose channels come in whole groups of 8: a thread takes 8 neighbouring channels with 16-byte loads, of
+// CONV_RUN rows one behind the other, whose inputs it holds in registers (a row a thread reads K rows for each it writes: 2,048 rows of
+// 6,144 channels, K = 4, 38 us; 19 us so, 75 MB).  A workgroup is 64 lanes of channels by CONV_ROWS such runs; the taps of its 512
+// channels, one contiguous stretch of the [C, K] table, come through LDS once (each thread's 8 K taps a word further along, so that the lanes
+// read different banks) instead of as 8 K scattered words per thread.  Sums in ascending j, as above.
+// KT: K, as many rows as that in registers; 0: any K, a row at a time.
+// unit.D > 0: channels 0 .. 2 unit.G unit.D are heads of unit.D that are made unit vectors, x / sqrt(sum x^2 + eps), those of the first half
+// times q_scale, in rows from unit.first on (what the delta rule reads; a head is unit.D / 8 neighbouring lanes).
+constexpr int CONV_ROWS = 4, CONV_LANES = 64, CONV_RUN = 4;
+struct ConvUnit {
+  int G, D, first;
+  float q_scale, eps;
+};
+__device__ __forceinline__ float lanes_sum(float v, int lanes) {
+  return lanes == 16 ? group_sum<16>(v) : (lanes == 8 ? group_sum<8>(v) : (lanes == 4 ? group_sum<4>(v) : group_sum<2>(v)));
+}
+template <typename TO, int KT>
 __global__ __launch_bounds__(CONV_ROWS * CONV_LANES) void causal_conv_vec8_kernel(
     const bf16* __restrict__ in, long ld, const float* __restrict__ taps, const float* __restrict__ bias, float* __restrict__ state,
     long slot_stride, const int* __restrict__ row_req, const int* __restrict__ cu, const int* __restrict__ slot, TO* __restrict__ out,
-    long ld_out, int n_rows, int C, int K, int shift_state, int act, int residual) {
+    long ld_out, int n_rows, int C, int K_any, int shift_state, int act, int residual, ConvUnit unit) {
   extern __shared__ float s_taps[];    // [CONV_LANES][8 K + 1]
+  constexpr int RUN = KT ? CONV_RUN : 1;
+  const int K = KT ? KT : K_any;
   const int c0 = blockIdx.y * CONV_LANES * 8;
   const int span = min(CONV_LANES * 8, C - c0) * K;      // taps of this workgroup's channels
   const int tid = threadIdx.y * CONV_LANES + threadIdx.x;
   for (int i = tid; i < span; i += CONV_ROWS * CONV_LANES) s_taps[i + i / (8 * K)] = taps[(size_t)c0 * K + i];
   __syncthreads();
-  const int n = blockIdx.x * CONV_ROWS + threadIdx.y;
+  const int n0 = (blockIdx.x * CONV_ROWS + __builtin_amdgcn_readfirstlane(threadIdx.y)) * RUN;
   const int c = c0 + threadIdx.x * 8;
-  if (n >= n_rows || c >= C) return;
+  if (n0 >= n_rows || c >= C) return;
   const float* tp = s_taps + threadIdx.x * (8 * K + 1);
-  const int r = row_req[n], first = cu[r], t = n - first;
-  float* st = state + (size_t)slot[r] * slot_stride;
-  float acc[8] = {}, own[8] = {};
-  for (int j = 0; j < K; ++j) {
-    const int tt = t - (K - 1) + j;
-    float xv[8];
-    if (tt >= 0) {
-      unpack8(*(const uint4*)(in + (size_t)(first + tt) * ld + c), xv);
+  float tap[KT ? KT : 1][8];
+  uint4 raw[KT ? KT - 1 + RUN : 1];    // rows n0 - (K - 1) .. n0 + RUN - 1 of the step (those of an earlier request are not used)
+  if constexpr (KT > 0) {
+#pragma unroll
+    for (int j = 0; j < KT - 1 + RUN; ++j) raw[j] = *(const uint4*)(in + (size_t)min(max(n0 - (KT - 1) + j, 0), n_rows - 1) * ld + c);
+#pragma unroll
+    for (int j = 0; j < KT; ++j)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) tap[j][i] = tp[i * KT + j];
+  }
+#pragma unroll
+  for (int u = 0; u < RUN; ++u) {
+    const int n = n0 + u;
+    if (n >= n_rows) break;
+    const int r = row_req[n], first = cu[r], t = n - first;
+    float* st = state + (size_t)slot[r] * slot_stride;
+    float acc[8] = {}, own[8] = {};
+    auto add = [&](int j, const float* w, bool known, const uint4& x) {
+      const int tt = t - (K - 1) + j;
+      float xv[8];
+      if (tt >= 0) {
+        unpack8(known ? x : *(const uint4*)(in + (size_t)(first + tt) * ld + c), xv);
+      } else {
+        const float4 a = *(const float4*)(st + (size_t)(K - 1 + tt) * C + c), b = *(const float4*)(st + (size_t)(K - 1 + tt) * C + c + 4);
+        xv[0] = a.x; xv[1] = a.y; xv[2] = a.z; xv[3] = a.w; xv[4] = b.x; xv[5] = b.y; xv[6] = b.z; xv[7] = b.w;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        acc[i] = fmaf(w[i], xv[i], acc[i]);
+        own[i] = xv[i];
+      }
+      if (shift_state && j >= 1) {
+        *(float4*)(st + (size_t)(j - 1) * C + c) = make_float4(xv[0], xv[1], xv[2], xv[3]);
+        *(float4*)(st + (size_t)(j - 1) * C + c + 4) = make_float4(xv[4], xv[5], xv[6], xv[7]);
+      }
+    };
+    if constexpr (KT > 0) {
+#pragma unroll
+      for (int j = 0; j < KT; ++j) add(j, tap[j], true, raw[u + j]);
     } else {
-      const float4 a = *(const float4*)(st + (size_t)(K - 1 + tt) * C + c), b = *(const float4*)(st + (size_t)(K - 1 + tt) * C + c + 4);
-      xv[0] = a.x; xv[1] = a.y; xv[2] = a.z; xv[3] = a.w; xv[4] = b.x; xv[5] = b.y; xv[6] = b.z; xv[7] = b.w;
+      for (int j = 0; j < K; ++j) {
+        float w[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] = tp[i * K + j];
+        add(j, w, false, raw[0]);
+      }
+    }
+    if (bias) {
+      const float4 b0 = *(const float4*)(bias + c), b1 = *(const float4*)(bias + c + 4);
+      acc[0] += b0.x; acc[1] += b0.y; acc[2] += b0.z; acc[3] += b0.w; acc[4] += b1.x; acc[5] += b1.y; acc[6] += b1.z; acc[7] += b1.w;
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      acc[i] = fmaf(tp[i * K + j], xv[i], acc[i]);
-      own[i] = xv[i];
+      if (act == CONV_ACT_SILU) acc[i] = acc[i] * sigmoid_f(acc[i]);
+      if (residual) acc[i] += own[i];
     }
-    if (shift_state && j >= 1) {
-      *(float4*)(st + (size_t)(j - 1) * C + c) = make_float4(xv[0], xv[1], xv[2], xv[3]);
-      *(float4*)(st + (size_t)(j - 1) * C + c + 4) = make_float4(xv[4], xv[5], xv[6], xv[7]);
-    }
-  }
-  if (bias) {
-    const float4 b0 = *(const float4*)(bias + c), b1 = *(const float4*)(bias + c + 4);
-    acc[0] += b0.x; acc[1] += b0.y; acc[2] += b0.z; acc[3] += b0.w; acc[4] += b1.x; acc[5] += b1.y; acc[6] += b1.z; acc[7] += b1.w;
-  }
+    if (unit.D > 0 && n >= unit.first) {
+      float sum = 0.f;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    if (act == CONV_ACT_SILU) acc[i] = acc[i] * sigmoid_f(acc[i]);
-    if (residual) acc[i] += own[i];
-  }
-  TO* o = out + (size_t)n * ld_out + c;
-  if constexpr (sizeof(TO) == 2) {
-    *(uint4*)o = pack8(acc);
-  } else {
-    *(float4*)o = make_float4(acc[0], acc[1], acc[2], acc[3]);
-    *(float4*)(o + 4) = make_float4(acc[4], acc[5], acc[6], acc[7]);
+      for (int i = 0; i < 8; ++i) sum = fmaf(acc[i], acc[i], sum);
+      sum = lanes_sum(sum, unit.D / 8);
+      const float scale = (c < unit.G * unit.D ? unit.q_scale : 1.0f) / sqrtf(sum + unit.eps);
+      if (c < 2 * unit.G * unit.D) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[i] *= scale;
+      }
+    }
+    TO* o = out + (size_t)n * ld_out + c;
+    if constexpr (sizeof(TO) == 2) {
+      *(uint4*)o = pack8(acc);
+    } else {
+      *(float4*)o = make_float4(acc[0], acc[1], acc[2], acc[3]);
+      *(float4*)(o + 4) = make_float4(acc[4], acc[5], acc[6], acc[7]);
+    }
   }
 }
 
@@ -175,6 +226,25 @@ __global__ __launch_bounds__(64) void delta_prep_kernel(DeltaPrepArgs a) {
   } else if (lane == 0) {
     const float z = to_float(((const T*)a.a_head)[(size_t)n * a.ld_raw + h]) + a.dt_bias[h];
     a.decay[(size_t)n * a.H + h] = expf(-rate * softplus_f(z));
+  }
+}
+
+// beta and decay alone, for rows whose q and k the convolution has made unit vectors: a thread a head, or four channels of one.
+template <typename T, bool CH>
+__global__ __launch_bounds__(256) void delta_gates_kernel(DeltaPrepArgs a, long count) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= count) return;
+  const int per_head = CH ? a.D / 4 : 1;
+  const long at = i / per_head;                 // row H + head
+  const int n = (int)(at / a.H), h = (int)(at - (long)n * a.H), part = (int)(i - at * per_head);
+  const float rate = expf(a.a_log[h]);
+  if (part == 0) a.beta[at] = sigmoid_f(to_float(((const T*)a.beta_raw)[(size_t)n * a.ld_raw + h]));
+  if constexpr (CH) {
+    const float4 z = *(const float4*)(a.a_channel + (size_t)i * 4), b = *(const float4*)(a.dt_bias + h * a.D + part * 4);
+    *(float4*)(a.decay + (size_t)i * 4) = make_float4(expf(-rate * softplus_f(z.x + b.x)), expf(-rate * softplus_f(z.y + b.y)),
+                                                      expf(-rate * softplus_f(z.z + b.z)), expf(-rate * softplus_f(z.w + b.w)));
+  } else {
+    a.decay[at] = expf(-rate * softplus_f(to_float(((const T*)a.a_head)[(size_t)n * a.ld_raw + h]) + a.dt_bias[h]));
   }
 }
 
@@ -563,25 +633,48 @@ __global__ void double_exp_decay_kernel(float* __restrict__ z, const float* __re
     else return gibbs_fail(what ": unknown dtype %d", (dtype)); \
   } while (0)
 
+namespace {
+// Rows from which a thread of the wide kernel takes CONV_RUN of them (fewer are too few workgroups)
+constexpr int CONV_RUN_ROWS = 512;
+// (steps of few rows are served faster by the kernel with a thread per channel: more, shorter workgroups; measured at 8 rows)
+bool conv_vec8(const void* in, long ld, int dtype, const float* bias, const float* state, long slot_stride, const void* out, int out_f32, long ld_out,
+               int n_rows, int C, int K) {
+  return dtype == GIBBS_BF16 && n_rows >= 64 && C % 8 == 0 && ld % 8 == 0 && ((uintptr_t)in % 16) == 0 && ((uintptr_t)out % 16) == 0 &&
+         ld_out % (out_f32 ? 4 : 8) == 0 && slot_stride % 4 == 0 && ((uintptr_t)state % 16) == 0 && ((uintptr_t)bias % 16) == 0 && K <= 16;
+}
+}  // namespace
+
 // The general entry point: an optional bias [C], act 0 none / 1 silu, `residual` (the input is added to the result), and the
 // result as float32 (out_f32) or in the input's type, in rows of ld_out values.  `in` and `out` must not overlap.
-GIBBS_EXPORT int gibbs_causal_conv(const void* in, long ld, int dtype, const float* taps, const float* bias, float* state, long slot_stride,
+static int causal_conv(const void* in, long ld, int dtype, const float* taps, const float* bias, float* state, long slot_stride,
                                    const int* row_req, const int* cu, const int* slot, void* out, int out_f32, long ld_out, int n_rows,
-                                   int n_req, int C, int K, int act, int residual, int update_state, int single_rows, hipStream_t stream) {
+                                   int n_req, int C, int K, int act, int residual, int update_state, int single_rows, ConvUnit unit,
+                       hipStream_t stream) {
   // single_rows: every request brings exactly one row (a step of decoded tokens): the state moves on in the same kernel
   const int shift = update_state && single_rows && K > 1 && n_rows == n_req;
   GIBBS_REQUIRE(in && taps && state && out && n_rows > 0 && n_req > 0 && C > 0 && K >= 1 && ld >= C && ld_out >= C && slot_stride >= (long)(K - 1) * C,
                 "causal_conv: bad operands rows=%d requests=%d C=%d K=%d", n_rows, n_req, C, K);
   const dim3 rows(n_rows, ceil_div(C, 256)), reqs(n_req, ceil_div(C, 256));
 #define CONV_ARGS taps, bias, state, slot_stride, row_req, cu, slot
-  // (steps of few rows are served faster by the kernel with a thread per channel: more, shorter workgroups; measured at 8 rows)
-  const bool vec8 = dtype == GIBBS_BF16 && n_rows >= 64 && C % 8 == 0 && ld % 8 == 0 && ((uintptr_t)in % 16) == 0 && ((uintptr_t)out % 16) == 0 &&
-                    ld_out % (out_f32 ? 4 : 8) == 0 && slot_stride % 4 == 0 && ((uintptr_t)state % 16) == 0 && ((uintptr_t)bias % 16) == 0 && K <= 16;
+  const bool vec8 = conv_vec8(in, ld, dtype, bias, state, slot_stride, out, out_f32, ld_out, n_rows, C, K);
+  GIBBS_REQUIRE(vec8 || unit.D == 0, "causal_conv: unit vectors of operands that the wide kernel refuses");
   if (vec8) {
-    const dim3 grid(ceil_div(n_rows, CONV_ROWS), ceil_div(C, CONV_LANES * 8)), block(CONV_LANES, CONV_ROWS);
+    const int run = K >= 2 && K <= 4 && n_rows >= CONV_RUN_ROWS ? CONV_RUN : 1;
+    const dim3 grid(ceil_div(n_rows, CONV_ROWS * run), ceil_div(C, CONV_LANES * 8)), block(CONV_LANES, CONV_ROWS);
     const size_t lds = (size_t)CONV_LANES * (8 * K + 1) * sizeof(float);
-    if (out_f32) causal_conv_vec8_kernel<float><<<grid, block, lds, stream>>>((const bf16*)in, ld, CONV_ARGS, (float*)out, ld_out, n_rows, C, K, shift, act, residual);
-    else causal_conv_vec8_kernel<bf16><<<grid, block, lds, stream>>>((const bf16*)in, ld, CONV_ARGS, (bf16*)out, ld_out, n_rows, C, K, shift, act, residual);
+    auto launch = [&](auto type, auto length) {
+      typedef decltype(type) TO;
+      causal_conv_vec8_kernel<TO, decltype(length)::value><<<grid, block, lds, stream>>>((const bf16*)in, ld, CONV_ARGS, (TO*)out, ld_out, n_rows, C, K, shift, act,
+                                                                                        residual, unit);
+    };
+    auto by_length = [&](auto type) {
+      if (run == 1) launch(type, std::integral_constant<int, 0>{});
+      else if (K == 2) launch(type, std::integral_constant<int, 2>{});
+      else if (K == 3) launch(type, std::integral_constant<int, 3>{});
+      else launch(type, std::integral_constant<int, 4>{});
+    };
+    if (out_f32) by_length(float{});
+    else by_length(bf16{});
   } else if (out_f32 || dtype == GIBBS_F32)
     BY_DTYPE(dtype, "causal_conv",
              (causal_conv_silu_kernel<float, float><<<rows, 256, 0, stream>>>((const float*)in, ld, CONV_ARGS, (float*)out, ld_out, C, K, shift, act, residual)),
@@ -597,6 +690,26 @@ GIBBS_EXPORT int gibbs_causal_conv(const void* in, long ld, int dtype, const flo
              (causal_conv_state_kernel<bf16><<<reqs, 256, 0, stream>>>((const bf16*)in, ld, state, slot_stride, cu, slot, C, K)));
   GIBBS_LAUNCH_STATUS("causal_conv");
 }
+GIBBS_EXPORT int gibbs_causal_conv(const void* in, long ld, int dtype, const float* taps, const float* bias, float* state, long slot_stride,
+                                   const int* row_req, const int* cu, const int* slot, void* out, int out_f32, long ld_out, int n_rows,
+                                   int n_req, int C, int K, int act, int residual, int update_state, int single_rows, hipStream_t stream) {
+  return causal_conv(in, ld, dtype, taps, bias, state, slot_stride, row_req, cu, slot, out, out_f32, ld_out, n_rows, n_req, C, K, act, residual,
+                     update_state, single_rows, ConvUnit{}, stream);
+}
+// The delta rule's convolution: silu, float32 results, and in rows from `first` on q and k (2 G heads of D, the first channels) made unit vectors,
+// q times q_scale.  Whether it takes these operands:
+GIBBS_EXPORT int gibbs_delta_conv_takes(const void* in, long ld, int dtype, const float* state, long slot_stride, const float* out, int n_rows, int C, int K,
+                                        int D) {
+  return conv_vec8(in, ld, dtype, nullptr, state, slot_stride, out, 1, C, n_rows, C, K) && (D == 16 || D == 32 || D == 64 || D == 128);
+}
+GIBBS_EXPORT int gibbs_delta_conv(const void* in, long ld, int dtype, const float* taps, float* state, long slot_stride, const int* row_req, const int* cu,
+                                  const int* slot, float* out, int n_rows, int n_req, int C, int K, int single_rows, int first, int G, int D, float q_scale,
+                                  float unit_eps, hipStream_t stream) {
+  GIBBS_REQUIRE(G > 0 && first >= 0 && 2L * G * D <= C && gibbs_delta_conv_takes(in, ld, dtype, state, slot_stride, out, n_rows, C, K, D),
+                "delta_conv: bad operands rows=%d C=%d kv heads=%d D=%d", n_rows, C, G, D);
+  return causal_conv(in, ld, dtype, taps, nullptr, state, slot_stride, row_req, cu, slot, out, 1, C, n_rows, n_req, C, K, 1, 0, 1, single_rows,
+                     ConvUnit{G, D, first, q_scale, unit_eps}, stream);
+}
 GIBBS_EXPORT int gibbs_causal_conv_silu(const void* in, long ld, int dtype, const float* taps, float* state, long slot_stride,
                                         const int* row_req, const int* cu, const int* slot, float* out, int n_rows, int n_req,
                                         int C, int K, int update_state, int single_rows, hipStream_t stream) {
@@ -607,9 +720,20 @@ GIBBS_EXPORT int gibbs_causal_conv_silu(const void* in, long ld, int dtype, cons
 GIBBS_EXPORT int gibbs_delta_prep(float* q, float* k, long ldqk, const void* beta_raw, const void* a_head, long ld_raw, int dtype,
                                   const float* a_channel, const float* dt_bias, const float* a_log, float* beta, float* decay,
                                   int n_rows, int G, int H, int D, float q_scale, float unit_eps, hipStream_t stream) {
-  GIBBS_REQUIRE(q && k && beta_raw && (a_head || a_channel) && dt_bias && a_log && beta && decay && n_rows > 0 && G > 0 && H > 0 && D > 0,
+  // (q and k null: beta and decay alone)
+  GIBBS_REQUIRE((q ? k != nullptr : !k && (!a_channel || (D % 4 == 0 && ((uintptr_t)a_channel % 16) == 0 && ((uintptr_t)dt_bias % 16) == 0 && ((uintptr_t)decay % 16) == 0))) &&
+                    beta_raw && (a_head || a_channel) && dt_bias && a_log && beta && decay && n_rows > 0 && G > 0 && H > 0 && D > 0,
                 "delta_prep: bad operands rows=%d kv heads=%d heads=%d D=%d", n_rows, G, H, D);
   DeltaPrepArgs a{q, k, ldqk, beta_raw, ld_raw, a_channel ? nullptr : a_head, a_channel, dt_bias, a_log, beta, decay, G, H, D, q_scale, unit_eps};
+  if (!q) {
+    const long count = (long)n_rows * H * (a_channel ? D / 4 : 1);
+    const int blocks = (int)((count + 255) / 256);
+    if (a_channel)
+      BY_DTYPE(dtype, "delta_prep", (delta_gates_kernel<float, true><<<blocks, 256, 0, stream>>>(a, count)), (delta_gates_kernel<bf16, true><<<blocks, 256, 0, stream>>>(a, count)));
+    else
+      BY_DTYPE(dtype, "delta_prep", (delta_gates_kernel<float, false><<<blocks, 256, 0, stream>>>(a, count)), (delta_gates_kernel<bf16, false><<<blocks, 256, 0, stream>>>(a, count)));
+    GIBBS_LAUNCH_STATUS("delta_prep");
+  }
   const dim3 grid(n_rows, G + H);
   BY_DTYPE(dtype, "delta_prep", (delta_prep_kernel<float><<<grid, 64, 0, stream>>>(a)), (delta_prep_kernel<bf16><<<grid, 64, 0, stream>>>(a)));
   GIBBS_LAUNCH_STATUS("delta_prep");

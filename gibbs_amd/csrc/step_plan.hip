@@ -1056,8 +1056,6 @@ struct DeltaBody : Body {
     const bool channel = a2.w != nullptr;
     char* raw = (char*)e.linear(h, in, N, false, false, false, nullptr);
     float* qkv = (float*)e.take((long)N * C * 4);
-    RUN(e, gibbs_causal_conv_silu(raw, in.O, e.p.dtype, taps, conv_state, slot_stride, a.row_req, a.cu, a.slot, qkv, N, a.n_req, C, K, 1,
-                                  a.max_q == 1, a.stream));
     float* a_channel = channel ? (float*)e.linear(raw + (long)off_a * e.esize, a2, N, true, false, false, nullptr, in.O) : nullptr;
     void* gate2 = g2.w ? e.linear(raw + (long)off_g * e.esize, g2, N, false, false, false, nullptr, in.O) : nullptr;
     const void* gate = gate2 ? gate2 : raw + (long)off_g * e.esize;
@@ -1070,6 +1068,15 @@ struct DeltaBody : Body {
     const bool steps = e.bf16_run && gibbs_delta_step_takes(D, V) && slot_stride % 4 == 0 && ((uintptr_t)rule_state % 16) == 0;
     const int single = !steps ? 0 : (e.rows_are_requests() ? N : a.lead_single), lead = token_kernel_pays(false, single, H, D, V) ? single : 0;
     const int rest = N - lead, reqs = a.n_req - lead;
+    // (the convolution makes q and k unit vectors itself where its wide kernel runs: one pass over them less)
+    const bool unit = rest > 0 && D % 4 == 0 && ((uintptr_t)dt_bias % 16) == 0 &&
+                      gibbs_delta_conv_takes(raw, in.O, e.p.dtype, conv_state, slot_stride, qkv, N, C, K, D);
+    if (unit)
+      RUN(e, gibbs_delta_conv(raw, in.O, e.p.dtype, taps, conv_state, slot_stride, a.row_req, a.cu, a.slot, qkv, N, a.n_req, C, K, a.max_q == 1, lead, G, D,
+                              q_scale, unit_eps, a.stream));
+    else
+      RUN(e, gibbs_causal_conv_silu(raw, in.O, e.p.dtype, taps, conv_state, slot_stride, a.row_req, a.cu, a.slot, qkv, N, a.n_req, C, K, 1,
+                                    a.max_q == 1, a.stream));
     if (lead > 0)
       RUN(e, gibbs_delta_step(qkv, C, raw + (long)off_b * e.esize, raw + (long)off_a * e.esize, in.O, e.p.dtype, a_channel, dt_bias, a_log, gate, ld_gate, act,
                               gain, eps, rule_state, slot_stride, a.slot, y, lead, G, H, D, V, q_scale, unit_eps, a.stream));
@@ -1080,7 +1087,7 @@ struct DeltaBody : Body {
       float* o = (float*)e.take((long)rest * H * V * 4);
       float* q = qkv + (long)lead * C;
       const char* r = raw + (long)lead * in.O * e.esize;
-      RUN(e, gibbs_delta_prep(q, q + (long)G * D, C, r + (long)off_b * e.esize, r + (long)off_a * e.esize, in.O, e.p.dtype,
+      RUN(e, gibbs_delta_prep(unit ? nullptr : q, unit ? nullptr : q + (long)G * D, C, r + (long)off_b * e.esize, r + (long)off_a * e.esize, in.O, e.p.dtype,
                               a_channel ? a_channel + (long)lead * H * D : nullptr, dt_bias, a_log, beta, decay, rest, G, H, D, q_scale, unit_eps, a.stream));
       // (the rules address rows by cu, which counts the step's)
       float *b0 = beta - (long)lead * H, *d0 = decay - (long)lead * H * wide, *o0 = o - (long)lead * H * V;

@@ -551,6 +551,23 @@ def causal_conv_silu(x: torch.Tensor, taps: torch.Tensor, state: torch.Tensor, r
     return out
 
 
+def delta_conv(x: torch.Tensor, taps: torch.Tensor, state: torch.Tensor, row_req: torch.Tensor, cu: torch.Tensor, slot: torch.Tensor,
+               kv_heads: int, dim: int, q_scale: float, unit_eps: float, first: int = 0) -> torch.Tensor:
+    """`causal_conv_silu` of bfloat16 rows (64 and more) with its state moved on; in rows from `first` on the first 2 * kv_heads heads of `dim`
+    channels, q and k, are made unit vectors x / sqrt(sum x^2 + unit_eps), q times q_scale."""
+    require_cuda(x, taps, state, row_req, cu, slot)
+    n, c = x.shape
+    k = taps.shape[1]
+    assert x.is_contiguous() and taps.dtype == torch.float32 and taps.shape == (c, k) and taps.is_contiguous()
+    assert state.dtype == torch.float32 and state.stride(-1) == 1 and (k == 1 or state.shape[1:] == (k - 1, c))
+    n_req = cu.numel() - 1
+    _i32(row_req, n, "row_req"); _i32(cu, n_req + 1, "cu"); _i32(slot, n_req, "slot")
+    out = torch.empty((n, c), dtype=torch.float32, device=x.device)
+    call("gibbs_delta_conv", ptr(x), c, dtype_code(x.dtype), ptr(taps), ptr(state), state.stride(0), ptr(row_req), ptr(cu), ptr(slot), ptr(out),
+         n, n_req, c, k, int(n == n_req), first, kv_heads, dim, float(q_scale), float(unit_eps), stream())
+    return out
+
+
 def delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Tensor, decay: torch.Tensor, state: torch.Tensor,
                cu: torch.Tensor, slot: torch.Tensor, heads: int, kv_heads: int, chunks: bool = False) -> torch.Tensor:
     """The gated delta rule over ragged rows, all float32: q, k [N, kv_heads*D] (unit vectors, q scaled), v [N, heads*V],

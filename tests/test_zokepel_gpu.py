@@ -867,3 +867,41 @@ def test_command_line(dirs):
     dump = json.loads(proc.stdout)
     assert dump["architecture"] == "Zokepel" and dump["unconsumed"] == [] and dump["missing"] == []
     assert dump["derived"]["order"] == [0, 1, 2, 1, 2, 1, 2, 3]
+
+
+@pytest.mark.parametrize("lens", [[64], [1] * 70, [3, 1, 2, 1, 300, 1, 210], [517], [1, 1, 1, 509, 4]])
+@pytest.mark.parametrize("K,G,D,V", [(4, 2, 128, 40), (2, 3, 16, 8), (3, 1, 64, 24), (5, 2, 32, 72), (4, 5, 128, 600)])
+def test_delta_convolution_makes_unit_vectors(lens, K, G, D, V):
+    """Rows of several requests that meet inside a thread's run of rows, with and without history, few and many rows: the convolution is
+    `causal_conv_silu`'s (the same sums, taken one by one), q and k its results over their norms; a sum of D squares and the rest are
+    D + 8 roundings of 2^-24 at most."""
+    from gibbs_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(5)
+    N, C = sum(lens), 2 * G * D + V
+    x = torch.randn((N, C), generator=g, device="cuda").bfloat16()
+    taps = torch.randn((C, K), generator=g, device="cuda")
+    state = torch.randn((len(lens) + 1, K - 1, C), generator=g, device="cuda")
+    cu = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32, device="cuda")
+    row_req = torch.repeat_interleave(torch.arange(len(lens), device="cuda"), torch.tensor(lens, device="cuda")).to(torch.int32)
+    slot = torch.arange(1, len(lens) + 1, dtype=torch.int32, device="cuda").flip(0).contiguous()
+    first = 3 if len(lens) > 4 else 0
+    padded = [torch.cat([state[s].double(), x[a:b].double()]) for s, a, b in zip(slot.tolist(), cu.tolist(), cu.tolist()[1:])]
+    conv = torch.cat([sum(p[j:j + n] * taps[:, j].double() for j in range(K)) for p, n in zip(padded, lens)])
+    want = conv * torch.sigmoid(conv)
+    heads = want[first:, :2 * G * D].unflatten(1, (2, G, D))
+    unit = heads / torch.sqrt((heads * heads).sum(-1, keepdim=True) + 1e-6) * torch.tensor([0.25, 1.0], device="cuda", dtype=torch.float64)[:, None, None]
+    want[first:, :2 * G * D] = unit.flatten(1)
+    kept = state.clone()
+    got = ops.delta_conv(x, taps, state, row_req, cu, slot, G, D, 0.25, 1e-6, first)
+    err = (got.double() - want).abs()
+    # (the convolution's own K + 8 roundings are relative to the sum of its terms' magnitudes, at most 60 here; the norm passes them on)
+    assert err[:first].max().item() <= (K + 8) * 2.0 ** -24 * 60 if first else True
+    assert err[first:, 2 * G * D:].max().item() <= (K + 8) * 2.0 ** -24 * 60
+    head = got[first:, :2 * G * D].double().unflatten(1, (2, G, D)) - unit
+    terms = torch.cat([sum((p[j:j + n] * taps[:, j].double()).abs() for j in range(K)) for p, n in zip(padded, lens)])[first:, :2 * G * D].unflatten(1, (2, G, D))
+    scale = unit.norm(dim=-1) / (heads.norm(dim=-1) + 1e-30)
+    bound = 2.0 ** -24 * (2 * (K + 8) * terms.norm(dim=-1) * scale + (D + 8) * unit.norm(dim=-1))
+    assert (head.norm(dim=-1) <= bound).all()
+    for i, s in enumerate(slot.tolist()):
+        assert torch.equal(state[s], padded[i][-(K - 1):].float())
+    assert torch.equal(state[0], kept[0])
