@@ -52,7 +52,7 @@ __global__ void causal_conv_silu_kernel(const T* __restrict__ in, long ld, const
 
 // The same for bfloat16 inputs whose channels come in whole groups of 8: a thread takes 8 neighbouring channels with 16-byte loads, of
 // CONV_RUN rows one behind the other, whose inputs it holds in registers (a row a thread reads K rows for each it writes: 2,048 rows of
-// 6,144 channels, K = 4, 38 us; 19 us so, 75 MB).  A workgroup is 64 lanes of channels by CONV_ROWS such runs; the taps of its 512
+// 6,144 channels, K = 4, 30 us with a kernel of 25 us for the unit vectors behind it; 25 us so with them, half of it exponentials).  A workgroup is 64 lanes of channels by CONV_ROWS such runs; the taps of its 512
 // channels, one contiguous stretch of the [C, K] table, come through LDS once (each thread's 8 K taps a word further along, so that the lanes
 // read different banks) instead of as 8 K scattered words per thread.  Sums in ascending j, as above.
 // KT: K, as many rows as that in registers; 0: any K, a row at a time.
@@ -479,6 +479,30 @@ __global__ __launch_bounds__(64) void head_norm_gate_kernel(const float* __restr
     y[(size_t)n * H * V + c] = from_float<T>(row[j] * inv * gain[c % gain_len] * g);
   }
 }
+// The same for bfloat16 results and heads of 16, 32, 64 or 128 values in whole 16 bytes: V / 8 neighbouring lanes a head, 8 values each, so that
+// a wave has 4 to 32 heads on their way (a wave a head, 2,048 rows of 16 heads of 128: 16.4 us for 33 MB; 10.4 us so).
+__global__ __launch_bounds__(256) void head_norm_gate_vec8_kernel(const float* __restrict__ o, const float* __restrict__ gain, int gain_len,
+                                                                  const bf16* __restrict__ gate, long ld_gate, bf16* __restrict__ y, long heads, int H, int V,
+                                                                  float eps, int act) {
+  const int lanes = V / 8;
+  const long i = (long)blockIdx.x * 256 + threadIdx.x, at = i / lanes;      // row H + head
+  const long m = at < heads ? at : heads - 1;
+  const int j = (int)(i - at * lanes) * 8, n = (int)(m / H), c = (int)(m - (long)n * H) * V + j;
+  const float* row = o + m * V + j;
+  const float4 a = *(const float4*)row, b = *(const float4*)(row + 4);
+  const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) ss = fmaf(v[k], v[k], ss);
+  const float inv = 1.0f / sqrtf(lanes_sum(ss, lanes) / (float)V + eps);
+  const float4 ga = *(const float4*)(gain + c % gain_len), gb = *(const float4*)(gain + c % gain_len + 4);
+  const float gv[8] = {ga.x, ga.y, ga.z, ga.w, gb.x, gb.y, gb.z, gb.w};
+  float z[8], out[8];
+  if (gate) unpack8(*(const uint4*)(gate + (size_t)n * ld_gate + c), z);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) out[k] = v[k] * inv * gv[k] * (gate ? activate_gate(z[k], act) : 1.f);
+  if (at < heads) *(uint4*)(y + m * V + j) = pack8(out);
+}
 
 // ------------------------------------------------------------------------------------------------ one token per request
 // The delta rule for requests that bring one row each (row n is request n's), with what stands around it: the unit vectors, beta and
@@ -604,6 +628,48 @@ __global__ void token_shift_kernel(const T* __restrict__ h, const float* __restr
   if (keep_row) state[(size_t)slot[r] * slot_stride + c] = cur;   // (every request brings one row: it is the next step's previous row)
   for (int s = 0; s < n_mix; ++s)
     out[((size_t)s * N + n) * W + c] = from_float<T>(fmaf(prev - cur, mu[(size_t)s * W + c], cur));
+}
+// The same for bfloat16 rows in whole groups of 8 channels: 16 bytes a thread, RUN rows one behind the other, so that a weight is read once for
+// all of them (a channel a thread, 2,048 rows of 2,048 channels, 5 mixes: 28 us for 50 MB; 12.2 us so).
+template <int RUN>
+__global__ __launch_bounds__(256) void token_shift_vec8_kernel(const bf16* __restrict__ h, const float* __restrict__ mu, int n_mix, float* __restrict__ state,
+                                                               long slot_stride, const int* __restrict__ row_req, const int* __restrict__ cu,
+                                                               const int* __restrict__ slot, bf16* __restrict__ out, int N, int W, int keep_row) {
+  const int n0 = blockIdx.x * RUN, c = (blockIdx.y * 256 + threadIdx.x) * 8;
+  if (c >= W) return;
+  float row[RUN + 1][8], before[RUN][8];      // row[u]: row n0 + u - 1; before[u]: what stands in front of row n0 + u
+  uint4 raw[RUN + 1];
+#pragma unroll
+  for (int u = 0; u <= RUN; ++u) raw[u] = *(const uint4*)(h + (size_t)min(max(n0 + u - 1, 0), N - 1) * W + c);
+#pragma unroll
+  for (int u = 0; u <= RUN; ++u) unpack8(raw[u], row[u]);
+#pragma unroll
+  for (int u = 0; u < RUN; ++u) {
+    const int n = min(n0 + u, N - 1), r = row_req[n];
+    const bool inside = n > cu[r];
+    float* st = state + (size_t)slot[r] * slot_stride + c;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
+    if (!inside) a = *(const float4*)st, b = *(const float4*)(st + 4);
+    const float old[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) before[u][i] = inside ? row[u][i] : old[i];
+    if (keep_row && n0 + u < N) {
+      *(float4*)st = make_float4(row[u + 1][0], row[u + 1][1], row[u + 1][2], row[u + 1][3]);
+      *(float4*)(st + 4) = make_float4(row[u + 1][4], row[u + 1][5], row[u + 1][6], row[u + 1][7]);
+    }
+  }
+  for (int s = 0; s < n_mix; ++s) {
+    const float4 a = *(const float4*)(mu + (size_t)s * W + c), b = *(const float4*)(mu + (size_t)s * W + c + 4);
+    const float w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int u = 0; u < RUN; ++u) {
+      if (n0 + u >= N) break;
+      float y[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) y[i] = fmaf(before[u][i] - row[u + 1][i], w[i], row[u + 1][i]);
+      *(uint4*)(out + ((size_t)s * N + n0 + u) * W + c) = pack8(y);
+    }
+  }
 }
 template <typename T>
 __global__ void token_shift_state_kernel(const T* __restrict__ h, float* __restrict__ state, long slot_stride,
@@ -849,6 +915,12 @@ GIBBS_EXPORT int gibbs_head_norm_gate(const float* o, const float* gain, int gai
                                       int dtype, int n_rows, int H, int V, float eps, int act, hipStream_t stream) {
   GIBBS_REQUIRE(o && gain && y && n_rows > 0 && H > 0 && V > 0 && gain_len > 0 && (!gate || ld_gate >= (long)H * V) && (act == 0 || act == 1),
                 "head_norm_gate: bad operands rows=%d heads=%d V=%d", n_rows, H, V);
+  if (dtype == GIBBS_BF16 && (V == 16 || V == 32 || V == 64 || V == 128) && gain_len % 8 == 0 && ld_gate % 8 == 0 &&
+      (((uintptr_t)o | (uintptr_t)gain | (uintptr_t)gate | (uintptr_t)y) % 16) == 0) {
+    const long heads = (long)n_rows * H;
+    head_norm_gate_vec8_kernel<<<(unsigned)((heads * (V / 8) + 255) / 256), 256, 0, stream>>>(o, gain, gain_len, (const bf16*)gate, ld_gate, (bf16*)y, heads, H, V, eps, act);
+    GIBBS_LAUNCH_STATUS("head_norm_gate");
+  }
   const dim3 grid(n_rows, H);
   BY_DTYPE(dtype, "head_norm_gate",
            (head_norm_gate_kernel<float><<<grid, 64, 0, stream>>>(o, gain, gain_len, (const float*)gate, ld_gate, (float*)y, H, V, eps, act)),
@@ -863,7 +935,16 @@ GIBBS_EXPORT int gibbs_token_shift(const void* h, int dtype, const float* mu, in
   GIBBS_REQUIRE(h && mu && state && out && n_rows > 0 && n_req > 0 && W > 0 && n_mix > 0 && slot_stride >= W,
                 "token_shift: bad operands rows=%d requests=%d W=%d", n_rows, n_req, W);
   const dim3 rows(n_rows, ceil_div(W, 256)), reqs(n_req, ceil_div(W, 256));
-  BY_DTYPE(dtype, "token_shift",
+  // (few rows: a channel a thread is more, shorter workgroups)
+  if (dtype == GIBBS_BF16 && n_rows >= 64 && W % 8 == 0 && slot_stride % 4 == 0 && (((uintptr_t)h | (uintptr_t)mu | (uintptr_t)state | (uintptr_t)out) % 16) == 0) {
+    if (n_rows >= 1024)
+      token_shift_vec8_kernel<4><<<dim3(ceil_div(n_rows, 4), ceil_div(W, 2048)), 256, 0, stream>>>((const bf16*)h, mu, n_mix, state, slot_stride, row_req, cu, slot,
+                                                                                                  (bf16*)out, n_rows, W, keep);
+    else
+      token_shift_vec8_kernel<1><<<dim3(n_rows, ceil_div(W, 2048)), 256, 0, stream>>>((const bf16*)h, mu, n_mix, state, slot_stride, row_req, cu, slot, (bf16*)out,
+                                                                                     n_rows, W, keep);
+  } else
+    BY_DTYPE(dtype, "token_shift",
            (token_shift_kernel<float><<<rows, 256, 0, stream>>>((const float*)h, mu, n_mix, state, slot_stride, row_req, cu, slot, (float*)out, n_rows, W, keep)),
            (token_shift_kernel<bf16><<<rows, 256, 0, stream>>>((const bf16*)h, mu, n_mix, state, slot_stride, row_req, cu, slot, (bf16*)out, n_rows, W, keep)));
   if (update_state && !keep)

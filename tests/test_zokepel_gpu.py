@@ -905,3 +905,71 @@ def test_delta_convolution_makes_unit_vectors(lens, K, G, D, V):
     for i, s in enumerate(slot.tolist()):
         assert torch.equal(state[s], padded[i][-(K - 1):].float())
     assert torch.equal(state[0], kept[0])
+
+
+@pytest.mark.parametrize("n,nh,nkv,hd,vd,norm_dim,unit,every", [(1, 4, 1, 64, 64, 0, True, 7), (70, 16, 4, 128, 128, 0, True, 1024), (9, 3, 3, 16, 24, 13, True, 0),
+                                                              (33, 40, 8, 64, 128, 0, False, 5), (5, 2, 0, 32, 8, 0, True, 3), (3, 64, 64, 128, 128, 0, True, 2)])
+def test_unit_heads_in_whole_16_bytes_like_float32(n, nh, nkv, hd, vd, norm_dim, unit, every):
+    """bfloat16 heads eight channels a lane against the float32 kernel on the same values: one rounding to bfloat16 apart (2^-8), values unchanged."""
+    from gibbs_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(n + nh)
+    W = (nh + nkv) * hd + nkv * vd
+    x = torch.randn((n, W), generator=g, device="cuda").bfloat16()
+    page_size, pages = 4, 40
+    pos = torch.randint(0, 100, (n,), generator=g, device="cuda", dtype=torch.int32)
+    req = torch.zeros(n, dtype=torch.int32, device="cuda")
+    table = torch.randperm(pages, generator=g, device="cuda").to(torch.int32)[:25].reshape(1, -1).contiguous()
+    outs = []
+    for kind in (torch.float32, torch.bfloat16):
+        rows = x.to(kind).clone()
+        kp = torch.zeros((pages, nkv, page_size, hd), dtype=kind, device="cuda") if nkv else None
+        vp = torch.zeros((pages, nkv, page_size, vd), dtype=kind, device="cuda") if nkv else None
+        for i in range(n):        # (rows of one position would race for a place in the pages)
+            ops.qk_unit_kv(rows[i:i + 1], nh, nkv, hd, vd, kpages=kp, vpages=vp, table=table if nkv else None, pos=pos[i:i + 1], row_req=req[:1], eps=1e-6, unit=unit,
+                           temp_coef=0.1, temp_every=every, norm_dim=norm_dim)
+        outs.append([rows.float()] + ([kp.float(), vp.float()] if nkv else []))
+        if kind == torch.bfloat16:
+            again = x.clone()
+            ops.qk_unit_kv(again, nh, nkv, hd, vd, kpages=None, vpages=None, table=None, pos=pos, row_req=req, eps=1e-6, unit=unit, temp_coef=0.1, temp_every=every,
+                           norm_dim=norm_dim)
+            assert torch.equal(again, rows)
+    for want, got in zip(*outs):
+        assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-30).all()
+
+
+@pytest.mark.parametrize("n,H,V,gains", [(1, 1, 16, 16), (7, 3, 32, 96), (300, 16, 128, 128), (130, 5, 64, 64)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_head_norm_in_whole_16_bytes_like_float32(n, H, V, gains, gated):
+    """The bfloat16 kernel with a few lanes a head against the float32 kernel: one rounding to bfloat16 apart."""
+    from gibbs_amd.ops.lib import call, ptr, stream
+    g = torch.Generator(device="cuda").manual_seed(n)
+    o = torch.randn((n, H * V), generator=g, device="cuda")
+    gain = torch.randn(gains, generator=g, device="cuda")
+    gate = torch.randn((n, H * V + 8), generator=g, device="cuda").bfloat16()
+    outs = []
+    for kind, code in ((torch.float32, 0), (torch.bfloat16, 1)):
+        y, z = torch.empty((n, H * V), dtype=kind, device="cuda"), gate.to(kind)
+        call("gibbs_head_norm_gate", ptr(o), ptr(gain), gains, ptr(z) if gated else None, H * V + 8 if gated else 0, ptr(y), code, n, H, V, 1e-6, 0, stream())
+        outs.append(y.float())
+    assert ((outs[1] - outs[0]).abs() <= 2.0 ** -8 * outs[0].abs() + 1e-30).all()
+
+
+@pytest.mark.parametrize("lens", [[64], [1] * 66, [1025], [5, 1, 1, 1500, 2, 1]])
+@pytest.mark.parametrize("W,mixes", [(8, 1), (2056, 5)])
+def test_token_shift_in_whole_16_bytes_like_float32(lens, W, mixes):
+    """Eight channels a thread, a row or four of them, requests that meet inside a thread's rows: the float32 kernel's results rounded, to the bit, and its state."""
+    from gibbs_amd.ops.lib import call, ptr, stream
+    g = torch.Generator(device="cuda").manual_seed(W)
+    n = sum(lens)
+    h = torch.randn((n, W), generator=g, device="cuda").bfloat16()
+    mu = torch.randn((mixes, W), generator=g, device="cuda")
+    kept = torch.randn((len(lens) + 1, W), generator=g, device="cuda")
+    cu = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32, device="cuda")
+    req = torch.repeat_interleave(torch.arange(len(lens), device="cuda"), torch.tensor(lens, device="cuda")).to(torch.int32)
+    slot = torch.arange(1, len(lens) + 1, dtype=torch.int32, device="cuda").flip(0).contiguous()
+    outs = []
+    for kind, code in ((torch.float32, 0), (torch.bfloat16, 1)):
+        x, state, out = h.to(kind), kept.clone(), torch.empty((mixes, n, W), dtype=kind, device="cuda")
+        call("gibbs_token_shift", ptr(x), code, ptr(mu), mixes, ptr(state), W, ptr(req), ptr(cu), ptr(slot), ptr(out), n, len(lens), W, 1, int(n == len(lens)), stream())
+        outs.append((out, state))
+    assert torch.equal(outs[0][0].bfloat16(), outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
