@@ -109,6 +109,96 @@ __device__ __forceinline__ float wave_dot(const T* __restrict__ row, const float
   return out[0];
 }
 
+// One wave's choice for row n from its logits z [E] in LDS, which change; `score`: E floats more, for modes 1 and 2.
+// the `top` largest, in descending order, the lower index among equal logits (one wave: a lane scans its share of
+// the experts, the lanes' bests are folded by exchanges); a logit that was taken becomes NaN; then the softmax
+// over the chosen logits alone
+__device__ __forceinline__ void choose_experts(float* z, float* score, int n, int lane, const float* __restrict__ router_bias, int* __restrict__ chosen,
+                                               float* __restrict__ weight, int E, int top, int mode, float weight_scale) {
+  int* mine = chosen + (size_t)n * top;
+  float* wts = weight + (size_t)n * top;
+  if (mode == 2 && router_bias) {
+    for (int e = lane; e < E; e += WAVE) {
+      score[e] = 1.0f / (1.0f + expf(-z[e]));
+      z[e] = score[e] + router_bias[e];
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_wave_barrier();
+  }
+  if (mode == 1) {
+    // scores over all outputs; what is compared is the score plus the output's correction
+    float zmax = -INFINITY;
+    for (int e = lane; e < E; e += WAVE) zmax = fmaxf(zmax, z[e]);
+    zmax = wave_max(zmax);
+    float total = 0.f;
+    for (int e = lane; e < E; e += WAVE) total += expf(z[e] - zmax);
+    total = wave_sum(total);
+    for (int e = lane; e < E; e += WAVE) {
+      const float sc = expf(z[e] - zmax) / total;
+      score[e] = sc;
+      z[e] = sc + (router_bias ? router_bias[e] : 0.f);
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_wave_barrier();
+  }
+  // (lane c keeps choice c: a store to memory inside this chain is a wait for it at every turn; 8 rows of 16 experts, 4 chosen, scores over all: 9.3 us so,
+  // 8.2 without.  More choices than lanes go to memory as they are made.)
+  const bool kept = top <= WAVE;
+  int my_pick = -1;
+  float my_weight = 0.f, best = 0.f, sum = 0.f;
+  for (int c = 0; c < top; ++c) {
+    float pv = -INFINITY;
+    int pick = 0x7fffffff;
+    for (int e = lane; e < E; e += WAVE) {
+      const float v = z[e];
+      if (v == v && (v > pv || (v == pv && e < pick) || pick == 0x7fffffff)) { pv = v; pick = e; }
+    }
+#pragma unroll
+    for (int o = WAVE / 2; o > 0; o >>= 1) {
+      const float ov = __shfl_xor(pv, o, WAVE);
+      const int op = __shfl_xor(pick, o, WAVE);
+      if (op != 0x7fffffff && (pick == 0x7fffffff || ov > pv || (ov == pv && op < pick))) { pv = ov; pick = op; }
+    }
+    if (pick == 0x7fffffff) {   // (fewer usable logits than choices: the first expert not taken yet, with no weight)
+      __builtin_amdgcn_s_waitcnt(0);
+      for (int e = 0; e < E && pick == 0x7fffffff; ++e) {
+        bool taken = kept && __builtin_amdgcn_ballot_w64(lane < c && my_pick == e) != 0;
+        for (int d = 0; !kept && d < c; ++d) taken |= mine[d] == e;
+        if (!taken) pick = e;
+      }
+      pv = -INFINITY;
+    }
+    if (c == 0) best = pv;
+    const float w = (mode == 1 || (mode == 2 && router_bias)) ? score[pick]
+                    : (pv == -INFINITY ? 0.f : (mode == 2 ? 1.0f / (1.0f + expf(-pv)) : expf(pv - best)));
+    sum += w;
+    if (lane == c) {
+      my_pick = pick;
+      my_weight = w;
+    }
+    if (lane == 0) {
+      if (!kept) {
+        mine[c] = pick;
+        wts[c] = w;
+      }
+      z[pick] = __builtin_nanf("");
+    }
+    // (the wave's own LDS write above is read by its next scan)
+    if (kept) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    else __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_wave_barrier();
+  }
+  auto normed = [&](float w) { return mode == 2 ? w : (mode == 1 ? w / (sum + 1e-20f) * weight_scale : (sum > 0.f ? w / sum : 0.f)); };
+  if (kept) {
+    if (lane < top) {
+      mine[lane] = my_pick;
+      wts[lane] = normed(my_weight);
+    }
+  } else if (lane == 0) {
+    for (int c = 0; c < top; ++c) wts[c] = normed(wts[c]);
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(1024) void moe_route_kernel(const T* __restrict__ h, long ldh, const float* __restrict__ router,
                                                         const float* __restrict__ router_bias, const float* __restrict__ shared_gate,
@@ -140,76 +230,70 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(const T* __restrict__ h
   }
   __syncthreads();
   if (wave != 0) return;
-  // the `top` largest, in descending order, the lower index among equal logits (one wave: a lane scans its share of
-  // the experts, the lanes' bests are folded by exchanges); a logit that was taken becomes NaN; then the softmax
-  // over the chosen logits alone
-  int* mine = chosen + (size_t)n * top;
-  float* wts = weight + (size_t)n * top;
-  float* score = z + E;
-  if (mode == 2 && router_bias) {
-    for (int e = lane; e < E; e += WAVE) {
-      score[e] = 1.0f / (1.0f + expf(-z[e]));
-      z[e] = score[e] + router_bias[e];
+  choose_experts(z, z + E, n, lane, router_bias, chosen, weight, E, top, mode, weight_scale);
+}
+
+// Many rows: a workgroup of four waves takes four of them, a wave two experts' logits of all four rows at a time, so that a router's row is read
+// once for four rows (and a row's values once for two experts), and then a row's choice.  Sums as wave_dots makes them: the same bits.
+constexpr int ROUTE_ROWS = 4;
+template <typename T>
+__global__ __launch_bounds__(ROUTE_ROWS * WAVE) void moe_route_rows_kernel(const T* __restrict__ h, long ldh, const float* __restrict__ router,
+                                                                           const float* __restrict__ router_bias, const float* __restrict__ shared_gate,
+                                                                           int* __restrict__ chosen, float* __restrict__ weight, float* __restrict__ sgate, int N,
+                                                                           int W, int E, int top, int mode, float weight_scale) {
+  extern __shared__ float z[];   // [ROUTE_ROWS][E], and as many scores behind them
+  const int n0 = blockIdx.x * ROUTE_ROWS, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
+  const int vectors = E + (shared_gate ? 1 : 0);
+  const T* rows[ROUTE_ROWS];
+#pragma unroll
+  for (int r = 0; r < ROUTE_ROWS; ++r) rows[r] = h + (size_t)min(n0 + r, N - 1) * ldh;
+  for (int e = 2 * wave; e < vectors; e += 2 * ROUTE_ROWS) {
+    const float* w[2];
+#pragma unroll
+    for (int v = 0; v < 2; ++v) w[v] = min(e + v, vectors - 1) < E ? router + (size_t)min(e + v, vectors - 1) * W : shared_gate;
+    float s[2][ROUTE_ROWS] = {};
+    auto step = [&](const float4 (&a)[ROUTE_ROWS], const float4 (&b)[2]) {
+#pragma unroll
+      for (int v = 0; v < 2; ++v)
+#pragma unroll
+        for (int r = 0; r < ROUTE_ROWS; ++r) {
+          s[v][r] = fmaf(a[r].x, b[v].x, s[v][r]); s[v][r] = fmaf(a[r].y, b[v].y, s[v][r]);
+          s[v][r] = fmaf(a[r].z, b[v].z, s[v][r]); s[v][r] = fmaf(a[r].w, b[v].w, s[v][r]);
+        }
+    };
+    int k = lane * 4;
+    for (; k + WAVE * 4 < W; k += 2 * WAVE * 4) {
+      float4 a[2][ROUTE_ROWS], b[2][2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int r = 0; r < ROUTE_ROWS; ++r) a[u][r] = load4f(rows[r] + k + u * WAVE * 4);
+#pragma unroll
+        for (int v = 0; v < 2; ++v) b[u][v] = *(const float4*)(w[v] + k + u * WAVE * 4);
+      }
+      step(a[0], b[0]);
+      step(a[1], b[1]);
     }
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_wave_barrier();
-  }
-  if (mode == 1) {
-    // scores over all outputs; what is compared is the score plus the output's correction
-    float zmax = -INFINITY;
-    for (int e = lane; e < E; e += WAVE) zmax = fmaxf(zmax, z[e]);
-    zmax = wave_max(zmax);
-    float total = 0.f;
-    for (int e = lane; e < E; e += WAVE) total += expf(z[e] - zmax);
-    total = wave_sum(total);
-    for (int e = lane; e < E; e += WAVE) {
-      const float sc = expf(z[e] - zmax) / total;
-      score[e] = sc;
-      z[e] = sc + (router_bias ? router_bias[e] : 0.f);
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_wave_barrier();
-  }
-  float best = 0.f, sum = 0.f;
-  for (int c = 0; c < top; ++c) {
-    float pv = -INFINITY;
-    int pick = 0x7fffffff;
-    for (int e = lane; e < E; e += WAVE) {
-      const float v = z[e];
-      if (v == v && (v > pv || (v == pv && e < pick) || pick == 0x7fffffff)) { pv = v; pick = e; }
+    for (; k < W; k += WAVE * 4) {
+      float4 a[ROUTE_ROWS], b[2];
+#pragma unroll
+      for (int r = 0; r < ROUTE_ROWS; ++r) a[r] = load4f(rows[r] + k);
+#pragma unroll
+      for (int v = 0; v < 2; ++v) b[v] = *(const float4*)(w[v] + k);
+      step(a, b);
     }
 #pragma unroll
-    for (int o = WAVE / 2; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(pv, o, WAVE);
-      const int op = __shfl_xor(pick, o, WAVE);
-      if (op != 0x7fffffff && (pick == 0x7fffffff || ov > pv || (ov == pv && op < pick))) { pv = ov; pick = op; }
-    }
-    if (pick == 0x7fffffff) {   // (fewer usable logits than choices: the first expert not taken yet, with no weight)
-      for (int e = 0; e < E && pick == 0x7fffffff; ++e) {
-        bool taken = false;
-        for (int d = 0; d < c; ++d) taken |= mine[d] == e;
-        if (!taken) pick = e;
+    for (int v = 0; v < 2; ++v)
+#pragma unroll
+      for (int r = 0; r < ROUTE_ROWS; ++r) {
+        const float sum = wave_sum(s[v][r]);
+        if (lane != 0 || e + v >= vectors) continue;
+        if (e + v < E) z[r * E + e + v] = sum + ((router_bias && mode == 0) ? router_bias[e + v] : 0.f);
+        else if (n0 + r < N) sgate[n0 + r] = 1.0f / (1.0f + expf(-sum));
       }
-      pv = -INFINITY;
-    }
-    if (c == 0) best = pv;
-    const float w = (mode == 1 || (mode == 2 && router_bias)) ? score[pick]
-                    : (pv == -INFINITY ? 0.f : (mode == 2 ? 1.0f / (1.0f + expf(-pv)) : expf(pv - best)));
-    sum += w;
-    if (lane == 0) {
-      mine[c] = pick;
-      wts[c] = w;
-      z[pick] = __builtin_nanf("");
-    }
-    __builtin_amdgcn_s_waitcnt(0);   // (the wave's own LDS write above is read by its next scan)
-    __builtin_amdgcn_wave_barrier();
   }
-  if (lane == 0 && mode != 2) {
-    if (mode == 1)
-      for (int c = 0; c < top; ++c) wts[c] = wts[c] / (sum + 1e-20f) * weight_scale;
-    else
-      for (int c = 0; c < top; ++c) wts[c] = sum > 0.f ? wts[c] / sum : 0.f;
-  }
+  __syncthreads();
+  if (n0 + wave < N) choose_experts(z + wave * E, z + (ROUTE_ROWS + wave) * E, n0 + wave, lane, router_bias, chosen, weight, E, top, mode, weight_scale);
 }
 
 // ------------------------------------------------------------------------------------------------- group
@@ -838,7 +922,19 @@ GIBBS_EXPORT int gibbs_moe_route_scaled(const void* h, long ldh, int dtype, cons
   GIBBS_REQUIRE(E > 0 && E <= MOE_MAX_EXPERTS && top > 0 && top <= E, "moe_route: %d of %d experts (at most %d)", top, E, MOE_MAX_EXPERTS);
   GIBBS_REQUIRE(!shared_gate || sgate, "moe_route: a shared expert's gate needs its output");
   const size_t lds = (size_t)E * sizeof(float) * (mode != 0 ? 2 : 1);
-  // few rows: a wave per expert (and one for the shared expert's gate) up to 16 waves; many rows fill the chip with 4
+  // few rows: a wave per expert (and one for the shared expert's gate) up to 16 waves; many rows fill the chip with 4; more share the router
+  // (16 experts, a row / four rows a workgroup, us: 513 rows of 2,048 13.2 / 16.1, 1,024 15.8 / 13.3, 2,029 23.4 / 19.6, 4,096 of 1,024 27 / 16.0; many experts
+  // gain nothing, 700 rows of 2,048, 256 experts 113 / 121)
+  const bool share = n >= 1024 && E <= 32 && W % 4 == 0 && ldh % 4 == 0 && ((uintptr_t)h % 16) == 0 && ((uintptr_t)router % 16) == 0 && ((uintptr_t)shared_gate % 16) == 0;
+  if (share && (dtype == GIBBS_F32 || dtype == GIBBS_BF16)) {
+    const int blocks = ceil_div(n, ROUTE_ROWS);
+    const size_t all = 2 * ROUTE_ROWS * (size_t)E * sizeof(float);
+    if (dtype == GIBBS_F32)
+      moe_route_rows_kernel<float><<<blocks, ROUTE_ROWS * WAVE, all, stream>>>((const float*)h, ldh, router, router_bias, shared_gate, chosen, weight, sgate, n, W, E, top, mode, weight_scale);
+    else
+      moe_route_rows_kernel<bf16><<<blocks, ROUTE_ROWS * WAVE, all, stream>>>((const bf16*)h, ldh, router, router_bias, shared_gate, chosen, weight, sgate, n, W, E, top, mode, weight_scale);
+    GIBBS_LAUNCH_STATUS("moe_route");
+  }
   const int threads = n >= 512 ? 256 : WAVE * std::min(16, std::max(4, E + 1));
   if (dtype == GIBBS_F32)
     moe_route_kernel<float><<<n, threads, lds, stream>>>((const float*)h, ldh, router, router_bias, shared_gate, chosen, weight, sgate, W, E, top, mode, weight_scale);

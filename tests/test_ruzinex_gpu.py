@@ -438,6 +438,31 @@ def test_experts_sum_inside_the_sublayer_boundary(dtype, shared):
     assert np.abs(out.float().cpu().numpy() - want_out).max() <= (2e-5 if dtype == torch.float32 else 2e-2) * max(1.0, np.abs(want_out).max())
 
 
+@pytest.mark.parametrize("W,E,top,shared", [(2048, 16, 4, False), (260, 7, 7, True), (512, 32, 3, True), (4, 1, 1, False)])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_routes_of_many_rows_are_the_routes_of_few(W, E, top, shared, mode):
+    """Four rows a workgroup (1,024 rows and more, the last workgroup not full) against a workgroup a row: the same choices, weights and gates, to the bit,
+    with equal logits and a row that is no number among them."""
+    from gibbs_amd.ops.lib import call, ptr, stream
+    g = torch.Generator(device="cuda").manual_seed(W + mode)
+    n = 1031
+    h = torch.randn((n, W), generator=g, device="cuda").bfloat16()
+    h[513, 3] = float("nan")
+    router, bias, gate = (torch.randn(s, generator=g, device="cuda") * W ** -0.5 for s in ((E, W), (E,), (W,)))
+    if E > 2:
+        router[2], bias[2] = router[1], bias[1]
+    def route(rows):
+        m = rows.shape[0]
+        out = torch.full((m, top), -1, dtype=torch.int32, device="cuda"), torch.zeros((m, top), device="cuda"), torch.zeros(m, device="cuda")
+        call("gibbs_moe_route_scaled", ptr(rows), W, 1, ptr(router), ptr(bias), ptr(gate) if shared else None, *map(ptr, out), m, W, E, top, mode,
+             1.5 if mode == 1 else 1.0, stream())
+        return out
+    many, few = route(h), [torch.cat(x) for x in zip(route(h[:500]), route(h[500:1000].contiguous()), route(h[1000:].contiguous()))]
+    for a, b in zip(many, few):
+        assert torch.equal(torch.nan_to_num(a.float(), nan=7.0), torch.nan_to_num(b.float(), nan=7.0))
+    assert torch.equal(many[0].sort(-1).values.diff(dim=-1) > 0, torch.ones((n, top - 1), dtype=torch.bool, device="cuda"))      # no expert twice
+
+
 def test_a_rows_experts_do_not_depend_on_its_neighbours():
     """32-bit: the same row alone and among 200 others gives the same bits."""
     from gibbs_amd import Engine
