@@ -18,8 +18,8 @@
 //
 // A pair's result depends on nothing but its own row and expert (no sum runs over pairs), so where a pair lands
 // among its expert's pairs, which the atomic counters of `group` decide, changes no value: a row's result is the
-// same whatever else is in the batch.  Products: plain FMA in ascending k for float32 and for bfloat16 operands
-// that are not 16-byte aligned; on the matrix cores for aligned bfloat16, float32 accumulators, the activation in
+// same whatever else is in the batch.  Products: plain FMA in ascending k for operands that are not 16-byte aligned; float32 in three bfloat16
+// parts on the matrix cores (moe_f32.hip); on the matrix cores for aligned bfloat16, float32 accumulators, the activation in
 // float32: tiles of 16 pairs for steps of few pairs (the experts' matrices are streamed once, a workgroup's four
 // waves split k, operands straight from memory: rows of h and of every W are contiguous along k), tiles of 128
 // pairs beyond (inner sizes of whole tiles of 64 k: 128 pairs x 256 rows of W loaded straight into LDS, three tiles deep, a workgroup a
@@ -28,6 +28,10 @@
 #include "common.h"
 #include "activation.h"
 #include <algorithm>
+
+// (moe_f32.hip)
+bool moe_gemm_f32(const float* X, long ldx, int top, const int* sorted_pair, const int* tile_expert, long cap, int bm, const float* wa, const float* wb,
+                  const float* in_weight, float* Y, long ldy, int O, int I, int act, hipStream_t stream);
 
 namespace {
 constexpr int MOE_MAX_EXPERTS = 1024;
@@ -991,7 +995,8 @@ GIBBS_EXPORT int gibbs_moe_gemm_weighted(const void* X, long ldx, int top, const
     else { if (w_b) MOE_PLAIN(T, 16, true); else MOE_PLAIN(T, 16, false); }                \
   } while (0)
   if (dtype == GIBBS_F32) {
-    MOE_PLAIN_ANY(float);
+    if (!moe_gemm_f32((const float*)X, ldx, top, sorted_pair, tile_expert, cap, bm, (const float*)w_a, (const float*)w_b, in_weight, (float*)Y, ldy, O, I, act, stream))
+      MOE_PLAIN_ANY(float);
   } else if (dtype == GIBBS_BF16) {
     const bool aligned = I % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)X % 16) == 0 && ((uintptr_t)w_a % 16) == 0 && ((uintptr_t)w_b % 16) == 0;
     if (!aligned) {

@@ -1,0 +1,130 @@
+// The experts' products in float32, on the matrix cores in three parts (f32_parts.h): the order of a sum is gemm_f32.hip's and depends on the inner
+// size alone, so a pair's result is the same to the bit whatever tile it falls in and whatever else is in the step.
+//
+// A workgroup takes 16 FN places of one expert's stretch and 32 of its features (gated: 16 of both matrices), its eight waves a stretch of k
+// each, straight from memory into the operands' registers, where they are split; the waves' sums meet in LDS.  Bound by the stream of the
+// experts' matrices for few pairs, by what a compute unit brings in for many.  The loop is gemm_f32_split_kernel's.
+// Width 1,024, experts of 512, 4 of 16 (us, gated and back, vector units before / now): 20 rows 165 and 54 / 18 and 14, 1,000 rows 496
+// and 215 / 180 and 145.
+#include "activation.h"
+#include "f32_parts.h"
+
+namespace {
+template <bool GLU, int FN>
+__global__ __launch_bounds__(512) void moe_gemm_f32_kernel(const float* __restrict__ X, long ldx, int top, const int* __restrict__ sorted_pair,
+                                                           const int* __restrict__ tile_expert, int bm, const float* __restrict__ Wa,
+                                                           const float* __restrict__ Wb, long expert_stride, float* __restrict__ Y, long ldy, int O, int I, int act,
+                                                           const float* __restrict__ in_weight) {
+  constexpr int SETS = 4, FO = 2, FEATURES = GLU ? 16 : 32;
+  __shared__ __attribute__((aligned(16))) f32x4 s_sum[F32_SEGMENTS][FO * FN][WAVE];
+  const int p0 = blockIdx.y * 16 * FN, e = tile_expert[p0 / bm];
+  if (e < 0 || sorted_pair[p0] < 0) return;      // (an expert's pairs take the first places of its tiles)
+  const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), g = lane / 16, c = lane % 16;
+  const int o0 = blockIdx.x * FEATURES;
+  const int segments = f32_segments(I), segment = f32_segment(I);
+  const int first = wave * segment, last = wave < segments ? min(first + segment, I) : 0;
+  const float *wa = Wa + (size_t)e * expert_stride, *wb = GLU ? Wb + (size_t)e * expert_stride : wa;
+  // (the row of a place without a pair is some row of X, and its results are not stored)
+  auto row_of = [&](int place) {
+    const int pair = sorted_pair[place];
+    return X + (size_t)(pair < 0 ? 0 : (top > 0 ? pair / top : place)) * ldx;
+  };
+  const float* wp[FO];
+  const float* xp[FN];
+#pragma unroll
+  for (int i = 0; i < FO; ++i) wp[i] = GLU ? (i == 0 ? wa : wb) + (size_t)min(o0 + c, O - 1) * I : wa + (size_t)min(o0 + 16 * i + c, O - 1) * I;
+#pragma unroll
+  for (int i = 0; i < FN; ++i) xp[i] = row_of(p0 + 16 * i + c);
+  f32x4 fw[SETS][2][FO], fx[SETS][2][FN];
+  // (k beyond the matrix: its last four again, and X's made zero when they are used)
+  auto ask = [&](int set, int k0) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const int k = min(k0 + 8 * g + 4 * half, I - 4);
+#pragma unroll
+      for (int i = 0; i < FO; ++i) fw[set][half][i] = *(const f32x4*)(wp[i] + k);
+#pragma unroll
+      for (int i = 0; i < FN; ++i) fx[set][half][i] = *(const f32x4*)(xp[i] + k);
+    }
+  };
+  f32x4 acc[FO][FN] = {};
+  auto use = [&](int set, int k0) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const uint32_t keep = (uint32_t)((k0 + 8 * g + 4 * half - I) >> 31);
+#pragma unroll
+      for (int i = 0; i < FN; ++i) fx[set][half][i] = __builtin_bit_cast(f32x4, __builtin_bit_cast(u32x4, fx[set][half][i]) & keep);
+    }
+    bf16x8 pw[FO][3], px[FN][3];
+#pragma unroll
+    for (int i = 0; i < FO; ++i) split8(fw[set][0][i], fw[set][1][i], pw[i]);
+#pragma unroll
+    for (int i = 0; i < FN; ++i) split8(fx[set][0][i], fx[set][1][i], px[i]);
+#pragma unroll
+    for (int p = 0; p < F32_PRODUCTS; ++p)
+#pragma unroll
+      for (int i = 0; i < FO; ++i)
+#pragma unroll
+        for (int h = 0; h < FN; ++h) acc[i][h] = mfma_bf16(pw[i][F32_PART[p][0]], px[h][F32_PART[p][1]], acc[i][h]);
+  };
+  if (first < last) {
+    const int end = (last - first + 31) / 32 * 32 + first - 32;      // the wave's last block
+#pragma unroll
+    for (int s = 0; s < SETS; ++s) ask(s, min(first + 32 * s, end));
+    int k0 = first;
+    for (; k0 + 32 * (2 * SETS - 1) <= end; k0 += 32 * SETS) {
+#pragma unroll
+      for (int s = 0; s < SETS; ++s) {
+        __builtin_amdgcn_sched_barrier(0);
+        use(s, k0 + 32 * s);
+        ask(s, k0 + 32 * (s + SETS));
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < 2 * SETS - 1; ++s) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (k0 + 32 * s <= end) use(s % SETS, k0 + 32 * s);
+      if (s < SETS - 1 && k0 + 32 * (s + SETS) <= end) ask(s, k0 + 32 * (s + SETS));
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < FO; ++i)
+#pragma unroll
+    for (int h = 0; h < FN; ++h) s_sum[wave][i * FN + h][lane] = acc[i][h];
+  __syncthreads();
+  const bool wide = O % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)Y % 16) == 0;
+  // the whole sum of one of the workgroup's results, in float32 where it wants that
+  auto whole = [&](int t, const float* w, int col, const float* x) {
+    f32x4 total = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < segments; ++s) total += s_sum[s][t][lane];
+    if (__builtin_expect(wants_again(total), 0)) total = again4(x, w, I, 0, I, 0, col, 1, O, total);
+    return total;
+  };
+  for (int t = wave; t < (GLU ? FN : FO * FN); t += F32_SEGMENTS) {
+    const int place = p0 + 16 * (t % FN) + c, pair = sorted_pair[place], col = o0 + 16 * (t / FN) + 4 * g;
+    if (pair < 0) continue;
+    const float* x = row_of(place);
+    f32x4 v = whole(t, wa, col, x);
+    if constexpr (GLU) {
+      const f32x4 u = whole(FN + t, wb, col, x);
+      const float w = in_weight ? in_weight[pair] : 1.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = activate(w * v[i], act) * (w * u[i]);
+    }
+    store_f32x4(Y, ldy, place, col, place + 1, O, wide, v);
+  }
+}
+}  // namespace
+
+// gibbs_moe_gemm_weighted's float32 products where rows are whole 16 bytes (false: not these operands, nothing was done).
+bool moe_gemm_f32(const float* X, long ldx, int top, const int* sorted_pair, const int* tile_expert, long cap, int bm, const float* wa, const float* wb,
+                  const float* in_weight, float* Y, long ldy, int O, int I, int act, hipStream_t stream) {
+  if (I % 4 || ldx % 4 || (((uintptr_t)X | (uintptr_t)wa | (uintptr_t)wb) % 16)) return false;
+  const int fn = bm == 16 ? 1 : 2;      // (places a workgroup takes: many pairs read the matrices half as often)
+  const dim3 grid(ceil_div(O, wb ? 16 : 32), (unsigned)(cap / (16 * fn)));
+  if (cap / (16 * fn) > 65535) return false;
+  auto launch = [&](auto kernel) { kernel<<<grid, 512, 0, stream>>>(X, ldx, top, sorted_pair, tile_expert, bm, wa, wb, (long)O * I, Y, ldy, O, I, act, in_weight); };
+  if (wb) fn == 1 ? launch(moe_gemm_f32_kernel<true, 1>) : launch(moe_gemm_f32_kernel<true, 2>);
+  else fn == 1 ? launch(moe_gemm_f32_kernel<false, 1>) : launch(moe_gemm_f32_kernel<false, 2>);
+  return true;
+}

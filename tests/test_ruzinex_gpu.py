@@ -463,6 +463,47 @@ def test_routes_of_many_rows_are_the_routes_of_few(W, E, top, shared, mode):
     assert torch.equal(many[0].sort(-1).values.diff(dim=-1) > 0, torch.ones((n, top - 1), dtype=torch.bool, device="cuda"))      # no expert twice
 
 
+@pytest.mark.parametrize("O,I", [(8, 4), (33, 68), (96, 260), (512, 1024), (70, 2052)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_experts_products_in_float32(O, I, gated):
+    """float32 products of tiles of 16 and of 128 places, some without pairs: the same bits whatever the tile, within the error of a sum of I products in 32
+    bits (I 2^-24 of their magnitudes; gated: of both sums, silu's slope at most 1.1, and 16 roundings of its own); values that are no numbers come out
+    as in plain float32."""
+    from gibbs_amd.ops.lib import call, ptr, stream
+    g = torch.Generator(device="cuda").manual_seed(O + I)
+    x = torch.randn((60, I), generator=g, device="cuda")
+    wa, wb = (torch.randn((3, O, I), generator=g, device="cuda") * I ** -0.5 for _ in range(2))
+    weight = torch.rand(120, generator=g, device="cuda") + 0.5
+    def products(rows, bm, taken):
+        place = torch.full((2 * bm,), -1, dtype=torch.int32, device="cuda")
+        place[bm:bm + taken] = torch.arange(taken, dtype=torch.int32, device="cuda")      # pairs 0 .. of the second tile, two a row
+        y = torch.full((2 * bm, O + 3), 7.0, device="cuda")
+        call("gibbs_moe_gemm_weighted", ptr(rows), I, 2, ptr(place), ptr(torch.tensor([-1, 2], dtype=torch.int32, device="cuda")), 2 * bm, bm, ptr(wa),
+             ptr(wb) if gated else None, ptr(weight) if gated else None, ptr(y), O + 3, 0, O, I, 0, stream())
+        assert (y[:bm] == 7.0).all() and (y[bm + taken:] == 7.0).all() and (y[:, O:] == 7.0).all()
+        return y[bm:bm + taken, :O]
+    many = products(x, 128, 120)
+    for bm, taken in ((16, 16), (16, 3), (128, 33), (128, 1)):
+        assert torch.equal(products(x, bm, taken), many[:taken])
+    rows = x[torch.arange(120, device="cuda") // 2].double()
+    a, b = rows @ wa[2].double().T, rows @ wb[2].double().T
+    sum_a, sum_b = rows.abs() @ wa[2].double().abs().T, rows.abs() @ wb[2].double().abs().T
+    e = I * 2.0 ** -24
+    if gated:
+        w = weight[:, None].double()
+        a, b, sum_a, sum_b = w * a, w * b, w * sum_a, w * sum_b
+        want = a * torch.sigmoid(a) * b
+        bound = 1.1 * (e * sum_a * (b.abs() + e * sum_b) + e * sum_b * a.abs()) + 16 * 2.0 ** -24 * (a * b).abs()
+    else:
+        want, bound = a, e * sum_a
+    assert ((many.double() - want).abs() <= bound + 1e-30).all()
+    if not gated:
+        odd = x.clone()
+        odd[0, 1], odd[1, 2], odd[2, 3] = float("inf"), float("nan"), 3.4e38
+        got, want = products(odd, 16, 8), odd[torch.arange(8, device="cuda") // 2].double() @ wa[2].double().T
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf()[:2], want.isinf()[:2])
+
+
 def test_a_rows_experts_do_not_depend_on_its_neighbours():
     """32-bit: the same row alone and among 200 others gives the same bits."""
     from gibbs_amd import Engine
