@@ -12,7 +12,9 @@
 // A wave and tile at head size 64 is 128 matrix instructions of 32 cycles, and about as long again of exponentials and
 // of waits that nothing covers: a prompt of some thousand rows has one wave for each SIMD.  16 heads over 8 of the cache, head
 // size 64 (in brackets attention_plain.hip, whose lanes read a key each, uncoalesced, and every key once a row): 1,194 rows of a
-// prompt 112 us (1,348), 4,096 rows 646 us (11,963; 52 TFLOP/s), 64 rows after 1,000 keys 66 us (518).
+// prompt 112 us (1,348), 4,096 rows 646 us (11,963; 52 TFLOP/s), 64 rows after 1,000 keys 66 us (518).  Values of twice the
+// keys' size (VT): the same walk with V in pieces and pages of its own; 20 rows behind 200 keys, 8 heads over 2 of 64 and 128, 33 us (292 in the plain
+// kernel).
 #include "common.h"
 
 namespace {
@@ -49,19 +51,21 @@ struct F32Args {
   int wide_out;         // rows of `out` take 16-byte stores
 };
 
-// DT: head size = 16 * DT.  POW2: the page size is a power of two (a shift instead of a division, eight a tile).
-template <int DT, bool POW2>
+// DT: head size = 16 * DT, of values 16 * VT.  POW2: the page size is a power of two (a shift instead of a division, eight a tile).
+template <int DT, bool POW2, int VT>
 __global__ __launch_bounds__(THREADS) void attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ kpages,
                                                                 const float* __restrict__ vpages, float* __restrict__ out, F32Args a) {
-  constexpr int HD = 16 * DT;
-  constexpr int VEC = DT % 4 == 0 ? 4 : DT % 2 == 0 ? 2 : 1;
+  constexpr int HD = 16 * DT, VD = 16 * VT;
+  constexpr int VEC = VT % 4 == 0 ? 4 : VT % 2 == 0 ? 2 : 1;
   typedef __attribute__((__vector_size__(VEC * sizeof(float)))) float floatv;
   constexpr int LD = HD + 4;                                // 16 lanes on 16 rows with 16 bytes each: all 64 banks (head size 64)
-  constexpr int PER_KEY = HD / 4;                           // 16-byte chunks of a key
-  constexpr int CHUNKS = KEYS * PER_KEY / THREADS;          // of K (and of V) per thread and tile: DT
-  static_assert(CHUNKS * THREADS == KEYS * PER_KEY, "whole chunks");
+  constexpr int LDV = VD + 4;
+  constexpr int PER_KEY = HD / 4, PER_VALUE = VD / 4;       // 16-byte chunks of a key and of its value
+  constexpr int CHUNKS = KEYS * PER_KEY / THREADS;          // of K per thread and tile: DT
+  constexpr int VCHUNKS = KEYS * PER_VALUE / THREADS;       // of V: VT
+  static_assert(CHUNKS * THREADS == KEYS * PER_KEY && VCHUNKS * THREADS == KEYS * PER_VALUE, "whole chunks");
   __shared__ __attribute__((aligned(16))) float sK[KEYS][LD];
-  __shared__ __attribute__((aligned(16))) float sV[KEYS][LD];
+  __shared__ __attribute__((aligned(16))) float sV[KEYS][LDV];
 
   const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
   // Which request and which of its tiles: 64 requests at a time, a lane each (one after the other, each a wait for memory, 256 requests of one
@@ -105,38 +109,53 @@ __global__ __launch_bounds__(THREADS) void attention_f32_kernel(const float* __r
   const int wave_first = p0 + min(wave * 16, rows_here - 1), wave_last = p0 + min(wave * 16 + 15, rows_here - 1);
   const int wave_lo = first_of(wave_first), wave_lo_last = first_of(wave_last);   // (first_of never falls)
 
-  floatx4 o[DT];
+  floatx4 o[VT];
 #pragma unroll
-  for (int t = 0; t < DT; ++t) o[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < VT; ++t) o[t] = floatx4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
 
-  // chunk i of this thread: key (tid + 256 i) / PER_KEY of the tile; keys past the last one repeat it, and are zero in LDS
-  int page[CHUNKS];
-  floatx4 kreg[CHUNKS], vreg[CHUNKS];
+  // chunk i of this thread: key (tid + 256 i) / PER_KEY of the tile (of V: / PER_VALUE); keys past the last one repeat it, and are zero in LDS
+  int page[CHUNKS], vpage[VT == DT ? 1 : VCHUNKS];
+  floatx4 kreg[CHUNKS], vreg[VCHUNKS];
   auto key_of = [&](int kt, int i) { return kt * KEYS + (tid + i * THREADS) / PER_KEY; };
+  auto value_of = [&](int kt, int i) { return kt * KEYS + (tid + i * THREADS) / PER_VALUE; };
   auto page_of = [&](int key) { return POW2 ? key >> a.page_shift : key / a.page_size; };
   auto ask_pages = [&](int kt) {
 #pragma unroll
     for (int i = 0; i < CHUNKS; ++i) page[i] = table[page_of(min(key_of(kt, i), last_pos))];
+    if constexpr (VT != DT) {
+#pragma unroll
+      for (int i = 0; i < VCHUNKS; ++i) vpage[i] = table[page_of(min(value_of(kt, i), last_pos))];
+    }
+  };
+  // the place of key `key` in its page `pg` of the pool (never outside the pool)
+  auto slot_of = [&](int pg, int key) {
+    return ((size_t)min(max(pg, 0), a.num_pages - 1) * a.nkv + kvh) * a.page_size + (key - page_of(key) * a.page_size);
   };
   auto ask_tile = [&](int kt) {
 #pragma unroll
     for (int i = 0; i < CHUNKS; ++i) {
-      const int key = min(key_of(kt, i), last_pos);
-      const int pg = min(max(page[i], 0), a.num_pages - 1);   // never read outside the pool
-      const size_t off = (((size_t)pg * a.nkv + kvh) * a.page_size + (key - page_of(key) * a.page_size)) * HD + (tid + i * THREADS) % PER_KEY * 4;
+      const size_t off = slot_of(page[i], min(key_of(kt, i), last_pos)) * HD + (tid + i * THREADS) % PER_KEY * 4;
       kreg[i] = *(const floatx4*)(kpages + off);
-      vreg[i] = *(const floatx4*)(vpages + off);
+      if constexpr (VT == DT) vreg[i] = *(const floatx4*)(vpages + off);
+    }
+    if constexpr (VT != DT) {
+#pragma unroll
+      for (int i = 0; i < VCHUNKS; ++i)
+        vreg[i] = *(const floatx4*)(vpages + slot_of(vpage[i], min(value_of(kt, i), last_pos)) * VD + (tid + i * THREADS) % PER_VALUE * 4);
     }
   };
   auto store_tile = [&](int kt) {
+    const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < CHUNKS; ++i) {
       const int c = tid + i * THREADS;
-      const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
-      const bool there = key_of(kt, i) <= last_pos;
-      *(floatx4*)&sK[c / PER_KEY][c % PER_KEY * 4] = there ? kreg[i] : zero;
-      *(floatx4*)&sV[c / PER_KEY][c % PER_KEY * 4] = there ? vreg[i] : zero;
+      *(floatx4*)&sK[c / PER_KEY][c % PER_KEY * 4] = key_of(kt, i) <= last_pos ? kreg[i] : zero;
+    }
+#pragma unroll
+    for (int i = 0; i < VCHUNKS; ++i) {
+      const int c = tid + i * THREADS;
+      *(floatx4*)&sV[c / PER_VALUE][c % PER_VALUE * 4] = value_of(kt, i) <= last_pos ? vreg[i] : zero;
     }
   };
 
@@ -189,7 +208,7 @@ __global__ __launch_bounds__(THREADS) void attention_f32_kernel(const float* __r
       float probe = 0.f;
       each([&](float s, int key) { return key <= pos_row && key >= lo_row ? s : -INFINITY; });
 #pragma unroll
-      for (int s = 0; s < DT; ++s)
+      for (int s = 0; s < VT; ++s)
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           const floatx4 v = *(const floatx4*)&sV[c * 16 + lr][s * 16 + g * 4];
@@ -217,7 +236,7 @@ __global__ __launch_bounds__(THREADS) void attention_f32_kernel(const float* __r
       }
     if (__builtin_amdgcn_ballot_w64(keep != 1.f) != 0) {
 #pragma unroll
-      for (int t = 0; t < DT; ++t)
+      for (int t = 0; t < VT; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[t][i] *= keep;
     }
@@ -228,7 +247,7 @@ __global__ __launch_bounds__(THREADS) void attention_f32_kernel(const float* __r
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int u = 0; u < DT / VEC; ++u) {
+          for (int u = 0; u < VT / VEC; ++u) {
             const floatv v = *(const floatv*)&sV[c * 16 + g * 4 + i][u * 16 * VEC + lr * VEC];
 #pragma unroll
             for (int e = 0; e < VEC; ++e) o[u * VEC + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e], s4[c][i], o[u * VEC + e], 0, 0, 0);
@@ -245,7 +264,7 @@ __global__ __launch_bounds__(THREADS) void attention_f32_kernel(const float* __r
             const float w = __shfl(s4[c][i], gg * 16 + lr, WAVE);
             if (key0 + row > pos_row || key0 + row < lo_row) continue;
 #pragma unroll
-            for (int t = 0; t < DT; ++t)
+            for (int t = 0; t < VT; ++t)
 #pragma unroll
               for (int k = 0; k < 4; ++k) o[t][k] = fmaf(w, sV[row][t / VEC * 16 * VEC + (g * 4 + k) * VEC + t % VEC], o[t][k]);
           }
@@ -256,9 +275,9 @@ __global__ __launch_bounds__(THREADS) void attention_f32_kernel(const float* __r
   if (wave * 16 + lr >= rows_here) return;
   if (a.sink) l += expf(a.sink[head] - m);
   const float inv = 1.0f / l;
-  float* dst = out + (size_t)(n0 + my_row) * a.ldo + (size_t)head * HD;
+  float* dst = out + (size_t)(n0 + my_row) * a.ldo + (size_t)head * VD;
 #pragma unroll
-  for (int u = 0; u < DT / VEC; ++u)
+  for (int u = 0; u < VT / VEC; ++u)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       float* to = dst + u * 16 * VEC + (g * 4 + i) * VEC;
@@ -275,18 +294,21 @@ __global__ __launch_bounds__(THREADS) void attention_f32_kernel(const float* __r
 }
 }  // namespace
 
+GIBBS_EXPORT int gibbs_attention_f32_takes(int hd, int vd) { return hd >= 16 && hd <= 128 && hd % 16 == 0 && (vd == hd || (vd == 2 * hd && hd <= 64)); }
+
 // q: float32 rows (stride ldq), rows of request r are cu[r] .. cu[r + 1] at positions ctx[r] ..; pages [num_pages, nkv, page_size,
-// hd] (keys and values of one head size, a multiple of 16 up to 128); out: row stride ldo.  cu may start above 0 (the requests of a
+// hd] and [num_pages, nkv, page_size, vd] (keys of a multiple of 16 up to 128, values of that size or, for keys up to 64, of twice that); out: row stride ldo.  cu may start above 0 (the requests of a
 // step from some request on); n_rows counts the rows from there.  The other operands are gibbs_attention_plain_masked's.
-GIBBS_EXPORT int gibbs_attention_f32(const void* q, const void* kpages, const void* vpages, void* out, const int* cu, const int* ctx,
+GIBBS_EXPORT int gibbs_attention_f32_values(const void* q, const void* kpages, const void* vpages, void* out, const int* cu, const int* ctx,
                                      const int* table, int n_req, int max_pages, int page_size, int num_pages, int n_rows, int nh,
-                                     int nkv, int hd, long ldq, long ldo, float scale, int window, const float* slopes, const float* bias,
+                                     int nkv, int hd, int vd, long ldq, long ldo, float scale, int window, const float* slopes, const float* bias,
                                      int bias_len, const float* sink, int chunk, float softcap, hipStream_t stream) {
   GIBBS_REQUIRE(n_rows >= 0 && n_req >= 0 && nh > 0 && nkv > 0 && nh % nkv == 0 && nh <= 65535, "attention_f32: bad sizes rows=%d requests=%d heads=%d kv=%d",
                 n_rows, n_req, nh, nkv);
   GIBBS_REQUIRE(hd % 16 == 0 && hd >= 16 && hd <= 128, "attention_f32: head size %d must be a multiple of 16 up to 128", hd);
+  GIBBS_REQUIRE(gibbs_attention_f32_takes(hd, vd), "attention_f32: values of %d beside keys of %d", vd, hd);
   GIBBS_REQUIRE(ldq % 4 == 0 && ((uintptr_t)q | (uintptr_t)kpages | (uintptr_t)vpages) % 16 == 0, "attention_f32: rows must be 16-byte aligned");
-  GIBBS_REQUIRE(ldq >= (long)nh * hd && ldo >= (long)nh * hd, "attention_f32: row strides shorter than heads * hd");
+  GIBBS_REQUIRE(ldq >= (long)nh * hd && ldo >= (long)nh * vd, "attention_f32: row strides shorter than heads * hd");
   GIBBS_REQUIRE(page_size > 0 && max_pages > 0 && num_pages > 0 && window >= 0, "attention_f32: bad cache geometry");
   GIBBS_REQUIRE(!bias || bias_len > 0, "attention_f32: an empty table of score biases");
   GIBBS_REQUIRE(chunk >= 0 && !(chunk > 0 && window > 0) && softcap >= 0.f, "attention_f32: a window of %d with chunks of %d, scores capped at %g", window, chunk, softcap);
@@ -297,21 +319,30 @@ GIBBS_EXPORT int gibbs_attention_f32(const void* q, const void* kpages, const vo
   const dim3 grid(ceil_div(n_rows, ROWS) + n_req, nh);
   const float *qq = (const float*)q, *kk = (const float*)kpages, *vv = (const float*)vpages;
   float* oo = (float*)out;
-#define F32_ATTENTION(DT)                                                                                             \
+#define F32_ATTENTION(DT, VT)                                                                                         \
   do {                                                                                                                \
-    if (page_shift >= 0) attention_f32_kernel<DT, true><<<grid, THREADS, 0, stream>>>(qq, kk, vv, oo, a);              \
-    else attention_f32_kernel<DT, false><<<grid, THREADS, 0, stream>>>(qq, kk, vv, oo, a);                             \
+    if (page_shift >= 0) attention_f32_kernel<DT, true, VT><<<grid, THREADS, 0, stream>>>(qq, kk, vv, oo, a);          \
+    else attention_f32_kernel<DT, false, VT><<<grid, THREADS, 0, stream>>>(qq, kk, vv, oo, a);                         \
   } while (0)
+  const bool twice = vd != hd;
   switch (hd / 16) {
-    case 1: F32_ATTENTION(1); break;
-    case 2: F32_ATTENTION(2); break;
-    case 3: F32_ATTENTION(3); break;
-    case 4: F32_ATTENTION(4); break;
-    case 5: F32_ATTENTION(5); break;
-    case 6: F32_ATTENTION(6); break;
-    case 7: F32_ATTENTION(7); break;
-    default: F32_ATTENTION(8); break;
+    case 1: if (twice) F32_ATTENTION(1, 2); else F32_ATTENTION(1, 1); break;
+    case 2: if (twice) F32_ATTENTION(2, 4); else F32_ATTENTION(2, 2); break;
+    case 3: if (twice) F32_ATTENTION(3, 6); else F32_ATTENTION(3, 3); break;
+    case 4: if (twice) F32_ATTENTION(4, 8); else F32_ATTENTION(4, 4); break;
+    case 5: F32_ATTENTION(5, 5); break;
+    case 6: F32_ATTENTION(6, 6); break;
+    case 7: F32_ATTENTION(7, 7); break;
+    default: F32_ATTENTION(8, 8); break;
   }
 #undef F32_ATTENTION
   GIBBS_LAUNCH_STATUS("attention_f32");
+}
+
+GIBBS_EXPORT int gibbs_attention_f32(const void* q, const void* kpages, const void* vpages, void* out, const int* cu, const int* ctx,
+                                     const int* table, int n_req, int max_pages, int page_size, int num_pages, int n_rows, int nh,
+                                     int nkv, int hd, long ldq, long ldo, float scale, int window, const float* slopes, const float* bias,
+                                     int bias_len, const float* sink, int chunk, float softcap, hipStream_t stream) {
+  return gibbs_attention_f32_values(q, kpages, vpages, out, cu, ctx, table, n_req, max_pages, page_size, num_pages, n_rows, nh, nkv, hd, hd, ldq, ldo, scale,
+                                    window, slopes, bias, bias_len, sink, chunk, softcap, stream);
 }

@@ -36,6 +36,11 @@ int gibbs_attention_f32(const void* q, const void* kpages, const void* vpages, v
                         int n_req, int max_pages, int page_size, int num_pages, int n_rows, int nh, int nkv, int hd, long ldq, long ldo,
                         float scale, int window, const float* slopes, const float* bias, int bias_len, const float* sink, int chunk,
                         float softcap, hipStream_t stream);
+int gibbs_attention_f32_takes(int hd, int vd);
+int gibbs_attention_f32_values(const void* q, const void* kpages, const void* vpages, void* out, const int* cu, const int* ctx, const int* table,
+                               int n_req, int max_pages, int page_size, int num_pages, int n_rows, int nh, int nkv, int hd, int vd, long ldq, long ldo,
+                               float scale, int window, const float* slopes, const float* bias, int bias_len, const float* sink, int chunk,
+                               float softcap, hipStream_t stream);
 int gibbs_attention_plain_masked(const void* q, const void* kpages, const void* vpages, void* out, int dtype, const int* pos,
                                  const int* row_req, const int* table, int max_pages, int page_size, int num_pages, int n_rows,
                                  int nh, int nkv, int hd, int vd, long ldq, long ldo, float scale, int window, const float* slopes,

@@ -722,11 +722,11 @@ void* attend_prepared(Exec& e, const PagedAttention& t, void* raw, long ldq, lon
   } else if (fast_bf16 && a.max_q == 1 && t.hd % 8 == 0 && t.hd <= 256 && (!t.bias || matrix_sizes)) {
     decode_attention(e, t, raw, ldq, N, a.pos, a.row_req, att);
   } else {
-    // float32 rows of one head size take the matrix-core kernel, decoded tokens too: with one row of its 16 in use it still walks
+    // float32 rows of one head size, or with values of twice that, take the matrix-core kernel, decoded tokens too: with one row of its 16 in use it still walks
     // 1,000 keys in 60 us, and the kernel with a wave a row, whose lanes read a key each, in 360 (64 keys: 10 and 17 us)
-    if (e.p.dtype == GIBBS_F32 && matrix_sizes && t.vd == t.hd && ldq % 4 == 0 && ((uintptr_t)raw | (uintptr_t)t.kpages | (uintptr_t)t.vpages) % 16 == 0)
-      RUN(e, gibbs_attention_f32(raw, t.kpages, t.vpages, att, a.cu, a.ctx, table, a.n_req, width, t.page_size, t.num_pages, N, t.nh, t.nkv,
-                                 t.hd, ldq, ldo, t.scale, t.window, t.slopes, t.bias, t.bias_len, t.sink, t.chunk, t.softcap, a.stream));
+    if (e.p.dtype == GIBBS_F32 && gibbs_attention_f32_takes(t.hd, t.vd) && ldq % 4 == 0 && ((uintptr_t)raw | (uintptr_t)t.kpages | (uintptr_t)t.vpages) % 16 == 0)
+      RUN(e, gibbs_attention_f32_values(raw, t.kpages, t.vpages, att, a.cu, a.ctx, table, a.n_req, width, t.page_size, t.num_pages, N, t.nh, t.nkv,
+                                 t.hd, t.vd, ldq, ldo, t.scale, t.window, t.slopes, t.bias, t.bias_len, t.sink, t.chunk, t.softcap, a.stream));
     else
       RUN(e, gibbs_attention_plain_masked(raw, t.kpages, t.vpages, att, e.p.dtype, a.pos, a.row_req, table, width, t.page_size, t.num_pages,
                                           N, t.nh, t.nkv, t.hd, t.vd, ldq, ldo, t.scale, t.window, t.slopes, t.bias, t.bias_len, t.sink,

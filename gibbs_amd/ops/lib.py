@@ -69,6 +69,9 @@ _SIGNATURES = {
     "gibbs_attention_plain_masked": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int,
                                      c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_long, c_long, c_float, c_int, c_void_p,
                                      c_void_p, c_int, c_void_p, c_int, c_float, c_void_p],
+    "gibbs_attention_f32_values": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
+                                   c_int, c_int, c_int, c_int, c_long, c_long, c_float, c_int, c_void_p, c_void_p, c_int, c_void_p, c_int, c_float,
+                                   c_void_p],
     "gibbs_attention_f32": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                             c_int, c_int, c_int, c_long, c_long, c_float, c_int, c_void_p, c_void_p, c_int, c_void_p, c_int, c_float,
                             c_void_p],

@@ -539,6 +539,50 @@ def test_attention_float32_portions(nh, nkv, hd, page, extra):
         assert (want - got)[want.isfinite()].abs().max() <= 1e-4 * max(1.0, float(want[want.isfinite()].abs().max()))
 
 
+@pytest.mark.parametrize("nh,nkv,hd,page,extra", [
+    (4, 2, 64, 16, {}), (2, 1, 16, 8, {"window": 50}), (3, 1, 48, 7, {"chunk": 40}), (4, 4, 32, 32, {"softcap": 2.0, "sink": True}),
+    (2, 2, 64, 5, {"slopes": True, "bias": True}), (1, 1, 64, 16, {"window": 1})])
+def test_attention_float32_values_twice_as_wide_as_keys(nh, nkv, hd, page, extra):
+    """The portions, masks and bounds of the test above with values of 2 hd; a request's rows alone and among the others, the same bits."""
+    from gibbs_amd import ops
+    from gibbs_amd.ops.lib import call, ptr, stream
+    vd = 2 * hd
+    seq_lens, q_lens = [333, 9, 130, 77, 64, 128], [150, 9, 2, 1, 64, 63]
+    kp, _, table, _, _ = paged_setup(torch.float32, nkv, hd, page, seq_lens, 400, seed=11)
+    vp = rnd(kp.shape[0], nkv, page, vd, dtype=torch.float32, seed=12)
+    ctx = [s - q for s, q in zip(seq_lens, q_lens)]
+    cu = np.concatenate([[0], np.cumsum(q_lens)])
+    n, R = int(cu[-1]), len(q_lens)
+    q = rnd(n, nh * hd + 4, dtype=torch.float32, seed=9)
+    pos = i32([c + t for c, ql in zip(ctx, q_lens) for t in range(ql)])
+    row_req = i32([r for r, ql in enumerate(q_lens) for _ in range(ql)])
+    opt = dict(extra)
+    for name, shape in (("sink", (nh,)), ("slopes", (nh,)), ("bias", (19, nh))):
+        if name in opt:
+            opt[name] = rnd(*shape, dtype=torch.float32, seed=3)
+    bias = opt.get("bias")
+    cud, ctxd = i32(cu), i32(ctx)
+    def run(first, count):
+        got = torch.full((n, nh * vd + 1), 7.0, device="cuda")
+        call("gibbs_attention_f32_values", ptr(q), ptr(kp), ptr(vp), ptr(got), ptr(cud[first:]), ptr(ctxd[first:]), ptr(table[first:]), count, table.shape[1], page,
+             kp.shape[0], int(cu[first + count] - cu[first]), nh, nkv, hd, vd, q.stride(0), nh * vd + 1, float(hd ** -0.5), int(opt.get("window", 0)),
+             ptr(opt.get("slopes")), ptr(bias), 0 if bias is None else bias.shape[0], ptr(opt.get("sink")), int(opt.get("chunk", 0)),
+             float(opt.get("softcap", 0.0)), stream())
+        assert (got[:, -1] == 7.0).all() and (got[:int(cu[first])] == 7.0).all() and (got[int(cu[first + count]):] == 7.0).all()
+        return got[:, :-1]
+    for poisoned in (False, True):
+        if poisoned:
+            key = seq_lens[0] - 3        # a key that the first request's last three rows see
+            vp[int(table[0, key // page]), :, key % page] = float("inf")
+        want, got = ops.attention_plain(q, n, nh, nkv, hd, kp, vp, table, R, pos, row_req, hd ** -0.5, **opt), run(0, R)
+        finite = want.isfinite()
+        assert torch.equal(finite, got.isfinite())
+        assert (want - got)[finite].abs().max() <= 1e-4 * max(1.0, float(want[finite].abs().max()))
+        for r in range(R):
+            a, b = int(cu[r]), int(cu[r + 1])
+            assert torch.equal(torch.nan_to_num(run(r, 1)[a:b], nan=5.0), torch.nan_to_num(got[a:b], nan=5.0))
+
+
 def test_attention_float32_many_requests():
     """150 requests of 1 to 130 rows in one call: each one's rows are those of a call of its own, to the bit (the workgroups find their request among
     64 at a time)."""
