@@ -72,7 +72,7 @@ __global__ __launch_bounds__(256) void shortconv_kernel(
 // The same with 16 bytes of channels (8 bfloat16, 4 float32) per thread and the window kept in registers:
 // a prompt portion is a pass over 3 + 1 values per (row, channel), bound by memory traffic.
 // K is a template parameter (2..4, what LFM2 checkpoints use); other lengths take the kernel above.
-// (float32, 1,194 rows of 1,024 channels: 31.7 us a channel a thread, K loads and products a row; 5.0 us so.)
+// (float32, 1,194 rows of 1,024 channels: 31.7 us a channel a thread, K loads and products a row; 6.1 us so.)
 constexpr int TLV = 8;   // rows per tile (>= K - 1)
 constexpr int RU = 4;    // rows whose loads are in flight together
 
