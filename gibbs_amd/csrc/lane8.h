@@ -3,6 +3,7 @@
 // position encoding in that layout.
 #pragma once
 #include "common.h"
+#include <type_traits>
 
 constexpr int EPL = 8;  // head-dim elements per lane (16 bytes of bfloat16)
 
@@ -48,6 +49,84 @@ __device__ __forceinline__ float group_sum(float v) {
   if (LPK >= 16) v += dpp_move<0x140>(v); // row_mirror
   if (LPK >= 32) v += __shfl_xor(v, 16, WAVE);
   return v;
+}
+
+// The value of lane (lane ^ MASK), MASK 1, 2, 4 or 8, likewise without LDS.
+template <int MASK>
+__device__ __forceinline__ float lane_xor(float v) {
+  static_assert(MASK == 1 || MASK == 2 || MASK == 4 || MASK == 8, "inside a row of 16 lanes");
+  if (MASK == 1) return dpp_move<0xB1>(v);
+  if (MASK == 2) return dpp_move<0x4E>(v);
+  if (MASK == 4) return dpp_move<0x1B>(dpp_move<0x141>(v));   // (i -> 7 - i, then quad_perm [3,2,1,0]: i -> i ^ 7 ^ 3)
+  return dpp_move<0x128>(v);                                  // (row_ror:8)
+}
+// The sum of a head's squares with its 8 LPK elements 8 to a lane, to the bit as a wave with one element a lane makes it (lane l: the squares of
+// elements l and l + 64 in that order, then wave_sum): kernels of both layouts give a head the same norm.  Element 8 j + i is lane j's value
+// i, so wave_sum's halves, quarters and eighths are lanes, and what it adds last are the values inside a lane.  Every such step over lanes
+// halves the values that a lane still has instead of adding all of them twice (a + b and b + a are the same bits), so that 10 moves do for 8
+// values in 8 lanes where a sum of each lane's own total takes 3.
+template <int LPK>
+__device__ __forceinline__ float head_squares(const float* v, int lane) {
+  static_assert(LPK == 2 || LPK == 4 || LPK == 8 || LPK == 16, "heads of 16, 32, 64 or 128");
+  float s[8];
+  if constexpr (LPK == 16) {        // elements l and l + 64 lie 8 lanes apart: each of the two lanes takes four of the eight pairs
+    const bool low = (lane & 8) == 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float own = low ? v[i] : v[4 + i], got = lane_xor<8>(low ? v[4 + i] : v[i]);
+      const float first = low ? own : got, second = low ? got : own;
+      s[i] = fmaf(second, second, fmaf(first, first, 0.f));
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s[i] = fmaf(v[i], v[i], 0.f);
+  }
+  // a lane with the bit set goes on with the upper half of its N values
+  auto halve = [&](auto mask, auto count) {
+    constexpr int M = decltype(mask)::value, H = decltype(count)::value / 2;
+    const bool low = (lane & M) == 0;
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      const float give = low ? s[H + i] : s[i], own = low ? s[i] : s[H + i];
+      s[i] = own + lane_xor<M>(give);
+    }
+  };
+  auto add = [&](auto mask, auto count) {
+#pragma unroll
+    for (int i = 0; i < decltype(count)::value; ++i) s[i] += lane_xor<decltype(mask)::value>(s[i]);
+  };
+  using std::integral_constant;
+  integral_constant<int, 1> one;
+  integral_constant<int, 2> two;
+  integral_constant<int, 4> four;
+  integral_constant<int, 8> eight;
+  if constexpr (LPK == 16) {
+    halve(four, four);
+    halve(two, two);
+    add(one, one);
+    add(eight, one);      // (the values of a lane: those of 4, 2 and 1 apart, which the halvings put into lanes)
+    add(four, one);
+    add(two, one);
+    return s[0];
+  } else if constexpr (LPK == 8) {
+    halve(four, eight);
+    halve(two, four);
+    halve(one, two);
+    add(four, one);
+    add(two, one);
+    add(one, one);
+    return s[0];
+  } else if constexpr (LPK == 4) {
+    halve(two, eight);
+    halve(one, four);
+    add(two, two);
+    add(one, two);
+    return s[0] + s[1];
+  } else {
+    halve(one, eight);
+    add(one, four);
+    return (s[0] + s[2]) + (s[1] + s[3]);
+  }
 }
 
 __device__ __forceinline__ bool finite(float x) { return x * 0.f == 0.f; }

@@ -46,8 +46,9 @@ __global__ __launch_bounds__(64) void qk_unit_kv_kernel(T* __restrict__ rows, lo
   }
 }
 
-// The same for bfloat16 heads of 8 LPK channels in whole 16 bytes: a workgroup a row, LPK lanes a head of q or k and vd / 8 a head of v, 8 channels each
-// (a wave a head, 2,048 rows of 32 heads over 8 of 64: 24.5 us; 9.0 us so).
+// The same for bfloat16 heads of 8 LPK channels in whole 16 bytes: a workgroup a row, LPK lanes a head of q or k and vd / 8 a head of v, 8 channels each,
+// the norms the same bits (a wave a head, 2,048 rows of 32 heads over 8 of 64: 24.5 us; 9.4 us so.  The order of the squares' sum is 0.4 us of that, and 0.6 of
+// 5.4 us at 8 rows).
 template <int LPK>
 __global__ void qk_unit_kv_vec8_kernel(bf16* __restrict__ rows, long ld, bf16* __restrict__ kpages, bf16* __restrict__ vpages, const int* __restrict__ pos,
                                        const int* __restrict__ row_req, const int* __restrict__ table, int max_pages, int page_size, int num_pages, int nh,
@@ -65,11 +66,9 @@ __global__ void qk_unit_kv_vec8_kernel(bf16* __restrict__ rows, long ld, bf16* _
       continue;
     }
     const int head = i / LPK, e = i % LPK * 8;
-    float v[8], ss = 0.f;
+    float v[8];
     unpack8(*(const uint4*)(row + (size_t)i * 8), v);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) ss = fmaf(v[k], v[k], ss);
-    float scale = unit ? 1.0f / sqrtf(group_sum<LPK>(ss) / (float)norm_dim + eps) : 1.0f;
+    float scale = unit ? 1.0f / sqrtf(head_squares<LPK>(v, threadIdx.x) / (float)norm_dim + eps) : 1.0f;
     if (head < nh && temp_every > 0) scale *= temp;
 #pragma unroll
     for (int k = 0; k < 8; ++k) v[k] *= scale;

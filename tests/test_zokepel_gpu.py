@@ -973,3 +973,29 @@ def test_token_shift_in_whole_16_bytes_like_float32(lens, W, mixes):
         call("gibbs_token_shift", ptr(x), code, ptr(mu), mixes, ptr(state), W, ptr(req), ptr(cu), ptr(slot), ptr(out), n, len(lens), W, 1, int(n == len(lens)), stream())
         outs.append((out, state))
     assert torch.equal(outs[0][0].bfloat16(), outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("hd", [16, 32, 64, 128])
+@pytest.mark.parametrize("unit,every", [(True, 7), (True, 0), (False, 3)])
+def test_unit_heads_in_whole_16_bytes_are_the_general_kernels(hd, unit, every):
+    """Rows of whole 16 bytes and the same rows two values further apart, which take the kernel with a wave a head: rows and pages are the same bits, with an infinity
+    and a NaN among them.  (A norm that is one float32 step off moves one of some 2^16 bfloat16 results, so there are over a million.)"""
+    from gibbs_amd.ops.lib import call, ptr, stream
+    g = torch.Generator(device="cuda").manual_seed(hd)
+    n, nh, nkv, vd, page_size, pages = 1031 * 128 // hd, 8, 3, 24, 16, 600
+    W = (nh + nkv) * hd + nkv * vd
+    x = torch.randn((n, W), generator=g, device="cuda").bfloat16()
+    x[3, 1], x[9, nh * hd + 5] = float("inf"), float("nan")
+    pos = torch.arange(n, dtype=torch.int32, device="cuda")
+    req = torch.zeros(n, dtype=torch.int32, device="cuda")
+    table = torch.randperm(pages, generator=g, device="cuda").to(torch.int32)[:520].reshape(1, -1).contiguous()
+    outs = []
+    for ld in (W, W + 2):
+        rows = torch.zeros((n, ld), dtype=torch.bfloat16, device="cuda")
+        rows[:, :W] = x
+        kp, vp = (torch.zeros((pages, nkv, page_size, d), dtype=torch.bfloat16, device="cuda") for d in (hd, vd))
+        call("gibbs_qk_unit_kv", ptr(rows), ld, ptr(kp), ptr(vp), 1, ptr(pos), ptr(req), ptr(table), 520, page_size, pages, n, nh, nkv, hd, vd, 1e-6, int(unit),
+             hd - 3, 0.1, every, stream())
+        outs.append([t.contiguous().nan_to_num(nan=5.0, posinf=7.0, neginf=-7.0) for t in (rows[:, :W], kp, vp)])
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
