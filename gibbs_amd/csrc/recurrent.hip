@@ -52,17 +52,23 @@ __global__ void causal_conv_silu_kernel(const T* __restrict__ in, long ld, const
 
 // The same for bfloat16 inputs whose channels come in whole groups of 8: a thread takes 8 neighbouring channels with 16-byte loads, of
 // CONV_RUN rows one behind the other, whose inputs it holds in registers (a row a thread reads K rows for each it writes: 2,048 rows of
-// 6,144 channels, K = 4, 30 us with a kernel of 25 us for the unit vectors behind it; 25 us so with them, half of it exponentials).  A workgroup is 64 lanes of channels by CONV_ROWS such runs; the taps of its 512
+// 6,144 channels, K = 4, 30 us with a kernel of 25 us for the unit vectors behind it; 26 us so with them, half of it exponentials, one the
+// order of the squares' sum).  A workgroup is 64 lanes of channels by CONV_ROWS such runs; the taps of its 512
 // channels, one contiguous stretch of the [C, K] table, come through LDS once (each thread's 8 K taps a word further along, so that the lanes
 // read different banks) instead of as 8 K scattered words per thread.  Sums in ascending j, as above.
 // KT: K, as many rows as that in registers; 0: any K, a row at a time.
 // unit.D > 0: channels 0 .. 2 unit.G unit.D are heads of unit.D that are made unit vectors, x / sqrt(sum x^2 + eps), those of the first half
-// times q_scale, in rows from unit.first on (what the delta rule reads; a head is unit.D / 8 neighbouring lanes).
+// times q_scale, in rows from unit.first on (what the delta rule reads, to the bit as delta_prep_kernel makes them; a head is unit.D / 8
+// neighbouring lanes).
 constexpr int CONV_ROWS = 4, CONV_LANES = 64, CONV_RUN = 4;
 struct ConvUnit {
   int G, D, first;
   float q_scale, eps;
 };
+__device__ __forceinline__ float lanes_squares(const float* v, int lanes) {
+  const int lane = threadIdx.x % WAVE;
+  return lanes == 16 ? head_squares<16>(v, lane) : (lanes == 8 ? head_squares<8>(v, lane) : (lanes == 4 ? head_squares<4>(v, lane) : head_squares<2>(v, lane)));
+}
 __device__ __forceinline__ float lanes_sum(float v, int lanes) {
   return lanes == 16 ? group_sum<16>(v) : (lanes == 8 ? group_sum<8>(v) : (lanes == 4 ? group_sum<4>(v) : group_sum<2>(v)));
 }
@@ -140,10 +146,7 @@ __global__ __launch_bounds__(CONV_ROWS * CONV_LANES) void causal_conv_vec8_kerne
       if (residual) acc[i] += own[i];
     }
     if (unit.D > 0 && n >= unit.first) {
-      float sum = 0.f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) sum = fmaf(acc[i], acc[i], sum);
-      sum = lanes_sum(sum, unit.D / 8);
+      const float sum = lanes_squares(acc, unit.D / 8);
       const float scale = (c < unit.G * unit.D ? unit.q_scale : 1.0f) / sqrtf(sum + unit.eps);
       if (c < 2 * unit.G * unit.D) {
 #pragma unroll

@@ -999,3 +999,32 @@ def test_unit_heads_in_whole_16_bytes_are_the_general_kernels(hd, unit, every):
         outs.append([t.contiguous().nan_to_num(nan=5.0, posinf=7.0, neginf=-7.0) for t in (rows[:, :W], kp, vp)])
     for a, b in zip(*outs):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("lens", [[64], [3, 1, 2, 1, 300, 1, 210], [1] * 515])
+@pytest.mark.parametrize("K,G,D,V", [(4, 2, 128, 40), (2, 3, 16, 8), (3, 1, 64, 24), (5, 2, 32, 72)])
+def test_delta_convolution_is_the_convolution_and_then_the_unit_vectors(lens, K, G, D, V):
+    """One kernel against the two that it stands for, whose results a row's do not differ from whichever way a step takes: rows and states to the bit, with
+    an infinity, a NaN and a head of zeros among the rows; 512 rows and more (four a thread) of a request each, which move all their states on, too."""
+    from gibbs_amd import ops
+    from gibbs_amd.ops.lib import call, ptr, stream
+    g = torch.Generator(device="cuda").manual_seed(D)
+    N, C, H = sum(lens), 2 * G * D + V, 2 * G
+    x = torch.randn((N, C), generator=g, device="cuda").bfloat16()
+    x[1, 2], x[2, 3], x[7:14, :D] = float("inf"), float("nan"), 0.0
+    taps = torch.randn((C, K), generator=g, device="cuda")
+    state = torch.randn((len(lens) + 1, K - 1, C), generator=g, device="cuda")
+    cu = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32, device="cuda")
+    row_req = torch.repeat_interleave(torch.arange(len(lens), device="cuda"), torch.tensor(lens, device="cuda")).to(torch.int32)
+    slot = torch.arange(1, len(lens) + 1, dtype=torch.int32, device="cuda").flip(0).contiguous()
+    first, other = (3 if len(lens) > 4 else 0), state.clone()
+    got = ops.delta_conv(x, taps, state, row_req, cu, slot, G, D, 0.25, 1e-6, first)
+    want = ops.causal_conv_silu(x, taps, other, row_req, cu, slot)
+    rest, m = want[first:], N - first
+    raw = torch.zeros((m, 2 * H), dtype=torch.bfloat16, device="cuda")
+    gates = torch.zeros(H, device="cuda")
+    beta, decay = torch.empty((m, H), device="cuda"), torch.empty((m, H), device="cuda")
+    call("gibbs_delta_prep", ptr(rest), ptr(rest[:, G * D:]), C, ptr(raw), ptr(raw[:, H:]), 2 * H, 1, None, ptr(gates), ptr(gates), ptr(beta), ptr(decay), m, G, H, D,
+         0.25, 1e-6, stream())
+    for a, b in ((got, want), (state, other)):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(nan=7.0), b.nan_to_num(nan=7.0))
