@@ -69,9 +69,6 @@ __device__ __forceinline__ float lanes_squares(const float* v, int lanes) {
   const int lane = threadIdx.x % WAVE;
   return lanes == 16 ? head_squares<16>(v, lane) : (lanes == 8 ? head_squares<8>(v, lane) : (lanes == 4 ? head_squares<4>(v, lane) : head_squares<2>(v, lane)));
 }
-__device__ __forceinline__ float lanes_sum(float v, int lanes) {
-  return lanes == 16 ? group_sum<16>(v) : (lanes == 8 ? group_sum<8>(v) : (lanes == 4 ? group_sum<4>(v) : group_sum<2>(v)));
-}
 template <typename TO, int KT>
 __global__ __launch_bounds__(CONV_ROWS * CONV_LANES) void causal_conv_vec8_kernel(
     const bf16* __restrict__ in, long ld, const float* __restrict__ taps, const float* __restrict__ bias, float* __restrict__ state,
@@ -483,7 +480,8 @@ __global__ __launch_bounds__(64) void head_norm_gate_kernel(const float* __restr
   }
 }
 // The same for bfloat16 results and heads of 16, 32, 64 or 128 values in whole 16 bytes: V / 8 neighbouring lanes a head, 8 values each, so that
-// a wave has 4 to 32 heads on their way (a wave a head, 2,048 rows of 16 heads of 128: 16.4 us for 33 MB; 10.4 us so).
+// a wave has 4 to 32 heads on their way (a wave a head, 2,048 rows of 16 heads of 128: 16.4 us for 33 MB; 10.9 us so, 0.5 of them
+// for the order of the squares' sum, which is the other kernel's).
 __global__ __launch_bounds__(256) void head_norm_gate_vec8_kernel(const float* __restrict__ o, const float* __restrict__ gain, int gain_len,
                                                                   const bf16* __restrict__ gate, long ld_gate, bf16* __restrict__ y, long heads, int H, int V,
                                                                   float eps, int act) {
@@ -494,10 +492,7 @@ __global__ __launch_bounds__(256) void head_norm_gate_vec8_kernel(const float* _
   const float* row = o + m * V + j;
   const float4 a = *(const float4*)row, b = *(const float4*)(row + 4);
   const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-  float ss = 0.f;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) ss = fmaf(v[k], v[k], ss);
-  const float inv = 1.0f / sqrtf(lanes_sum(ss, lanes) / (float)V + eps);
+  const float inv = 1.0f / sqrtf(lanes_squares(v, lanes) / (float)V + eps);
   const float4 ga = *(const float4*)(gain + c % gain_len), gb = *(const float4*)(gain + c % gain_len + 4);
   const float gv[8] = {ga.x, ga.y, ga.z, ga.w, gb.x, gb.y, gb.z, gb.w};
   float z[8], out[8];

@@ -1028,3 +1028,22 @@ def test_delta_convolution_is_the_convolution_and_then_the_unit_vectors(lens, K,
          0.25, 1e-6, stream())
     for a, b in ((got, want), (state, other)):
         assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(nan=7.0), b.nan_to_num(nan=7.0))
+
+
+@pytest.mark.parametrize("V", [16, 32, 64, 128])
+@pytest.mark.parametrize("gated", [False, True])
+def test_head_norm_in_whole_16_bytes_is_the_general_kernels(V, gated):
+    """Results in whole 16 bytes and the same results one value further on, which take the kernel with a wave a head: the same bits, with an infinity, a NaN and a
+    head of zeros.  (Over a million results: a norm that is one float32 step off moves one of some 2^16.)"""
+    from gibbs_amd.ops.lib import call, ptr, stream
+    g = torch.Generator(device="cuda").manual_seed(V)
+    H, n = 8, 1031 * 128 // V
+    o = torch.randn((n, H * V), generator=g, device="cuda")
+    o[3, 1], o[9, V + 5], o[11, :V] = float("inf"), float("nan"), 0.0
+    gain, gate = torch.randn(V, generator=g, device="cuda"), torch.randn((n, H * V), generator=g, device="cuda").bfloat16()
+    outs = []
+    for shift in (0, 1):
+        y = torch.zeros(n * H * V + 8, dtype=torch.bfloat16, device="cuda")[shift:shift + n * H * V]
+        call("gibbs_head_norm_gate", ptr(o), ptr(gain), V, ptr(gate) if gated else None, H * V if gated else 0, ptr(y), 1, n, H, V, 1e-6, 1, stream())
+        outs.append(y.clone())
+    assert torch.equal(outs[0].isnan(), outs[1].isnan()) and torch.equal(outs[0].nan_to_num(nan=7.0), outs[1].nan_to_num(nan=7.0))
