@@ -54,6 +54,67 @@ __device__ __forceinline__ void split8(f32x4 x, f32x4 y, bf16x8* p) {
 constexpr int F32_PRODUCTS = 6;
 __device__ constexpr int F32_PART[F32_PRODUCTS][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
 
+// One wave's stretch first .. last of a product of 16 FO rows of W with 16 FN of X, straight from memory into the operands' registers, where they are
+// split: lane (g, c) reads rows c of wp's and xp's blocks of 16, k 8 g .. 8 g + 7 of a block of 32 (rows of whole 16 bytes, I of them at least 4).
+// Four blocks are on their way, and a block is split as soon as it is there (8 rows x 1,024 features, inner size 1,024: 5.6 us; 6.3
+// where the first use waited for all loads).
+template <int FO, int FN>
+__device__ __forceinline__ void f32_stretch(const float* const (&wp)[FO], const float* const (&xp)[FN], int first, int last, int I, int g, f32x4 (&acc)[FO][FN]) {
+  constexpr int SETS = 4;
+  f32x4 fw[SETS][2][FO], fx[SETS][2][FN];
+  // (k beyond the matrix: its last four again, and X's made zero when they are used)
+  auto ask = [&](int set, int k0) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const int k = min(k0 + 8 * g + 4 * half, I - 4);
+#pragma unroll
+      for (int i = 0; i < FO; ++i) fw[set][half][i] = *(const f32x4*)(wp[i] + k);
+#pragma unroll
+      for (int i = 0; i < FN; ++i) fx[set][half][i] = *(const f32x4*)(xp[i] + k);
+    }
+  };
+  auto use = [&](int set, int k0) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const uint32_t keep = (uint32_t)((k0 + 8 * g + 4 * half - I) >> 31);
+#pragma unroll
+      for (int i = 0; i < FN; ++i) fx[set][half][i] = __builtin_bit_cast(f32x4, __builtin_bit_cast(u32x4, fx[set][half][i]) & keep);
+    }
+    bf16x8 pw[FO][3], px[FN][3];
+#pragma unroll
+    for (int i = 0; i < FO; ++i) split8(fw[set][0][i], fw[set][1][i], pw[i]);
+#pragma unroll
+    for (int i = 0; i < FN; ++i) split8(fx[set][0][i], fx[set][1][i], px[i]);
+#pragma unroll
+    for (int p = 0; p < F32_PRODUCTS; ++p)
+#pragma unroll
+      for (int i = 0; i < FO; ++i)
+#pragma unroll
+        for (int h = 0; h < FN; ++h) acc[i][h] = mfma_bf16(pw[i][F32_PART[p][0]], px[h][F32_PART[p][1]], acc[i][h]);
+  };
+  // (the first loads stand behind no branch, or the first block's use would wait for all of them: blocks behind a wave's last are that one again)
+  if (first < last) {
+    const int end = (last - first + 31) / 32 * 32 + first - 32;      // the wave's last block
+#pragma unroll
+    for (int s = 0; s < SETS; ++s) ask(s, min(first + 32 * s, end));
+    int k0 = first;
+    for (; k0 + 32 * (2 * SETS - 1) <= end; k0 += 32 * SETS) {
+#pragma unroll
+      for (int s = 0; s < SETS; ++s) {
+        __builtin_amdgcn_sched_barrier(0);
+        use(s, k0 + 32 * s);
+        ask(s, k0 + 32 * (s + SETS));
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < 2 * SETS - 1; ++s) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (k0 + 32 * s <= end) use(s % SETS, k0 + 32 * s);
+      if (s < SETS - 1 && k0 + 32 * (s + SETS) <= end) ask(s, k0 + 32 * (s + SETS));
+    }
+  }
+}
+
 __device__ __forceinline__ bool wants_again(float x) { return !(fabsf(x) <= 3.4028234e38f) || (x != 0.f && fabsf(x) < 0x1p-100f); }
 // One element in plain float32 (a sum that is NaN stays NaN).
 __device__ __forceinline__ float again(const float* a, const float* w, int I) {

@@ -149,15 +149,12 @@ __global__ __launch_bounds__(64 * WO * WN, OCC) void gemm_f32_tile_kernel(const 
     }
 }
 
-// Few rows or few tiles: a workgroup takes 16 FO features x 16 FN rows and its eight waves a stretch of k each, straight from
-// memory into the operands' registers, where they are split (no barrier before the sums meet in LDS).  Bound by the stream of
-// W (one row group) or by what comes through L2.  Four blocks of 32 k are on their way, and a block is split as soon as it is there (8 rows
-// x 1,024 features, inner size 1,024: 5.6 us; 6.3 where the first use waited for all loads).
+// Few rows or few tiles: a workgroup takes 16 FO features x 16 FN rows and its eight waves a stretch of k each (f32_stretch; no barrier before
+// the sums meet in LDS).  Bound by the stream of W (one row group) or by what comes through L2.
 template <int FO, int FN>
 __global__ __launch_bounds__(512) void gemm_f32_split_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                              float* __restrict__ C, int N, int O, int I, long lda, long ldw,
                                                              long ldc, int wide) {
-  constexpr int SETS = 4;
   __shared__ __attribute__((aligned(16))) f32x4 s_sum[F32_SEGMENTS][FO * FN][WAVE];
   const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), g = lane / 16, c = lane % 16;
   const int o0 = blockIdx.x * 16 * FO, n0 = blockIdx.y * 16 * FN;
@@ -169,59 +166,8 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(const float* __rest
   for (int i = 0; i < FO; ++i) wp[i] = W + (size_t)min(o0 + 16 * i + c, O - 1) * ldw;
 #pragma unroll
   for (int i = 0; i < FN; ++i) xp[i] = A + (size_t)min(n0 + 16 * i + c, N - 1) * lda;
-  f32x4 fw[SETS][2][FO], fx[SETS][2][FN];
-  // (k beyond the matrix: its last four again, and A's made zero when they are used)
-  auto ask = [&](int set, int k0) {
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const int k = min(k0 + 8 * g + 4 * half, I - 4);
-#pragma unroll
-      for (int i = 0; i < FO; ++i) fw[set][half][i] = *(const f32x4*)(wp[i] + k);
-#pragma unroll
-      for (int i = 0; i < FN; ++i) fx[set][half][i] = *(const f32x4*)(xp[i] + k);
-    }
-  };
   f32x4 acc[FO][FN] = {};
-  auto use = [&](int set, int k0) {
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const uint32_t keep = (uint32_t)((k0 + 8 * g + 4 * half - I) >> 31);
-#pragma unroll
-      for (int i = 0; i < FN; ++i) fx[set][half][i] = __builtin_bit_cast(f32x4, __builtin_bit_cast(u32x4, fx[set][half][i]) & keep);
-    }
-    bf16x8 pw[FO][3], px[FN][3];
-#pragma unroll
-    for (int i = 0; i < FO; ++i) split8(fw[set][0][i], fw[set][1][i], pw[i]);
-#pragma unroll
-    for (int i = 0; i < FN; ++i) split8(fx[set][0][i], fx[set][1][i], px[i]);
-#pragma unroll
-    for (int p = 0; p < F32_PRODUCTS; ++p)
-#pragma unroll
-      for (int i = 0; i < FO; ++i)
-#pragma unroll
-        for (int h = 0; h < FN; ++h) acc[i][h] = mfma_bf16(pw[i][F32_PART[p][0]], px[h][F32_PART[p][1]], acc[i][h]);
-  };
-  // (the first loads stand behind no branch, or the first block's use would wait for all of them: blocks behind a wave's last are that one again)
-  if (first < last) {
-    const int end = (last - first + 31) / 32 * 32 + first - 32;      // the wave's last block
-#pragma unroll
-    for (int s = 0; s < SETS; ++s) ask(s, min(first + 32 * s, end));
-    int k0 = first;
-    for (; k0 + 32 * (2 * SETS - 1) <= end; k0 += 32 * SETS) {
-#pragma unroll
-      for (int s = 0; s < SETS; ++s) {
-        __builtin_amdgcn_sched_barrier(0);
-        use(s, k0 + 32 * s);
-        ask(s, k0 + 32 * (s + SETS));
-      }
-    }
-#pragma unroll
-    for (int s = 0; s < 2 * SETS - 1; ++s) {
-      __builtin_amdgcn_sched_barrier(0);
-      if (k0 + 32 * s <= end) use(s % SETS, k0 + 32 * s);
-      if (s < SETS - 1 && k0 + 32 * (s + SETS) <= end) ask(s, k0 + 32 * (s + SETS));
-    }
-  }
+  f32_stretch(wp, xp, first, last, I, g, acc);
 #pragma unroll
   for (int i = 0; i < FO; ++i)
 #pragma unroll

@@ -2,8 +2,8 @@
 // size alone, so a pair's result is the same to the bit whatever tile it falls in and whatever else is in the step.
 //
 // A workgroup takes 16 FN places of one expert's stretch and 32 of its features (gated: 16 of both matrices), its eight waves a stretch of k
-// each, straight from memory into the operands' registers, where they are split; the waves' sums meet in LDS.  Bound by the stream of the
-// experts' matrices for few pairs, by what a compute unit brings in for many.  The loop is gemm_f32_split_kernel's.
+// each (f32_stretch); the waves' sums meet in LDS.  Bound by the stream of the experts' matrices for few pairs, by what a compute unit brings
+// in for many.
 // Width 1,024, experts of 512, 4 of 16 (us, gated and back, vector units before / now): 20 rows 165 and 54 / 18 and 14, 1,000 rows 496
 // and 215 / 180 and 145.
 #include "activation.h"
@@ -15,7 +15,7 @@ __global__ __launch_bounds__(512) void moe_gemm_f32_kernel(const float* __restri
                                                            const int* __restrict__ tile_expert, int bm, const float* __restrict__ Wa,
                                                            const float* __restrict__ Wb, long expert_stride, float* __restrict__ Y, long ldy, int O, int I, int act,
                                                            const float* __restrict__ in_weight) {
-  constexpr int SETS = 4, FO = 2, FEATURES = GLU ? 16 : 32;
+  constexpr int FO = 2, FEATURES = GLU ? 16 : 32;
   __shared__ __attribute__((aligned(16))) f32x4 s_sum[F32_SEGMENTS][FO * FN][WAVE];
   const int p0 = blockIdx.y * 16 * FN, e = tile_expert[p0 / bm];
   if (e < 0 || sorted_pair[p0] < 0) return;      // (an expert's pairs take the first places of its tiles)
@@ -35,58 +35,8 @@ __global__ __launch_bounds__(512) void moe_gemm_f32_kernel(const float* __restri
   for (int i = 0; i < FO; ++i) wp[i] = GLU ? (i == 0 ? wa : wb) + (size_t)min(o0 + c, O - 1) * I : wa + (size_t)min(o0 + 16 * i + c, O - 1) * I;
 #pragma unroll
   for (int i = 0; i < FN; ++i) xp[i] = row_of(p0 + 16 * i + c);
-  f32x4 fw[SETS][2][FO], fx[SETS][2][FN];
-  // (k beyond the matrix: its last four again, and X's made zero when they are used)
-  auto ask = [&](int set, int k0) {
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const int k = min(k0 + 8 * g + 4 * half, I - 4);
-#pragma unroll
-      for (int i = 0; i < FO; ++i) fw[set][half][i] = *(const f32x4*)(wp[i] + k);
-#pragma unroll
-      for (int i = 0; i < FN; ++i) fx[set][half][i] = *(const f32x4*)(xp[i] + k);
-    }
-  };
   f32x4 acc[FO][FN] = {};
-  auto use = [&](int set, int k0) {
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const uint32_t keep = (uint32_t)((k0 + 8 * g + 4 * half - I) >> 31);
-#pragma unroll
-      for (int i = 0; i < FN; ++i) fx[set][half][i] = __builtin_bit_cast(f32x4, __builtin_bit_cast(u32x4, fx[set][half][i]) & keep);
-    }
-    bf16x8 pw[FO][3], px[FN][3];
-#pragma unroll
-    for (int i = 0; i < FO; ++i) split8(fw[set][0][i], fw[set][1][i], pw[i]);
-#pragma unroll
-    for (int i = 0; i < FN; ++i) split8(fx[set][0][i], fx[set][1][i], px[i]);
-#pragma unroll
-    for (int p = 0; p < F32_PRODUCTS; ++p)
-#pragma unroll
-      for (int i = 0; i < FO; ++i)
-#pragma unroll
-        for (int h = 0; h < FN; ++h) acc[i][h] = mfma_bf16(pw[i][F32_PART[p][0]], px[h][F32_PART[p][1]], acc[i][h]);
-  };
-  if (first < last) {
-    const int end = (last - first + 31) / 32 * 32 + first - 32;      // the wave's last block
-#pragma unroll
-    for (int s = 0; s < SETS; ++s) ask(s, min(first + 32 * s, end));
-    int k0 = first;
-    for (; k0 + 32 * (2 * SETS - 1) <= end; k0 += 32 * SETS) {
-#pragma unroll
-      for (int s = 0; s < SETS; ++s) {
-        __builtin_amdgcn_sched_barrier(0);
-        use(s, k0 + 32 * s);
-        ask(s, k0 + 32 * (s + SETS));
-      }
-    }
-#pragma unroll
-    for (int s = 0; s < 2 * SETS - 1; ++s) {
-      __builtin_amdgcn_sched_barrier(0);
-      if (k0 + 32 * s <= end) use(s % SETS, k0 + 32 * s);
-      if (s < SETS - 1 && k0 + 32 * (s + SETS) <= end) ask(s, k0 + 32 * (s + SETS));
-    }
-  }
+  f32_stretch(wp, xp, first, last, I, g, acc);
 #pragma unroll
   for (int i = 0; i < FO; ++i)
 #pragma unroll
