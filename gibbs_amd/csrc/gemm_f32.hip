@@ -10,9 +10,12 @@
 // order.  Both kernels below keep to this whatever tile an element falls in, so a row's result does not depend on how many
 // other rows the call holds, and the stretches may be given to different waves.
 //
-// Values without three such parts.  An infinity or a NaN, and what rounds up to infinity, leaves NaN in its parts, and below
-// 2^-110 the low part is lost to bfloat16's smallest value; results that are not finite or closer to 0 than 2^-100 are therefore
-// taken again in plain float32 (`again`), from the operands as they are.
+// Values without three such parts.  An infinity or a NaN, and what rounds up to infinity, leaves NaN in its parts, and digits under 2^-133 (of
+// values under 2^-110) are lost to bfloat16's smallest value.  What is left of a value behind its second part shows such digits (`collect`:
+// half an instruction a value); the rows of A and of W that have any, and the results that are not finite, are taken again on the 32-bit
+// matrix instruction from the operands as they are, blocks of 16 x 16 with one such result at a time (`again`).  That depends on a result's own
+// two rows alone.  1,194 rows, 9,216 x 1,024 (us, in brackets one lane a result along its rows): none 154, one row with an infinity 250 (664),
+// every row with one 892 (6,840); 8 rows of 1,024 x 1,024 5.4, all again 19 (118).
 //
 // The plain kernel (vector units, ascending k) takes what these refuse: rows that are no whole number of 16 bytes, and
 // bfloat16 operands (float32 accumulation) of any size and stride.
@@ -55,6 +58,7 @@ __global__ __launch_bounds__(64 * WO * WN, OCC) void gemm_f32_tile_kernel(const 
     src[i] = i < NW ? W + (size_t)min(o0 + r0 + ROWS * i, O - 1) * ldw : A + (size_t)min(n0 + r0 + ROWS * (i - NW), N - 1) * lda;
   f32x4 raw[NP];
   bf16x2 part[3][2];
+  uint32_t left[NP] = {};      // (of this thread's rows)
   // (k beyond I: the last four k again, made zero where they are taken up.  No branch may stand there: with one, every wait became a
   // wait for all loads, and the kernel took 1.3 to 1.8 times as long)
   auto ask = [&](int i, int k0) { raw[i] = *(const f32x4*)(src[i] + min(k0 + quad, I - 4)); };
@@ -83,7 +87,11 @@ __global__ __launch_bounds__(64 * WO * WN, OCC) void gemm_f32_tile_kernel(const 
       x[2] = x2;
       x[3] = x3;
     }
-    if constexpr (s == 6) ask(i, next);
+    if constexpr (s == 6) {
+      left[i] = collect(collect(left[i], x[0], x[1]), x[2], x[3]);
+      asm("" : "+v"(left[i]));      // (now: put off, it keeps every remainder in a register)
+      ask(i, next);
+    }
     if constexpr (s == 7) {
 #pragma unroll
       for (int q = 0; q < 3; ++q) *(u32x2*)&s_p[buf + q * PART + ROWS * i * F32_BK + at] = u32x2{__builtin_bit_cast(uint32_t, part[q][0]), __builtin_bit_cast(uint32_t, part[q][1])};
@@ -139,14 +147,45 @@ __global__ __launch_bounds__(64 * WO * WN, OCC) void gemm_f32_tile_kernel(const 
 #pragma unroll
       for (int h = 0; h < FN; ++h) total[i][h] += acc[i][h];
   }
+  // which of the tile's rows have lost digits: hardly ever one
+  uint32_t any = 0;
+#pragma unroll
+  for (int i = 0; i < NP; ++i) any |= left[i];
+  const bool lost = __syncthreads_or(digits_lost(any));
+  int* s_lost = (int*)s_p;      // [BO + BN] (behind the last stretch's barrier, and behind the one above)
+  if (__builtin_expect(lost, 0)) {
+    for (int i = threadIdx.x; i < BO + BN; i += T) s_lost[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      if (digits_lost(left[i])) s_lost[ROWS * i + r0] = 1;
+    __syncthreads();
+  }
+  static_assert(FO * FN * 4 <= 32, "a bit for each of a lane's results");
+  uint32_t want = 0;
 #pragma unroll
   for (int i = 0; i < FO; ++i)
 #pragma unroll
     for (int h = 0; h < FN; ++h) {
-      const int row = n0 + wn + 16 * h + c, col = o0 + wo + 16 * i + 4 * g;
-      if (__builtin_expect(wants_again(total[i][h]), 0)) total[i][h] = again4(A, W, I, lda, ldw, row, col, N, O, total[i][h]);
-      store_f32x4(C, ldc, row, col, N, O, wide, total[i][h]);
+      uint32_t w_lost = 0;
+      if (lost) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w_lost |= (uint32_t)s_lost[wo + 16 * i + 4 * g + j] << j;
+      }
+      want |= wants_again(total[i][h], lost && s_lost[BO + wn + 16 * h + c], w_lost) << (4 * (i * FN + h));
+      store_f32x4(C, ldc, n0 + wn + 16 * h + c, o0 + wo + 16 * i + 4 * g, N, O, wide, total[i][h]);
     }
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(want != 0) == 0, 1)) return;
+#pragma unroll 1
+  for (int b = 0; b < FO * FN; ++b) {
+    const uint32_t mine = want >> (4 * b) & 15;
+    if (__builtin_amdgcn_ballot_w64(mine != 0) == 0) continue;
+    const int row = n0 + wn + 16 * (b % FN) + c, col = o0 + wo + 16 * (b / FN);
+    const f32x4 y = again(W + (size_t)min(col + c, O - 1) * ldw, A + (size_t)min(row, N - 1) * lda, I, g, mine);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if ((mine >> j & 1) && row < N && col + 4 * g + j < O) C[(size_t)row * ldc + col + 4 * g + j] = y[j];
+  }
 }
 
 // Few rows or few tiles: a workgroup takes 16 FO features x 16 FN rows and its eight waves a stretch of k each (f32_stretch; no barrier before
@@ -156,6 +195,7 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(const float* __rest
                                                              float* __restrict__ C, int N, int O, int I, long lda, long ldw,
                                                              long ldc, int wide) {
   __shared__ __attribute__((aligned(16))) f32x4 s_sum[F32_SEGMENTS][FO * FN][WAVE];
+  __shared__ __attribute__((aligned(16))) uint64_t s_lost[F32_SEGMENTS];
   const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), g = lane / 16, c = lane % 16;
   const int o0 = blockIdx.x * 16 * FO, n0 = blockIdx.y * 16 * FN;
   const int segments = f32_segments(I), segment = f32_segment(I);
@@ -167,18 +207,24 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(const float* __rest
 #pragma unroll
   for (int i = 0; i < FN; ++i) xp[i] = A + (size_t)min(n0 + 16 * i + c, N - 1) * lda;
   f32x4 acc[FO][FN] = {};
-  f32_stretch(wp, xp, first, last, I, g, acc);
+  uint32_t left[FO + FN] = {};
+  f32_stretch(wp, xp, first, last, I, g, acc, left);
+  const uint64_t my_lost = rows_lost(left);
+  if (lane == 0) s_lost[wave] = my_lost;
 #pragma unroll
   for (int i = 0; i < FO; ++i)
 #pragma unroll
     for (int h = 0; h < FN; ++h) s_sum[wave][i * FN + h][lane] = acc[i][h];
   __syncthreads();
+  uint64_t lost = 0;
+#pragma unroll
+  for (int s = 0; s < F32_SEGMENTS; ++s) lost |= s_lost[s];
   for (int t = wave; t < FO * FN; t += F32_SEGMENTS) {
     f32x4 total = {0.f, 0.f, 0.f, 0.f};
     for (int s = 0; s < segments; ++s) total += s_sum[s][t][lane];
-    const int row = n0 + 16 * (t % FN) + c, col = o0 + 16 * (t / FN) + 4 * g;
-    if (__builtin_expect(wants_again(total), 0)) total = again4(A, W, I, lda, ldw, row, col, N, O, total);
-    store_f32x4(C, ldc, row, col, N, O, wide, total);
+    const int row = n0 + 16 * (t % FN) + c, col = o0 + 16 * (t / FN);
+    total = whole_f32(total, lost, t / FN, FO + t % FN, g, c, I, [&] { return W + (size_t)min(col + c, O - 1) * ldw; }, [&] { return A + (size_t)min(row, N - 1) * lda; });
+    store_f32x4(C, ldc, row, col + 4 * g, N, O, wide, total);
   }
 }
 

@@ -17,6 +17,7 @@ __global__ __launch_bounds__(512) void moe_gemm_f32_kernel(const float* __restri
                                                            const float* __restrict__ in_weight) {
   constexpr int FO = 2, FEATURES = GLU ? 16 : 32;
   __shared__ __attribute__((aligned(16))) f32x4 s_sum[F32_SEGMENTS][FO * FN][WAVE];
+  __shared__ __attribute__((aligned(16))) uint64_t s_lost[F32_SEGMENTS];
   const int p0 = blockIdx.y * 16 * FN, e = tile_expert[p0 / bm];
   if (e < 0 || sorted_pair[p0] < 0) return;      // (an expert's pairs take the first places of its tiles)
   const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), g = lane / 16, c = lane % 16;
@@ -36,32 +37,36 @@ __global__ __launch_bounds__(512) void moe_gemm_f32_kernel(const float* __restri
 #pragma unroll
   for (int i = 0; i < FN; ++i) xp[i] = row_of(p0 + 16 * i + c);
   f32x4 acc[FO][FN] = {};
-  f32_stretch(wp, xp, first, last, I, g, acc);
+  uint32_t left[FO + FN] = {};
+  f32_stretch(wp, xp, first, last, I, g, acc, left);
+  const uint64_t my_lost = rows_lost(left);
+  if (lane == 0) s_lost[wave] = my_lost;
 #pragma unroll
   for (int i = 0; i < FO; ++i)
 #pragma unroll
     for (int h = 0; h < FN; ++h) s_sum[wave][i * FN + h][lane] = acc[i][h];
   __syncthreads();
   const bool wide = O % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)Y % 16) == 0;
-  // the whole sum of one of the workgroup's results, in float32 where it wants that
+  uint64_t lost = 0;
+#pragma unroll
+  for (int s = 0; s < F32_SEGMENTS; ++s) lost |= s_lost[s];
+  // the whole sum of one of the workgroup's blocks of results (features from `col` on)
   auto whole = [&](int t, const float* w, int col, const float* x) {
     f32x4 total = {0.f, 0.f, 0.f, 0.f};
     for (int s = 0; s < segments; ++s) total += s_sum[s][t][lane];
-    if (__builtin_expect(wants_again(total), 0)) total = again4(x, w, I, 0, I, 0, col, 1, O, total);
-    return total;
+    return whole_f32(total, lost, t / FN, FO + t % FN, g, c, I, [&] { return w + (size_t)min(col + c, O - 1) * I; }, [&] { return x; });
   };
   for (int t = wave; t < (GLU ? FN : FO * FN); t += F32_SEGMENTS) {
-    const int place = p0 + 16 * (t % FN) + c, pair = sorted_pair[place], col = o0 + 16 * (t / FN) + 4 * g;
-    if (pair < 0) continue;
+    const int place = p0 + 16 * (t % FN) + c, pair = sorted_pair[place], col = o0 + 16 * (t / FN);
     const float* x = row_of(place);
     f32x4 v = whole(t, wa, col, x);
     if constexpr (GLU) {
       const f32x4 u = whole(FN + t, wb, col, x);
-      const float w = in_weight ? in_weight[pair] : 1.f;
+      const float w = in_weight && pair >= 0 ? in_weight[pair] : 1.f;
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] = activate(w * v[i], act) * (w * u[i]);
     }
-    store_f32x4(Y, ldy, place, col, place + 1, O, wide, v);
+    if (pair >= 0) store_f32x4(Y, ldy, place, col + 4 * g, place + 1, O, wide, v);
   }
 }
 }  // namespace

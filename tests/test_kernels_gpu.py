@@ -113,6 +113,44 @@ def test_gemm_f32_values_without_three_bfloat16_parts(shape):
     assert got[~big & ~want.isnan() & (want.abs() < 3.3e38)].isfinite().all()
 
 
+@pytest.mark.parametrize("shape", [(5, 96, 512), (40, 1000, 516), (200, 2112, 100), (70, 48, 4), (700, 2112, 512)])
+def test_gemm_f32_keeps_the_digits_of_small_operands(shape):
+    """Operands with bits under 2^-133, which three bfloat16 do not hold, against operands large enough that the results are ordinary, from either side, in
+    single rows and in single columns.  An error of I additions, each of at most 2^-24 of a partial sum that is no larger than the whole in the root mean
+    square, is 2^-24 sqrt(I) of the whole, row by row (three products instead of six are at 4e-6, parts without these digits up to 2e-2), and 2^-149
+    a product where float32 ends.  A row's bits are its own, in whatever company and kernel."""
+    from gibbs_amd import ops
+    n, o, i = shape
+    a0, w0 = rnd(n, i), rnd(o, i, seed=1)
+    def check(a, w, what):
+        got = ops.gemm_f32(a, w)
+        want = a.double() @ w.double().t()
+        bound = 2.0 ** -24 * (1 + i ** 0.5) * want.norm(dim=1) + i * 2.0 ** -149 * o ** 0.5
+        err = (got.double() - want).norm(dim=1)
+        assert (err <= bound).all(), (shape, what, float((err / want.norm(dim=1)).max()))
+        for m in (1, 17, 70):
+            if m < n:
+                assert torch.equal(ops.gemm_f32(a[:m].contiguous(), w), got[:m]), (shape, what, m)
+        return got
+    for small, large in ((-107, 20), (-112, 0), (-120, 27), (-124, 30), (-124, 124), (-130, 40), (-140, 60), (-70, -66)):
+        check(a0 * 2.0 ** small, w0 * 2.0 ** large, (small, large))
+        check(a0 * 2.0 ** large, w0 * 2.0 ** small, (large, small))
+    plain = ops.gemm_f32(a0, w0)
+    a = a0.clone()
+    a[n // 2] *= 2.0 ** -125
+    got = check(a, w0, "a small row")
+    keep = torch.arange(n, device="cuda") != n // 2
+    assert torch.equal(got[keep], plain[keep])
+    w = w0.clone()
+    w[o // 3] *= 2.0 ** -125
+    got = check(a0, w, "a small feature")
+    keep = torch.arange(o, device="cuda") != o // 3
+    assert torch.equal(got[:, keep], plain[:, keep])
+    a, w = a0 * 2.0 ** -10, w0.clone()
+    a[:, i // 2], w[:, i // 2] = a0[:, i // 2] * 2.0 ** -123, w0[:, i // 2] * 2.0 ** 124
+    check(a, w, "small values that count")
+
+
 def test_gemm_f32_as_many_rows_as_the_plain_kernel_takes():
     """4,194,240 rows, which is where the plain kernel's grid ends, of few features: the tiles that cut k over their waves have no grid for them."""
     from gibbs_amd import ops

@@ -504,6 +504,37 @@ def test_experts_products_in_float32(O, I, gated):
         assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf()[:2], want.isinf()[:2])
 
 
+@pytest.mark.parametrize("O,I", [(33, 68), (96, 260), (512, 1024)])
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("small,large", [(-120, 120), (-130, 124), (124, -124)])
+def test_experts_products_in_float32_keep_the_digits_of_small_operands(O, I, gated, small, large):
+    """Rows or matrices with bits under 2^-133, which three bfloat16 do not hold, and results of the order of 1: the same bits whatever the tile, and the
+    error of I additions, each of at most 2^-24 of a partial sum no larger than the whole in the root mean square (gated: of both sums and some
+    roundings more)."""
+    from gibbs_amd.ops.lib import call, ptr, stream
+    g = torch.Generator(device="cuda").manual_seed(O + I)
+    x = torch.randn((60, I), generator=g, device="cuda")
+    x[::2] *= 2.0 ** small
+    x[1::2] *= 2.0 ** -large
+    wa, wb = (torch.randn((3, O, I), generator=g, device="cuda") * I ** -0.5 * 2.0 ** large for _ in range(2))
+    def products(bm, taken):
+        place = torch.full((2 * bm,), -1, dtype=torch.int32, device="cuda")
+        place[bm:bm + taken] = torch.arange(taken, dtype=torch.int32, device="cuda")      # pairs 0 .. of the second tile, two a row
+        y = torch.full((2 * bm, O + 3), 7.0, device="cuda")
+        call("gibbs_moe_gemm_weighted", ptr(x), I, 2, ptr(place), ptr(torch.tensor([-1, 2], dtype=torch.int32, device="cuda")), 2 * bm, bm, ptr(wa),
+             ptr(wb) if gated else None, None, ptr(y), O + 3, 0, O, I, 0, stream())
+        assert (y[:bm] == 7.0).all() and (y[bm + taken:] == 7.0).all() and (y[:, O:] == 7.0).all()
+        return y[bm:bm + taken, :O]
+    many = products(128, 120)
+    for bm, taken in ((16, 16), (16, 3), (128, 33)):
+        assert torch.equal(products(bm, taken), many[:taken])
+    rows = x[torch.arange(120, device="cuda") // 2].double()
+    a, b = rows @ wa[2].double().T, rows @ wb[2].double().T
+    want = a * torch.sigmoid(a) * b if gated else a
+    err = (many.double() - want).norm(dim=1) / want.norm(dim=1)
+    assert (err <= 2.0 ** -24 * (1 + I ** 0.5) * (4 if gated else 1)).all(), float(err.max())
+
+
 def test_a_rows_experts_do_not_depend_on_its_neighbours():
     """32-bit: the same row alone and among 200 others gives the same bits."""
     from gibbs_amd import Engine
