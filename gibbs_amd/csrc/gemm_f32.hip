@@ -286,8 +286,12 @@ void launch_split(const float* A, const float* W, float* C, int N, int O, int I,
 }
 
 // The variants, and which one takes a shape.  A compute unit works through ceil(tiles / 256) tiles; one tile alone takes `alone`, one among
-// others on the same unit `loaded` (us at an inner size of 1,024; measured), so the least of max(alone, rounds * loaded) is taken; both grow with
-// the inner size alike.  Features x rows of a tile; the last three cut k over their waves and serve few rows.
+// others on the same unit `loaded` (us at an inner size of 1,024; measured), so the least of max(alone, rounds * loaded) is taken.  Over 1,024
+// that order of the variants stays; under it a split tile's waves have four blocks of k or fewer, which are not enough to hide what one
+// waits for, and it costs 1.4 times its share.  (77 shapes of 1 to 544 rows and 256 to 6,144 features at 13 inner sizes of 32 to 768, the variant
+// taken over the best one, without and with that: in the mean 1.06 and 1.01, at most 2.10 and 1.21; 100 rows x 4,096 features, us:
+// inner size 128 10.5 / 6.0, 252 11.9 / 8.6, 512 18.3 / 12.0; inner size 1,024: 1.003, at most 1.05.)
+// Features x rows of a tile; the last three cut k over their waves and serve few rows.
 // (1,194 rows, us, on the matrix cores' 32-bit instruction / in three parts: 9,216 features x 1,024 227 / 156, 1,024 x 4,608 154 / 123, 1,024 x
 // 1,024 38 / 34, 3,072 x 1,024 84 / 50; 333 rows: 9,216 x 1,024 82 / 49; 8 rows: 9,216 x 1,024 11.8 / 12.1, 1,024 x 4,608 15.0 / 15.9, 1,024 x 1,024 5.3 / 5.6
 // before the kernels' arguments came in registers, which gives that back: a decoded token of the 350M shape takes as long as it did.
@@ -310,7 +314,7 @@ bool launch_f32(const float* A, const float* W, float* C, int N, int O, int I, l
   for (const F32Variant& v : F32_VARIANTS) {
     if (v.split && ceil_div(N, v.rows) > 65535) continue;
     const long tiles = (long)ceil_div(N, v.rows) * ceil_div(O, v.features);
-    const float cost = fmaxf(v.alone, (float)((tiles + 255) / 256) * v.loaded);
+    const float cost = fmaxf(v.alone, (float)((tiles + 255) / 256) * v.loaded) * (v.split && I < 1024 ? 1.4f : 1.f);
     if (!best || cost < least) {
       best = &v;
       least = cost;
