@@ -926,10 +926,12 @@ GIBBS_EXPORT int gibbs_moe_route_scaled(const void* h, long ldh, int dtype, cons
   GIBBS_REQUIRE(E > 0 && E <= MOE_MAX_EXPERTS && top > 0 && top <= E, "moe_route: %d of %d experts (at most %d)", top, E, MOE_MAX_EXPERTS);
   GIBBS_REQUIRE(!shared_gate || sgate, "moe_route: a shared expert's gate needs its output");
   const size_t lds = (size_t)E * sizeof(float) * (mode != 0 ? 2 : 1);
-  // few rows: a wave per expert (and one for the shared expert's gate) up to 16 waves; many rows fill the chip with 4; more share the router
-  // (16 experts, a row / four rows a workgroup, us: 513 rows of 2,048 13.2 / 16.1, 1,024 15.8 / 13.3, 2,029 23.4 / 19.6, 4,096 of 1,024 27 / 16.0; many experts
-  // gain nothing, 700 rows of 2,048, 256 experts 113 / 121)
-  const bool share = n >= 1024 && E <= 32 && W % 4 == 0 && ldh % 4 == 0 && ((uintptr_t)h % 16) == 0 && ((uintptr_t)router % 16) == 0 && ((uintptr_t)shared_gate % 16) == 0;
+  // few rows: a wave per expert (and one for the shared expert's gate) up to 16 waves; many rows fill the chip with 4; more share the router.
+  // A row / four rows a workgroup, us, where the line lies: 8 experts 1,280 rows of 1,024 13.0 / 13.6, 1,536 13.8 / 13.7, of 256 12.7 / 12.5, of 2,048 768
+  // 13.0 / 13.0, 1,024 13.6 / 12.9; 32 experts 1,024 rows of 1,024 18.2 / 20.4, 1,536 24.5 / 22.5, of 512 21.8 / 20.1, of 2,048 768 22.6 / 23.0, 1,024 26.0 /
+  // 23.1; 64 experts 1,536 rows of 1,024 38.3 / 33.4, 1,024 of 2,048 41.6 / 36.3, 4,096 127 / 62; 256 experts 1,024 rows of 2,048 138 / 120, 4,096 484 / 206,
+  // 512 experts 1,024 rows 264 / 272
+  const bool share = (n >= 1536 || (n >= 1024 && W >= 2048)) && E <= 256 && W % 4 == 0 && ldh % 4 == 0 && ((uintptr_t)h % 16) == 0 && ((uintptr_t)router % 16) == 0 && ((uintptr_t)shared_gate % 16) == 0;
   if (share && (dtype == GIBBS_F32 || dtype == GIBBS_BF16)) {
     const int blocks = ceil_div(n, ROUTE_ROWS);
     const size_t all = 2 * ROUTE_ROWS * (size_t)E * sizeof(float);

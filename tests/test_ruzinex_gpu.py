@@ -463,6 +463,27 @@ def test_routes_of_many_rows_are_the_routes_of_few(W, E, top, shared, mode):
     assert torch.equal(many[0].sort(-1).values.diff(dim=-1) > 0, torch.ones((n, top - 1), dtype=torch.bool, device="cuda"))      # no expert twice
 
 
+@pytest.mark.parametrize("n,W,E,top", [(1535, 64, 40, 3), (1536, 64, 40, 3), (1539, 260, 7, 7), (1025, 2048, 33, 8), (1601, 36, 256, 70), (1601, 36, 257, 70), (1537, 4, 256, 256)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_routes_of_many_rows_among_any_number_of_experts(n, W, E, top, dtype):
+    """Where rows begin to share the router, more experts than lanes, more choices than lanes, all of the most experts that do and one more: a row's
+    route is that of a call of few rows, to the bit."""
+    from gibbs_amd.ops.lib import call, ptr, stream
+    g = torch.Generator(device="cuda").manual_seed(n + E)
+    h = torch.randn((n, W), generator=g, device="cuda").to(dtype)
+    router, bias, gate = (torch.randn(s, generator=g, device="cuda") * W ** -0.5 for s in ((E, W), (E,), (W,)))
+    for mode in (0, 1, 2):
+        def route(rows):
+            m = rows.shape[0]
+            out = torch.full((m, top), -1, dtype=torch.int32, device="cuda"), torch.zeros((m, top), device="cuda"), torch.zeros(m, device="cuda")
+            call("gibbs_moe_route_scaled", ptr(rows), W, int(dtype == torch.bfloat16), ptr(router), ptr(bias), ptr(gate), *map(ptr, out), m, W, E, top, mode,
+                 1.5 if mode == 1 else 1.0, stream())
+            return out
+        many, few = route(h), [torch.cat(x) for x in zip(*(route(part.contiguous()) for part in h.split(500)))]
+        for a, b in zip(many, few):
+            assert torch.equal(a, b), mode
+
+
 @pytest.mark.parametrize("O,I", [(8, 4), (33, 68), (96, 260), (512, 1024), (70, 2052)])
 @pytest.mark.parametrize("gated", [False, True])
 def test_experts_products_in_float32(O, I, gated):
