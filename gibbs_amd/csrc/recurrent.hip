@@ -52,10 +52,10 @@ __global__ void causal_conv_silu_kernel(const T* __restrict__ in, long ld, const
 
 // The same for bfloat16 inputs whose channels come in whole groups of 8: a thread takes 8 neighbouring channels with 16-byte loads, of
 // CONV_RUN rows one behind the other, whose inputs it holds in registers (a row a thread reads K rows for each it writes: 2,048 rows of
-// 6,144 channels, K = 4, 30 us with a kernel of 25 us for the unit vectors behind it; 26 us so with them, half of it exponentials, one the
-// order of the squares' sum).  A workgroup is 64 lanes of channels by CONV_ROWS such runs; the taps of its 512
-// channels, one contiguous stretch of the [C, K] table, come through LDS once (each thread's 8 K taps a word further along, so that the lanes
-// read different banks) instead of as 8 K scattered words per thread.  Sums in ascending j, as above.
+// 6,144 channels, K = 4, 30 us with a kernel of 25 us for the unit vectors behind it; 26 us so with them, half of it exponentials, one
+// the order of the squares' sum).  A workgroup is 64 lanes of channels by CONV_ROWS such runs; the taps of its 512 channels, one
+// contiguous stretch of the [C, K] table, come through LDS once (each thread's 8 K taps a word further along, so that the lanes read
+// different banks) instead of as 8 K scattered words per thread.  Sums in ascending j, as above.
 // KT: K, as many rows as that in registers; 0: any K, a row at a time.
 // unit.D > 0: channels 0 .. 2 unit.G unit.D are heads of unit.D that are made unit vectors, x / sqrt(sum x^2 + eps), those of the first half
 // times q_scale, in rows from unit.first on (what the delta rule reads, to the bit as delta_prep_kernel makes them; a head is unit.D / 8
@@ -698,8 +698,12 @@ __global__ void double_exp_decay_kernel(float* __restrict__ z, const float* __re
   } while (0)
 
 namespace {
-// Rows from which a thread of the wide kernel takes CONV_RUN of them (fewer are too few workgroups)
-constexpr int CONV_RUN_ROWS = 512;
+// Whether a thread of the wide kernel takes CONV_RUN rows: where they leave workgroups enough, which is rows times channels.  A row / four rows a thread,
+// without and with unit vectors, us: K = 4, 4,096 rows of 1,024 10.3 / 11.7 and 13.6 / 15.2, 1,024 of 2,048 6.7 / 8.4 and 9.2 / 11.6, 2,048 of 2,048 10.6 /
+// 11.4 and 14.3 / 14.9, 3,072 of 2,048 16.5 / 13.7 and 19.9 / 18.0, 640 of 6,144 10.2 / 10.8 and 13.2 / 14.4, 768 of 6,144 13.5 / 12.4 and 17.6 / 16.4, 2,048 of
+// 6,144 27.2 / 23.0 and 30.7 / 28.2, 256 of 12,288 8.6 / 9.6, 384 of 12,288 13.9 / 11.6; K = 3, 768 of 6,144 11.5 / 11.3 and 15.0 / 15.1; K = 2, which saves one
+// row in three, 2,048 of 4,096 15.7 / 15.9 and 18.2 / 19.8, 2,048 of 6,144 20.9 / 18.8 and 23.7 / 23.0.
+bool conv_runs(long rows, int C, int K) { return K >= 2 && K <= 4 && rows * C >= (K == 2 ? 12L << 20 : 9L << 19); }
 // (steps of few rows are served faster by the kernel with a thread per channel: more, shorter workgroups; measured at 8 rows)
 bool conv_vec8(const void* in, long ld, int dtype, const float* bias, const float* state, long slot_stride, const void* out, int out_f32, long ld_out,
                int n_rows, int C, int K) {
@@ -723,7 +727,7 @@ static int causal_conv(const void* in, long ld, int dtype, const float* taps, co
   const bool vec8 = conv_vec8(in, ld, dtype, bias, state, slot_stride, out, out_f32, ld_out, n_rows, C, K);
   GIBBS_REQUIRE(vec8 || unit.D == 0, "causal_conv: unit vectors of operands that the wide kernel refuses");
   if (vec8) {
-    const int run = K >= 2 && K <= 4 && n_rows >= CONV_RUN_ROWS ? CONV_RUN : 1;
+    const int run = conv_runs(n_rows, C, K) ? CONV_RUN : 1;
     const dim3 grid(ceil_div(n_rows, CONV_ROWS * run), ceil_div(C, CONV_LANES * 8)), block(CONV_LANES, CONV_ROWS);
     const size_t lds = (size_t)CONV_LANES * (8 * K + 1) * sizeof(float);
     auto launch = [&](auto type, auto length) {

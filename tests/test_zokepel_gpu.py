@@ -1005,7 +1005,7 @@ def test_unit_heads_in_whole_16_bytes_are_the_general_kernels(hd, unit, every):
 @pytest.mark.parametrize("K,G,D,V", [(4, 2, 128, 40), (2, 3, 16, 8), (3, 1, 64, 24), (5, 2, 32, 72)])
 def test_delta_convolution_is_the_convolution_and_then_the_unit_vectors(lens, K, G, D, V):
     """One kernel against the two that it stands for, whose results a row's do not differ from whichever way a step takes: rows and states to the bit, with
-    an infinity, a NaN and a head of zeros among the rows; 512 rows and more (four a thread) of a request each, which move all their states on, too."""
+    an infinity, a NaN and a head of zeros among the rows; rows of a request each, which move all their states on, too."""
     from gibbs_amd import ops
     from gibbs_amd.ops.lib import call, ptr, stream
     g = torch.Generator(device="cuda").manual_seed(D)
@@ -1028,6 +1028,33 @@ def test_delta_convolution_is_the_convolution_and_then_the_unit_vectors(lens, K,
          0.25, 1e-6, stream())
     for a, b in ((got, want), (state, other)):
         assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(nan=7.0), b.nan_to_num(nan=7.0))
+
+
+@pytest.mark.parametrize("K,C", [(4, 9216), (3, 4608), (2, 24640), (4, 4616)])
+@pytest.mark.parametrize("lens", [[1] * 1027, [1026], [3, 1, 2, 1, 700, 1, 4, 313]])
+def test_convolution_of_four_rows_a_thread_is_float32s(K, C, lens):
+    """Rows and channels enough that a thread takes four rows: bfloat16 rows against the same values in float32, a channel a thread, to the bit (sums are
+    float32 in ascending order in both); requests that meet inside a thread's rows, and one row of each with its state moved on in the same kernel.  With unit
+    vectors (heads of 128, the first channels) the other channels are the same bits, and q and k unit vectors."""
+    from gibbs_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(K)
+    N = sum(lens)
+    x = torch.randn((N, C), generator=g, device="cuda").bfloat16()
+    x[1, 2], x[5, C - 1] = float("inf"), float("nan")
+    taps = torch.randn((C, K), generator=g, device="cuda")
+    state = torch.randn((len(lens) + 1, K - 1, C), generator=g, device="cuda")
+    cu = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32, device="cuda")
+    row_req = torch.repeat_interleave(torch.arange(len(lens), device="cuda"), torch.tensor(lens, device="cuda")).to(torch.int32)
+    slot = torch.arange(1, len(lens) + 1, dtype=torch.int32, device="cuda").flip(0).contiguous()
+    states = [state.clone() for _ in range(3)]
+    want = ops.causal_conv_silu(x.float(), taps, states[0], row_req, cu, slot)
+    got = ops.causal_conv_silu(x, taps, states[1], row_req, cu, slot)
+    unit = ops.delta_conv(x, taps, states[2], row_req, cu, slot, 2, 128, 0.25, 1e-6, 2)
+    same = lambda a, b: torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(nan=7.0), b.nan_to_num(nan=7.0))
+    assert same(got, want) and same(states[1], states[0]) and same(states[2], states[0])
+    assert same(unit[:, 512:], want[:, 512:]) and same(unit[:2], want[:2])
+    heads = unit[2:, :512].unflatten(1, (4, 128)).double().norm(dim=-1)[8:]
+    assert (heads - torch.tensor([0.25, 0.25, 1.0, 1.0], device="cuda")).abs().max() < 1e-5
 
 
 @pytest.mark.parametrize("V", [16, 32, 64, 128])
