@@ -937,9 +937,13 @@ GIBBS_EXPORT int gibbs_token_shift(const void* h, int dtype, const float* mu, in
   GIBBS_REQUIRE(h && mu && state && out && n_rows > 0 && n_req > 0 && W > 0 && n_mix > 0 && slot_stride >= W,
                 "token_shift: bad operands rows=%d requests=%d W=%d", n_rows, n_req, W);
   const dim3 rows(n_rows, ceil_div(W, 256)), reqs(n_req, ceil_div(W, 256));
-  // (few rows: a channel a thread is more, shorter workgroups)
-  if (dtype == GIBBS_BF16 && n_rows >= 64 && W % 8 == 0 && slot_stride % 4 == 0 && (((uintptr_t)h | (uintptr_t)mu | (uintptr_t)state | (uintptr_t)out) % 16) == 0) {
-    if (n_rows >= 1024)
+  // A channel a thread / eight channels, a row / four rows, us (few values: a channel a thread is more, shorter workgroups): 5 mixes, 64 rows of 2,048 2.58 /
+  // 3.13 / 4.61, 256 of 2,048 3.63 / 3.69 / 5.04, 512 of 1,024 3.71 / 3.70 / 4.79, 1,024 of 2,048 8.89 / 6.06 / 7.19, 1,536 of 2,048 14.8 / 9.24 / 9.18, 3,072 of
+  // 1,024 14.7 / 9.40 / 8.97, 2,048 of 2,048 19.8 / 11.2 / 10.8; one mix, whose weights are few to read again, 256 of 2,048 2.42 / 2.15 / 2.91, 2,048 of
+  // 2,048 8.1 / 4.0 / 4.2, 3,072 of 2,048 13.1 / 5.7 / 5.1
+  const long values = (long)n_rows * W;
+  if (dtype == GIBBS_BF16 && values >= 1L << 19 && W % 8 == 0 && slot_stride % 4 == 0 && (((uintptr_t)h | (uintptr_t)mu | (uintptr_t)state | (uintptr_t)out) % 16) == 0) {
+    if (values >= (n_mix > 1 ? 3L : 6L) << 20)
       token_shift_vec8_kernel<4><<<dim3(ceil_div(n_rows, 4), ceil_div(W, 2048)), 256, 0, stream>>>((const bf16*)h, mu, n_mix, state, slot_stride, row_req, cu, slot,
                                                                                                   (bf16*)out, n_rows, W, keep);
     else

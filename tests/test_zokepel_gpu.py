@@ -1030,6 +1030,28 @@ def test_delta_convolution_is_the_convolution_and_then_the_unit_vectors(lens, K,
         assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(nan=7.0), b.nan_to_num(nan=7.0))
 
 
+@pytest.mark.parametrize("lens", [[1] * 1027, [1026], [5, 1, 1, 700, 2, 1, 330]])
+@pytest.mark.parametrize("W,mixes", [(512, 5), (3072, 2), (3080, 5), (6152, 1)])
+def test_token_shift_of_many_values_is_float32s(lens, W, mixes):
+    """Eight channels a thread, of a row (the first width) and of four, where rows and channels are enough for that: the float32 kernel's results rounded, to the bit,
+    and its state; requests that meet inside a thread's rows, and rows of a request each, whose states one thread reads and moves on."""
+    from gibbs_amd.ops.lib import call, ptr, stream
+    g = torch.Generator(device="cuda").manual_seed(W)
+    n = sum(lens)
+    h = torch.randn((n, W), generator=g, device="cuda").bfloat16()
+    mu = torch.randn((mixes, W), generator=g, device="cuda")
+    kept = torch.randn((len(lens) + 1, W), generator=g, device="cuda")
+    cu = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32, device="cuda")
+    req = torch.repeat_interleave(torch.arange(len(lens), device="cuda"), torch.tensor(lens, device="cuda")).to(torch.int32)
+    slot = torch.arange(1, len(lens) + 1, dtype=torch.int32, device="cuda").flip(0).contiguous()
+    outs = []
+    for kind, code in ((torch.float32, 0), (torch.bfloat16, 1)):
+        x, state, out = h.to(kind), kept.clone(), torch.empty((mixes, n, W), dtype=kind, device="cuda")
+        call("gibbs_token_shift", ptr(x), code, ptr(mu), mixes, ptr(state), W, ptr(req), ptr(cu), ptr(slot), ptr(out), n, len(lens), W, 1, int(n == len(lens)), stream())
+        outs.append((out, state))
+    assert torch.equal(outs[0][0].bfloat16(), outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
 @pytest.mark.parametrize("K,C", [(4, 9216), (3, 4608), (2, 24640), (4, 4616)])
 @pytest.mark.parametrize("lens", [[1] * 1027, [1026], [3, 1, 2, 1, 700, 1, 4, 313]])
 def test_convolution_of_four_rows_a_thread_is_float32s(K, C, lens):
