@@ -47,8 +47,8 @@ __global__ __launch_bounds__(64) void qk_unit_kv_kernel(T* __restrict__ rows, lo
 }
 
 // The same for bfloat16 heads of 8 LPK channels in whole 16 bytes: a workgroup a row, LPK lanes a head of q or k and vd / 8 a head of v, 8 channels each,
-// the norms the same bits (a wave a head, 2,048 rows of 32 heads over 8 of 64: 24.5 us; 9.4 us so.  The order of the squares' sum is 0.4 us of that, and 0.6 of
-// 5.4 us at 8 rows).
+// the norms the same bits (a wave a head, 2,048 rows of 32 heads over 8 of 64: 23.9 us; 7.7 us so, 0.25 of them for the order of the squares' sum; 8 rows
+// 2.7 / 2.6).
 template <int LPK>
 __global__ void qk_unit_kv_vec8_kernel(bf16* __restrict__ rows, long ld, bf16* __restrict__ kpages, bf16* __restrict__ vpages, const int* __restrict__ pos,
                                        const int* __restrict__ row_req, const int* __restrict__ table, int max_pages, int page_size, int num_pages, int nh,

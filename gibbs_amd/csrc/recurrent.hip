@@ -480,8 +480,8 @@ __global__ __launch_bounds__(64) void head_norm_gate_kernel(const float* __restr
   }
 }
 // The same for bfloat16 results and heads of 16, 32, 64 or 128 values in whole 16 bytes: V / 8 neighbouring lanes a head, 8 values each, so that
-// a wave has 4 to 32 heads on their way (a wave a head, 2,048 rows of 16 heads of 128: 16.4 us for 33 MB; 10.9 us so, 0.5 of them
-// for the order of the squares' sum, which is the other kernel's).
+// a wave has 4 to 32 heads on their way, and the norms are the other kernel's to the bit (a wave a head, 2,048 rows of 16 heads of 128: 13.9 us for 33 MB;
+// 8.0 us so, 0.6 of them for the order of the squares' sum).
 __global__ __launch_bounds__(256) void head_norm_gate_vec8_kernel(const float* __restrict__ o, const float* __restrict__ gain, int gain_len,
                                                                   const bf16* __restrict__ gate, long ld_gate, bf16* __restrict__ y, long heads, int H, int V,
                                                                   float eps, int act) {
@@ -917,9 +917,11 @@ GIBBS_EXPORT int gibbs_head_norm_gate(const float* o, const float* gain, int gai
                                       int dtype, int n_rows, int H, int V, float eps, int act, hipStream_t stream) {
   GIBBS_REQUIRE(o && gain && y && n_rows > 0 && H > 0 && V > 0 && gain_len > 0 && (!gate || ld_gate >= (long)H * V) && (act == 0 || act == 1),
                 "head_norm_gate: bad operands rows=%d heads=%d V=%d", n_rows, H, V);
-  if (dtype == GIBBS_BF16 && (V == 16 || V == 32 || V == 64 || V == 128) && gain_len % 8 == 0 && ld_gate % 8 == 0 &&
+  // (a wave a head / a few lanes a head, us: 8 rows of 16 heads of 128 2.6 / 3.1, 64 2.8 / 3.2, 256 3.9 / 3.3; 64 rows of 32 heads of 64 2.7 / 3.1, 256 4.3 / 3.2; 256
+  // rows of 8 heads of 16 2.7 / 3.0, 2,048 6.2 / 3.0)
+  const long heads = (long)n_rows * H;
+  if (dtype == GIBBS_BF16 && heads >= 4096 && (V == 16 || V == 32 || V == 64 || V == 128) && gain_len % 8 == 0 && ld_gate % 8 == 0 &&
       (((uintptr_t)o | (uintptr_t)gain | (uintptr_t)gate | (uintptr_t)y) % 16) == 0) {
-    const long heads = (long)n_rows * H;
     head_norm_gate_vec8_kernel<<<(unsigned)((heads * (V / 8) + 255) / 256), 256, 0, stream>>>(o, gain, gain_len, (const bf16*)gate, ld_gate, (bf16*)y, heads, H, V, eps, act);
     GIBBS_LAUNCH_STATUS("head_norm_gate");
   }
