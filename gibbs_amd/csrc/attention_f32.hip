@@ -14,7 +14,7 @@
 // size 64 (in brackets attention_plain.hip, whose lanes read a key each, uncoalesced, and every key once a row): 1,194 rows of a
 // prompt 112 us (1,348), 4,096 rows 646 us (11,963; 52 TFLOP/s), 64 rows after 1,000 keys 66 us (518).  Values of twice the
 // keys' size (VT): the same walk with V in pieces and pages of its own; 20 rows behind 200 keys, 8 heads over 2 of 64 and 128, 33 us (292 in the plain
-// kernel).
+// kernel); 8 rows behind 20 9.4 (12.4), 63 8.7 (31); one row behind 7 keys 9.2 (6.9), 20 rows of a prompt 9.4 (11.9): a tile of 64 keys is walked whole.
 #include "common.h"
 
 namespace {

@@ -1,9 +1,11 @@
 // True 32-bit matrix product for the float32 path:  C[n, o] = sum_k A[n, k] * W[o, k], on the matrix cores' bfloat16
 // instruction.  A float32 is exactly the sum of three bfloat16 (8 + 8 + 8 bits: high = round(x), middle = round(x - high),
-// low = x - high - middle, all differences exact), and a product of two such sums is nine products, of which the six down to
-// 2^-18 of the whole are taken: what is left out is below 2^-26 of it, a fourth of a float32 product's own rounding.  Six
-// products at 16 times the rate of v_mfma_f32_16x16x4_f32, and 6 additions to a float32 sum for 32 k where that instruction
-// makes 8.
+// low = x - high - middle, all differences exact), and a product of two such sums is nine products (the method of Henry, Tang and
+// Heinecke, "Leveraging the bfloat16 artificial intelligence datatype for higher-precision computations", 2019), of which the six
+// largest are taken, down to high by low at 2^-17 of the whole.  What is left out, middle by low both ways and low by low, is 2^-24 of a product at
+// most (a float32 rounding, where the 32-bit instruction has none before its addition) and 2^-27.4 in the root mean square.  Six products at 16 times the
+// rate of v_mfma_f32_16x16x4_f32, and 6 additions to a float32 sum for 32 k where that instruction makes 8, which is why a sum's
+// error is smaller all the same: relative to the norm, inner size 1,024 2.1e-7 there / 1.6e-7, 4,608 4.3e-7 / 3.7e-7.
 //
 // The order of a sum.  k is cut into f32_segments(I) stretches of f32_segment(I) values; inside one the sum runs through
 // blocks of 32 k in ascending order, the six products of a block smallest first; the stretches' sums are added in ascending
@@ -294,8 +296,7 @@ void launch_split(const float* A, const float* W, float* C, int N, int O, int I,
 // Features x rows of a tile; the last three cut k over their waves and serve few rows.
 // (1,194 rows, us, on the matrix cores' 32-bit instruction / in three parts: 9,216 features x 1,024 227 / 156, 1,024 x 4,608 154 / 123, 1,024 x
 // 1,024 38 / 34, 3,072 x 1,024 84 / 50; 333 rows: 9,216 x 1,024 82 / 49; 8 rows: 9,216 x 1,024 11.8 / 12.1, 1,024 x 4,608 15.0 / 15.9, 1,024 x 1,024 5.3 / 5.6
-// before the kernels' arguments came in registers, which gives that back: a decoded token of the 350M shape takes as long as it did.
-// Error against 64 bits, relative, the same two: inner size 1,024 2.1e-7 / 1.6e-7, 4,608 4.3e-7 / 3.7e-7.)
+// before the kernels' arguments came in registers, which gives that back: a decoded token of the 350M shape takes as long as it did.)
 struct F32Variant {
   int features, rows;
   float alone, loaded;
