@@ -467,11 +467,13 @@ def test_routes_of_many_rows_are_the_routes_of_few(W, E, top, shared, mode):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_routes_of_many_rows_among_any_number_of_experts(n, W, E, top, dtype):
     """Where rows begin to share the router, more experts than lanes, more choices than lanes, all of the most experts that do and one more: a row's
-    route is that of a call of few rows, to the bit."""
+    route is that of a call of few rows, to the bit, with equal logits and a row that is no number among them."""
     from gibbs_amd.ops.lib import call, ptr, stream
     g = torch.Generator(device="cuda").manual_seed(n + E)
     h = torch.randn((n, W), generator=g, device="cuda").to(dtype)
     router, bias, gate = (torch.randn(s, generator=g, device="cuda") * W ** -0.5 for s in ((E, W), (E,), (W,)))
+    h[513, 3] = float("nan")
+    router[2], bias[2] = router[1], bias[1]
     for mode in (0, 1, 2):
         def route(rows):
             m = rows.shape[0]
@@ -481,7 +483,7 @@ def test_routes_of_many_rows_among_any_number_of_experts(n, W, E, top, dtype):
             return out
         many, few = route(h), [torch.cat(x) for x in zip(*(route(part.contiguous()) for part in h.split(500)))]
         for a, b in zip(many, few):
-            assert torch.equal(a, b), mode
+            assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(nan=7.0), b.nan_to_num(nan=7.0)), mode
 
 
 @pytest.mark.parametrize("O,I", [(8, 4), (33, 68), (96, 260), (512, 1024), (70, 2052)])
