@@ -643,6 +643,9 @@ __global__ __launch_bounds__(NW * WAVE, GT <= 4 ? (NW == 8 ? 4 : 3) : 2) void at
   }
 }
 
+}  // namespace
+#include "attention_tiles.h"
+namespace {
 template <int LPK, bool RAW, int NW, bool MM>
 void launch_decode(int gt, dim3 grid, hipStream_t stream, const bf16* q, bf16* k, bf16* v, float* partial, bf16* out,
                    const DecodeArgs& a) {
@@ -701,7 +704,9 @@ int run_decode(const bf16* q, bf16* kpages, bf16* vpages, bf16* out, float* part
   const long ids = (bound + a.page_size - 1) / a.page_size;
   a.ids_whole = a.window == 0 && a.chunk == 0 && ids <= SEG_PAGES;
   a.n_ids = (int)min(ids, (long)a.max_pages);
-  if (lanes <= 2) launch_waves<2, RAW>(waves, mm, gt, grid, stream, q, kpages, vpages, partial, out, a);
+  // (the tiles' kernel keeps no page ids: no slice is too long for it)
+  if ((mm || kind == 0) && tiles_take<RAW>(a, kind, q, kpages, vpages, out, partial)) run_tiles<RAW>(a, n_rows, waves, stream, q, kpages, vpages, out, partial);
+  else if (lanes <= 2) launch_waves<2, RAW>(waves, mm, gt, grid, stream, q, kpages, vpages, partial, out, a);
   else if (lanes <= 4) launch_waves<4, RAW>(waves, mm, gt, grid, stream, q, kpages, vpages, partial, out, a);
   else if (lanes <= 8) launch_waves<8, RAW>(waves, mm, gt, grid, stream, q, kpages, vpages, partial, out, a);
   else if (lanes <= 16) launch_waves<16, RAW>(waves, mm, gt, grid, stream, q, kpages, vpages, partial, out, a);

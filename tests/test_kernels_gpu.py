@@ -1057,6 +1057,47 @@ def test_attention_decode_fused(nh, nkv, hd, rot, page, window, variant, n_split
     close(got, want, dtype, "fused decode attention", bf16=8e-3)
 
 
+@pytest.mark.parametrize("raw", [False, True])
+@pytest.mark.parametrize("n_splits,waves", [(1, 4), (1, 8), (5, 4), (None, None)])
+@pytest.mark.parametrize("nh,nkv,hd,page,window", [(2, 2, 64, 16, None), (4, 2, 64, 64, 33), (8, 1, 64, 16, 700), (1, 1, 128, 16, None),
+                                                   (4, 2, 128, 32, 70), (8, 1, 128, 16, 31)])
+def test_attention_decode_in_tiles(nh, nkv, hd, page, window, n_splits, waves, raw):
+    """Heads of 64 and 128 in groups of 1 to 8, rows that end on either side of a tile of 32 keys and of a page, a row of more tiles than
+    a wave holds page ids for (4,400 keys are 138 tiles: 35 a wave), windows that begin inside a tile; in the pages, everything
+    that no row may see is NaN.  Raw rows also at positions behind the table of rotation factors."""
+    from gibbs_amd import ops
+    from gibbs_amd.parts.rope import rope_inv_freq
+    dtype = torch.bfloat16
+    seq_lens = [4400, 1, 16, 17, 32, 33, 96, 97]
+    n = len(seq_lens)
+    kp, vp, table, ks, vs = paged_setup(dtype, nkv, hd, page, seq_lens, 320, seed=13)
+    kp[kp == 50], vp[vp == -50] = float("nan"), float("nan")
+    pos = i32([l - 1 for l in seq_lens])
+    scale = 1 / math.sqrt(hd)
+    qkv = rnd(n, (nh + 2 * nkv) * hd, dtype=dtype, seed=9)
+    if raw:
+        inv = torch.from_numpy(rope_inv_freq(hd, 10000.0, "f32")).to(DEV)
+        gains = rnd(hd, seed=1) * 0.1 + 1, rnd(hd, seed=2) * 0.1 + 1
+        kp2, vp2, q = kp.clone(), vp.clone(), qkv.clone()
+        ops.qk_rope_kv(q, n, nh, nkv, hd, q_gain=gains[0], k_gain=gains[1], eps=1e-6, inv_freq=inv, rotary_dim=hd, variant="half_split", pos=pos,
+                       row_req=i32(list(range(n))), kpages=kp2, vpages=vp2, table=table, n_req=n)
+        out = ops.attention_decode_fused(qkv, n, nh, nkv, hd, kp, vp, table, n, pos, i32(list(range(n))), scale, q_gain=gains[0], k_gain=gains[1], eps=1e-6,
+                                         inv_freq=inv, rotary_dim=hd, variant="half_split", window=window, max_seq=4400, n_splits=n_splits, waves=waves,
+                                         cos_sin=ops.rope_table(inv, 33))
+        for r, l in enumerate(seq_lens):      # the new keys and values, and nothing else in the pages
+            pg = table[r, (l - 1) // page].item()
+            ks[r][l - 1], vs[r][l - 1] = kp2[pg, :, (l - 1) % page], vp2[pg, :, (l - 1) % page]
+        close(kp.nan_to_num(0), kp2.nan_to_num(0), dtype, "new keys in the pages", bf16=8e-3)
+        assert torch.equal(vp.nan_to_num(7), vp2.nan_to_num(7))
+    else:
+        q = qkv
+        out = ops.attention_decode(q, n, nh, nkv, hd, kp, vp, table, n, pos, None, scale, window, max_seq=4400, n_splits=n_splits, waves=waves)
+    for r, l in enumerate(seq_lens):
+        want = attention_reference(q[r:r + 1, :nh * hd].view(1, nh, hd), ks[r], vs[r], [l - 1], scale, window)
+        # (the weights and the output are bfloat16: 2^-9 of the largest value each, and 2^-8 for a raw row's keys and queries)
+        close(out[r].view(1, nh, hd), want, dtype, f"row of {l} keys", bf16=1e-2)
+
+
 @pytest.mark.parametrize("n_rows,nh,nkv,hd,n_splits", [(64, 32, 8, 64, 8), (3, 6, 2, 48, 5), (2, 4, 1, 128, 40),
                                                        (4200, 8, 8, 16, 2)])
 def test_slices_merged_by_the_last_to_finish_or_by_a_second_kernel(n_rows, nh, nkv, hd, n_splits):
