@@ -98,7 +98,9 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
   floatx4 (*red)[FT][RG][NT][WAVE] = reinterpret_cast<floatx4 (*)[FT][RG][NT][WAVE]>(smem);
   bf16x8* stage = reinterpret_cast<bf16x8*>(smem) + (size_t)(threadIdx.x / WAVE) * NT * 16 * CH;
   __shared__ float red_ss[WAVES][NT][16];
-  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  // (the wave's number as a scalar: its share of k, and where its operands of W begin, are then scalar arithmetic beside the
+  // vector units, which two waves of a SIMD share: 100 instructions in front of the first loads were 0.4 us of each call)
+  const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int r = lane % 16, g = lane / 16;
   const int o0 = blockIdx.x * ROWS * FT;
   // the wave's share of k, in whole MFMA steps of 32 (workgroups of 8 features: in pairs of steps)
@@ -119,39 +121,40 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
   const int k_begin = wave * per_wave * KU;
   const int k_end = min(a.I, k_begin + per_wave * KU);
 
-  // Where a lane's A operands lie: wrow + a_off(step), the step being the number of the 32-k tile (pairs: of
-  // the 64-k pair) from the start of k.  One expression for all layouts, so that no branch stands between loads:
+  // Where a lane's A operands lie: wrow (a scalar, in tile order) + a_off(step) + a_lane, the step being the number of the
+  // 32-k tile (pairs: of the 64-k pair) from the start of k.  One expression for all layouts, so that no branch stands between loads:
   //   j = min(step * a_unit + koff, a_limit);  offset = (j >> a_sh) * a_mul + (j & a_sh) * 64 - koff
   //   16-row tiles: tile j, 512 elements each.  Pair layout read by 16 features: pair j / 2, half j % 2.
   //   Row-major: element j of the row (a_unit elements per step).
-  bool row_ok[FT];
   const bf16* wrow[FT][RG];
+  uint32_t a_lane[FT];      // bytes
   int koff = 0, a_unit = 1, a_sh = 0, a_mul = 512;
   int a_limit = (k_end - 1) / KU;
   const int r8 = r % 8, half = r / 8;
 #pragma unroll
   for (int f = 0; f < FT; ++f) {
-    row_ok[f] = r < ROWS && o0 + f * ROWS + r < a.O;
+    a_lane[f] = lane * 16;
 #pragma unroll
     for (int q = 0; q < RG; ++q) {
       if (a.packed == 2) {
         // 8-row tiles of two k tiles: [row group][8-row tile][pair][g][half][r8][8]
         const size_t tiles8 = 2 * a.group_tiles;
-        if (PAIR) {
-          wrow[f][q] = a.W + ((q * tiles8 + o0 / 8) * a.ktiles) * 512 + lane * 8;
-        } else {
-          const size_t o8 = min((size_t)(o0 + f * ROWS) / 8 + half, tiles8 - 1);   // (beyond the last tile: unused rows)
-          wrow[f][q] = a.W + ((q * tiles8 + o8) * a.ktiles) * 512 + (g * 16 + r8) * 8;
+        const size_t o8 = (size_t)(o0 + f * ROWS) / 8;
+        wrow[f][q] = a.W + ((q * tiles8 + o8) * a.ktiles) * 512;
+        if (!PAIR) {
+          // (16 features: the tile behind o8 too; beyond the last tile: unused rows)
+          a_lane[f] = (half && o8 + 1 < tiles8 ? (uint32_t)a.ktiles * 1024 : 0u) + (g * 16 + r8) * 16;
           a_sh = 1;
         }
       } else if (a.packed) {
         // 16-row tiles (never read by workgroups of 8 features: the layout follows the number of rows)
         const int o_tile = min((o0 + f * ROWS) / 16, (int)a.group_tiles - 1);   // (beyond the last tile: unused rows)
-        wrow[f][q] = a.W + (((size_t)q * a.group_tiles + o_tile) * a.ktiles) * 512 + lane * 8;
+        wrow[f][q] = a.W + (((size_t)q * a.group_tiles + o_tile) * a.ktiles) * 512;
       } else {
-        const int row = PAIR ? (o0 + r8 < a.O ? o0 + r8 : 0) : (row_ok[f] ? o0 + f * ROWS + r : 0);
+        const int row = PAIR ? (o0 + r8 < a.O ? o0 + r8 : 0) : (r < ROWS && o0 + f * ROWS + r < a.O ? o0 + f * ROWS + r : 0);
         koff = (PAIR ? half * 32 : 0) + g * 8;
         wrow[f][q] = a.W + ((size_t)q * a.group_stride + row) * a.ldw + koff;
+        a_lane[f] = 0;
         a_unit = KU; a_limit = a.I - 8; a_mul = 1;
       }
     }
@@ -166,7 +169,7 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
   for (int t = 0; t < NT; ++t) {
     const int n = BP ? t * 8 + r8 : t * 16 + r;
     x_ok[t] = n < a.N;
-    xrow[t] = a.X + (size_t)(x_ok[t] ? n : 0) * a.ldx + (BP ? half * 32 : 0) + g * 8;
+    xrow[t] = a.X + (size_t)(x_ok[t] ? n : 0) * a.ldx;
   }
   // What the epilogue reads besides the product is asked for behind the first loads of the operands: the
   // product hides the latency (the state row hangs on a slot index, two dependent loads, and wave 0 would
@@ -223,7 +226,10 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
   // ranges and wraps around (the order of a feature's additions is fixed by its workgroup).
   const int n_iter = (k_end - k_begin + 32 * U - 1) / (32 * U);
   const int first_iter = (STAGE && n_iter > 0 && a.rotate) ? (int)(blockIdx.x % n_iter) : 0;
-  auto k_of = [&](int it) { return k_begin + ((it + first_iter) % n_iter) * 32 * U; };
+  auto k_of = [&](int it) {
+    const int at = it + first_iter;     // (first_iter < n_iter, and 0 without staging)
+    return k_begin + (STAGE && at >= n_iter ? at - n_iter : at) * 32 * U;
+  };
 
   // Operands live in registers for one iteration of U MFMA steps.  As soon as a step's operands have been
   // used, the same registers are asked for the next iteration's step: a wave keeps U steps of loads in
@@ -241,15 +247,29 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
   // before them: their registers would cost a second resident workgroup, or spill)
   constexpr bool ROLL_S = NT <= 2;
   bf16x8 av[UA][FT][RG], bv[UB][NT], sv[NT][LPT];
+  // (W in tile order: a load is a descriptor, the lane's 16 bytes and a scalar offset, no vector arithmetic; the offsets of a
+  // workgroup's tiles, one tile of rows over the whole of k, stay far below 4 GB)
+  __amdgpu_buffer_rsrc_t wbuf[FT][RG];
+  if constexpr (TILED) {
+#pragma unroll
+    for (int f = 0; f < FT; ++f)
+#pragma unroll
+      for (int q = 0; q < RG; ++q) wbuf[f][q] = __builtin_amdgcn_make_buffer_rsrc((void*)wrow[f][q], 0, 0x7fffffff, 0x00020000);
+  }
   auto load_a = [&](int k, int u) {   // u: the iteration's A operand
     const long off = a_off(k / KU + u);
 #pragma unroll
     for (int f = 0; f < FT; ++f)
 #pragma unroll
-      for (int q = 0; q < RG; ++q) av[u][f][q] = *(const bf16x8*)(wrow[f][q] + off);
+      for (int q = 0; q < RG; ++q) {
+        if constexpr (TILED) av[u][f][q] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(wbuf[f][q], a_lane[f], (int)off * 2, 0));
+        else av[u][f][q] = *(const bf16x8*)(wrow[f][q] + off);
+      }
   };
+  // (loads return in the order they were asked for: they stay in the order below, arithmetic may move across)
+  auto in_order = [] { __builtin_amdgcn_sched_barrier(0x7 | 0x8 | 0x380); };
   auto load_b = [&](int k, int u) {
-    const int kc = min(k + u * (BP ? 64 : 32) + xoff, a.I - 8) - xoff;
+    const uint32_t kc = min(k + u * (BP ? 64 : 32) + xoff, a.I - 8);
 #pragma unroll
     for (int t = 0; t < NT; ++t) bv[u][t] = *(const bf16x8*)(xrow[t] + kc);
   };
@@ -281,7 +301,7 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
 #pragma unroll
         for (int t = 0; t < NT; ++t) stage[(t * LPT + i) * WAVE + lane] = k_ok ? sv[t][i] : zero;
       }
-      if (ROLL_S && more) load_s(k_next);
+      if (ROLL_S && more) { load_s(k_next); in_order(); }
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -317,7 +337,10 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
           }
           if (more) load_a(k_next, 2 * u + 1);
         }
-        if (more) load_b(k_next, u);
+        if (more) {
+          load_b(k_next, u);
+          in_order();
+        }
       }
     } else {
 #pragma unroll
@@ -337,34 +360,62 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
               acc[f][q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[PAIR ? u / 2 : u][f][q], b, acc[f][q][t], 0, 0, 0);
           }
       }
-      if (more) {
+      if (more && (!STAGE || ROLL_S)) {
         if (!PAIR) load_a(k_next, u);
         else if (u % 2 == 1) load_a(k_next, u / 2);
         if (!STAGE) load_b(k_next, u);
+        in_order();
       }
     }
     }
-    if (STAGE && !ROLL_S && more) load_s(k_next);
+    if (STAGE && !ROLL_S && more) {   // (the rows of X first: they go to LDS before the first product)
+      load_s(k_next);
+      in_order();
+#pragma unroll
+      for (int u = 0; u < UA; ++u) load_a(k_next, u);
+    }
   };
+  // (what other loads of the epilogue hang on goes first: it arrives before the operands, and the state rows' loads need
+  // not wait for those)
+  int slot_epi = 0, before_epi = 0;
+  if (EPI == EPI_CONV && KC > 1 && epi_lane) { slot_epi = a.slot[n_epi]; before_epi = a.ctx[n_epi]; }
   if (n_iter > 0) {
     const int k = k_of(0);
-    if (STAGE) load_s(k);
+    if (STAGE) { load_s(k); in_order(); }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (u < UA) load_a(k, u);
       if (!STAGE && u < UB) load_b(k, u);
+      in_order();
     }
   }
-  if (EPI == EPI_RESIDUAL) {
+  // (a lane's four features in one load each where rows and pointers allow it)
+  const bool epi_vec = a.y_vec && o_epi + 3 < a.O;
+  auto load4 = [&](float (&to)[4], const float* from) {
+    if (epi_vec) {
+      const floatx4 v = epi_lane ? *(const floatx4*)from : floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) pre_x[i] = (epi_lane && o_epi + i < a.O) ? a.x[(size_t)n_epi * a.O + o_epi + i] : 0.f;
-  }
+      for (int i = 0; i < 4; ++i) to[i] = v[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) to[i] = (epi_lane && o_epi + i < a.O) ? from[i] : 0.f;
+    }
+  };
+  if (EPI == EPI_RESIDUAL && wave < FT * NT) load4(pre_x, a.x + (size_t)n_epi * a.O + o_epi);
   if (EPI == EPI_ACT && a.mult) {
     const int id = epi_lane ? min(max(a.ids[n_epi], 0), a.vocab - 1) : 0;      // (never read outside the table)
 #pragma unroll
     for (int i = 0; i < 4; ++i) pre_x[i] = (epi_lane && o_epi + i < a.O) ? (float)a.mult[(size_t)id * a.mult_ld + o_epi + i] : 0.f;
   }
-  if (EPI == EPI_CONV && KC > 1) {
+  if (EPI == EPI_CONV && KC > 1 && wave < FT * NT) {
+    const float* st = a.state + (size_t)slot_epi * a.slot_stride + o_epi;
+#pragma unroll
+    for (int j = 0; j < KH; ++j) {
+      // (rows before the start of a request are zero)
+      load4(pre_hist[j], st + (size_t)j * a.O);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) pre_hist[j][i] = before_epi - (KC - 1) + j >= 0 ? pre_hist[j][i] : 0.f;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const bool ok = epi_lane && o_epi + i < a.O;
@@ -372,13 +423,6 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
       for (int j = 0; j < KC; ++j) pre_taps[j][i] = ok ? a.taps[(size_t)(o_epi + i) * KC + j] : 0.f;
       pre_bias[i] = (ok && a.bias) ? a.bias[o_epi + i] : 0.f;
     }
-    const float* st = a.state + (size_t)(epi_lane ? a.slot[n_epi] : 0) * a.slot_stride;
-    const int before = epi_lane ? a.ctx[n_epi] : 0;
-#pragma unroll
-    for (int j = 0; j < KH; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        pre_hist[j][i] = (epi_lane && o_epi + i < a.O && before - (KC - 1) + j >= 0) ? st[(size_t)j * a.O + o_epi + i] : 0.f;
   }
 
   if (n_iter > 0) {
@@ -404,36 +448,53 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
       if (g == r / 4) red_ss[wave][t][r] = d;   // (paired B operands: rows 8..15 are rows 0..7 at k + 32)
     }
   }
-  // the waves' partial products meet in LDS; wave f * NT + t adds those of its tile in the order of the waves
-  // (8 features: lanes g < 2 hold them in the first accumulator, lanes g >= 2 in the second; lane l < 32 then
-  // adds what lane l + 32 left)
+  // the waves' partial products meet in LDS; wave f * NT + t adds those of its tile in the order of the waves.  With 8 features
+  // a wave's own two halves are added first: lanes g < 2 hold the first, lanes g >= 2 the second, in the second accumulator, or
+  // (paired B operands) 8 columns on in the same one.
 #pragma unroll
   for (int f = 0; f < FT; ++f)
 #pragma unroll
     for (int q = 0; q < RG; ++q)
 #pragma unroll
-      for (int t = 0; t < NT; ++t) red[wave][f][q][t][lane] = (PAIR && !BP && g >= 2) ? acc_hi[PAIR ? q : 0][t] : acc[f][q][t];
+      for (int t = 0; t < NT; ++t) {
+        floatx4 v = acc[f][q][t];
+        if (PAIR) {
+          const floatx4 second = BP ? v : acc_hi[PAIR ? q : 0][t];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const uint32_t x = __float_as_uint(second[i]);
+            uint32_t up = __builtin_amdgcn_permlane32_swap(x, x, false, false)[1];      // (lanes below 32: what lane + 32 holds)
+            if (BP) up = __builtin_amdgcn_update_dpp(0, (int)up, 0x128 /* row_ror:8 */, 0xf, 0xf, false);
+            v[i] += __uint_as_float(up);
+          }
+        }
+        red[wave][f][q][t][lane] = v;
+      }
   __syncthreads();
   if (wave >= FT * NT) return;
-  // (paired B operands: the second half of feature (g, i) and row r is at rows + 8, columns + 8 of the tile)
-  const int partner = BP ? (lane + 40) & 63 : (lane & 31) + 32;   // (8 features only)
+  // (every read is asked for before the first is used: one by one they were 0.3 us at the end of each call)
+  floatx4 part[WAVES][RG];
+  float squares[WAVES][BP ? 2 : 1];
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    if (RMS) {
+      squares[w][0] = red_ss[w][t_epi][r];
+      if (BP) squares[w][BP ? 1 : 0] = red_ss[w][t_epi][(r + 8) & 15];
+    }
+#pragma unroll
+    for (int q = 0; q < RG; ++q) part[w][q] = red[w][f_epi][q][t_epi][lane];
+  }
+  __builtin_amdgcn_sched_barrier(0);
   floatx4 sum[RG];
 #pragma unroll
   for (int q = 0; q < RG; ++q) {
-    sum[q] = red[0][f_epi][q][t_epi][lane];
-    if (PAIR) sum[q] += red[0][f_epi][q][t_epi][partner];
+    sum[q] = part[0][q];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) sum[q] += part[w][q];
   }
-#pragma unroll
-  for (int w = 1; w < WAVES; ++w)
-#pragma unroll
-    for (int q = 0; q < RG; ++q) {
-      sum[q] += red[w][f_epi][q][t_epi][lane];
-      if (PAIR) sum[q] += red[w][f_epi][q][t_epi][partner];
-    }
 
   // D[feature g*4 + i][row r] of the tile: lane holds 4 consecutive features of one row
   {
-    const int t = t_epi;
     const int n = n_epi;
     const int o = o_epi;
     if (n >= a.N || r >= TILE_ROWS || g * 4 >= ROWS || o >= a.O) return;
@@ -441,7 +502,7 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
     if (RMS) {
       float tot = 0.f;
 #pragma unroll
-      for (int w = 0; w < WAVES; ++w) tot += red_ss[w][t][r] + (BP ? red_ss[w][t][(r + 8) & 15] : 0.f);
+      for (int w = 0; w < WAVES; ++w) tot += squares[w][0] + (BP ? squares[w][BP ? 1 : 0] : 0.f);
       scale = __builtin_amdgcn_rsqf(tot * a.inv_I + a.eps);   // (1 ulp: the outputs are rounded to bfloat16, or added to a stream that is)
     }
     const bool full = o + 3 < a.O;
@@ -476,16 +537,33 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
       bf16* y = a.Y + (size_t)n * a.ldy + o;
       bf16 v[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = (bf16)(activate(sum[0][i], a.act) * (a.mult ? pre_x[i] : 1.0f));
+      for (int i = 0; i < 4; ++i) pre_x[i] = a.mult ? pre_x[i] : 1.0f;
+      if (a.act == ACT_GELU_TANH) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (bf16)(activate(sum[0][i], ACT_GELU_TANH) * pre_x[i]);
+      } else if (a.act == ACT_RELU_SQUARED) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (bf16)(activate(sum[0][i], ACT_RELU_SQUARED) * pre_x[i]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (bf16)(activate(sum[0][i], a.act) * pre_x[i]);
+      }
       if (full && a.y_vec) *(bf16x4*)y = bf16x4{v[0], v[1], v[2], v[3]};
       else for (int i = 0; i < 4 && o + i < a.O; ++i) y[i] = v[i];
     } else if (EPI == EPI_GLU) {
       bf16* y = a.Y + (size_t)n * a.ldy + o;
       bf16 v[4];
+      // (which activation is asked once, not for each value: the jumps between them were 0.7 to 1.1 us at the end of a call)
+      const floatx4 gt = sum[0] * scale, up = sum[RG > 1 ? 1 : 0] * scale;
+      if (a.act == ACT_SILU) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float gt = sum[0][i] * scale, up = sum[RG > 1 ? 1 : 0][i] * scale;
-        v[i] = (bf16)(a.act == ACT_CLAMPED_SWISH ? clamped_swish_product(gt, up, a.act_alpha, a.act_limit) : activate_to_bf16(gt, a.act) * up);
+        for (int i = 0; i < 4; ++i) v[i] = (bf16)(activate_to_bf16(gt[i], ACT_SILU) * up[i]);
+      } else if (a.act == ACT_CLAMPED_SWISH) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (bf16)clamped_swish_product(gt[i], up[i], a.act_alpha, a.act_limit);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (bf16)(activate(gt[i], a.act) * up[i]);
       }
       if (full && a.y_vec) *(bf16x4*)y = bf16x4{v[0], v[1], v[2], v[3]};
       else for (int i = 0; i < 4 && o + i < a.O; ++i) y[i] = v[i];
