@@ -5,6 +5,7 @@
 #include <stdint.h>
 #include <stdio.h>
 #include <stdarg.h>
+#include <type_traits>
 
 typedef __bf16 bf16;
 
@@ -39,15 +40,46 @@ template <> __device__ __forceinline__ bf16 from_float<bf16>(float v) { return (
 
 constexpr int WAVE = 64;
 
+// What lane (lane ^ MASK) holds, by moves between lanes of the vector units (4 to 12 cycles) instead of a trip through LDS (some 120,
+// and such exchanges come six in a row).  All 64 lanes take part.
+template <int MASK>
+__device__ __forceinline__ uint32_t lane_xor_bits(uint32_t v) {
+  static_assert(MASK == 1 || MASK == 2 || MASK == 4 || MASK == 8 || MASK == 16 || MASK == 32, "one bit of the lane's number");
+  if constexpr (MASK >= 16) {
+    const auto both = [&] {
+      if constexpr (MASK == 32) return __builtin_amdgcn_permlane32_swap(v, v, false, false);
+      else return __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    }();      // [0]: of each pair of halves the lower one's value in both, [1]: the upper one's
+    return (threadIdx.x & MASK) ? both[0] : both[1];
+  } else if constexpr (MASK == 4) {      // (lane i -> 7 - i, then quads reversed: i -> i ^ 7 ^ 3)
+    return __builtin_amdgcn_update_dpp(0, __builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true), 0x1B, 0xf, 0xf, true);
+  } else {
+    constexpr int CTRL = MASK == 1 ? 0xB1 : (MASK == 2 ? 0x4E : 0x128);      // quad_perm [1,0,3,2], [2,3,0,1], row_ror:8
+    return __builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
+  }
+}
+template <int MASK>
+__device__ __forceinline__ float lane_xor_float(float v) { return __uint_as_float(lane_xor_bits<MASK>(__float_as_uint(v))); }
+// f(v, what lane ^ 32 has), then lane ^ 16, 8, 4, 2, 1: every lane gets the same result of a commutative f.
+template <typename T, typename F>
+__device__ __forceinline__ T wave_fold(T v, F f) {
+  static_assert(sizeof(T) == 4, "a register");
+  const auto bits = [](T x) { return __builtin_bit_cast(uint32_t, x); };
+  const auto from = [](uint32_t x) { return __builtin_bit_cast(T, x); };
+  const auto a = __builtin_amdgcn_permlane32_swap(bits(v), bits(v), false, false);
+  v = f(from(a[0]), from(a[1]));
+  const auto b = __builtin_amdgcn_permlane16_swap(bits(v), bits(v), false, false);
+  v = f(from(b[0]), from(b[1]));
+  v = f(v, from(lane_xor_bits<8>(bits(v))));
+  v = f(v, from(lane_xor_bits<4>(bits(v))));
+  v = f(v, from(lane_xor_bits<2>(bits(v))));
+  return f(v, from(lane_xor_bits<1>(bits(v))));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-  return v;
+  return wave_fold(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = WAVE / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, WAVE));
-  return v;
+  return wave_fold(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Sum over a block of up to 1024 threads; every thread gets the result.  `scratch` holds
@@ -59,6 +91,17 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
   __syncthreads();
   if (lane == 0) scratch[wave] = v;
   __syncthreads();
+  // (read side by side where their number is a usual one: one by one they were a tenth of a microsecond each)
+  auto together = [&](auto count) {
+    float part[decltype(count)::value], total = 0.f;
+#pragma unroll
+    for (int i = 0; i < decltype(count)::value; ++i) part[i] = scratch[i];
+#pragma unroll
+    for (int i = 0; i < decltype(count)::value; ++i) total += part[i];
+    return total;
+  };
+  if (n_waves == 8) return together(std::integral_constant<int, 8>{});
+  if (n_waves == 4) return together(std::integral_constant<int, 4>{});
   float total = 0.f;
   for (int i = 0; i < n_waves; ++i) total += scratch[i];
   return total;

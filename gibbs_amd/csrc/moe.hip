@@ -157,12 +157,17 @@ __device__ __forceinline__ void choose_experts(float* z, float* score, int n, in
       const float v = z[e];
       if (v == v && (v > pv || (v == pv && e < pick) || pick == 0x7fffffff)) { pv = v; pick = e; }
     }
-#pragma unroll
-    for (int o = WAVE / 2; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(pv, o, WAVE);
-      const int op = __shfl_xor(pick, o, WAVE);
-      if (op != 0x7fffffff && (pick == 0x7fffffff || ov > pv || (ov == pv && op < pick))) { pv = ov; pick = op; }
-    }
+    auto meet = [&](float ov, int op) {
+      const bool other = op != 0x7fffffff && (pick == 0x7fffffff || ov > pv || (ov == pv && op < pick));
+      pv = other ? ov : pv;
+      pick = other ? op : pick;
+    };
+    meet(lane_xor_float<32>(pv), lane_xor_bits<32>(pick));
+    meet(lane_xor_float<16>(pv), lane_xor_bits<16>(pick));
+    meet(lane_xor_float<8>(pv), lane_xor_bits<8>(pick));
+    meet(lane_xor_float<4>(pv), lane_xor_bits<4>(pick));
+    meet(lane_xor_float<2>(pv), lane_xor_bits<2>(pick));
+    meet(lane_xor_float<1>(pv), lane_xor_bits<1>(pick));
     if (pick == 0x7fffffff) {   // (fewer usable logits than choices: the first expert not taken yet, with no weight)
       __builtin_amdgcn_s_waitcnt(0);
       for (int e = 0; e < E && pick == 0x7fffffff; ++e) {

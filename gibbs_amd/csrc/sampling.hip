@@ -19,12 +19,17 @@ __device__ __forceinline__ bool better(float v, int i, float bv, int bi) {
 
 // Best (value, index) over the block under `better`; all threads get it.
 __device__ __forceinline__ void block_best(float& v, int& i, float* sv, int* si) {
-#pragma unroll
-  for (int o = WAVE / 2; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(v, o, WAVE);
-    const int oi = __shfl_xor(i, o, WAVE);
-    if (better(ov, oi, v, i)) { v = ov; i = oi; }
-  }
+  auto meet = [&](float ov, int oi) {
+    const bool other = better(ov, oi, v, i);
+    v = other ? ov : v;
+    i = other ? oi : i;
+  };
+  meet(lane_xor_float<32>(v), lane_xor_bits<32>(i));
+  meet(lane_xor_float<16>(v), lane_xor_bits<16>(i));
+  meet(lane_xor_float<8>(v), lane_xor_bits<8>(i));
+  meet(lane_xor_float<4>(v), lane_xor_bits<4>(i));
+  meet(lane_xor_float<2>(v), lane_xor_bits<2>(i));
+  meet(lane_xor_float<1>(v), lane_xor_bits<1>(i));
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   __syncthreads();
   if (lane == 0) { sv[wave] = v; si[wave] = i; }
@@ -163,13 +168,10 @@ __global__ __launch_bounds__(THREADS) void sample_kernel(const float* __restrict
   const int per_wave = (k + WAVES - 1) / WAVES;
   unsigned rest = mine, nth = 0;
   for (int c = 0; c < per_wave; ++c) {
-    nth = rest;
-#pragma unroll
-    for (int o = WAVE / 2; o > 0; o >>= 1) nth = max(nth, (unsigned)__shfl_xor((int)nth, o, WAVE));
+    nth = wave_fold(rest, [](unsigned a, unsigned b) { return max(a, b); });
     if (rest == nth) rest = 0;
   }
-#pragma unroll
-  for (int o = WAVE / 2; o > 0; o >>= 1) valid += __shfl_xor(valid, o, WAVE);
+  valid = wave_fold(valid, [](int a, int b) { return a + b; });
   __syncthreads();
   if (lane == 0) {
     wave_low[wave] = nth;
@@ -311,6 +313,13 @@ __global__ __launch_bounds__(THREADS) void decode_tail_kernel(const float* __res
   __shared__ int s_token;
   const int i = blockIdx.x;
   const bool padding = live && live[i] == 0;
+  // (what one thread keeps count of, and what it reads for that, is asked for before the walk over the logits)
+  int step = 0, at = 0, cached = 0;
+  float draw = 0.f;
+  if (threadIdx.x == 0 && !padding) {
+    step = steps[i]; at = pos[i]; cached = ctx[i];
+    if (u && step + 1 < capacity) draw = u_all[(size_t)(step + 1) * n + i];
+  }
   int token = 0;
   if (logits && !padding) {
     const float* row = logits + (size_t)i * ld;
@@ -326,11 +335,10 @@ __global__ __launch_bounds__(THREADS) void decode_tail_kernel(const float* __res
     if (logits && !padding) ids[i] = token;
     else token = ids[i];
     if (!padding) {
-      const int step = steps[i];
       if (step < capacity) log[(size_t)step * n + i] = token;
-      pos[i] += 1;
-      ctx[i] += 1;
-      if (u && step + 1 < capacity) u[i] = u_all[(size_t)(step + 1) * n + i];
+      pos[i] = at + 1;
+      ctx[i] = cached + 1;
+      if (u && step + 1 < capacity) u[i] = draw;
       steps[i] = step + 1;
     }
     s_token = token;
