@@ -18,7 +18,7 @@ __global__ void embed_kernel(const T* __restrict__ table, const int* __restrict_
   id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
   const T* row = table + (size_t)id * hidden;
   float* out = x + (size_t)n * hidden;
-  for (int i = threadIdx.x; i < hidden; i += blockDim.x) {
+  for (int i = blockIdx.y * blockDim.x + threadIdx.x; i < hidden; i += gridDim.y * blockDim.x) {
     float v = to_float(row[i]) * scale;
     if (inv_freq && i / 2 < hidden / 2) {
       const float angle = (float)pos[n] * inv_freq[i / 2];
@@ -37,11 +37,14 @@ GIBBS_EXPORT int gibbs_embed_general(const void* table, int dtype, const int* id
   GIBBS_REQUIRE(n >= 0 && hidden > 0 && vocab > 0, "embed: bad sizes n=%d hidden=%d vocab=%d", n, hidden, vocab);
   GIBBS_REQUIRE(!inv_freq || pos, "embed: a position vector needs the rows' positions");
   if (n == 0) return 0;
+  // (a row's sines are long code that each thread walks once for each of its columns: few rows share theirs out over workgroups.  8 rows of
+  // 2,048 with a position vector, us: a workgroup a row 10.2, eight 2.9)
   const int threads = hidden >= 1024 ? 256 : 64;
+  const dim3 grid(n, inv_freq && n <= 128 ? ceil_div(hidden, threads) : 1);
   if (dtype == GIBBS_F32)
-    embed_kernel<float><<<n, threads, 0, stream>>>((const float*)table, ids, x, (bf16*)mirror, hidden, vocab, scale, pos, inv_freq, keep);
+    embed_kernel<float><<<grid, threads, 0, stream>>>((const float*)table, ids, x, (bf16*)mirror, hidden, vocab, scale, pos, inv_freq, keep);
   else if (dtype == GIBBS_BF16)
-    embed_kernel<bf16><<<n, threads, 0, stream>>>((const bf16*)table, ids, x, (bf16*)mirror, hidden, vocab, scale, pos, inv_freq, keep);
+    embed_kernel<bf16><<<grid, threads, 0, stream>>>((const bf16*)table, ids, x, (bf16*)mirror, hidden, vocab, scale, pos, inv_freq, keep);
   else
     return gibbs_fail("embed: unknown dtype %d", dtype);
   GIBBS_LAUNCH_STATUS("embed");

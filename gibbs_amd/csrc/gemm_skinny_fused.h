@@ -44,6 +44,7 @@ struct FusedArgs {
   float* Yf;
   int y_vec;   // a lane's four features take one store (rows and pointers are aligned for it)
   long ldy;
+  long y_apart;   // MANY: values of Y from one product to the next
   // RESIDUAL
   float* x;   // [N, O] float32, updated in place
   bf16* xb;   // [N, O] mirror
@@ -70,7 +71,9 @@ struct FusedArgs {
 // than one or two MFMA tiles: X is re-read from L2 by every workgroup, so a workgroup should use
 // each B operand for more of W).  Wave f * NT + t sums tile f of features and tile t of rows over the waves
 // and runs its epilogue.
-template <bool TILED, int NT, int RG, int ROWS, int FT, int WAVES, bool RMS, int EPI, int KC, bool STAGE, bool BP = false>
+// MANY: several products of one size in a launch, the second dimension of the grid: matrices one behind the other in tile order, `rotate`
+// values of X from one's rows to the next's (0: the same rows), y_apart of Y.
+template <bool TILED, int NT, int RG, int ROWS, int FT, int WAVES, bool RMS, int EPI, int KC, bool STAGE, bool BP = false, bool MANY = false>
 __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const bf16* W, const bf16* X, int N, int O, int I, int packed,
                                                                          int ktiles, int rotate, long group_tiles, long ldx,
                                                                          long ldw, FusedArgs rest) {
@@ -83,6 +86,12 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
   // TILED: W is in tile order (pairs for workgroups of 8 features, else whichever the matrix has); not TILED:
   // row-major.  Known at compile time, the other layouts' address arithmetic is not in the way of the first loads.
   a.packed = TILED ? (ROWS == 8 ? 2 : (packed == 2 ? 2 : 1)) : 0;
+  static_assert(!MANY || (TILED && RG == 1 && EPI == EPI_STORE), "several products: of matrices in tile order, stored");
+  if constexpr (MANY) {
+    a.W += (size_t)blockIdx.y * group_tiles * ktiles * (a.packed == 2 ? 1024 : 512);
+    a.X += (size_t)blockIdx.y * rotate;
+    a.rotate = 1;
+  }
   static_assert(FT * NT <= WAVES && (FT == 1 || EPI == EPI_STORE || EPI == EPI_GLU), "several tiles: store and GLU only; a wave per tile of the result");
   // STAGE (more than a few rows of X): a wave brings its part of X in through LDS, 128 contiguous bytes or
   // more of a row per request instead of the 64 that a lane group of an MFMA operand covers (the memory
@@ -515,6 +524,7 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
       }
     } else if (EPI == EPI_STORE) {
       bf16* y = a.Y + (size_t)n * a.ldy + o;
+      if constexpr (MANY) y += blockIdx.y * a.y_apart;
       if (full && a.ldy % 4 == 0) {
         *(bf16x4*)y = bf16x4{(bf16)(sum[0][0] * scale), (bf16)(sum[0][1] * scale), (bf16)(sum[0][2] * scale),
                              (bf16)(sum[0][3] * scale)};
@@ -632,37 +642,37 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
 
 #define FUSED_KERNEL_ARGS(a) (a).W, (a).X, (a).N, (a).O, (a).I, (a).packed, (a).ktiles, (a).rotate, (a).group_tiles, (a).ldx, (a).ldw, (a)
 
-template <bool TILED, int NT, bool ST, int RG, bool RMS, int EPI, int KC>
-void launch_rows(const FusedArgs& a, hipStream_t s) {
+template <bool TILED, int NT, bool ST, int RG, bool RMS, int EPI, int KC, bool MANY>
+void launch_rows(const FusedArgs& a, int products, hipStream_t s) {
   constexpr int tiles2_from = 192;   // pairs of tiles from which a workgroup takes two (measured at 33 to 64 rows)
   if constexpr (NT >= 2 && (EPI == EPI_STORE || EPI == EPI_GLU)) {
     // many rows of X: two tiles of 16 features per workgroup where that still leaves enough workgroups
     // (also where single tiles would need a second round of workgroups that pairs do not: 257 to 383 tiles)
     if (a.O / 32 >= tiles2_from || (ceil_div(a.O, 16) > 256 && a.O / 32 >= 128)) {
-      gemm_skinny_fused_kernel<TILED, NT, RG, 16, 2, 8, RMS, EPI, KC, ST><<<ceil_div(a.O, 32), 8 * WAVE, 0, s>>>(FUSED_KERNEL_ARGS(a));
+      gemm_skinny_fused_kernel<TILED, NT, RG, 16, 2, 8, RMS, EPI, KC, ST, false, MANY><<<dim3(ceil_div(a.O, 32), products), 8 * WAVE, 0, s>>>(FUSED_KERNEL_ARGS(a));
       return;
     }
   }
   // few features: halve the rows per workgroup so that every compute unit gets one
   if ((NT <= 2 || EPI == EPI_CONV) && pair_layout(a.O)) {
     if constexpr (NT == 1 && !ST) {   // paired B operands: one tile of 8 rows of X, or two
-      if (a.N <= 8) gemm_skinny_fused_kernel<TILED, 1, RG, 8, 1, 8, RMS, EPI, KC, ST, true><<<ceil_div(a.O, 8), 8 * WAVE, 0, s>>>(FUSED_KERNEL_ARGS(a));
-      else gemm_skinny_fused_kernel<TILED, 2, RG, 8, 1, 8, RMS, EPI, KC, ST, true><<<ceil_div(a.O, 8), 8 * WAVE, 0, s>>>(FUSED_KERNEL_ARGS(a));
+      if (a.N <= 8) gemm_skinny_fused_kernel<TILED, 1, RG, 8, 1, 8, RMS, EPI, KC, ST, true, MANY><<<dim3(ceil_div(a.O, 8), products), 8 * WAVE, 0, s>>>(FUSED_KERNEL_ARGS(a));
+      else gemm_skinny_fused_kernel<TILED, 2, RG, 8, 1, 8, RMS, EPI, KC, ST, true, MANY><<<dim3(ceil_div(a.O, 8), products), 8 * WAVE, 0, s>>>(FUSED_KERNEL_ARGS(a));
     } else {
-      gemm_skinny_fused_kernel<TILED, NT, RG, 8, 1, 8, RMS, EPI, KC, ST><<<ceil_div(a.O, 8), 8 * WAVE, 0, s>>>(FUSED_KERNEL_ARGS(a));
+      gemm_skinny_fused_kernel<TILED, NT, RG, 8, 1, 8, RMS, EPI, KC, ST, false, MANY><<<dim3(ceil_div(a.O, 8), products), 8 * WAVE, 0, s>>>(FUSED_KERNEL_ARGS(a));
     }
   } else {
     if constexpr (NT == 1 && !ST) {
-      if (a.N <= 8) gemm_skinny_fused_kernel<TILED, 1, RG, 16, 1, 8, RMS, EPI, KC, ST, true><<<ceil_div(a.O, 16), 8 * WAVE, 0, s>>>(FUSED_KERNEL_ARGS(a));
-      else gemm_skinny_fused_kernel<TILED, 2, RG, 16, 1, 8, RMS, EPI, KC, ST, true><<<ceil_div(a.O, 16), 8 * WAVE, 0, s>>>(FUSED_KERNEL_ARGS(a));
+      if (a.N <= 8) gemm_skinny_fused_kernel<TILED, 1, RG, 16, 1, 8, RMS, EPI, KC, ST, true, MANY><<<dim3(ceil_div(a.O, 16), products), 8 * WAVE, 0, s>>>(FUSED_KERNEL_ARGS(a));
+      else gemm_skinny_fused_kernel<TILED, 2, RG, 16, 1, 8, RMS, EPI, KC, ST, true, MANY><<<dim3(ceil_div(a.O, 16), products), 8 * WAVE, 0, s>>>(FUSED_KERNEL_ARGS(a));
     } else {
-      gemm_skinny_fused_kernel<TILED, NT, RG, 16, 1, 8, RMS, EPI, KC, ST><<<ceil_div(a.O, 16), 8 * WAVE, 0, s>>>(FUSED_KERNEL_ARGS(a));
+      gemm_skinny_fused_kernel<TILED, NT, RG, 16, 1, 8, RMS, EPI, KC, ST, false, MANY><<<dim3(ceil_div(a.O, 16), products), 8 * WAVE, 0, s>>>(FUSED_KERNEL_ARGS(a));
     }
   }
 }
 
-template <bool TILED, int RG, bool RMS, int EPI, int KC = 0>
-void launch_nt(const FusedArgs& a, hipStream_t s) {
+template <bool TILED, int RG, bool RMS, int EPI, int KC = 0, bool MANY = false>
+void launch_nt(const FusedArgs& a, hipStream_t s, int products = 1) {
   // Up to 16 rows of X come straight into paired B operands, except 9 to 16 rows where the product has no more
   // workgroups than the chip has compute units: those come through LDS.  Measured over whole decode steps of
   // three model shapes (hidden sizes 1024, 2048 and 2048 with wider feed-forwards): products of up to 2048
@@ -672,11 +682,11 @@ void launch_nt(const FusedArgs& a, hipStream_t s) {
   constexpr int one_round = 256;   // workgroups of 8 features that get a compute unit each
   const bool staged = a.N > 8 && ceil_div(a.O, 8) <= one_round;
   const int nt = ceil_div(a.N, 16);
-  if (nt == 1 && !staged) launch_rows<TILED, 1, false, RG, RMS, EPI, KC>(a, s);
-  else if (nt == 1) launch_rows<TILED, 1, true, RG, RMS, EPI, KC>(a, s);
-  else if (nt == 2) launch_rows<TILED, 2, true, RG, RMS, EPI, KC>(a, s);
-  else if (nt == 3) launch_rows<TILED, 3, true, RG, RMS, EPI, KC>(a, s);
-  else launch_rows<TILED, 4, true, RG, RMS, EPI, KC>(a, s);
+  if (nt == 1 && !staged) launch_rows<TILED, 1, false, RG, RMS, EPI, KC, MANY>(a, products, s);
+  else if (nt == 1) launch_rows<TILED, 1, true, RG, RMS, EPI, KC, MANY>(a, products, s);
+  else if (nt == 2) launch_rows<TILED, 2, true, RG, RMS, EPI, KC, MANY>(a, products, s);
+  else if (nt == 3) launch_rows<TILED, 3, true, RG, RMS, EPI, KC, MANY>(a, products, s);
+  else launch_rows<TILED, 4, true, RG, RMS, EPI, KC, MANY>(a, products, s);
 }
 
 template <bool TILED, bool RMS>

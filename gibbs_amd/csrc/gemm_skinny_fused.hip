@@ -62,6 +62,22 @@ int gibbs_skinny_store_as(const void* X, const void* W, void* Y, int out_dtype, 
   GIBBS_LAUNCH_STATUS("skinny_store");
 }
 
+// `products` of these in one launch: W holds as many matrices [O, I] one behind the other, each in tile order by itself; product p reads the rows at
+// X + p x_apart (0: the same rows) and writes at Y + p y_apart.  Four of 8 rows x 2,048 x 2,048 take 7.5 us so, and 17.5 one after
+// the other: a launch's path from its first instruction to its last store is 3 us whatever it multiplies.
+GIBBS_EXPORT int gibbs_skinny_store_many(const void* X, long x_apart, const void* W, int products, void* Y, long y_apart, int N, int O, int I,
+                                         long ldx, long ldy, hipStream_t stream) {
+  if (check_common("skinny_store_many", X, W, N, O, I, ldx, 0)) return 1;
+  GIBBS_REQUIRE(ldy >= O, "skinny_store_many: output rows shorter than %d", O);
+  GIBBS_REQUIRE(products > 0 && products <= 65535 && x_apart >= 0 && x_apart % 8 == 0 && x_apart <= 0x7fffffffl && y_apart >= 0 && y_apart % 4 == 0 && ((uintptr_t)Y % 8) == 0,
+                "skinny_store_many: %d products, %ld and %ld values apart", products, x_apart, y_apart);
+  FusedArgs a{};
+  a.W = (const bf16*)W; a.X = (const bf16*)X; a.N = N; a.O = O; a.I = I; a.ldx = ldx; note_layout(a);
+  a.Y = (bf16*)Y; a.ldy = ldy; a.y_apart = y_apart; a.rotate = (int)x_apart;
+  launch_nt<true, 1, false, EPI_STORE, 0, true>(a, stream, products);
+  GIBBS_LAUNCH_STATUS("skinny_store_many");
+}
+
 // x[n, o] += sum_k X[n, k] W[o, k];  xb[n, o] = bfloat16(x[n, o]).  x: [N, O] float32, xb: [N, O] bfloat16.
 GIBBS_EXPORT int gibbs_skinny_residual(const void* X, const void* W, float* x, void* xb, int N, int O, int I, long ldx,
                                        long ldw, hipStream_t stream) {
@@ -104,7 +120,7 @@ GIBBS_EXPORT int gibbs_skinny_act(const void* X, const void* W, void* Y, int N, 
                                   const void* mult, long mult_ld, const int* ids, int vocab, hipStream_t stream) {
   if (check_common("skinny_act", X, W, N, O, I, ldx, ldw)) return 1;
   GIBBS_REQUIRE(ldy >= O, "skinny_act: output rows shorter than %d", O);
-  GIBBS_REQUIRE((act >= 0 && act < ACT_COUNT) || act == ACT_RELU_SQUARED, "skinny_act: unknown activation %d", act);
+  GIBBS_REQUIRE((act >= 0 && act < ACT_COUNT) || act == ACT_RELU_SQUARED || act == ACT_TANH, "skinny_act: unknown activation %d", act);
   GIBBS_REQUIRE(!mult || (ids && vocab > 0 && mult_ld >= O), "skinny_act: a table without the rows' tokens, or rows of %ld entries", mult_ld);
   FusedArgs a{};
   a.W = (const bf16*)W; a.X = (const bf16*)X; a.N = N; a.O = O; a.I = I; a.ldw = ldw; a.ldx = ldx; note_layout(a);

@@ -252,6 +252,8 @@ int gibbs_token_shift(const void* h, int dtype, const float* mu, int n_mix, floa
                       hipStream_t stream);
 int gibbs_tanh_rows(const float* in, void* out, int dtype, long count, hipStream_t stream);
 int gibbs_double_exp_decay(float* z, const float* bias, long count, int C, hipStream_t stream);
+int gibbs_add_rmsnorm_mirror(float* x, const void* delta, int parts, long apart, const float* gain, float eps, void* out, void* mirror, int dtype,
+                             int n, int hidden, hipStream_t stream);
 int gibbs_add_rmsnorm(float* x, const void* delta, const float* gain, float eps, void* out, int dtype, const int* rows,
                       int n_out, int hidden, hipStream_t stream);
 int gibbs_add_partials_rmsnorm(float* x, const float* partials, int n_partials, long partial_stride, const float* gain,
@@ -269,6 +271,8 @@ int gibbs_gemm_library(const void* A, const void* W, void* C, int N, int O, int 
                        hipStream_t stream);
 int gibbs_gemm_skinny(const void* X, const void* W, void* Y, int out_dtype, int N, int O, int I, long ldx, long ldw,
                       long ldy, int k_splits, hipStream_t stream);
+int gibbs_skinny_store_many(const void* X, long x_apart, const void* W, int products, void* Y, long y_apart, int N, int O, int I, long ldx,
+                            long ldy, hipStream_t stream);
 int gibbs_skinny_store(const void* X, const void* W, void* Y, int N, int O, int I, long ldx, long ldw, long ldy, int rms,
                        float eps, hipStream_t stream);
 int gibbs_skinny_residual(const void* X, const void* W, float* x, void* xb, int N, int O, int I, long ldx, long ldw,

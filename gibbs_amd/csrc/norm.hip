@@ -52,7 +52,7 @@ __device__ __forceinline__ void store4(bf16* p, float4 v) {
 template <typename T, int CHUNKS, typename D = T>
 __global__ void add_rmsnorm_vec_kernel(float* __restrict__ x, const D* __restrict__ delta,
                                        const float* __restrict__ gain, float eps, T* __restrict__ out,
-                                       const int* __restrict__ rows, int hidden, int write_x, int parts = 0, long apart = 0) {
+                                       const int* __restrict__ rows, int hidden, int write_x, int parts = 0, long apart = 0, bf16* __restrict__ mirror = nullptr) {
   __shared__ float scratch[16];
   const int m = blockIdx.x;
   const int r = rows ? rows[m] : m;
@@ -75,6 +75,7 @@ __global__ void add_rmsnorm_vec_kernel(float* __restrict__ x, const D* __restric
         v[c].x += d.x; v[c].y += d.y; v[c].z += d.z; v[c].w += d.w;
         if (write_x) *(float4*)(xr + i) = v[c];
       }
+      if (mirror) store4(mirror + (size_t)r * hidden + i, v[c]);
       ss += v[c].x * v[c].x + v[c].y * v[c].y + v[c].z * v[c].z + v[c].w * v[c].w;
     }
   }
@@ -94,16 +95,16 @@ __global__ void add_rmsnorm_vec_kernel(float* __restrict__ x, const D* __restric
 
 template <typename T, typename D = T>
 bool launch_vec(float* x, const D* delta, const float* gain, float eps, T* out, const int* rows, int n_out, int hidden,
-                int write_x, hipStream_t stream, int parts = 0, long apart = 0) {
+                int write_x, hipStream_t stream, int parts = 0, long apart = 0, bf16* mirror = nullptr) {
   if (hidden % 4 || ((uintptr_t)x % 16) || (gain && ((uintptr_t)gain % 16)) || ((uintptr_t)out % (4 * sizeof(T))) ||
-      (delta && ((uintptr_t)delta % (4 * sizeof(D)))) || apart % 4)
+      (delta && ((uintptr_t)delta % (4 * sizeof(D)))) || apart % 4 || ((uintptr_t)mirror % 8))
     return false;
   const int threads = hidden >= 2048 ? 512 : (hidden >= 512 ? 256 : 64);
   const int chunks = ceil_div(hidden, 4 * threads);
-  if (chunks == 1) add_rmsnorm_vec_kernel<T, 1, D><<<n_out, threads, 0, stream>>>(x, delta, gain, eps, out, rows, hidden, write_x, parts, apart);
-  else if (chunks == 2) add_rmsnorm_vec_kernel<T, 2, D><<<n_out, threads, 0, stream>>>(x, delta, gain, eps, out, rows, hidden, write_x, parts, apart);
-  else if (chunks <= 4) add_rmsnorm_vec_kernel<T, 4, D><<<n_out, threads, 0, stream>>>(x, delta, gain, eps, out, rows, hidden, write_x, parts, apart);
-  else if (chunks <= 8) add_rmsnorm_vec_kernel<T, 8, D><<<n_out, threads, 0, stream>>>(x, delta, gain, eps, out, rows, hidden, write_x, parts, apart);
+  if (chunks == 1) add_rmsnorm_vec_kernel<T, 1, D><<<n_out, threads, 0, stream>>>(x, delta, gain, eps, out, rows, hidden, write_x, parts, apart, mirror);
+  else if (chunks == 2) add_rmsnorm_vec_kernel<T, 2, D><<<n_out, threads, 0, stream>>>(x, delta, gain, eps, out, rows, hidden, write_x, parts, apart, mirror);
+  else if (chunks <= 4) add_rmsnorm_vec_kernel<T, 4, D><<<n_out, threads, 0, stream>>>(x, delta, gain, eps, out, rows, hidden, write_x, parts, apart, mirror);
+  else if (chunks <= 8) add_rmsnorm_vec_kernel<T, 8, D><<<n_out, threads, 0, stream>>>(x, delta, gain, eps, out, rows, hidden, write_x, parts, apart, mirror);
   else return false;
   return true;
 }
@@ -125,6 +126,20 @@ GIBBS_EXPORT int gibbs_add_rmsnorm(float* x, const void* delta, const float* gai
   } else {
     return gibbs_fail("rmsnorm: unknown dtype %d", dtype);
   }
+  GIBBS_LAUNCH_STATUS("rmsnorm");
+}
+
+// The same of all n rows (bfloat16), and what x then holds rounded to bfloat16, which a fused product reads: a kernel less than
+// gibbs_residual_add behind it (2 to 5 us of a decode step).  parts: 0 no delta, 1 bfloat16 rows, 2 and more float32 partial sums `apart` values
+// from one to the next.  Returns 0 when it was queued, -1 when the sizes or addresses do not allow it (nothing was queued), 1 on an error.
+GIBBS_EXPORT int gibbs_add_rmsnorm_mirror(float* x, const void* delta, int parts, long apart, const float* gain, float eps, void* out, void* mirror, int dtype,
+                                          int n, int hidden, hipStream_t stream) {
+  GIBBS_REQUIRE(x && out && mirror && n >= 0 && hidden > 0 && parts >= 0 && (parts == 0 || delta), "rmsnorm: bad sizes n=%d hidden=%d partials=%d", n, hidden, parts);
+  if (n == 0) return 0;
+  if (dtype != GIBBS_BF16) return -1;
+  const bool queued = parts >= 2 ? launch_vec<bf16, float>(x, (const float*)delta, gain, eps, (bf16*)out, nullptr, n, hidden, 1, stream, parts, apart, (bf16*)mirror)
+                                 : launch_vec<bf16>(x, parts ? (const bf16*)delta : nullptr, gain, eps, (bf16*)out, nullptr, n, hidden, 1, stream, 0, 0, (bf16*)mirror);
+  if (!queued) return -1;
   GIBBS_LAUNCH_STATUS("rmsnorm");
 }
 

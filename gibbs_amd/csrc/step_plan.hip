@@ -47,6 +47,7 @@ long ceil_div_l(long a, long b) { return (a + b - 1) / b; }
 constexpr int FUSED_ROWS = 64;            // rows that the few-row products (and so the fused decode kernels) take
 constexpr int SKINNY_ROWS = 64;           // rows up to which a plain product takes the weight-streaming kernel
 constexpr int SKINNY_ROWS_F32_OUT = 48;   // the same for float32 output (the head: it streams faster than the tiled product)
+constexpr int ACT_TANGENT = 6;            // (activation.h: ACT_TANH)
 constexpr int ACT_CLAMPED = 4;            // the gated feed-forward's clamped activation (activation.h: ACT_CLAMPED_SWISH)
 constexpr int SSD_CHUNKED_ROWS = 256;     // rows of one request from which the state-space rule runs in chunks
 constexpr int GATED_CHUNKED_ROWS = 96;    // rows of a request from which the gated outer-product rule runs in chunks
@@ -341,6 +342,8 @@ struct Exec {
   // next half is a fused one): two kernels less than a delta that is written, added and mirrored (null: it stays a delta).
   float* into = nullptr;
   void** into_mirror = nullptr;
+  // Where a norm of all rows may leave a bfloat16 mirror of x (null: nobody reads one).
+  void** mirror_out = nullptr;
   // a mixer's last product: its delta, or nothing pending if it went into the stream
   Pending leave(const void* y, const Matrix& m);
   // x += y @ W^T with the mirror kept (the last product of a fused half of a layer)
@@ -536,6 +539,18 @@ struct RmsNorm : NormPart {
   void* run(Exec& e, float* x, Pending& pending, const int* rows, int n_out) const override {
     const int H = e.p.hidden;
     void* out = e.take((long)n_out * H * e.esize);
+    if (e.mirror_out && !rows && H % 4 == 0 && H <= 16384) {
+      void* mirror = e.take((long)n_out * H * 2);
+      int done = e.dry || e.status ? 0 : gibbs_add_rmsnorm_mirror(x, pending.data, pending.parts, (long)n_out * H, gain, eps, out, mirror, e.p.dtype, n_out, H, e.a.stream);
+      if (done > 0) e.status = 1;
+      if (done == 0) {
+        *e.mirror_out = mirror;
+        e.give(pending.data);
+        pending = Pending{};
+        return out;
+      }
+      e.give(mirror);
+    }
     if (pending.parts >= 2)
       RUN(e, gibbs_add_partials_rmsnorm(x, (const float*)pending.data, pending.parts, (long)e.a.n_rows * H, gain, eps, out, e.p.dtype,
                                         rows, n_out, H, e.a.stream));
@@ -674,7 +689,15 @@ struct ConvBody : Body {
   }
   Pending general(Exec& e, void* h) const override {
     const int N = e.a.n_rows;
-    void* y = convolve(e, e.linear(h, in, N, false, false, false, nullptr));
+    void* bcx;
+    if (e.bf16_run && N <= SKINNY_ROWS && in_packed3 && C % 4 == 0 && aligned_for_matrix_cores(h, in.I, in_packed3, in.I)) {
+      // (few rows: the three groups of the tile-ordered copy are three products of the same rows)
+      bcx = e.take((long)N * 3 * C * 2);
+      RUN(e, gibbs_skinny_store_many(h, 0, in_packed3, 3, bcx, C, N, C, in.I, in.I, 3 * C, e.a.stream));
+    } else {
+      bcx = e.linear(h, in, N, false, false, false, nullptr);
+    }
+    void* y = convolve(e, bcx);
     Pending delta = e.leave(y, out);
     e.give(y);
     return delta;
@@ -916,7 +939,7 @@ struct AttnBody : Body {
   }
   Pending general(Exec& e, void* h) const override {
     const int N = e.a.n_rows;
-    void* raw = e.linear(h, qkv, N, false, false, false, nullptr);
+    void* raw = e.linear(h, qkv, N, false, false, true, nullptr);
     void* att = attend(e, raw);
     e.give(raw);
     Pending delta = e.leave(att, out);
@@ -1074,10 +1097,10 @@ struct DeltaBody : Body {
     const GibbsStepArgs& a = e.a;
     const int N = a.n_rows, C = 2 * G * D + H * V;
     const bool channel = a2.w != nullptr;
-    char* raw = (char*)e.linear(h, in, N, false, false, false, nullptr);
+    char* raw = (char*)e.linear(h, in, N, false, false, true, nullptr);
     float* qkv = (float*)e.take((long)N * C * 4);
-    float* a_channel = channel ? (float*)e.linear(raw + (long)off_a * e.esize, a2, N, true, false, false, nullptr, in.O) : nullptr;
-    void* gate2 = g2.w ? e.linear(raw + (long)off_g * e.esize, g2, N, false, false, false, nullptr, in.O) : nullptr;
+    float* a_channel = channel ? (float*)e.linear(raw + (long)off_a * e.esize, a2, N, true, false, true, nullptr, in.O) : nullptr;
+    void* gate2 = g2.w ? e.linear(raw + (long)off_g * e.esize, g2, N, false, false, true, nullptr, in.O) : nullptr;
     const void* gate = gate2 ? gate2 : raw + (long)off_g * e.esize;
     const long ld_gate = gate2 ? (long)H * V : in.O;
     const int act = g2.w ? 1 : 0;
@@ -1143,6 +1166,7 @@ struct DeltaBody : Body {
 // read-out is divided by its root mean square, multiplied by a gain and silu(g), and projected back.
 struct TimeMixBody : Body {
   Matrix wr, wk, wv, wg, w1, w2, out;
+  const void* rkvg_packed = nullptr;   // r, k, v and g in tile order, one behind the other
   int H = 0, D = 0;
   const float* mu = nullptr;         // [5, hidden]: r, k, v, g, w
   const float* w0 = nullptr;         // [H D]
@@ -1163,16 +1187,22 @@ struct TimeMixBody : Body {
     const long apart = ((long)N * C * e.esize + 255) / 256 * 256 / e.esize;      // values from one to the next
     char* rows = (char*)e.take(4 * apart * e.esize);
     char *r = rows, *k = r + apart * e.esize, *v = k + apart * e.esize, *g = v + apart * e.esize;
-    e.linear_into(mixes, wr, N, false, false, r);
-    e.linear_into(mixes + one, wk, N, false, false, k);
-    e.linear_into(mixes + 2 * one, wv, N, false, false, v);
-    e.linear_into(mixes + 3 * one, wg, N, false, false, g);
-    float* z = (float*)e.linear(mixes + 4 * one, w1, N, true, false, false, nullptr);
-    e.give(mixes);
     void* t = e.take((long)N * w1.O * e.esize);
-    RUN(e, gibbs_tanh_rows(z, t, e.p.dtype, (long)N * w1.O, a.stream));
-    e.give(z);
-    float* w = (float*)e.linear(t, w2, N, true, false, false, nullptr);
+    if (e.bf16_run && N <= SKINNY_ROWS && rkvg_packed && W % 8 == 0) {
+      // few rows: the four products in one launch, and the tangent as the fifth's epilogue (seven launches are three)
+      RUN(e, gibbs_skinny_store_many(mixes, (long)N * W, rkvg_packed, 4, r, apart, N, C, W, W, C, a.stream));
+      RUN(e, gibbs_skinny_act(mixes + 4 * one, w1.packed ? w1.packed : w1.w, t, N, w1.O, W, W, w1.packed ? 0 : W, w1.O, ACT_TANGENT, nullptr, 0, nullptr, 0, a.stream));
+    } else {
+      e.linear_into(mixes, wr, N, false, false, r);
+      e.linear_into(mixes + one, wk, N, false, false, k);
+      e.linear_into(mixes + 2 * one, wv, N, false, false, v);
+      e.linear_into(mixes + 3 * one, wg, N, false, false, g);
+      float* z = (float*)e.linear(mixes + 4 * one, w1, N, true, false, false, nullptr);
+      RUN(e, gibbs_tanh_rows(z, t, e.p.dtype, (long)N * w1.O, a.stream));
+      e.give(z);
+    }
+    e.give(mixes);
+    float* w = (float*)e.linear(t, w2, N, true, false, true, nullptr);
     e.give(t);
     void* y = e.take((long)N * C * e.esize);
     // Requests at the head of the batch that bring one row each (row n is request n's) take the row kernel; the others run in chunks where
@@ -1662,9 +1692,17 @@ void Exec::run() {
         break;
       }
       case Plan::OP_NORM:
-        rows[op.result] = p.norms[op.norm]->run(*this, x, pending, nullptr, N);
-        give(mirror);      // (x has taken what was pending: its mirror is stale)
-        mirror = nullptr;
+        {
+          // (a half that reads x itself in the fused kernels follows: its mirror leaves in the same pass)
+          const Plan::Op* next = i + 1 < last && p.ops[i + 1].kind == Plan::OP_HALF ? &p.ops[i + 1] : nullptr;
+          float next_eps = 0.f;
+          void* made = nullptr;
+          mirror_out = next && few_rows && p.bodies[next->body]->fusable(fused_step) && p.norms[next->norm]->folded_rms(&next_eps) ? &made : nullptr;
+          rows[op.result] = p.norms[op.norm]->run(*this, x, pending, nullptr, N);
+          mirror_out = nullptr;
+          give(mirror);      // (x has taken what was pending: its mirror is stale)
+          mirror = made;
+        }
         break;
       case Plan::OP_BODY:
         deltas[op.result] = p.bodies[op.body]->general(*this, rows[op.value]);
@@ -1989,7 +2027,7 @@ GIBBS_EXPORT int gibbs_plan_body_attention(void* plan, const void* w_qkv, const 
     return -1;
   }
   auto t = std::make_unique<AttnBody>();
-  t->qkv = Matrix{w_qkv, nullptr, (nh + (owns ? 2 * nkv : 0)) * hd, p->hidden}; t->qkv_packed = p_qkv;
+  t->qkv = Matrix{w_qkv, p_qkv, (nh + (owns ? 2 * nkv : 0)) * hd, p->hidden}; t->qkv_packed = p_qkv;
   t->out = Matrix{w_out, p_out, p->hidden, nh * hd};
   t->nh = nh; t->nkv = nkv; t->hd = hd; t->scale = scale; t->window = window; t->q_gain = q_gain; t->k_gain = k_gain; t->qk_eps = qk_eps;
   t->inv_freq = inv_freq; t->rot = inv_freq ? rot : 0; t->variant = variant; t->cos_sin = cos_sin; t->table_len = table_len;
@@ -2427,10 +2465,10 @@ GIBBS_EXPORT int gibbs_plan_body_delta(void* plan, const GibbsDeltaSpec* d) {
     return -1;
   }
   auto b = std::make_unique<DeltaBody>();
-  b->in = Matrix{d->w_in, nullptr, d->in_rows, p->hidden};
-  b->out = Matrix{d->w_out, nullptr, p->hidden, d->heads * d->vdim};
-  if (d->w_a2) b->a2 = Matrix{d->w_a2, nullptr, d->heads * d->dim, d->a_rank};
-  if (d->w_g2) b->g2 = Matrix{d->w_g2, nullptr, d->heads * d->vdim, d->g_rank};
+  b->in = Matrix{d->w_in, d->p_in, d->in_rows, p->hidden};
+  b->out = Matrix{d->w_out, d->p_out, p->hidden, d->heads * d->vdim};
+  if (d->w_a2) b->a2 = Matrix{d->w_a2, d->p_a2, d->heads * d->dim, d->a_rank};
+  if (d->w_g2) b->g2 = Matrix{d->w_g2, d->p_g2, d->heads * d->vdim, d->g_rank};
   b->H = d->heads; b->G = d->kv_heads; b->D = d->dim; b->V = d->vdim; b->K = d->taps_per_channel;
   b->off_b = d->off_b; b->off_a = d->off_a; b->off_g = d->off_g;
   b->taps = d->taps; b->dt_bias = d->dt_bias; b->a_log = d->a_log; b->gain = d->gain;
@@ -2455,8 +2493,9 @@ GIBBS_EXPORT int gibbs_plan_body_time_mix(void* plan, const GibbsTimeMixSpec* d)
   const int C = d->heads * d->dim, W = p->hidden;
   auto b = std::make_unique<TimeMixBody>();
   b->wr = Matrix{d->w_r, nullptr, C, W}; b->wk = Matrix{d->w_k, nullptr, C, W}; b->wv = Matrix{d->w_v, nullptr, C, W};
-  b->wg = Matrix{d->w_g, nullptr, C, W}; b->w1 = Matrix{d->w_1, nullptr, d->rank, W}; b->w2 = Matrix{d->w_2, nullptr, C, d->rank};
-  b->out = Matrix{d->w_out, nullptr, W, C};
+  b->wg = Matrix{d->w_g, nullptr, C, W}; b->w1 = Matrix{d->w_1, d->p_1, d->rank, W}; b->w2 = Matrix{d->w_2, d->p_2, C, d->rank};
+  b->out = Matrix{d->w_out, d->p_out, W, C};
+  b->rkvg_packed = d->p_rkvg;
   b->H = d->heads; b->D = d->dim; b->mu = d->mu; b->w0 = d->w0; b->bonus = d->bonus; b->gain = d->gain;
   b->shift_state = d->shift_state; b->rule_state = d->rule_state; b->slot_stride = d->slot_stride; b->eps = d->eps;
   p->bodies.push_back(std::move(b));

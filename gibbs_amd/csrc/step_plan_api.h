@@ -111,6 +111,7 @@ int gibbs_plan_glu_clamped(void* plan, int body, float alpha, float limit);
 // heads vdim, taps_per_channel], the last one the current token's.
 struct GibbsDeltaSpec {
   const void* w_in; const void* w_out; const void* w_a2; const void* w_g2;
+  const void* p_in; const void* p_out; const void* p_a2; const void* p_g2;   // the same in tile order (bfloat16), or null
   const float* taps; const float* dt_bias; const float* a_log; const float* gain;
   float* conv_state; float* rule_state; long slot_stride;
   int in_rows, heads, kv_heads, dim, vdim, taps_per_channel, off_b, off_a, off_g, a_rank, g_rank;
@@ -122,6 +123,7 @@ int gibbs_plan_body_delta(void* plan, const struct GibbsDeltaSpec* spec);
 // [heads*dim, rank], w_out [hidden, heads*dim]; mu [5, hidden] (r, k, v, g, w); w0, gain [heads*dim]; bonus [heads, dim].
 struct GibbsTimeMixSpec {
   const void* w_r; const void* w_k; const void* w_v; const void* w_g; const void* w_1; const void* w_2; const void* w_out;
+  const void* p_rkvg; const void* p_1; const void* p_2; const void* p_out;   // in tile order (bfloat16), r, k, v and g one behind the other; or null
   const float* mu; const float* w0; const float* bonus; const float* gain;
   float* shift_state; float* rule_state; long slot_stride;
   int heads, dim, rank;

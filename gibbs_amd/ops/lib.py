@@ -35,6 +35,8 @@ _SIGNATURES = {
                           c_void_p],
     "gibbs_add_partials_rmsnorm": [c_void_p, c_void_p, c_int, c_long, c_void_p, c_float, c_void_p, c_int, c_void_p,
                                    c_int, c_int, c_void_p],
+    "gibbs_skinny_store_many": [c_void_p, c_long, c_void_p, c_int, c_void_p, c_long, c_int, c_int, c_int, c_long, c_long, c_void_p],
+    "gibbs_add_rmsnorm_mirror": [c_void_p, c_void_p, c_int, c_long, c_void_p, c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
     "gibbs_skinny_store": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_int, c_float,
                            c_void_p],
     "gibbs_skinny_residual": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_void_p],

@@ -80,6 +80,9 @@ class ParallelNormsBlock(Block):
         if self.pair:
             for norm in (self.left_out, self.right_out):
                 norm.gain = norm.gain * 0.5
+        if rt.act_dtype == torch.bfloat16:
+            for role in ("left", "right") if self.pair else ("mixer",):
+                self.named[role].pack_matrices()
         if "ffn" in self.named and rt.act_dtype == torch.bfloat16:
             if rt.fold_gains and hasattr(self.norm2, "fold_gain") and hasattr(self.ffn, "fold_input_gain"):
                 self.ffn.fold_input_gain(self.norm2.fold_gain())

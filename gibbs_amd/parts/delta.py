@@ -22,6 +22,7 @@ from typing import List, Sequence
 
 import torch
 
+from .. import ops
 from ..cache.needs import StateNeed
 from ..weights.loader import FLOAT32, TensorDecl, WeightStore
 from .base import Mixer, Runtime, register_mixer
@@ -100,6 +101,7 @@ class GatedDeltaMixer(Mixer):
         self.w_out = weights[t["o"]]
         self.conv_taps = torch.cat([weights[t["q_taps"]], weights[t["k_taps"]], weights[t["v_taps"]]], dim=0).contiguous()
         self.a_log, self.dt_bias, self.gain = weights[t["A_log"]], weights[t["dt_bias"]], weights[t["norm"]]
+        self.packed = [None] * 4
 
     def matrices(self):
         return [m for m in (self.w_in, self.w_a2, self.w_g2, self.w_out) if m is not None]
@@ -117,6 +119,9 @@ class GatedDeltaMixer(Mixer):
     def state_bytes(self) -> int:
         """Bytes of state that a decoded token reads and writes."""
         return 2 * 4 * (self.heads * self.dim * self.vdim + (self.taps - 1) * self.conv_channels)
+
+    def pack_matrices(self) -> None:
+        self.packed = [None if w is None else ops.PackedWeight(w) for w in (self.w_in, self.w_out, self.w_a2, self.w_g2)]
 
     def emit(self, plan, cache) -> int:
         rule = cache.states[RULE_STATE]

@@ -37,6 +37,7 @@ class StepArgs(ctypes.Structure):
 class DeltaSpec(ctypes.Structure):
     """GibbsDeltaSpec of csrc/step_plan_api.h."""
     _fields_ = [("w_in", c_void_p), ("w_out", c_void_p), ("w_a2", c_void_p), ("w_g2", c_void_p),
+                ("p_in", c_void_p), ("p_out", c_void_p), ("p_a2", c_void_p), ("p_g2", c_void_p),
                 ("taps", c_void_p), ("dt_bias", c_void_p), ("a_log", c_void_p), ("gain", c_void_p),
                 ("conv_state", c_void_p), ("rule_state", c_void_p), ("slot_stride", c_long),
                 ("in_rows", c_int), ("heads", c_int), ("kv_heads", c_int), ("dim", c_int), ("vdim", c_int),
@@ -47,7 +48,8 @@ class DeltaSpec(ctypes.Structure):
 class TimeMixSpec(ctypes.Structure):
     """GibbsTimeMixSpec of csrc/step_plan_api.h."""
     _fields_ = [("w_r", c_void_p), ("w_k", c_void_p), ("w_v", c_void_p), ("w_g", c_void_p), ("w_1", c_void_p), ("w_2", c_void_p),
-                ("w_out", c_void_p), ("mu", c_void_p), ("w0", c_void_p), ("bonus", c_void_p), ("gain", c_void_p),
+                ("w_out", c_void_p), ("p_rkvg", c_void_p), ("p_1", c_void_p), ("p_2", c_void_p), ("p_out", c_void_p),
+                ("mu", c_void_p), ("w0", c_void_p), ("bonus", c_void_p), ("gain", c_void_p),
                 ("shift_state", c_void_p), ("rule_state", c_void_p), ("slot_stride", c_long),
                 ("heads", c_int), ("dim", c_int), ("rank", c_int), ("eps", ctypes.c_float)]
 
@@ -500,6 +502,7 @@ class NativePlan:
         assert rule_state.dtype == torch.float32 and conv_state.dtype == torch.float32 and rule_state.stride(0) == conv_state.stride(0)
         d = DeltaSpec()
         d.w_in, d.w_out, d.w_a2, d.w_g2 = self._held(m.w_in, m.w_out, m.w_a2, m.w_g2)
+        d.p_in, d.p_out, d.p_a2, d.p_g2 = self._held(*m.packed)
         d.taps, d.dt_bias, d.a_log, d.gain = self._held(m.conv_taps, m.dt_bias, m.a_log, m.gain)
         d.conv_state, d.rule_state, d.slot_stride = conv_state.data_ptr(), rule_state.data_ptr(), int(rule_state.stride(0))
         self.keep += [conv_state, rule_state]
@@ -514,6 +517,7 @@ class NativePlan:
         assert rule_state.dtype == torch.float32 and shift_state.dtype == torch.float32 and rule_state.stride(0) == shift_state.stride(0)
         d = TimeMixSpec()
         d.w_r, d.w_k, d.w_v, d.w_g, d.w_1, d.w_2, d.w_out = self._held(m.w_r, m.w_k, m.w_v, m.w_g, m.w_1, m.w_2, m.w_out)
+        d.p_rkvg, d.p_1, d.p_2, d.p_out = self._held(*m.packed)
         d.mu, d.w0, d.bonus, d.gain = self._held(m.mu, m.w0, m.bonus, m.gain)
         d.shift_state, d.rule_state, d.slot_stride = shift_state.data_ptr(), rule_state.data_ptr(), int(rule_state.stride(0))
         self.keep += [shift_state, rule_state]

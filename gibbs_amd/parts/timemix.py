@@ -18,6 +18,7 @@ from typing import List, Sequence
 
 import torch
 
+from .. import ops
 from ..cache.needs import StateNeed
 from ..weights.loader import FLOAT32, TensorDecl, WeightStore
 from .base import Mixer, Runtime, register_mixer
@@ -55,6 +56,7 @@ class TimeMixMixer(Mixer):
         self.w_r, self.w_k, self.w_v, self.w_g = (weights[t[s]] for s in ("r", "k", "v", "g"))
         self.w_1, self.w_2, self.w_out = weights[t["w1"]], weights[t["w2"]], weights[t["o"]]
         self.w0, self.bonus, self.gain = weights[t["w0"]], weights[t["u"]].contiguous(), weights[t["norm"]]
+        self.packed = [None] * 4
 
     def matrices(self):
         return [self.w_r, self.w_k, self.w_v, self.w_g, self.w_1, self.w_2, self.w_out]
@@ -68,6 +70,10 @@ class TimeMixMixer(Mixer):
 
     def state_bytes(self) -> int:
         return 2 * 4 * (self.heads * self.dim * self.dim + self.hidden)
+
+    def pack_matrices(self) -> None:
+        four = ops.PackedWeight(torch.cat([self.w_r, self.w_k, self.w_v, self.w_g], dim=0), groups=4)
+        self.packed = [four, ops.PackedWeight(self.w_1), ops.PackedWeight(self.w_2), ops.PackedWeight(self.w_out)]
 
     def emit(self, plan, cache) -> int:
         return plan.time_mix(self, shift_state=cache.states[SHIFT_STATE], rule_state=cache.states[RULE_STATE])

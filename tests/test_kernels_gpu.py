@@ -1057,6 +1057,40 @@ def test_attention_decode_fused(nh, nkv, hd, rot, page, window, variant, n_split
     close(got, want, dtype, "fused decode attention", bf16=8e-3)
 
 
+@pytest.mark.parametrize("n", [1, 8, 9, 16, 33, 64])
+@pytest.mark.parametrize("o,i,products,apart", [(8, 64, 3, True), (72, 200, 4, True), (520, 40, 2, False), (4104, 96, 2, True)])
+def test_several_products_of_one_size_in_a_launch(n, o, i, products, apart):
+    """Every product's rows as they come from a launch of their own, to the bit: matrices in either tile order, one or two tiles of rows and
+    more, rows of X shared or one's behind the other's, results side by side in wider rows."""
+    from gibbs_amd import ops
+    from gibbs_amd.ops.lib import call, ptr, stream
+    x = rnd(products if apart else 1, n, i, dtype=torch.bfloat16, seed=1)
+    w = rnd(products * o, i, dtype=torch.bfloat16, seed=2)
+    packed = ops.PackedWeight(w, groups=products)
+    y = torch.zeros(n, products * o, dtype=torch.bfloat16, device=DEV)
+    call("gibbs_skinny_store_many", ptr(x), n * i if apart else 0, ptr(packed.data), products, ptr(y), o, n, o, i, i, products * o, stream())
+    for p in range(products):
+        rows = x[p if apart else 0].contiguous()
+        assert torch.equal(y[:, p * o:(p + 1) * o], ops.skinny_store(rows, ops.PackedWeight(w[p * o:(p + 1) * o].contiguous()))), p
+        # (a bfloat16 result of float32 sums)
+        close(y[:, p * o:(p + 1) * o], rows.double() @ w[p * o:(p + 1) * o].double().T, torch.bfloat16, f"product {p}", bf16=8e-3)
+
+
+@pytest.mark.parametrize("parts", [0, 1, 3])
+@pytest.mark.parametrize("hidden", [4, 516, 2048, 5000])
+def test_norm_that_leaves_a_mirror(hidden, parts):
+    """x, the normed rows and x in bfloat16 in one kernel: the bits of the two that it stands for."""
+    from gibbs_amd import ops
+    from gibbs_amd.ops.lib import call, dtype_code, ptr, stream
+    n = 5
+    x, gain = rnd(n, hidden, seed=1), rnd(hidden, seed=2)
+    delta = None if parts == 0 else rnd(n, hidden, dtype=torch.bfloat16, seed=3) if parts == 1 else rnd(parts, n, hidden, seed=3)
+    x1, out, mirror = x.clone(), torch.empty(n, hidden, dtype=torch.bfloat16, device=DEV), torch.empty(n, hidden, dtype=torch.bfloat16, device=DEV)
+    want = ops.add_rmsnorm(x, delta, gain, 1e-5, torch.bfloat16)
+    call("gibbs_add_rmsnorm_mirror", ptr(x1), ptr(delta), parts, n * hidden, ptr(gain), 1e-5, ptr(out), ptr(mirror), dtype_code(torch.bfloat16), n, hidden, stream())
+    assert torch.equal(x1, x) and torch.equal(out, want) and torch.equal(mirror, x.to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("raw", [False, True])
 @pytest.mark.parametrize("n_splits,waves", [(1, 4), (1, 8), (5, 4), (None, None)])
 @pytest.mark.parametrize("nh,nkv,hd,page,window", [(2, 2, 64, 16, None), (4, 2, 64, 64, 33), (8, 1, 64, 16, 700), (1, 1, 128, 16, None),
