@@ -166,6 +166,11 @@ int gibbs_rmsnorm_rows_sum_add_read(float* x, const void* in, int parts, long pa
 int gibbs_rows_terms(const void* in, int parts, const float* bias, float scale, const void* in2, int parts2, float scale2, float* out,
                      int dtype, int n, int hidden, hipStream_t stream);
 // ---- moe.hip: mixture of experts
+int gibbs_moe_direct_takes(int n, int top, int E, int W, int F);
+int gibbs_moe_route_placed(const void* h, long ldh, int dtype, const float* router, const float* router_bias, const float* shared_gate, int* chosen,
+                           float* weight, float* sgate, int* place, int matrices, int n, int W, int E, int top, int mode, float weight_scale, hipStream_t stream);
+int gibbs_moe_gemm_direct(const void* X, long ldx, int top, const int* chosen, int pairs, int E, const void* w_a, const void* w_b, const float* in_weight, void* Y,
+                          long ldy, int O, int I, int act, hipStream_t stream);
 int gibbs_moe_route_scaled(const void* h, long ldh, int dtype, const float* router, const float* router_bias, const float* shared_gate,
                            int* chosen, float* weight, float* sgate, int n, int W, int E, int top, int mode, float weight_scale,
                            hipStream_t stream);

@@ -118,7 +118,8 @@ __device__ __forceinline__ float wave_dot(const T* __restrict__ row, const float
 // the experts, the lanes' bests are folded by exchanges); a logit that was taken becomes NaN; then the softmax
 // over the chosen logits alone
 __device__ __forceinline__ void choose_experts(float* z, float* score, int n, int lane, const float* __restrict__ router_bias, int* __restrict__ chosen,
-                                               float* __restrict__ weight, int E, int top, int mode, float weight_scale) {
+                                               float* __restrict__ weight, int E, int top, int mode, float weight_scale, int* __restrict__ place = nullptr,
+                                               int matrices = 0) {
   int* mine = chosen + (size_t)n * top;
   float* wts = weight + (size_t)n * top;
   if (mode == 2 && router_bias) {
@@ -202,6 +203,7 @@ __device__ __forceinline__ void choose_experts(float* z, float* score, int n, in
     if (lane < top) {
       mine[lane] = my_pick;
       wts[lane] = normed(my_weight);
+      if (place) place[(size_t)n * top + lane] = my_pick < matrices ? n * top + lane : -1;
     }
   } else if (lane == 0) {
     for (int c = 0; c < top; ++c) wts[c] = normed(wts[c]);
@@ -212,7 +214,7 @@ template <typename T>
 __global__ __launch_bounds__(1024) void moe_route_kernel(const T* __restrict__ h, long ldh, const float* __restrict__ router,
                                                         const float* __restrict__ router_bias, const float* __restrict__ shared_gate,
                                                         int* __restrict__ chosen, float* __restrict__ weight, float* __restrict__ sgate,
-                                                        int W, int E, int top, int mode, float weight_scale) {
+                                                        int W, int E, int top, int mode, float weight_scale, int* __restrict__ place, int matrices) {
   extern __shared__ float z[];   // [E] (mode 1 and 2: and the scores behind them, [E])
   const int n = blockIdx.x, wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, n_waves = blockDim.x / WAVE;
   const T* row = h + (size_t)n * ldh;
@@ -239,7 +241,7 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(const T* __restrict__ h
   }
   __syncthreads();
   if (wave != 0) return;
-  choose_experts(z, z + E, n, lane, router_bias, chosen, weight, E, top, mode, weight_scale);
+  choose_experts(z, z + E, n, lane, router_bias, chosen, weight, E, top, mode, weight_scale, place, matrices);
 }
 
 // Many rows: a workgroup of four waves takes four of them, a wave two experts' logits of all four rows at a time, so that a router's row is read
@@ -421,79 +423,125 @@ typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 
-// Few pairs: a tile is 16 places, a workgroup takes 32 features of it (of both matrices, GLU) and its four waves a
+// Few pairs: a tile is 16 places, a workgroup takes 32 features of it (GLU: 16, of both matrices) and its four waves a
 // quarter of k each, so that the experts' matrices, which are read once, are spread over many workgroups; the waves'
-// sums meet in LDS and the first wave adds them in wave order.  W is the first operand of the 16 x 16 x 32 product (the
+// sums meet in LDS and are added in wave order.  W is the first operand of the 16 x 16 x 32 product (the
 // tile is Y^T = W X^T): lane l holds 8 values along k of feature or place l % 16, and its four results are four
-// neighbouring features of place l % 16.  Operands come straight from memory.
-template <bool GLU>
-__global__ __launch_bounds__(256) void moe_gemm_few_kernel(const bf16* __restrict__ X, long ldx, int top, const int* __restrict__ sorted_pair,
+// neighbouring features of place l % 16.  Operands come straight from memory.  Measured (16 experts of 1,024 at width 2,048, 4 chosen; us, gated and
+// back): 1 row 13.7 and 6.7 with loads under conditions, 32 features and one wave's tail, 10.1 and 5.6 now; 8 rows (126 and 63 MB) 34.8 and
+// 13.7, now 29.7 and 13.1; 16 gated features a workgroup or 32: 1 row 10.1 / 11.7, 8 rows 29.7 / 31.4, 32 rows 33.6 / 34.3; back, 8 rows 13.7 / 13.1.
+// DIRECT (at most 64 pairs, an expert at most 16 of them): no grouping in front: blockIdx.y is the expert, `sorted_pair` holds each pair's choice, and
+// places are the pairs' own numbers.
+template <bool GLU, bool DIRECT>
+__global__ __launch_bounds__(256) void moe_gemm_few_kernel(const bf16* __restrict__ X, const int* __restrict__ sorted_pair,
                                                            const int* __restrict__ tile_expert, const bf16* __restrict__ Wa,
-                                                           const bf16* __restrict__ Wb, long expert_stride, bf16* __restrict__ Y, long ldy,
-                                                           int O, int I, int act, const float* __restrict__ in_weight) {
-  constexpr int NF = 2, NA = GLU ? 2 * NF : NF;    // feature tiles of 16 a workgroup; accumulators a wave
-  __shared__ float part[4][NA][WAVE][4];
-  const int tile = blockIdx.y, e = tile_expert[tile];
-  if (e < 0) return;
-  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, lr = lane % 16, lg = lane / 16;
-  const int place = tile * 16 + lr;
+                                                           const bf16* __restrict__ Wb, int top, int I, long ldx, long expert_stride, bf16* __restrict__ Y,
+                                                           long ldy, int O, int act, const float* __restrict__ in_weight, int pairs) {
+  constexpr int NF = GLU ? 1 : 2, NA = GLU ? 2 * NF : NF;    // feature tiles of 16 a workgroup; accumulators a wave
+  __shared__ __attribute__((aligned(16))) floatx4 part[4][NA][WAVE];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, lr = lane % 16, lg = lane / 16;
+  int e, pair, place;
+  if constexpr (DIRECT) {
+    e = blockIdx.y;
+    const bool mine = lane < pairs && sorted_pair[min(lane, pairs - 1)] == e;
+    const uint64_t all = __builtin_amdgcn_ballot_w64(mine);
+    if (all == 0) return;
+    // the expert's pairs, in ascending order, to lanes 0, 1, ...; every lane then takes its place's
+    const int rank = __popcll(all & ((1ull << lane) - 1));
+    const int sent = __builtin_amdgcn_ds_permute((mine ? rank : WAVE - 1) * 4, lane);
+    pair = __builtin_amdgcn_ds_bpermute(lr * 4, sent);
+    if (lr >= __popcll(all)) pair = -1;
+    place = pair < 0 ? 0 : pair;
+  } else {
+    e = tile_expert[blockIdx.y];
+    place = blockIdx.y * 16 + lr;
+    pair = sorted_pair[place];
+    if (e < 0) return;
+  }
   const int col0 = blockIdx.x * (16 * NF);
-  const int pair = sorted_pair[place];
-  const long src = pair < 0 ? -1 : (top > 0 ? pair / top : place);
-  const bf16* xr = X + (size_t)(src < 0 ? 0 : src) * ldx;
-  const bf16* wa = Wa + (size_t)e * expert_stride;
-  const bf16* wb = GLU ? Wb + (size_t)e * expert_stride : nullptr;
-  const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+  const int src = pair < 0 ? 0 : (top > 0 ? pair / top : place);      // (a place without a pair: some row, its results are not stored)
+  const bf16* xr = X + (size_t)src * ldx;
+  const bf16* w[NA];
+#pragma unroll
+  for (int t = 0; t < NA; ++t) w[t] = (GLU && t >= NF ? Wb : Wa) + (size_t)e * expert_stride + (size_t)min(col0 + t % NF * 16 + lr, O - 1) * I;
   floatx4 acc[NA];
 #pragma unroll
   for (int t = 0; t < NA; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
   // wave w takes the stretches of 64 along k whose number is w modulo 4, in ascending order.  A lane group holds 16
   // neighbouring values of a stretch as the operands of two products (the order along k inside a product is free as long as
-  // both operands agree), so that the wave asks for whole lines of 128 bytes of every row; two stretches at a time
-#pragma unroll 2
-  for (int k0 = wave * 64; k0 < I; k0 += 256) {
-    bf16x8 x8[2], a8[2][NF], b8[2][NF];
+  // both operands agree), so that the wave asks for whole lines of 128 bytes of every row; two stretches on their way.  No load stands
+  // under a condition (each would be waited for alone): k beyond I reads the rows' last values, and X's are made zero.
+  const int n = I > wave * 64 ? (I - wave * 64 + 255) / 256 : 0;      // this wave's stretches
+  bf16x8 x8[2][2], w8[2][2][NA];
+  auto ask = [&](int set, int it) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const int k = k0 + lg * 16 + u * 8;
-      x8[u] = (src >= 0 && k < I) ? *(const bf16x8*)(xr + k) : zero8;
+      const uint32_t k = min(it * 256 + wave * 64 + lg * 16 + u * 8, I - 8);
+      x8[set][u] = *(const bf16x8*)(xr + k);
 #pragma unroll
-      for (int t = 0; t < NF; ++t) {
-        const int col = col0 + t * 16 + lr;
-        const bool in = col < O && k < I;
-        a8[u][t] = in ? *(const bf16x8*)(wa + (size_t)col * I + k) : zero8;
-        if (GLU) b8[u][t] = in ? *(const bf16x8*)(wb + (size_t)col * I + k) : zero8;
-      }
+      for (int t = 0; t < NA; ++t) w8[set][u][t] = *(const bf16x8*)(w[t] + k);
     }
+  };
+  auto use = [&](int set, int it) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < 2; ++u) {
+      if (it * 256 + wave * 64 + 64 > I && it * 256 + wave * 64 + lg * 16 + u * 8 >= I) x8[set][u] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-      for (int t = 0; t < NF; ++t) {
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a8[u][t], x8[u], acc[t], 0, 0, 0);
-        if (GLU) acc[NF + t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b8[u][t], x8[u], acc[NF + t], 0, 0, 0);
-      }
+      for (int t = 0; t < NA; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w8[set][u][t], x8[set][u], acc[t], 0, 0, 0);
+    }
+  };
+  if (n > 0) {
+    ask(0, 0);
+    ask(1, min(1, n - 1));
+    int it = 0;
+    for (; it + 2 < n; it += 2) {
+      use(0, it);
+      ask(0, it + 2);
+      __builtin_amdgcn_sched_barrier(0x7 | 0x8 | 0x380);
+      use(1, it + 1);
+      ask(1, min(it + 3, n - 1));
+      __builtin_amdgcn_sched_barrier(0x7 | 0x8 | 0x380);
+    }
+    use(0, it);
+    if (it + 1 < n) use(1, it + 1);
   }
 #pragma unroll
-  for (int t = 0; t < NA; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) part[wave][t][lane][i] = acc[t][i];
+  for (int t = 0; t < NA; ++t) part[wave][t][lane] = acc[t];
   __syncthreads();
-  if (wave != 0 || src < 0) return;
+  if (wave >= NF || pair < 0) return;      // wave t writes features t * 16 .. + 16
   const float pw = (GLU && in_weight) ? in_weight[pair] : 1.f;
+  floatx4 pa[4], pb[4];
 #pragma unroll
-  for (int t = 0; t < NF; ++t)
+  for (int v = 0; v < 4; ++v) {
+    pa[v] = part[v][wave][lane];
+    if (GLU) pb[v] = part[v][GLU ? NF + wave : 0][lane];
+  }
+  floatx4 a = {0.f, 0.f, 0.f, 0.f}, b = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int col = col0 + t * 16 + lg * 4 + i;
-      if (col >= O) continue;
-      float a = 0.f, b = 0.f;
+  for (int v = 0; v < 4; ++v) {
+    a += pa[v];
+    if (GLU) b += pb[v];
+  }
+  if (GLU) {
+    // (which activation is asked once, not for each value)
+    a *= pw;
+    if (act == ACT_SILU) {
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        a += part[w][t][lane][i];
-        if (GLU) b += part[w][NF + t][lane][i];
-      }
-      Y[(size_t)place * ldy + col] = (bf16)(GLU ? activate(pw * a, act) * (pw * b) : a);
+      for (int i = 0; i < 4; ++i) a[i] = activate(a[i], ACT_SILU) * (pw * b[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) a[i] = activate(a[i], act) * (pw * b[i]);
     }
+  }
+  const int col = col0 + wave * 16 + lg * 4;
+  bf16* y = Y + (size_t)place * ldy + col;
+  if (col + 3 < O && ldy % 4 == 0 && ((uintptr_t)Y % 8) == 0) {
+    *(bf16x4*)y = bf16x4{(bf16)a[0], (bf16)a[1], (bf16)a[2], (bf16)a[3]};
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (col + i < O) y[i] = (bf16)a[i];
+  }
 }
 
 // Many pairs: a tile is 128 places, a workgroup of NW waves computes 128 places x BN rows of W (GLU: BN / 2 features of both
@@ -918,6 +966,12 @@ GIBBS_EXPORT long gibbs_moe_capacity(int n_pairs, int E, int bm) {
 // Tiles of pairs: 16 while the matrices are streamed for few pairs each (at most 64 an expert on average), 128 beyond.
 GIBBS_EXPORT int gibbs_moe_tile(int n_pairs, int E) { return (long)n_pairs <= 64L * E ? 16 : 128; }
 
+// Few rows, whose products need no grouping (gibbs_moe_gemm_direct): at most 16, so that an expert has at most one of each row's pairs, a tile, and
+// 64 pairs, one for each lane of a wave.
+GIBBS_EXPORT int gibbs_moe_direct_takes(int n, int top, int E, int W, int F) {
+  return n > 0 && n <= 16 && n * top <= WAVE && E <= 65535 && W % 8 == 0 && F % 8 == 0;
+}
+
 // mode 0: the largest logits (+ bias), weights by the softmax over the chosen; mode 1: scores by the softmax over all E
 // outputs, the largest of score + router_bias (a correction that only the choice sees), weights the chosen scores over their sum;
 // mode 2: scores by the sigmoid of every output alone, the largest of score + router_bias, weights the chosen scores.
@@ -925,6 +979,14 @@ GIBBS_EXPORT int gibbs_moe_tile(int n_pairs, int E) { return (long)n_pairs <= 64
 GIBBS_EXPORT int gibbs_moe_route_scaled(const void* h, long ldh, int dtype, const float* router, const float* router_bias,
                                         const float* shared_gate, int* chosen, float* weight, float* sgate, int n, int W, int E, int top,
                                         int mode, float weight_scale, hipStream_t stream) {
+  return gibbs_moe_route_placed(h, ldh, dtype, router, router_bias, shared_gate, chosen, weight, sgate, nullptr, 0, n, W, E, top, mode, weight_scale, stream);
+}
+// The same, and for products without grouping place [n, top] (null: none): the pair's own number, or -1 where its choice is none of the
+// first `matrices` (an identity expert).  At most 1,023 rows and 64 choices.
+GIBBS_EXPORT int gibbs_moe_route_placed(const void* h, long ldh, int dtype, const float* router, const float* router_bias,
+                                        const float* shared_gate, int* chosen, float* weight, float* sgate, int* place, int matrices, int n, int W, int E, int top,
+                                        int mode, float weight_scale, hipStream_t stream) {
+  GIBBS_REQUIRE(!place || (n < 1024 && top <= WAVE), "moe_route: places for %d rows of %d choices", n, top);
   GIBBS_REQUIRE(weight_scale == 1.0f || mode == 1, "moe_route: weights times %g go with the scores' softmax over all outputs", weight_scale);
   GIBBS_REQUIRE(mode >= 0 && mode <= 2, "moe_route: mode %d", mode);
   GIBBS_REQUIRE(h && router && chosen && weight && n > 0 && W > 0 && ldh >= W, "moe_route: bad operands n=%d width=%d", n, W);
@@ -948,9 +1010,9 @@ GIBBS_EXPORT int gibbs_moe_route_scaled(const void* h, long ldh, int dtype, cons
   }
   const int threads = n >= 512 ? 256 : WAVE * std::min(16, std::max(4, E + 1));
   if (dtype == GIBBS_F32)
-    moe_route_kernel<float><<<n, threads, lds, stream>>>((const float*)h, ldh, router, router_bias, shared_gate, chosen, weight, sgate, W, E, top, mode, weight_scale);
+    moe_route_kernel<float><<<n, threads, lds, stream>>>((const float*)h, ldh, router, router_bias, shared_gate, chosen, weight, sgate, W, E, top, mode, weight_scale, place, matrices);
   else if (dtype == GIBBS_BF16)
-    moe_route_kernel<bf16><<<n, threads, lds, stream>>>((const bf16*)h, ldh, router, router_bias, shared_gate, chosen, weight, sgate, W, E, top, mode, weight_scale);
+    moe_route_kernel<bf16><<<n, threads, lds, stream>>>((const bf16*)h, ldh, router, router_bias, shared_gate, chosen, weight, sgate, W, E, top, mode, weight_scale, place, matrices);
   else
     return gibbs_fail("moe_route: unknown dtype %d", dtype);
   GIBBS_LAUNCH_STATUS("moe_route");
@@ -1013,17 +1075,35 @@ GIBBS_EXPORT int gibbs_moe_gemm_weighted(const void* X, long ldx, int top, const
               : launch_tiled<false>((const bf16*)X, ldx, top, sorted_pair, tile_expert, tiles, (const bf16*)w_a, nullptr, stride, (bf16*)Y, ldy, O, I, act, nullptr, stream))
         return 1;
     } else if (w_b) {
-      moe_gemm_few_kernel<true><<<dim3(ceil_div(O, 32), tiles), 256, 0, stream>>>((const bf16*)X, ldx, top, sorted_pair, tile_expert, (const bf16*)w_a,
-                                                                                 (const bf16*)w_b, stride, (bf16*)Y, ldy, O, I, act, in_weight);
+      moe_gemm_few_kernel<true, false><<<dim3(ceil_div(O, 16), tiles), 256, 0, stream>>>((const bf16*)X, sorted_pair, tile_expert, (const bf16*)w_a, (const bf16*)w_b,
+                                                                                        top, I, ldx, stride, (bf16*)Y, ldy, O, act, in_weight, 0);
     } else {
-      moe_gemm_few_kernel<false><<<dim3(ceil_div(O, 32), tiles), 256, 0, stream>>>((const bf16*)X, ldx, top, sorted_pair, tile_expert, (const bf16*)w_a,
-                                                                                  nullptr, stride, (bf16*)Y, ldy, O, I, act, nullptr);
+      moe_gemm_few_kernel<false, false><<<dim3(ceil_div(O, 32), tiles), 256, 0, stream>>>((const bf16*)X, sorted_pair, tile_expert, (const bf16*)w_a, nullptr, top, I,
+                                                                                         ldx, stride, (bf16*)Y, ldy, O, act, nullptr, 0);
     }
   } else {
     return gibbs_fail("moe_gemm: unknown dtype %d", dtype);
   }
 #undef MOE_PLAIN_ANY
 #undef MOE_PLAIN
+  GIBBS_LAUNCH_STATUS("moe_gemm");
+}
+
+// The products of few rows (gibbs_moe_direct_takes) straight from their choices `chosen` [pairs], bfloat16: row i of Y is pair i's result; X's rows are the step's
+// (gated: w_b given, row pair / top) or the pairs' own (w_b null).  Choices of E and beyond have no result.
+GIBBS_EXPORT int gibbs_moe_gemm_direct(const void* X, long ldx, int top, const int* chosen, int pairs, int E, const void* w_a, const void* w_b,
+                                       const float* in_weight, void* Y, long ldy, int O, int I, int act, hipStream_t stream) {
+  GIBBS_REQUIRE(X && chosen && w_a && Y && O > 0 && I > 0 && ldx >= I && ldy >= O && top > 0, "moe_gemm: bad operands O=%d I=%d", O, I);
+  GIBBS_REQUIRE(pairs > 0 && pairs <= WAVE && pairs % top == 0 && pairs / top <= 16 && E > 0 && E <= 65535, "moe_gemm: %d pairs of %d a row without grouping", pairs, top);
+  GIBBS_REQUIRE(act >= 0 && act < ACT_COUNT && (!in_weight || w_b), "moe_gemm: bad activation, or weights on the inputs of an ungated product");
+  GIBBS_REQUIRE(I % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)X % 16) == 0 && ((uintptr_t)w_a % 16) == 0 && ((uintptr_t)w_b % 16) == 0, "moe_gemm: rows of whole 16 bytes");
+  const long stride = (long)O * I;
+  if (w_b)
+    moe_gemm_few_kernel<true, true><<<dim3(ceil_div(O, 16), E), 256, 0, stream>>>((const bf16*)X, chosen, nullptr, (const bf16*)w_a, (const bf16*)w_b, top, I, ldx, stride,
+                                                                                 (bf16*)Y, ldy, O, act, in_weight, pairs);
+  else
+    moe_gemm_few_kernel<false, true><<<dim3(ceil_div(O, 32), E), 256, 0, stream>>>((const bf16*)X, chosen, nullptr, (const bf16*)w_a, nullptr, 0, I, ldx, stride, (bf16*)Y,
+                                                                                  ldy, O, act, nullptr, pairs);
   GIBBS_LAUNCH_STATUS("moe_gemm");
 }
 

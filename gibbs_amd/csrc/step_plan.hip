@@ -1544,6 +1544,7 @@ struct MoeBody : Body {
   const void* down = nullptr;           // [E, hidden, F]
   int E = 0, top = 0, F = 0, act = 0;
   Matrix shared_gate_up, shared_down;   // the shared expert (w null: none): [2 SF, hidden], [hidden, SF]
+  const void* shared_gate_up_packed2 = nullptr;
   int SF = 0, shared_act = 0;
   const float* shared_gate = nullptr;   // [hidden] float32, or null: the shared expert is added as it is
   // mode 1: scores by a softmax over all router outputs, the choice by score + router_bias, weights the chosen scores over
@@ -1554,25 +1555,33 @@ struct MoeBody : Body {
   bool weigh_input = false;   // the weight multiplies the expert's input (its gate and up products) instead of its result
   Pending general(Exec& e, void* h) const override {
     const int N = e.a.n_rows, W = e.p.hidden, pairs = N * top;
+    const bool direct = e.bf16_run && gibbs_moe_direct_takes(N, top, E, W, F) && (((uintptr_t)h | (uintptr_t)gate | (uintptr_t)up | (uintptr_t)down) % 16) == 0;
     const int bm = gibbs_moe_tile(pairs, E);
-    const long cap = gibbs_moe_capacity(pairs, E, bm);
+    const long cap = direct ? pairs : gibbs_moe_capacity(pairs, E, bm);      // rows of the pairs' results
     int* chosen = (int*)e.take((long)pairs * 4);
     float* weight = (float*)e.take((long)pairs * 4);
     float* sgate = shared_gate ? (float*)e.take((long)N * 4) : nullptr;
-    RUN(e, gibbs_moe_route_scaled(h, W, e.p.dtype, router, router_bias, shared_gate, chosen, weight, sgate, N, W, E + identity, top, mode, weight_scale, e.a.stream));
-    int* sorted = (int*)e.take(cap * 4);
     int* place = (int*)e.take((long)pairs * 4);
-    int* tile_expert = (int*)e.take(cap / bm * 4);
-    RUN(e, gibbs_moe_group(chosen, pairs, E, bm, sorted, place, tile_expert, cap, e.a.stream));
-    e.give(chosen);
+    RUN(e, gibbs_moe_route_placed(h, W, e.p.dtype, router, router_bias, shared_gate, chosen, weight, sgate, direct ? place : nullptr, E, N, W, E + identity, top, mode,
+                                  weight_scale, e.a.stream));
+    int *sorted = nullptr, *tile_expert = nullptr;
+    if (!direct) {
+      sorted = (int*)e.take(cap * 4);
+      tile_expert = (int*)e.take(cap / bm * 4);
+      RUN(e, gibbs_moe_group(chosen, pairs, E, bm, sorted, place, tile_expert, cap, e.a.stream));
+    }
     void* mid = e.take(cap * F * e.esize);
-    RUN(e, gibbs_moe_gemm_weighted(h, W, top, sorted, tile_expert, cap, bm, gate, up, weigh_input ? weight : nullptr, mid, F, e.p.dtype, F, W, act, e.a.stream));
+    const float* weighed = weigh_input ? weight : nullptr;
+    if (direct) RUN(e, gibbs_moe_gemm_direct(h, W, top, chosen, pairs, E, gate, up, weighed, mid, F, F, W, act, e.a.stream));
+    else RUN(e, gibbs_moe_gemm_weighted(h, W, top, sorted, tile_expert, cap, bm, gate, up, weighed, mid, F, e.p.dtype, F, W, act, e.a.stream));
     if (weigh_input) {
       e.give(weight);
       weight = nullptr;
     }
     void* y = e.take(cap * W * e.esize);
-    RUN(e, gibbs_moe_gemm(mid, F, 0, sorted, tile_expert, cap, bm, down, nullptr, y, W, e.p.dtype, W, F, 0, e.a.stream));
+    if (direct) RUN(e, gibbs_moe_gemm_direct(mid, F, top, chosen, pairs, E, down, nullptr, nullptr, y, W, W, F, 0, e.a.stream));
+    else RUN(e, gibbs_moe_gemm(mid, F, 0, sorted, tile_expert, cap, bm, down, nullptr, y, W, e.p.dtype, W, F, 0, e.a.stream));
+    e.give(chosen);
     e.give(mid);
     e.give(sorted);
     e.give(tile_expert);
@@ -1580,13 +1589,14 @@ struct MoeBody : Body {
     if (shared_gate_up.w) {
       void* sy = e.take((long)N * SF * e.esize);
       if (e.few_rows && W % 8 == 0 && SF % 8 == 0) {
-        RUN(e, gibbs_skinny_glu_general(h, shared_gate_up.w, sy, N, SF, W, W, W, SF, 0, 0.f, shared_act, 0.f, 0.f, e.a.stream));
+        RUN(e, gibbs_skinny_glu_general(h, shared_gate_up_packed2 ? shared_gate_up_packed2 : shared_gate_up.w, sy, N, SF, W, W, shared_gate_up_packed2 ? 0 : W, SF, 0, 0.f,
+                                        shared_act, 0.f, 0.f, e.a.stream));
       } else {
         void* gu = e.linear(h, shared_gate_up, N, false, false, false, nullptr);
         RUN(e, gibbs_glu(gu, sy, e.p.dtype, N, SF, shared_act, e.a.stream));
         e.give(gu);
       }
-      shared = e.linear(sy, shared_down, N, false, false, false, nullptr);
+      shared = e.linear(sy, shared_down, N, false, false, true, nullptr);
       e.give(sy);
     }
     Pending delta{e.take((long)N * W * e.esize), 1};
@@ -2434,7 +2444,8 @@ GIBBS_EXPORT int gibbs_plan_body_moe(void* plan, const GibbsMoeSpec* d) {
   b->E = d->experts; b->top = d->top; b->F = d->F; b->act = d->act;
   if (d->shared_gate_up) {
     b->shared_gate_up = Matrix{d->shared_gate_up, nullptr, 2 * d->shared_F, p->hidden};
-    b->shared_down = Matrix{d->shared_down, nullptr, p->hidden, d->shared_F};
+    b->shared_gate_up_packed2 = d->p_shared_gate_up;
+    b->shared_down = Matrix{d->shared_down, d->p_shared_down, p->hidden, d->shared_F};
     b->SF = d->shared_F; b->shared_act = d->shared_act; b->shared_gate = d->shared_gate;
   }
   p->bodies.push_back(std::move(b));

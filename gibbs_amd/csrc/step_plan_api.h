@@ -98,6 +98,7 @@ struct GibbsMoeSpec {
   const float* router; const float* router_bias;
   const void* gate; const void* up; const void* down;
   const void* shared_gate_up; const void* shared_down; const float* shared_gate;
+  const void* p_shared_gate_up; const void* p_shared_down;   // in tile order (gate and up each by itself; bfloat16), or null
   int experts, top, F, act, shared_F, shared_act;
 };
 int gibbs_plan_body_moe(void* plan, const struct GibbsMoeSpec* spec);

@@ -125,6 +125,9 @@ _SIGNATURES = {
     "gibbs_rmsnorm_rows_sum_add_read": [c_void_p, c_void_p, c_int, c_long, c_void_p, c_float, c_void_p, c_int, c_float, c_void_p, c_float, c_int,
                                         c_void_p, c_int, c_int, c_int, c_void_p],
     "gibbs_rows_terms": [c_void_p, c_int, c_void_p, c_float, c_void_p, c_int, c_float, c_void_p, c_int, c_int, c_int, c_void_p],
+    "gibbs_moe_route_placed": [c_void_p, c_long, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
+                               c_int, c_int, c_float, c_void_p],
+    "gibbs_moe_gemm_direct": [c_void_p, c_long, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_int, c_int, c_int, c_void_p],
     "gibbs_moe_route_scaled": [c_void_p, c_long, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                c_int, c_float, c_void_p],
     "gibbs_head_norm_gate": [c_void_p, c_void_p, c_int, c_void_p, c_long, c_void_p, c_int, c_int, c_int, c_int, c_float, c_int, c_void_p],

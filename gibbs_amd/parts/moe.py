@@ -89,7 +89,7 @@ class MoeFeedForward(FeedForward):
         self.w_gate = torch.stack([weights[n] for n in t["gate"]]).contiguous()
         self.w_up = torch.stack([weights[n] for n in t["up"]]).contiguous()
         self.w_down = torch.stack([weights[n] for n in t["down"]]).contiguous()
-        self.shared_gate_up = self.shared_down = self.shared_gate = None
+        self.shared_gate_up = self.shared_down = self.shared_gate = self.p_shared_gate_up = self.p_shared_down = None
         if self.shared_inter:
             self.shared_gate_up = torch.cat([weights[t["shared_gate"]], weights[t["shared_up"]]], dim=0).contiguous()
             self.shared_down = weights[t["shared_down"]].contiguous()
@@ -110,6 +110,11 @@ class MoeFeedForward(FeedForward):
 
     def small_tensors(self):
         return [t for t in (self.router_bias, self.shared_gate) if t is not None]
+
+    def pack_matrices(self) -> None:
+        if self.shared_inter:
+            self.p_shared_gate_up = ops.PackedWeight(self.shared_gate_up, groups=2)
+            self.p_shared_down = ops.PackedWeight(self.shared_down)
 
     def emit(self, plan) -> int:
         return plan.moe(self)

@@ -107,6 +107,7 @@ class MoeSpec(ctypes.Structure):
     """GibbsMoeSpec of csrc/step_plan_api.h."""
     _fields_ = [("router", c_void_p), ("router_bias", c_void_p), ("gate", c_void_p), ("up", c_void_p), ("down", c_void_p),
                 ("shared_gate_up", c_void_p), ("shared_down", c_void_p), ("shared_gate", c_void_p),
+                ("p_shared_gate_up", c_void_p), ("p_shared_down", c_void_p),
                 ("experts", c_int), ("top", c_int), ("F", c_int), ("act", c_int), ("shared_F", c_int), ("shared_act", c_int)]
 
 
@@ -477,6 +478,7 @@ class NativePlan:
         d = MoeSpec()
         d.router, d.router_bias, d.gate, d.up, d.down = self._held(m.router, m.router_bias, m.w_gate, m.w_up, m.w_down)
         d.shared_gate_up, d.shared_down, d.shared_gate = self._held(m.shared_gate_up, m.shared_down, m.shared_gate)
+        d.p_shared_gate_up, d.p_shared_down = self._held(m.p_shared_gate_up, m.p_shared_down)
         d.experts, d.top, d.F, d.act = m.experts, m.top, m.inter, ACTIVATIONS[m.activation]
         d.shared_F, d.shared_act = m.shared_inter, ACTIVATIONS[m.shared_activation]
         body = self._made(L.library().gibbs_plan_body_moe(self.handle, ctypes.byref(d)))

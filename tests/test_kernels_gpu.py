@@ -1076,6 +1076,45 @@ def test_several_products_of_one_size_in_a_launch(n, o, i, products, apart):
         close(y[:, p * o:(p + 1) * o], rows.double() @ w[p * o:(p + 1) * o].double().T, torch.bfloat16, f"product {p}", bf16=8e-3)
 
 
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("n,top,experts,identity,width,inner", [(1, 1, 1, 0, 8, 8), (3, 4, 5, 2, 72, 40), (16, 4, 16, 0, 264, 520), (16, 4, 4, 0, 1024, 136),
+                                                                 (8, 8, 9, 3, 256, 64)])
+def test_few_rows_experts_without_grouping(n, top, experts, identity, width, inner, weighted):
+    """Places are the pairs' own numbers (-1: an identity expert), and every pair's gated and returned rows have the bits that the grouped
+    products give them: one pair and 64, an expert that all rows choose, experts that none does, sizes beside the tiles and the
+    stretches of k."""
+    from gibbs_amd.ops.lib import call, dtype_code, library, ptr, stream
+    bf = torch.bfloat16
+    h, router = rnd(n, width, dtype=bf, seed=1), rnd(experts + identity, width, seed=2)
+    wa, wb, wd = rnd(experts, inner, width, dtype=bf, seed=3), rnd(experts, inner, width, dtype=bf, seed=4), rnd(experts, width, inner, dtype=bf, seed=5)
+    pairs = n * top
+    new = lambda *shape, dtype=torch.int32: torch.full(shape, 77, dtype=dtype, device=DEV)
+    chosen, weight, place = new(pairs), new(pairs, dtype=torch.float32), new(pairs)
+    call("gibbs_moe_route_placed", ptr(h), width, dtype_code(bf), ptr(router), None, None, ptr(chosen), ptr(weight), None, ptr(place), experts, n, width,
+         experts + identity, top, 1, 1.0, stream())
+    own = torch.arange(pairs, dtype=torch.int32, device=DEV)
+    assert torch.equal(place, torch.where(chosen < experts, own, -torch.ones_like(own)))
+    tile = 16
+    cap = int(library().gibbs_moe_capacity(pairs, experts, tile))
+    order, at, tiles = new(cap), new(pairs), new(cap // tile)
+    call("gibbs_moe_group", ptr(chosen), pairs, experts, tile, ptr(order), ptr(at), ptr(tiles), cap, stream())
+    scale = ptr(weight) if weighted else None
+    grouped, direct = new(cap, inner, dtype=bf), new(pairs, inner, dtype=bf)
+    call("gibbs_moe_gemm_weighted", ptr(h), width, top, ptr(order), ptr(tiles), cap, tile, ptr(wa), ptr(wb), scale, ptr(grouped), inner, dtype_code(bf), inner, width, 0, stream())
+    call("gibbs_moe_gemm_direct", ptr(h), width, top, ptr(chosen), pairs, experts, ptr(wa), ptr(wb), scale, ptr(direct), inner, inner, width, 0, stream())
+    has = chosen < experts
+    assert torch.equal(direct[has], grouped[at[has].long()])
+    back, out = new(cap, width, dtype=bf), new(pairs, width, dtype=bf)
+    call("gibbs_moe_gemm", ptr(grouped), inner, 0, ptr(order), ptr(tiles), cap, tile, ptr(wd), None, ptr(back), width, dtype_code(bf), width, inner, 0, stream())
+    call("gibbs_moe_gemm_direct", ptr(direct), inner, top, ptr(chosen), pairs, experts, ptr(wd), None, None, ptr(out), width, width, inner, 0, stream())
+    assert torch.equal(out[has], back[at[has].long()])
+    # (against float64: sums of bfloat16 products in float32, a rounding to bfloat16 at the end)
+    for i in torch.nonzero(has).flatten().tolist()[:6]:
+        e, x, w = int(chosen[i]), h[i // top].double(), float(weight[i]) if weighted else 1.0
+        g, u = w * (wa[e].double() @ x), w * (wb[e].double() @ x)
+        close(direct[i], F.silu(g) * u, bf, f"pair {i}", bf16=8e-3)
+
+
 @pytest.mark.parametrize("parts", [0, 1, 3])
 @pytest.mark.parametrize("hidden", [4, 516, 2048, 5000])
 def test_norm_that_leaves_a_mirror(hidden, parts):
