@@ -554,6 +554,9 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
       } else if (a.act == ACT_RELU_SQUARED) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = (bf16)(activate(sum[0][i], ACT_RELU_SQUARED) * pre_x[i]);
+      } else if (a.act == ACT_TANH) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (bf16)(tanhf(sum[0][i]) * pre_x[i]);
       } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = (bf16)(activate(sum[0][i], a.act) * pre_x[i]);
