@@ -38,7 +38,7 @@ GIBBS_EXPORT int gibbs_embed_general(const void* table, int dtype, const int* id
   GIBBS_REQUIRE(!inv_freq || pos, "embed: a position vector needs the rows' positions");
   if (n == 0) return 0;
   // (a row's sines are long code that each thread walks once for each of its columns: few rows share theirs out over workgroups.  8 rows of
-  // 2,048 with a position vector, us: a workgroup a row 10.2, eight 2.9)
+  // 2,048 with a position vector, us: a workgroup a row 10.2, eight 4.8)
   const int threads = hidden >= 1024 ? 256 : 64;
   const dim3 grid(n, inv_freq && n <= 128 ? ceil_div(hidden, threads) : 1);
   if (dtype == GIBBS_F32)

@@ -63,7 +63,7 @@ int gibbs_skinny_store_as(const void* X, const void* W, void* Y, int out_dtype, 
 }
 
 // `products` of these in one launch: W holds as many matrices [O, I] one behind the other, each in tile order by itself; product p reads the rows at
-// X + p x_apart (0: the same rows) and writes at Y + p y_apart.  Four of 8 rows x 2,048 x 2,048 take 7.5 us so, and 17.5 one after
+// X + p x_apart (0: the same rows) and writes at Y + p y_apart.  Four of 8 rows x 2,048 x 2,048 take 9.4 us so, and 17.8 one after
 // the other: a launch's path from its first instruction to its last store is 3 us whatever it multiplies.
 GIBBS_EXPORT int gibbs_skinny_store_many(const void* X, long x_apart, const void* W, int products, void* Y, long y_apart, int N, int O, int I,
                                          long ldx, long ldy, hipStream_t stream) {

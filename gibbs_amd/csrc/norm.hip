@@ -39,6 +39,24 @@ __device__ __forceinline__ float4 load4(const bf16* p) {
   const bf16x4 v = *(const bf16x4*)p;
   return make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
 }
+// v += the partial sums `first` .. parts - 1 at p, `apart` elements from one to the next, in ascending order.  Eight or four are asked for before the
+// first is added (beyond the last: the last one again, not added): one after the other, each is a trip to memory, 0.3 us.  45 rows of
+// 1,024 in 12 parts, added and normed: 6.1 -> 4.6 us.
+template <typename D>
+__device__ __forceinline__ void add_parts4(float4& v, const D* p, int first, int parts, size_t apart) {
+  auto some = [&](auto count, int s) {
+    constexpr int N = decltype(count)::value;
+    float4 m[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) m[u] = load4(p + (size_t)min(s + u, parts - 1) * apart);
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+      if (s + u < parts) { v.x += m[u].x; v.y += m[u].y; v.z += m[u].z; v.w += m[u].w; }
+  };
+  int s = first;
+  for (; parts - s > 4; s += 8) some(std::integral_constant<int, 8>{}, s);
+  if (s < parts) some(std::integral_constant<int, 4>{}, s);
+}
 __device__ __forceinline__ void store4(float* p, float4 v) { *(float4*)p = v; }
 __device__ __forceinline__ void store4(bf16* p, float4 v) {
   typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
@@ -68,10 +86,7 @@ __global__ void add_rmsnorm_vec_kernel(float* __restrict__ x, const D* __restric
       v[c] = *(const float4*)(xr + i);
       if (dr) {
         float4 d = load4(dr + i);
-        for (int s = 1; s < parts; ++s) {
-          const float4 more = load4(dr + s * apart + i);
-          d.x += more.x; d.y += more.y; d.z += more.z; d.w += more.w;
-        }
+        add_parts4(d, dr + i, 1, parts, apart);
         v[c].x += d.x; v[c].y += d.y; v[c].z += d.z; v[c].w += d.w;
         if (write_x) *(float4*)(xr + i) = v[c];
       }
@@ -313,10 +328,7 @@ template <typename T>
 __device__ __forceinline__ float4 sum_parts4(const void* in, int parts, size_t part_stride, size_t i) {
   if (parts == 1) return load4((const T*)in + i);
   float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int s = 0; s < parts; ++s) {
-    const float4 d = *(const float4*)((const float*)in + s * part_stride + i);
-    v.x += d.x; v.y += d.y; v.z += d.z; v.w += d.w;
-  }
+  add_parts4(v, (const float*)in + i, 0, parts, part_stride);
   return v;
 }
 template <typename T, int CHUNKS, int FROM, int READ>
