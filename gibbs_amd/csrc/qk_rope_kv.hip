@@ -20,6 +20,11 @@
 #include "lane8.h"
 
 namespace {
+// Up to one workgroup of 256 a compute unit, a lane group takes one head and not four.  Four heads / one, us, by lanes in all: heads of 64, 16 + 2 x 8 of
+// them, 11,520 (45 rows) 7.4 / 5.6, 65,536 7.7 / 5.3, 131,072 7.9 / 6.6, 262,144 8.6 / 9.9; heads of 128, 32 + 2 x 8, 34,560 8.1 / 6.0, 61,440
+// 8.1 / 6.0, 98,304 8.3 / 8.1, 147,456 8.3 / 10.4.
+constexpr long FEW_LANES = 1 << 16;
+
 enum { ROPE_HALF_SPLIT = 0, ROPE_INTERLEAVED = 1 };
 
 struct QkRopeArgs {
@@ -120,6 +125,8 @@ __global__ __launch_bounds__(256) void qk_rope_kv_bf16x8_kernel(bf16* __restrict
   const int hd = a.hd;
   const bool active = item_ok && e0 < hd;
   const int p = a.pos[n];
+  // (few rows: asked for beside the position, so that what hangs on both is one trip later, not two; many rows: 14.6 -> 15.6 us with it)
+  const int req = HPI == 1 && kpages ? a.row_req[n] : 0;
   bf16* row = qkv + (size_t)n * a.ld + e0;
   uint4 raw[HPI];
 #pragma unroll
@@ -128,7 +135,7 @@ __global__ __launch_bounds__(256) void qk_rope_kv_bf16x8_kernel(bf16* __restrict
   // the page of the row's position, if a head of this item goes there
   int page = -1;
   if (kpages && active && hs0 + HPI > a.nh) {
-    page = a.table[(size_t)a.row_req[n] * a.max_pages + p / a.page_size];
+    page = a.table[(size_t)(HPI == 1 ? req : a.row_req[n]) * a.max_pages + p / a.page_size];
     if (page >= a.num_pages) page = -1;  // the host never asks for another; never write outside
   }
   const Rot8 rt = rotation8(e0, a.inv_freq, a.rot, a.variant, p, a.cs_table, a.table_len);
@@ -202,17 +209,22 @@ GIBBS_EXPORT int gibbs_qk_rope_kv(void* qkv, void* kpages, void* vpages, int dty
                       ((uintptr_t)qkv % 16) == 0;
   if (lanes8) {
     const int lanes = hd / EPL;
-    const long items = (long)n_rows * ceil_div(slots, 4);   // a lane group takes four consecutive heads of a row
+    // a lane group takes four consecutive heads of a row, or one where four would leave most of the chip idle
+    const long heads = (long)n_rows * slots;
+    const bool few = heads * lanes <= FEW_LANES;
+    const long items = few ? heads : (long)n_rows * ceil_div(slots, 4);
     GIBBS_REQUIRE(items < (1l << 31) - 64, "qk_rope_kv: %d rows of %d heads are more than the kernel numbers", n_rows, slots);
-#define GIBBS_ROPE8(LPK)                                                                                   \
-  qk_rope_kv_bf16x8_kernel<LPK, 4><<<ceil_div(items, 4 * (WAVE / LPK)), 256, 0, stream>>>((bf16*)qkv, (bf16*)kpages, \
-                                                                                           (bf16*)vpages, a, n_rows)
-    if (lanes <= 2) GIBBS_ROPE8(2);
-    else if (lanes <= 4) GIBBS_ROPE8(4);
-    else if (lanes <= 8) GIBBS_ROPE8(8);
-    else if (lanes <= 16) GIBBS_ROPE8(16);
-    else GIBBS_ROPE8(32);
-#undef GIBBS_ROPE8
+    const auto queue = [&](auto group) {
+      constexpr int LPK = decltype(group)::value;
+      const unsigned blocks = ceil_div(items, 4 * (WAVE / LPK));
+      if (few) qk_rope_kv_bf16x8_kernel<LPK, 1><<<blocks, 256, 0, stream>>>((bf16*)qkv, (bf16*)kpages, (bf16*)vpages, a, n_rows);
+      else qk_rope_kv_bf16x8_kernel<LPK, 4><<<blocks, 256, 0, stream>>>((bf16*)qkv, (bf16*)kpages, (bf16*)vpages, a, n_rows);
+    };
+    if (lanes <= 2) queue(std::integral_constant<int, 2>{});
+    else if (lanes <= 4) queue(std::integral_constant<int, 4>{});
+    else if (lanes <= 8) queue(std::integral_constant<int, 8>{});
+    else if (lanes <= 16) queue(std::integral_constant<int, 16>{});
+    else queue(std::integral_constant<int, 32>{});
   } else if (dtype == GIBBS_F32)
     qk_rope_kv_kernel<float><<<grid, 256, 0, stream>>>((float*)qkv, (float*)kpages, (float*)vpages, a);
   else if (dtype == GIBBS_BF16)

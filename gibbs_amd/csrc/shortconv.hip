@@ -74,7 +74,7 @@ __global__ __launch_bounds__(256) void shortconv_kernel(
 // K is a template parameter (2..4, what LFM2 checkpoints use); other lengths take the kernel above.
 // (float32, 1,194 rows of 1,024 channels: 31.7 us a channel a thread, K loads and products a row; 6.1 us so.)
 constexpr int TLV = 8;   // rows per tile (>= K - 1)
-constexpr int RU = 4;    // rows whose loads are in flight together
+constexpr int RU = 4;    // rows whose loads are in flight together, and rows per tile where rows are few
 
 __device__ __forceinline__ void unpack16(const uint4& raw, float (&f)[8]) {
   const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
@@ -101,7 +101,7 @@ __device__ __forceinline__ uint4 pack16(const float (&f)[4]) {
   return make_uint4(__float_as_uint(f[0]), __float_as_uint(f[1]), __float_as_uint(f[2]), __float_as_uint(f[3]));
 }
 
-template <typename T, int K>
+template <typename T, int K, int ROWS>
 __global__ __launch_bounds__(64) void shortconv_vec_kernel(
     const T* __restrict__ bcx, const float* __restrict__ taps, const float* __restrict__ bias,
     float* __restrict__ state, long slot_stride, const int* __restrict__ cu, const int* __restrict__ ctx,
@@ -115,7 +115,7 @@ __global__ __launch_bounds__(64) void shortconv_vec_kernel(
     tile -= lead_single;
     for (r = lead_single; r < n_req; ++r) {
       q = cu[r + 1] - cu[r];
-      const int t = (q + TLV - 1) / TLV;
+      const int t = (q + ROWS - 1) / ROWS;
       if (tile < t) break;
       tile -= t;
     }
@@ -148,13 +148,10 @@ __global__ __launch_bounds__(64) void shortconv_vec_kernel(
       for (int i = 0; i < V; ++i) out[i] = have ? st[(size_t)(K - 1 + tp) * C + c0 + i] : 0.f;
     }
   };
-  const int t0 = tile * TLV, t_end = min(q, t0 + TLV);
-  float win[K][V];  // win[j]: B * x of row t - (K-1) + j
-#pragma unroll
-  for (int j = 0; j < K - 1; ++j) bx_at(t0 - (K - 1) + j, win[j + 1]);
-  for (int tg = t0; tg < t_end; tg += RU) {
-    // the loads of RU rows first, then their arithmetic: a wave is alone with its rows' latency
-    uint4 rb[RU], rx[RU], rc[RU];
+  const int t0 = tile * ROWS, t_end = min(q, t0 + ROWS);
+  // the loads of RU rows first, then their arithmetic: a wave is alone with its rows' latency
+  uint4 rb[RU], rx[RU], rc[RU];
+  auto ask = [&](int tg) {
 #pragma unroll
     for (int u = 0; u < RU; ++u) {
       rb[u] = rx[u] = rc[u] = make_uint4(0, 0, 0, 0);
@@ -165,6 +162,13 @@ __global__ __launch_bounds__(64) void shortconv_vec_kernel(
         rx[u] = *(const uint4*)(row + 2 * C);
       }
     }
+  };
+  ask(t0);   // (in front of the window's loads, which branch: one trip to memory for both)
+  float win[K][V];  // win[j]: B * x of row t - (K-1) + j
+#pragma unroll
+  for (int j = 0; j < K - 1; ++j) bx_at(t0 - (K - 1) + j, win[j + 1]);
+  for (int tg = t0; tg < t_end; tg += RU) {
+    if (tg != t0) ask(tg);
 #pragma unroll
     for (int u = 0; u < RU; ++u) {
       const int t = tg + u;
@@ -221,10 +225,16 @@ GIBBS_EXPORT int gibbs_shortconv(const void* bcx, const float* taps, const float
   const int vec = dtype == GIBBS_F32 ? 4 : 8;
   if (C % vec == 0 && K <= 4 && ((uintptr_t)bcx % 16) == 0 && ((uintptr_t)y % 16) == 0 && (dtype == GIBBS_BF16 || tiles(TLV) <= 65535)) {
     GIBBS_REQUIRE(tiles(TLV) <= 65535, "shortconv: too many row tiles (%d)", (int)tiles(TLV));
-    const dim3 vgrid(ceil_div(C, vec * 64), tiles(TLV));
+    const int columns = ceil_div(C, vec * 64);
+    // Tiles of 8 rows / of 4, us: bfloat16, 1,024 channels, 45 rows 5.5 / 4.5, 512 6.0 / 5.0, 2,048 7.6 / 6.9; 2,048 channels, 45 rows 5.7 / 4.8, 1,024 7.6 / 7.0,
+    // 2,048 10.0 / 9.9; float32, 1,024 channels, 45 rows 4.5 / 3.9, 1,024 6.6 / 6.3, 2,048 8.9 / 9.0.  (Larger: a tile's K - 1 rows in front of it are read again.)
+    const bool few = (size_t)rest_rows * C <= (size_t)(dtype == GIBBS_F32 ? 1 : 2) << 20 && tiles(RU) <= 65535;
+    const dim3 vgrid(columns, tiles(few ? RU : TLV));
     auto launch = [&](auto type, auto length) {
       typedef decltype(type) T;
-      shortconv_vec_kernel<T, decltype(length)::value><<<vgrid, 64, 0, stream>>>((const T*)bcx, taps, bias, state, slot_stride, cu, ctx, slot, (T*)y, n_req, C, lead_single);
+      constexpr int L = decltype(length)::value;
+      if (few) shortconv_vec_kernel<T, L, RU><<<vgrid, 64, 0, stream>>>((const T*)bcx, taps, bias, state, slot_stride, cu, ctx, slot, (T*)y, n_req, C, lead_single);
+      else shortconv_vec_kernel<T, L, TLV><<<vgrid, 64, 0, stream>>>((const T*)bcx, taps, bias, state, slot_stride, cu, ctx, slot, (T*)y, n_req, C, lead_single);
     };
     auto by_length = [&](auto type) {
       if (K == 2) launch(type, std::integral_constant<int, 2>{});

@@ -333,6 +333,26 @@ def test_shortconv_ragged_with_state(dtype, K, C, bias):
         close(state[slot], full[-(K - 1):], torch.float32, "state", f32=1e-6)
     assert torch.all(state[1] == 7.0), "a slot of no request was written"
 
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("C,over", [(64, 1), (1024, 1), (1024, 5)])
+def test_shortconv_tiles_of_few_and_of_many_rows(dtype, C, over):
+    """Where rows stop being few (4 MB of values): the rows of a request are to the bit those of the same request a few rows longer, and its state that of
+    the same rows brought by two calls."""
+    from gibbs_amd import ops
+    line = (1 << (20 if dtype == torch.float32 else 21)) // C
+    taps, x = rnd(C, 3, seed=4), rnd(line + over, 3 * C, dtype=dtype, seed=5)
+    def run(*cuts):
+        state, rows, at = torch.full((1, 2, C), 7.0, device=DEV), [], 0
+        for cut in cuts:
+            rows.append(ops.shortconv(x[at:cut].contiguous(), taps, None, state, i32([0, cut - at]), i32([at]), i32([0]), cut - at, 1))
+            at = cut
+        return torch.cat(rows), state
+    few, few_state = run(line)
+    many, many_state = run(line + over)
+    rest, rest_state = run(line, line + over)
+    assert torch.equal(few, many[:line]) and torch.equal(rest, many) and torch.equal(rest_state, many_state)
+    assert torch.equal(few_state[0], (x[line - 2:line, :C].float() * x[line - 2:line, 2 * C:].float()))
+
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("C", [24, 520])
@@ -725,6 +745,31 @@ def test_qk_rope_kv(dtype, variant, nh, nkv, hd, rot, table_len):
         close(kp[pg, :, p % page], kr[i], dtype, "k page", bf16=8e-3)
         assert torch.equal(vp[pg, :, p % page], v0[i])
     assert kp.float().abs().sum(dim=(1, 3)).count_nonzero().item() == n, "exactly one page slot per row was written"
+
+@pytest.mark.parametrize("nh,nkv,hd", [(16, 8, 64), (3, 1, 48), (6, 1, 256), (5, 2, 16)])
+def test_qk_rope_kv_one_head_or_four_a_lane_group(nh, nkv, hd):
+    """Where rows stop being few (65,536 lanes of 8 values): rows and cache pages are to the bit those of a call with some more rows."""
+    from gibbs_amd import ops
+    from gibbs_amd.parts.rope import rope_inv_freq
+    line = (1 << 16) // ((nh + 2 * nkv) * (hd // 8))
+    rows, page = line + 3, 64
+    pages = rows // page + 1
+    x, qg, kg = rnd(rows, (nh + 2 * nkv) * hd, dtype=torch.bfloat16), rnd(hd, seed=1) + 1, rnd(hd, seed=2) + 1
+    inv = torch.from_numpy(rope_inv_freq(hd, 10000.0, "f32")).to(DEV)
+    table = i32([np.random.default_rng(3).permutation(pages).tolist()])
+    def run(n):
+        qkv = x[:n].clone()
+        kp, vp = (torch.zeros(pages, nkv, page, hd, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+        ops.qk_rope_kv(qkv, n, nh, nkv, hd, q_gain=qg, k_gain=kg, eps=1e-6, inv_freq=inv, rotary_dim=hd, variant="half_split",
+                       pos=i32(list(range(n))), row_req=i32([0] * n), kpages=kp, vpages=vp, table=table, n_req=1, cos_sin=ops.rope_table(inv, 128))
+        for r in range(n, rows):
+            assert not kp[table[0, r // page].item(), :, r % page].any()
+        return qkv[:, :nh * hd], kp, vp
+    few, many = run(line), run(rows)
+    for r in range(line, rows):
+        many[1][table[0, r // page].item(), :, r % page] = 0
+        many[2][table[0, r // page].item(), :, r % page] = 0
+    assert torch.equal(few[0], many[0][:line]) and torch.equal(few[1], many[1]) and torch.equal(few[2], many[2])
 
 
 def plain_qk(x, gain, positions, inv, eps):
