@@ -107,6 +107,23 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
   return total;
 }
 
+// first + part[apart] + part[2 apart] + ... (`more` of them), in this order, read from LDS eight or four at a time: one by one each is a
+// trip of its own, 60 ns.
+__device__ __forceinline__ float strided_sum(float first, const float* part, int more, int apart) {
+  auto some = [&](auto count, int g) {
+    constexpr int N = decltype(count)::value;
+    float m[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) m[u] = part[min(g + u, more) * apart];
+#pragma unroll
+    for (int u = 0; u < N; ++u) first = g + u <= more ? first + m[u] : first;
+  };
+  int g = 1;
+  for (; more - g >= 4; g += 8) some(std::integral_constant<int, 8>{}, g);
+  if (g <= more) some(std::integral_constant<int, 4>{}, g);
+  return first;
+}
+
 // Every file of the library sees the entry points' prototypes, so that a definition whose signature has
 // drifted from what the native step (step_plan.hip) calls does not compile.
 #include "kernels.h"

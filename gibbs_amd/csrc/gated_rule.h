@@ -164,8 +164,7 @@ __global__ __launch_bounds__(STEP_THREADS) void gated_rule_rows_kernel(RuleArgs 
     __syncthreads();
     float ss = 0.f;
     for (int j = tid; j < V; j += STEP_THREADS) {
-      float t = part[j];
-      for (int g = 1; g < groups; ++g) t += part[g * V + j];
+      float t = strided_sum(part[j], part + j, groups - 1, V);
       part[j] = t;
       ss = fmaf(t, t, ss);
     }

@@ -157,8 +157,7 @@ __global__ __launch_bounds__(STEP_THREADS) void matrix_lstm_rows_kernel(LstmArgs
     const float inv_den = 1.0f / (fmaxf(fabsf(nq), expf(-m)) + TINY);
     float ss = 0.f;
     for (int j = tid; j < V; j += STEP_THREADS) {
-      float t = part[j];
-      for (int g = 1; g < groups; ++g) t += part[g * V + j];
+      float t = strided_sum(part[j], part + j, groups - 1, V);
       t *= inv_den;
       part[j] = t;
       ss = fmaf(t, t, ss);

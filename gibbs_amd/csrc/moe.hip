@@ -210,6 +210,47 @@ __device__ __forceinline__ void choose_experts(float* z, float* score, int n, in
   }
 }
 
+// The same for at most WAVE experts, a lane each (`correction`: this lane's router_bias, asked for by the caller in front of the logits; 0
+// where there is none): a lane counts the experts in front of its own, by descending value and ascending index, NaN behind all, and hands
+// its own to the lane of that place.  The same choices, weights and bits: the order is the one in which the turns above take them.  A turn is
+// a chain of 0.4 us (LDS, six exchanges, LDS), an expert counted 10 ns: 8 rows of 16 experts, 4 chosen, scores over all, logits included, 8.3 -> 6.7 us;
+// 1,992 rows 18.7 -> 16.4.
+__device__ __forceinline__ void choose_in_lanes(const float* z, float correction, bool corrected, int n, int lane, int* __restrict__ chosen, float* __restrict__ weight,
+                                                int E, int top, int mode, float weight_scale, int* __restrict__ place, int matrices) {
+  const bool expert = lane < E;
+  float v = expert ? z[lane] : -INFINITY, score = 0.f;
+  if (mode == 2 && corrected) {
+    score = 1.0f / (1.0f + expf(-v));
+    v = score + correction;
+  } else if (mode == 1) {
+    const float power = expf(v - wave_max(v));
+    score = power / wave_sum(expert ? power : 0.f);
+    v = score + correction;
+  }
+  // (whole numbers in the order of the values; both zeros are one number, and NaN lies under -inf)
+  const int bits = __float_as_int(v + 0.f), key = v == v ? bits ^ ((bits >> 31) & 0x7fffffff) : (int)0x80000000;
+  int ahead = expert ? 0 : lane;
+#pragma unroll 8
+  for (int e = 0; e < E; ++e) {
+    const int other = __builtin_amdgcn_readlane(key, e);
+    ahead += expert && other >= key + (e >= lane ? 1 : 0) ? 1 : 0;
+  }
+  const int pick = __builtin_amdgcn_ds_permute(ahead * 4, lane);
+  float pv = __int_as_float(__builtin_amdgcn_ds_permute(ahead * 4, __float_as_int(v)));
+  score = __int_as_float(__builtin_amdgcn_ds_permute(ahead * 4, __float_as_int(score)));
+  if (!(pv == pv)) pv = -INFINITY;
+  const float best = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pv), 0));
+  const float w = (mode == 1 || (mode == 2 && corrected)) ? score
+                  : (pv == -INFINITY ? 0.f : (mode == 2 ? 1.0f / (1.0f + expf(-pv)) : expf(pv - best)));
+  float sum = 0.f;
+  for (int c = 0; c < top; ++c) sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), c));
+  if (lane < top) {
+    chosen[(size_t)n * top + lane] = pick;
+    weight[(size_t)n * top + lane] = mode == 2 ? w : (mode == 1 ? w / (sum + 1e-20f) * weight_scale : (sum > 0.f ? w / sum : 0.f));
+    if (place) place[(size_t)n * top + lane] = pick < matrices ? n * top + lane : -1;
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(1024) void moe_route_kernel(const T* __restrict__ h, long ldh, const float* __restrict__ router,
                                                         const float* __restrict__ router_bias, const float* __restrict__ shared_gate,
@@ -219,6 +260,7 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(const T* __restrict__ h
   const int n = blockIdx.x, wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, n_waves = blockDim.x / WAVE;
   const T* row = h + (size_t)n * ldh;
   const bool vec = W % 4 == 0 && ldh % 4 == 0 && ((uintptr_t)h % 16) == 0 && ((uintptr_t)router % 16) == 0 && ((uintptr_t)shared_gate % 16) == 0;
+  const float correction = router_bias && mode != 0 && wave == 0 && lane < E ? router_bias[lane] : 0.f;
   // the last wave also has the shared expert's gate: with its last expert's logit in one pass over the row
   bool gate_left = shared_gate && wave == n_waves - 1;
   for (int e = wave; e < E; e += n_waves) {
@@ -241,7 +283,8 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(const T* __restrict__ h
   }
   __syncthreads();
   if (wave != 0) return;
-  choose_experts(z, z + E, n, lane, router_bias, chosen, weight, E, top, mode, weight_scale, place, matrices);
+  if (E <= WAVE) choose_in_lanes(z, correction, router_bias != nullptr, n, lane, chosen, weight, E, top, mode, weight_scale, place, matrices);
+  else choose_experts(z, z + E, n, lane, router_bias, chosen, weight, E, top, mode, weight_scale, place, matrices);
 }
 
 // Many rows: a workgroup of four waves takes four of them, a wave two experts' logits of all four rows at a time, so that a router's row is read
@@ -255,6 +298,7 @@ __global__ __launch_bounds__(ROUTE_ROWS * WAVE) void moe_route_rows_kernel(const
   extern __shared__ float z[];   // [ROUTE_ROWS][E], and as many scores behind them
   const int n0 = blockIdx.x * ROUTE_ROWS, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
   const int vectors = E + (shared_gate ? 1 : 0);
+  const float correction = router_bias && mode != 0 && lane < E ? router_bias[lane] : 0.f;
   const T* rows[ROUTE_ROWS];
 #pragma unroll
   for (int r = 0; r < ROUTE_ROWS; ++r) rows[r] = h + (size_t)min(n0 + r, N - 1) * ldh;
@@ -304,7 +348,9 @@ __global__ __launch_bounds__(ROUTE_ROWS * WAVE) void moe_route_rows_kernel(const
       }
   }
   __syncthreads();
-  if (n0 + wave < N) choose_experts(z + wave * E, z + (ROUTE_ROWS + wave) * E, n0 + wave, lane, router_bias, chosen, weight, E, top, mode, weight_scale);
+  if (n0 + wave >= N) return;
+  if (E <= WAVE) choose_in_lanes(z + wave * E, correction, router_bias != nullptr, n0 + wave, lane, chosen, weight, E, top, mode, weight_scale, nullptr, 0);
+  else choose_experts(z + wave * E, z + (ROUTE_ROWS + wave) * E, n0 + wave, lane, router_bias, chosen, weight, E, top, mode, weight_scale);
 }
 
 // ------------------------------------------------------------------------------------------------- group

@@ -508,7 +508,7 @@ __global__ __launch_bounds__(256) void head_norm_gate_vec8_kernel(const float* _
 // thread (tx, group) holds columns 4 tx .. and rows group, group + groups, ... in registers from the load to the store; the two sums over
 // the key channels meet in LDS in group order.  Bound by its chain (state and operands arrive, two sums, the norm), not by the state's
 // bytes.  8 requests, 16 heads of 128 x 128: the walk, whose lanes read 16 bytes of a state's row at a time, took 14.5 us and the kernels
-// around it 8.7; this one 9.9.
+// around it 8.7; this one 9.5.
 struct DeltaStepArgs {
   const float* qkv; long ld;            // convolved rows: q [G D], k [G D], v [H V]
   const void* beta_raw; const void* a_head; long ld_raw;
@@ -567,8 +567,7 @@ __global__ __launch_bounds__(STEP_THREADS) void delta_step_kernel(DeltaStepArgs 
     __syncthreads();
     float t = 0.f;
     if (j < V) {
-      t = part[j];
-      for (int g = 1; g < groups; ++g) t += part[g * V + j];
+      t = strided_sum(part[j], part + j, groups - 1, V);
     }
     return t;
   };

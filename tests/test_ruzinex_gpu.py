@@ -485,6 +485,50 @@ def test_routes_of_many_rows_among_any_number_of_experts(n, W, E, top, dtype):
         for a, b in zip(many, few):
             assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(nan=7.0), b.nan_to_num(nan=7.0)), mode
 
+@pytest.mark.parametrize("E,top", [(1, 1), (7, 7), (16, 4), (63, 5), (64, 64), (65, 9)])
+@pytest.mark.parametrize("mode,corrected", [(0, True), (1, False), (1, True), (2, False), (2, True)])
+def test_choices_among_equal_infinite_and_no_numbers(E, top, mode, corrected):
+    """A lane an expert up to a wave's lanes, turns beyond: the experts by descending score and ascending index, NaN last, where scores are whole numbers (both
+    zeros among them), -inf, +inf and NaN; weights within 16 roundings of 32 bits of those in 64 (no power here has an argument beyond 8)."""
+    from gibbs_amd.ops.lib import call, ptr, stream
+    rng = np.random.default_rng(E * 8 + mode)
+    n, W = 40, 4
+    z = rng.integers(-4, 4, (n, E)).astype(np.float32)
+    z[:, ::3] *= -1.0                                         # (zeros of both signs)
+    odd = {3: [np.nan], 4: [-np.inf], 5: [np.nan, -np.inf], 6: [np.nan] * E, 7: [-np.inf] * E}
+    for r, values in odd.items():
+        z[r, rng.permutation(E)[:len(values)]] = values[:E]
+    bias = rng.integers(-2, 3, E).astype(np.float32) if corrected else None
+    got_c, got_w = [], []
+    for r in range(n):                                        # (a router of each row's own: its logits are its first column, exactly)
+        router = np.zeros((E, W), np.float32)
+        router[:, 0] = z[r]
+        h = torch.tensor([[1.0, 0.0, 0.0, 0.0]], device="cuda")
+        c, w = torch.full((1, top), -1, dtype=torch.int32, device="cuda"), torch.zeros((1, top), device="cuda")
+        rt, bs = torch.tensor(router, device="cuda"), torch.tensor(bias, device="cuda") if corrected else None
+        call("gibbs_moe_route_scaled", ptr(h), W, 0, ptr(rt), ptr(bs) if corrected else None, None, ptr(c), ptr(w), None, 1, W, E, top, mode, 1.0, stream())
+        got_c.append(c[0].cpu().numpy()), got_w.append(w[0].cpu().numpy())
+    for r in range(n):
+        with np.errstate(all="ignore"):
+            v = z[r].astype(np.float64) + (bias if corrected and mode == 0 else 0)
+            score = 1 / (1 + np.exp(-v)) if mode == 2 else np.exp(v - np.nanmax(v)) / np.exp(v - np.nanmax(v)).sum()
+            if mode == 1 or (mode == 2 and corrected):
+                ranked = score + (bias if corrected else 0)
+                # (scores that 32 bits cannot tell apart, or that 64 bits hold apart by rounding alone)
+                order = sorted(range(E), key=lambda e: (np.isnan(ranked[e]), -np.round(np.nan_to_num(ranked[e]), 6), e))
+            else:
+                order = sorted(range(E), key=lambda e: (np.isnan(v[e]), -np.nan_to_num(v[e], nan=0.0), e))
+            want = order[:top]
+            assert got_c[r].tolist() == want, (r, z[r])
+            if mode == 0:
+                p = np.where(np.isnan(v[want]) | (v[want] == -np.inf), 0.0, np.exp(v[want] - v[want[0]]))
+                weight = p / p.sum() if p.sum() > 0 else np.zeros(top)
+            elif mode == 1:
+                weight = score[want] / (score[want].sum() + 1e-20)
+            else:
+                weight = score[want] if corrected else np.where(np.isnan(v[want]) | (v[want] == -np.inf), 0.0, score[want])
+        np.testing.assert_allclose(got_w[r], weight, rtol=16 * 2.0 ** -24 + top * 2.0 ** -24, atol=1e-30)
+
 
 @pytest.mark.parametrize("O,I", [(8, 4), (33, 68), (96, 260), (512, 1024), (70, 2052)])
 @pytest.mark.parametrize("gated", [False, True])
