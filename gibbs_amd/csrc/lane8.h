@@ -168,6 +168,27 @@ __device__ __forceinline__ Rot8 rotation8(int e0, const float* inv_freq, int rot
   Rot8 r;
   const int half = rot / 2;
   const bool tabled = table && pos < table_len;
+  // (eight elements of the rotated part have neighbouring factors: a table's row is read 16 bytes at a time, not a pair at a time under
+  // a condition of its own.  The table is of pairs, its rows need not start at 16 bytes)
+  typedef float floatx4_8 __attribute__((ext_vector_type(4), aligned(8)));
+  if (inv_freq && tabled && e0 + EPL <= rot && half % EPL == 0) {
+    const float2* row = table + (size_t)pos * half + (variant == 1 ? e0 / 2 : (e0 < half ? e0 : e0 - half));
+    if (variant == 1) {
+#pragma unroll
+      for (int i = 0; i < EPL; i += 4) {
+        const floatx4_8 t = *(const floatx4_8*)(row + i / 2);
+        r.c[i] = r.c[i + 1] = t[0]; r.s[i] = r.s[i + 1] = t[1];
+        r.c[i + 2] = r.c[i + 3] = t[2]; r.s[i + 2] = r.s[i + 3] = t[3];
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < EPL; i += 2) {
+        const floatx4_8 t = *(const floatx4_8*)(row + i);
+        r.c[i] = t[0]; r.s[i] = t[1]; r.c[i + 1] = t[2]; r.s[i + 1] = t[3];
+      }
+    }
+    return r;
+  }
 #pragma unroll
   for (int i = 0; i < EPL; ++i) {
     const int e = e0 + i;

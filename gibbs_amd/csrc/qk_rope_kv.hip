@@ -20,10 +20,10 @@
 #include "lane8.h"
 
 namespace {
-// Up to one workgroup of 256 a compute unit, a lane group takes one head and not four.  Four heads / one, us, by lanes in all: heads of 64, 16 + 2 x 8 of
-// them, 11,520 (45 rows) 7.4 / 5.6, 65,536 7.7 / 5.3, 131,072 7.9 / 6.6, 262,144 8.6 / 9.9; heads of 128, 32 + 2 x 8, 34,560 8.1 / 6.0, 61,440
-// 8.1 / 6.0, 98,304 8.3 / 8.1, 147,456 8.3 / 10.4.
-constexpr long FEW_LANES = 1 << 16;
+// Up to six workgroups of 256 a compute unit, a lane group takes one head and not four.  Four heads / one, us, by lanes in all: heads of 64, 16 + 2 x 8 of
+// them, 11,520 (45 rows) 6.4 / 5.6, 65,536 6.5 / 5.4, 262,144 7.6 / 6.2; 32 + 2 x 8, 196,608 6.8 / 5.4, 393,216 9.1 / 8.0; heads of 128, 32 + 2 x 8, 61,440
+// 6.2 / 4.3, 196,608 6.6 / 5.3, 393,216 8.8 / 8.0, 786,432 11.9 / 12.5.
+constexpr long FEW_LANES = 3 << 17;
 
 enum { ROPE_HALF_SPLIT = 0, ROPE_INTERLEAVED = 1 };
 
@@ -104,11 +104,24 @@ __global__ __launch_bounds__(256) void qk_rope_kv_kernel(T* __restrict__ qkv, T*
   for (int e = 2 * half + lane; e < hd; e += WAVE) dst[e] = from_float<T>(normed(e));
 }
 
+__device__ __forceinline__ void gains8(const float* gain, int e0, bool active, float (&out)[EPL]) {
+  typedef float floatx4_4 __attribute__((ext_vector_type(4), aligned(4)));
+#pragma unroll
+  for (int i = 0; i < EPL; ++i) out[i] = 1.f;
+  if (!gain || !active) return;
+#pragma unroll
+  for (int i = 0; i < EPL; i += 4) {
+    const floatx4_4 t = *(const floatx4_4*)(gain + e0 + i);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) out[i + k] = t[k];
+  }
+}
+
 // bfloat16, hd and rot multiples of 16: LPK lanes per (row, HPI consecutive heads), 64 / LPK such items per wave.
 // A lane group takes several heads of its row, because what a head needs besides its own 16 bytes per lane (the
 // position, the rotation factors, the gains, the page) is the same for all of them and four times as many bytes.
-// (2,048 rows of 48 heads of 64: 16.0 -> 15.4 us, most of it from the 32-bit item numbers; without its stores and
-// rotation factors the kernel still takes 11.7 us, a chain of loads that each hang on the one before.)
+// (2,048 rows of 48 heads of 64: 15.1 us with the rotation factors and the gains read value by value, each under a condition of its own, 12.0
+// read 16 bytes at a time; what bounds it is the instructions of its three waves a SIMD, not the 25 MB, which are 5 us.)
 template <int LPK, int HPI>
 __global__ __launch_bounds__(256) void qk_rope_kv_bf16x8_kernel(bf16* __restrict__ qkv, bf16* __restrict__ kpages,
                                                                 bf16* __restrict__ vpages, QkRopeArgs a, int n_rows) {
@@ -140,11 +153,8 @@ __global__ __launch_bounds__(256) void qk_rope_kv_bf16x8_kernel(bf16* __restrict
   }
   const Rot8 rt = rotation8(e0, a.inv_freq, a.rot, a.variant, p, a.cs_table, a.table_len);
   float q_gain8[EPL], k_gain8[EPL];
-#pragma unroll
-  for (int i = 0; i < EPL; ++i) {
-    q_gain8[i] = (a.q_gain && active) ? a.q_gain[e0 + i] : 1.f;
-    k_gain8[i] = (a.k_gain && active) ? a.k_gain[e0 + i] : 1.f;
-  }
+  gains8(a.q_gain, e0, active, q_gain8);
+  gains8(a.k_gain, e0, active, k_gain8);
 #pragma unroll
   for (int i = 0; i < HPI; ++i) {
     const int hs = hs0 + i;

@@ -748,10 +748,10 @@ def test_qk_rope_kv(dtype, variant, nh, nkv, hd, rot, table_len):
 
 @pytest.mark.parametrize("nh,nkv,hd", [(16, 8, 64), (3, 1, 48), (6, 1, 256), (5, 2, 16)])
 def test_qk_rope_kv_one_head_or_four_a_lane_group(nh, nkv, hd):
-    """Where rows stop being few (65,536 lanes of 8 values): rows and cache pages are to the bit those of a call with some more rows."""
+    """Where rows stop being few (393,216 lanes of 8 values): rows and cache pages are to the bit those of a call with some more rows."""
     from gibbs_amd import ops
     from gibbs_amd.parts.rope import rope_inv_freq
-    line = (1 << 16) // ((nh + 2 * nkv) * (hd // 8))
+    line = (3 << 17) // ((nh + 2 * nkv) * (hd // 8))
     rows, page = line + 3, 64
     pages = rows // page + 1
     x, qg, kg = rnd(rows, (nh + 2 * nkv) * hd, dtype=torch.bfloat16), rnd(hd, seed=1) + 1, rnd(hd, seed=2) + 1
