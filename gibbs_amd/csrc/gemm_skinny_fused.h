@@ -457,49 +457,46 @@ __global__ __launch_bounds__(WAVES * WAVE) void gemm_skinny_fused_kernel(const b
       if (g == r / 4) red_ss[wave][t][r] = d;   // (paired B operands: rows 8..15 are rows 0..7 at k + 32)
     }
   }
-  // the waves' partial products meet in LDS; wave f * NT + t adds those of its tile in the order of the waves.  With 8 features
-  // a wave's own two halves are added first: lanes g < 2 hold the first, lanes g >= 2 the second, in the second accumulator, or
-  // (paired B operands) 8 columns on in the same one.
+  // the waves' partial products meet in LDS; wave f * NT + t adds those of its tile in the order of the waves
+  // (8 features: lanes g < 2 hold them in the first accumulator, lanes g >= 2 in the second; lane l < 32 then
+  // adds what lane l + 32 left, a wave's second half behind its first: the order is part of the result's bits)
 #pragma unroll
   for (int f = 0; f < FT; ++f)
 #pragma unroll
     for (int q = 0; q < RG; ++q)
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        floatx4 v = acc[f][q][t];
-        if (PAIR) {
-          const floatx4 second = BP ? v : acc_hi[PAIR ? q : 0][t];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const uint32_t x = __float_as_uint(second[i]);
-            uint32_t up = __builtin_amdgcn_permlane32_swap(x, x, false, false)[1];      // (lanes below 32: what lane + 32 holds)
-            if (BP) up = __builtin_amdgcn_update_dpp(0, (int)up, 0x128 /* row_ror:8 */, 0xf, 0xf, false);
-            v[i] += __uint_as_float(up);
-          }
-        }
-        red[wave][f][q][t][lane] = v;
-      }
+      for (int t = 0; t < NT; ++t) red[wave][f][q][t][lane] = (PAIR && !BP && g >= 2) ? acc_hi[PAIR ? q : 0][t] : acc[f][q][t];
   __syncthreads();
   if (wave >= FT * NT) return;
-  // (every read is asked for before the first is used: one by one they were 0.3 us at the end of each call)
-  floatx4 part[WAVES][RG];
+  // (paired B operands: the second half of feature (g, i) and row r is at rows + 8, columns + 8 of the tile)
+  const int partner = BP ? (lane + 40) & 63 : (lane & 31) + 32;   // (8 features only)
   float squares[WAVES][BP ? 2 : 1];
+  if (RMS) {
 #pragma unroll
-  for (int w = 0; w < WAVES; ++w) {
-    if (RMS) {
+    for (int w = 0; w < WAVES; ++w) {
       squares[w][0] = red_ss[w][t_epi][r];
       if (BP) squares[w][BP ? 1 : 0] = red_ss[w][t_epi][(r + 8) & 15];
     }
-#pragma unroll
-    for (int q = 0; q < RG; ++q) part[w][q] = red[w][f_epi][q][t_epi][lane];
   }
-  __builtin_amdgcn_sched_barrier(0);
+  // (the reads of AT_ONCE waves' products are asked for before the first is used: one by one they were 0.3 us at the end of each call)
+  constexpr int HALVES = PAIR ? 2 : 1, AT_ONCE = RG * HALVES > 3 ? WAVES / 2 : WAVES;
   floatx4 sum[RG];
 #pragma unroll
-  for (int q = 0; q < RG; ++q) {
-    sum[q] = part[0][q];
+  for (int w0 = 0; w0 < WAVES; w0 += AT_ONCE) {
+    floatx4 part[AT_ONCE][RG][HALVES];
 #pragma unroll
-    for (int w = 1; w < WAVES; ++w) sum[q] += part[w][q];
+    for (int w = 0; w < AT_ONCE; ++w)
+#pragma unroll
+      for (int q = 0; q < RG; ++q)
+#pragma unroll
+        for (int h = 0; h < HALVES; ++h) part[w][q][h] = red[w0 + w][f_epi][q][t_epi][h ? partner : lane];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < RG; ++q)
+#pragma unroll
+      for (int w = 0; w < AT_ONCE; ++w)
+#pragma unroll
+        for (int h = 0; h < HALVES; ++h) sum[q] = w0 + w + h == 0 ? part[w][q][h] : sum[q] + part[w][q][h];
   }
 
   // D[feature g*4 + i][row r] of the tile: lane holds 4 consecutive features of one row

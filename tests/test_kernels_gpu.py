@@ -998,6 +998,39 @@ def test_skinny_residual(n, o, i):
     assert torch.equal(x0, x), "tile-ordered weights: same sums"
 
 
+@pytest.mark.parametrize("n", [1, 8, 9, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("o,i", [(72, 1088), (72, 64), (4104, 520)])
+def test_few_row_products_add_waves_in_order_and_a_waves_halves_one_after_the_other(n, o, i):
+    """The order in which the eight waves' shares of k are added is part of the bits.  Workgroups of 8 features hold a share as two
+    sums, of the even and of the odd 32 of k: first + second of wave 0, + first of wave 1, + its second, and so on; workgroups of 16 one sum a wave.  A
+    share by itself is the product with X zero everywhere else (zeros add nothing).  Products of two and three row groups add like those of one."""
+    from gibbs_amd import ops
+    x, w = rnd(n, i, dtype=torch.bfloat16, seed=1), rnd(3 * o, i, dtype=torch.bfloat16, seed=2)
+    def product(rows, matrix):
+        total, mirror = torch.zeros(n, o, device=DEV), torch.empty(n, o, dtype=torch.bfloat16, device=DEV)
+        ops.skinny_residual(rows, ops.PackedWeight(matrix), total, mirror)
+        return total
+    pairs = ops.pair_layout(o) and n <= 32
+    unit = 64 if pairs else 32
+    share = -(-(-(-i // unit)) // 8) * unit
+    k = torch.arange(i, device=DEV)
+    want = torch.zeros(n, o, device=DEV)
+    for wave in range(8):
+        for half in range(2 if pairs else 1):
+            mine = (k // share == wave) & ((k // 32 % 2 == half) if pairs else True)
+            want += product(torch.where(mine, x, torch.zeros_like(x)), w[:o])
+    assert torch.equal(product(x, w[:o]), want)
+    if n > 8:      # (rows that pass through LDS: a wave starts elsewhere in its share with every number of row groups)
+        return
+    b, c, d = (product(x, w[g * o:(g + 1) * o].contiguous()) for g in range(3))
+    assert torch.equal(ops.skinny_glu(x, ops.PackedWeight(w[:2 * o].contiguous(), groups=2), activation="relu"), (b.relu() * c).to(torch.bfloat16))
+    taps = torch.zeros(o, 3, device=DEV)
+    taps[:, 2] = 1.0
+    state = torch.zeros(n, 2, o, device=DEV)
+    y = ops.skinny_conv(x, ops.PackedWeight(w, groups=3), taps, None, state, i32(list(range(n))), i32([0] * n))
+    assert torch.equal(state[:, 1], b * d) and torch.equal(y, (c * (b * d)).to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("n,f,i", [(1, 8192, 2048), (8, 200, 512), (40, 128, 72), (64, 256, 1024), (64, 6200, 256),
                                    (36, 8192, 2048),                        # two tiles a workgroup
                                    (5, 4100, 104), (8, 52, 40), (11, 4090, 72), (14, 2200, 104), (9, 60, 136)])
