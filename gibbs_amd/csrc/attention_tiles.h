@@ -6,17 +6,20 @@
 // path: an instruction of a wave takes 2 ns, a dependent access of memory 0.3 to 0.8 us, and the general kernel is 5,700
 // instructions long, with a branch for each element that may lie outside a head.  Here sizes are known when the kernel is
 // compiled, and
-//   * slices take tiles of 32 keys in turn (tile t belongs to slice t / NW % slices) instead of one stretch each, so that a
-//     wave knows its page ids' places without the row's position: ids and position are asked for together, the keys next;
+//   * where a row's keys are whole and in one slice, a wave knows its page ids' places without the row's position: ids and position
+//     are asked for together, the keys next;
 //   * a page id holds for 16 keys, so it is a scalar: the keys' and values' addresses are a scalar base and the lane's 16 bytes;
 //   * every wave prepares all query heads (and the row's own key) at once, a head to each group of lanes, instead of a head a
 //     wave: the queries reach the matrix operand by lane permutes, no LDS and no barrier in front of the walk;
 //   * the waves' results are folded, and the slices merged, by all threads, two elements each.
+// Which keys a slice and a wave take, and the order in which their results are folded, are the general kernel's: the bits of a row are the same
+// in both.  (Where the row's first key lies inside a tile, as a window has it, the tiles begin in front of it, at a multiple of 32, and
+// the bits are others.)
 //
-// Measured (us a call in a captured chain of calls, the general kernel -> this one, in the slices that each does best in):
-// 16 query heads of 64 in 8 groups, 1 row of 40 keys 6.9 -> 3.5, of 500 10.7 -> 5.2; 32 heads in 8, 1 row of 2,100 11.8 -> 6.5, of 16,000
-// 18.0 -> 12.0; 8 rows of 2,100 16.3 -> 10.8 (33 MB: 5.3 at the rate of a kernel that only reads); 64 rows of 1,000 32.4 -> 25.0
-// (131 MB: 21); 8 rows of 520 with a bias 10.5 -> 6.4, with a sink 9.9 -> 5.2; 16 heads of 128 in 4, 8 rows of 520 11.5 -> 6.9.
+// Measured (us a call in a captured chain of calls over caches of their own, the general kernel -> this one, both in the slices of 4 waves that
+// decode_splits gives): 16 query heads of 64 in 8 groups, 1 row of 40 keys 7.7 -> 4.4, of 500 11.1 -> 6.9; 32 heads in 8, 1 row of 2,100 12.5 -> 8.2, of
+// 16,000 21.0 -> 20.0 (64 slices, whose merge is 6); 8 rows of 2,100 17.2 -> 12.6 (33 MB: 5.3 at the rate of a kernel that only reads); 64 rows of 1,000
+// 34.8 -> 28.8 (131 MB: 21); 8 rows of 520 with a bias 11.8 -> 7.9, with a sink 10.6 -> 7.3; 16 heads of 128 in 4, 8 rows of 520 13.8 -> 8.4.
 #pragma once
 
 namespace {
@@ -26,6 +29,7 @@ struct TilesArgs {
   float* partial;
   long ldo;
   int num_pages, nh, nkv;
+  uint32_t per_tile;      // 2^32 over the waves of all slices, rounded up
   float scale;
   int merge_here;
   // raw rows
@@ -70,27 +74,34 @@ __global__ __launch_bounds__(NW * WAVE, HD == 64 ? 4 : 2) void attention_tiles_k
   const int p = pos_[row];
   __builtin_amdgcn_sched_barrier(0);                   // (asked for first)
   const int page_shift = packed & 63, n_splits = packed >> 8;
+  const uint32_t per_tile = a.per_tile;
   const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int grp = lane / LPK, sub = lane % LPK, e0 = sub * EPL;
   const int lr = lane % 16, g4 = lane / 16;
-  const int first = split * NW + wave;                 // the wave's tiles: first, first + step, ...
-  const int step = n_splits * NW;
-
   int req = row;
   if (packed & 128) {
     req = row_req[row];
     asm volatile("" : "+s"(req));                      // (waited for here, so that a step without a map waits for nothing)
   }
   const int* table = table_ + (size_t)req * max_pages;
-  // the first key that the row sees, and the tile it lies in (0 without waiting for the position)
-  int lo = 0, base = 0;
+  // the first key that the row sees, and the tile it lies in; the wave's tiles: first, first + NW, ... (0 and the wave without waiting for the
+  // position, where a row's keys are whole and in one slice)
+  int lo = 0, base = 0, first = wave, per_slice = 0;
   if (packed & 64) {
     lo = !RAW && a.chunk > 0 ? p - p % a.chunk : max(0, p - a.window + 1);
     base = lo / TILE * TILE;
   }
+  if (n_splits > 1) {
+    // ceil(tiles / (slices NW)) to each wave: a product in place of the division, at most one too many
+    const uint32_t waves = n_splits * NW, x = (uint32_t)max(0, p - base + TILE) / TILE + waves - 1;
+    uint32_t rounds = __umulhi(x, per_tile);
+    if (rounds * waves > x) --rounds;
+    per_slice = rounds * NW;
+    first = split * per_slice + wave;
+  }
   // lane l of the wave holds the page id of 16 keys: half l % 2 of its tile l / 2 (of 32 tiles at a time)
   auto ask_ids = [&](int round) {
-    const int key = base + (first + (round * 32 + lane / 2) * step) * TILE + 16 * (lane % 2);
+    const int key = base + (first + (round * 32 + lane / 2) * NW) * TILE + 16 * (lane % 2);
     return table[min(key >> page_shift, max_pages - 1)];
   };
   int ids = ask_ids(0);
@@ -128,7 +139,8 @@ __global__ __launch_bounds__(NW * WAVE, HD == 64 ? 4 : 2) void attention_tiles_k
     }
   }
 
-  const int n_tiles = (p - base + TILE) / TILE;
+  const int all_tiles = (p - base + TILE) / TILE;
+  const int n_tiles = n_splits > 1 ? min(all_tiles, (split + 1) * per_slice) : all_tiles;      // where the slice ends
   const int kv_bytes = kvh << page_shift;              // keys of a page in front of this head's (times HD * 2 bytes)
   uint4 kreg[LPT], vreg[LPT];
   float bnext[EXTRA ? 8 : 1];
@@ -241,7 +253,7 @@ __global__ __launch_bounds__(NW * WAVE, HD == 64 ? 4 : 2) void attention_tiles_k
   bf16 (*tV)[LDT] = tK + TILE;
   const float scale2 = a.scale * 1.44269504088896340736f;
   int j = 0, round = 0;
-  for (int tile = first; tile < n_tiles; tile += step) {
+  for (int tile = first; tile < n_tiles; tile += NW) {
     const int t0 = base + tile * TILE;
     // (what lies in a page outside the keys that the row sees may be anything: 0 times it need not be 0.  The row's own
     // key and value come from the registers)
@@ -264,12 +276,12 @@ __global__ __launch_bounds__(NW * WAVE, HD == 64 ? 4 : 2) void attention_tiles_k
 #pragma unroll
       for (int i = 0; i < 8; ++i) b8[i] = bnext[i];
     }
-    if (tile + step < n_tiles) {
+    if (tile + NW < n_tiles) {
       if (++j == 32) {
         j = 0;
         ids = ask_ids(++round);
       }
-      fetch(tile + step, j);
+      fetch(tile + NW, j);
     }
     __builtin_amdgcn_sched_barrier(0);  // the loads above stay ahead of the arithmetic below
     if (RAW && t0 + TILE > p) {   // the wave's last tile: the row's own key and value, here and in their page
@@ -373,30 +385,26 @@ __global__ __launch_bounds__(NW * WAVE, HD == 64 ? 4 : 2) void attention_tiles_k
     const int i = i0 + threadIdx.x;
     if (PAIRS % (NW * WAVE) != 0 && i >= PAIRS) break;
     const int g = i / (HD / 2), e = i % (HD / 2) * 2;
-    float ms[NW], M = -INFINITY;
+    auto values = [&](int w) { return *(const float2*)(reinterpret_cast<const float*>(s_tiles + (size_t)w * WAVE_LDS) + g * HD + e); };
+    float M = s_ml[0][g][0], L = s_ml[0][g][1], v[2] = {values(0).x, values(0).y};
 #pragma unroll
-    for (int w = 0; w < NW; ++w) { ms[w] = s_ml[w][g][0]; M = fmaxf(M, ms[w]); }
-    float L = 0.f, v0 = 0.f, v1 = 0.f;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const float2 x = *(const float2*)(reinterpret_cast<const float*>(s_tiles + (size_t)w * WAVE_LDS) + g * HD + e);
-      const float f = __expf(ms[w] - M);
-      L = fmaf(f, s_ml[w][g][1], L);
-      v0 = fmaf(f, x.x, v0);
-      v1 = fmaf(f, x.y, v1);
+    for (int w = 1; w < NW; ++w) {
+      const float2 x = values(w);
+      const float more[2] = {x.x, x.y};
+      fold<2>(M, L, v, s_ml[w][g][0], s_ml[w][g][1], more);
     }
     if (n_splits == 1) {
       if (EXTRA && a.sink) L += __expf(a.sink[kvh * GT + g] - M);
-      put(g, e, L, v0, v1);
+      put(g, e, L, v[0], v[1]);
     } else {
       float* ps = row_partial + ((size_t)g * n_splits + split) * (HD + 2);
       if (merge_here) {
         // another workgroup, on another L2, reads them in this same kernel: written through
         if (e == 0) store_through2(ps, M, L);
-        store_through2(ps + 2 + e, v0, v1);
+        store_through2(ps + 2 + e, v[0], v[1]);
       } else {
         if (e == 0) *(float2*)ps = make_float2(M, L);
-        *(float2*)(ps + 2 + e) = make_float2(v0, v1);
+        *(float2*)(ps + 2 + e) = make_float2(v[0], v[1]);
       }
     }
   }
@@ -463,7 +471,9 @@ bool tiles_take(const DecodeArgs& a, int kind, const bf16* q, const bf16* kpages
 }
 
 template <int HD, bool RAW, int NW, bool EXTRA>
-void launch_tiles(int G, dim3 grid, hipStream_t s, const bf16* q, bf16* k, const DecodeArgs& d, const TilesArgs& a) {
+void launch_tiles(int G, dim3 grid, hipStream_t s, const bf16* q, bf16* k, const DecodeArgs& d, TilesArgs a) {
+  const uint64_t waves = (uint64_t)d.n_splits * NW;
+  a.per_tile = (uint32_t)(((1ull << 32) + waves - 1) / waves);
   const uint32_t page_bytes = (uint32_t)d.nkv * d.page_size * HD * 2;
   const uint32_t packed = (uint32_t)d.n_splits << 8 | (d.row_req ? 128u : 0u) | (d.window > 0 || d.chunk > 0 ? 64u : 0u) | (uint32_t)d.page_shift;
 #define GIBBS_TILES(GT) attention_tiles_kernel<HD, GT, RAW, NW, EXTRA><<<grid, NW * WAVE, 0, s>>>(d.pos, d.table, d.row_req, k, q, (int)d.ldq, d.max_pages, page_bytes, packed, a)

@@ -1249,6 +1249,65 @@ def test_attention_decode_in_tiles(nh, nkv, hd, page, window, n_splits, waves, r
         close(out[r].view(1, nh, hd), want, dtype, f"row of {l} keys", bf16=1e-2)
 
 
+@pytest.mark.parametrize("n_splits,waves,kind", [(1, 4, 0), (1, 8, 0), (3, 8, 4), (5, 4, 2)])
+@pytest.mark.parametrize("nh,nkv,hd,page", [(2, 2, 64, 16), (4, 2, 64, 64), (8, 2, 64, 16), (8, 1, 64, 32), (1, 1, 128, 16), (4, 2, 128, 32), (8, 1, 128, 16)])
+@pytest.mark.parametrize("what", ["raw", "plain", "bias", "sink", "capped", "chunk", "all", "short chunk"])
+def test_tiles_give_the_bits_of_the_general_decode_kernel(nh, nkv, hd, page, n_splits, waves, kind, what):
+    """A row's keys are shared out over slices and waves, and their results folded, as in the kernel for any shape (which output rows of
+    an odd stride reach), so that a model's rows do not depend on which of the two takes a call.  Rows on either side of a tile and of a page,
+    one of more tiles than a wave holds page ids for; what no row sees is NaN.  Prepared rows with a bias whose table ends before the row's
+    keys do, a sink, capped scores and chunks, each also against float64 (a chunk inside which tiles do not begin: against that alone)."""
+    from gibbs_amd import ops
+    from gibbs_amd.ops.lib import call, ptr, stream
+    from gibbs_amd.parts.rope import rope_inv_freq
+    bf = torch.bfloat16
+    seq_lens = [4400, 1, 31, 32, 33, 96, 97, 1029]
+    n, raw = len(seq_lens), what == "raw"
+    kp, vp, table, ks, vs = paged_setup(bf, nkv, hd, page, seq_lens, 400, seed=3)
+    kp[kp == 50], vp[vp == -50] = float("nan"), float("nan")
+    pos = i32([l - 1 for l in seq_lens])
+    scale = 1 / math.sqrt(hd)
+    qkv = rnd(n, (nh + 2 * nkv) * hd, dtype=bf, seed=9)
+    every = what == "all"
+    bias = rnd(nh, 300, seed=4) / scale if what == "bias" or every else None
+    sink = rnd(nh, seed=5) if what == "sink" or every else None
+    softcap = 2.0 if what == "capped" or every else 0.0
+    chunk = {"chunk": 1024, "all": 96, "short chunk": 180}.get(what, 0)
+    inv = torch.from_numpy(rope_inv_freq(hd, 10000.0, "f32")).to(DEV)
+    gains, factors = (rnd(hd, seed=1) * 0.1 + 1, rnd(hd, seed=2) * 0.1 + 1), ops.rope_table(inv, 1000)
+
+    def run(ldo):
+        out, k, v = torch.zeros(n, ldo, dtype=bf, device=DEV), kp.clone(), vp.clone()
+        partial = torch.empty(n * nh * n_splits * (hd + 2), device=DEV)
+        cache = (ptr(table), table.shape[1], page, kp.shape[0], n, nh, nkv, hd, qkv.shape[1], ldo, scale, 0, n_splits, waves, kind, 4400)
+        if raw:
+            call("gibbs_attention_decode_fused", ptr(qkv), ptr(k), ptr(v), ptr(out), ptr(partial), ptr(gains[0]), ptr(gains[1]), 1e-6, ptr(inv), hd, 0,
+                 ptr(factors), 1000, ptr(pos), None, *cache, stream())
+        else:
+            call("gibbs_attention_decode_masked", ptr(qkv), ptr(k), ptr(v), ptr(out), ptr(partial), ptr(pos), None, *cache, ptr(bias), 300, ptr(sink), chunk,
+                 softcap, stream())
+        return out[:, :nh * hd], k, v
+
+    got, general = run(nh * hd), run(nh * hd + 1)
+    if chunk % 32 == 0:
+        for a, b in zip(got, general):
+            assert torch.equal(a.nan_to_num(7.0), b.nan_to_num(7.0))
+    if raw:
+        return
+    for r, l in enumerate(seq_lens):
+        lo = (l - 1) // chunk * chunk if chunk else 0
+        kk, vv = (x[r][lo:].double().repeat_interleave(nh // nkv, 1) for x in (ks, vs))
+        s = torch.einsum("hd,lhd->hl", qkv[r, :nh * hd].view(nh, hd).double(), kk) * scale
+        s = softcap * torch.tanh(s / softcap) if softcap else s
+        if bias is not None:
+            s = s + bias.double()[:, (l - 1 - torch.arange(lo, l, device=DEV)).clamp(max=299)] * scale
+        if sink is not None:
+            s = torch.cat([s, sink.double()[:, None]], 1)
+        want = torch.einsum("hl,lhd->hd", s.softmax(-1)[:, :l - lo], vv)
+        # (the weights and the output are bfloat16: 2^-9 of the largest value each)
+        close(got[0][r].view(nh, hd), want, bf, f"row of {l} keys", bf16=8e-3)
+
+
 @pytest.mark.parametrize("n_rows,nh,nkv,hd,n_splits", [(64, 32, 8, 64, 8), (3, 6, 2, 48, 5), (2, 4, 1, 128, 40),
                                                        (4200, 8, 8, 16, 2)])
 def test_slices_merged_by_the_last_to_finish_or_by_a_second_kernel(n_rows, nh, nkv, hd, n_splits):
