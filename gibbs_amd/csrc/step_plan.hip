@@ -71,26 +71,7 @@ int skinny_splits(int n_out, int inner, int want_blocks = 512, int features = 16
 // final fold), 8 waves on the vector units, 4 on the matrix cores (measured at batch 1 to 64, 2,048 to 8,192
 // keys).  The matrix-core walk keeps the page ids of a whole slice in LDS: caches longer than that are cut
 // into as many slices as it takes.  kind: 0 the kernel's choice of walk, 1 vector units, 2 matrix cores.
-//
-// Heads of 64 in groups of 1, 2, 4 or 8 take the kernel for tiles (attention_tiles.h; + 8 in `kind` says that a call does not,
-// for its rotation).  A wave of it passes a tile of 32 keys in 0.65 us (0.9 where memory is busy), and slices cost their merge,
-// 1.3 us; so slices share out as few tiles a wave as one round of workgroups of 8 waves over the chip allows, evenly, and
-// are left where they save no more than two tiles a wave.  Measured (us; slices of 8 waves, or of 4 as the rule above has
-// them): 1 row of 2,100 keys in 8 slices 6.5, in one 10.2 (8 of 4: 6.7); 8 rows of 2,100 in 3 11.0, in one 14.3 (8 of 4: 11.1); 1 row
-// of 16,000 in 32 12.5 (62 of 4: 15.1); 8 rows of 520 in one 5.2, in 2 6.3; 16 rows of 700 in one 8.5, in 2 9.7 (2 of 4: 9.6);
-// 32 rows of 2,000 (256 workgroups) in one 25.7 (one of 4: 27.9).  From 512 workgroups on 4 waves are enough: 64 rows of 1,000
-// 25.0, and 26.1 with 8.
 void decode_splits(int n_rows, int nkv, int group, int max_seq, int hd, int page_size, int kind, int* n_splits, int* waves) {
-  const bool tiles = !(kind & 8) && (kind & 3) != 1 && hd == 64 && (group == 1 || group == 2 || group == 4 || group == 8) &&
-                     page_size >= 16 && (page_size & (page_size - 1)) == 0;
-  if (tiles) {
-    const long blocks = std::max<long>(1, (long)n_rows * nkv), all = std::max<long>(1, ceil_div_l(max_seq, 32));
-    *waves = blocks >= 512 ? 4 : 8;
-    const long alone = ceil_div_l(all, 8);                       // tiles a wave in one slice
-    const long each = std::max<long>(1, ceil_div_l(alone, std::min<long>(64, ceil_div_l(256, blocks))));
-    *n_splits = alone - each <= 2 ? 1 : (int)ceil_div_l(alone, each);
-    return;
-  }
   kind &= 3;   // (+ 4 only says which kernel merges the slices)
   const bool matrix = kind != 1 && hd > 0 && hd % 16 == 0 && hd <= 128;
   const int gt = group >= 8 ? 8 : (group > 2 ? 4 : group);
@@ -839,8 +820,7 @@ struct AttnBody : Body {
   void* attend_decoded(Exec& e, const void* raw) const {
     const int N = e.a.n_rows;
     int n_splits, waves;
-    const bool tiles = !inv_freq || (variant == 0 && rot == hd && cos_sin);
-    decode_splits(N, nkv, nh / nkv, e.a.max_seq, hd, page_size, tiles ? 0 : 8, &n_splits, &waves);
+    decode_splits(N, nkv, nh / nkv, e.a.max_seq, hd, page_size, 0, &n_splits, &waves);
     float* partial = n_splits > 1 ? (float*)e.take(gibbs_attention_decode_workspace(N, nh, hd, n_splits) * 4) : nullptr;
     void* o = e.take((long)N * nh * hd * 2);
     RUN(e, gibbs_attention_decode_fused(raw, kpages, vpages, o, partial, q_gain, k_gain, qk_eps, inv_freq, rot, variant, cos_sin,

@@ -370,8 +370,7 @@ def attention_decode_fused(qkv: torch.Tensor, n_rows: int, nh: int, nkv: int, hd
         if rotary_dim % 16:
             raise KernelError(f"attention_decode_fused: rotary_dim {rotary_dim} must be a multiple of 16")
     if n_splits is None or waves is None:
-        tiles = inv_freq is None or (variant == "half_split" and rotary_dim == hd and cos_sin is not None)
-        auto_splits, auto_waves = decode_splits(n_rows, nkv, nh // nkv, max_seq, hd, kind, page_size, tiles)
+        auto_splits, auto_waves = decode_splits(n_rows, nkv, nh // nkv, max_seq, hd, kind, page_size)
         n_splits = auto_splits if n_splits is None else n_splits
         waves = auto_waves if waves is None else waves
     partial = None
@@ -623,13 +622,13 @@ def slices_workspace(n_rows: int, nh: int, hd: int, n_splits: int) -> int:
 
 
 def decode_splits(n_rows: int, nkv: int, group: int, max_seq: int, hd: int = 0, kind: str = "auto",
-                  page_size: int = 16, tiles: bool = True) -> tuple:
+                  page_size: int = 16) -> tuple:
     """(key slices per (row, kv head), waves per workgroup) that the native step would choose for the
-    decode attention (csrc/step_plan.hip).  `tiles` False: the call's rotation keeps it from the kernel for tiles."""
+    decode attention (csrc/step_plan.hip)."""
     import ctypes
     n_splits, waves = ctypes.c_int(0), ctypes.c_int(0)
-    library().gibbs_rule_decode_splits(n_rows, nkv, group, max_seq, hd, page_size, DECODE_KINDS[kind] + (0 if tiles else 8),
-                                       ctypes.byref(n_splits), ctypes.byref(waves))
+    library().gibbs_rule_decode_splits(n_rows, nkv, group, max_seq, hd, page_size, DECODE_KINDS[kind], ctypes.byref(n_splits),
+                                       ctypes.byref(waves))
     return n_splits.value, waves.value
 
 

@@ -1308,6 +1308,34 @@ def test_tiles_give_the_bits_of_the_general_decode_kernel(nh, nkv, hd, page, n_s
         close(got[0][r].view(nh, hd), want, bf, f"row of {l} keys", bf16=8e-3)
 
 
+@pytest.mark.parametrize("rows,nh,nkv,max_seq,kind", [(32, 32, 8, 8192, "auto"), (64, 16, 4, 10368, "auto"), (16, 8, 8, 16384, "auto"), (64, 8, 8, 16384, "mfma")])
+def test_decode_attention_of_many_rows_under_a_far_bound(rows, nh, nkv, max_seq, kind):
+    """Rows that fill the chip, under a bound on their keys beyond the page ids that one slice has room for: a bias on the scores, and the matrix
+    cores asked for, are taken with the slices of the rule.  (Rows share their pages: only the bound has to be far.)"""
+    from gibbs_amd import ops
+    from gibbs_amd.ops.lib import call, ptr, stream
+    bf, hd, page, keys = torch.bfloat16, 64, 16, 300
+    kp, vp, one, ks, vs = paged_setup(bf, nkv, hd, page, [keys], 24, seed=5)
+    table = torch.zeros(rows, max_seq // page, dtype=torch.int32, device=DEV)
+    table[:, :one.shape[1]] = one
+    pos = i32([(keys - 1) if r % 2 else r for r in range(rows)])
+    q, scale = rnd(rows, nh * hd, dtype=bf, seed=6), 0.125
+    bias = rnd(nh, 64, seed=7) / scale if kind == "auto" else None
+    n_splits, waves = ops.decode_splits(rows, nkv, nh // nkv, max_seq, hd, kind, page)
+    partial = torch.empty(max(1, ops.slices_workspace(rows, nh, hd, n_splits)), device=DEV)
+    out = torch.zeros(rows, nh * hd, dtype=bf, device=DEV)
+    call("gibbs_attention_decode_masked", ptr(q), ptr(kp), ptr(vp), ptr(out), ptr(partial), ptr(pos), None, ptr(table), table.shape[1], page, kp.shape[0],
+         rows, nh, nkv, hd, nh * hd, nh * hd, scale, 0, n_splits, waves, ops.DECODE_KINDS[kind], max_seq, ptr(bias), 64, None, 0, 0.0, stream())
+    kk, vv = ks[0].double().repeat_interleave(nh // nkv, 1), vs[0].double().repeat_interleave(nh // nkv, 1)
+    for r in range(rows):
+        p = pos[r].item()
+        s = torch.einsum("hd,lhd->hl", q[r].view(nh, hd).double(), kk[:p + 1]) * scale
+        if bias is not None:
+            s = s + bias.double()[:, (p - torch.arange(p + 1, device=DEV)).clamp(max=63)] * scale
+        # (the weights and the output are bfloat16: 2^-9 of the largest value each)
+        close(out[r].view(nh, hd), torch.einsum("hl,lhd->hd", s.softmax(-1), vv[:p + 1]), bf, f"row {r}", bf16=8e-3)
+
+
 @pytest.mark.parametrize("n_rows,nh,nkv,hd,n_splits", [(64, 32, 8, 64, 8), (3, 6, 2, 48, 5), (2, 4, 1, 128, 40),
                                                        (4200, 8, 8, 16, 2)])
 def test_slices_merged_by_the_last_to_finish_or_by_a_second_kernel(n_rows, nh, nkv, hd, n_splits):

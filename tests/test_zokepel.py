@@ -167,3 +167,19 @@ def test_decoded_tokens_of_many_small_heads_keep_the_three_kernels(time_mix, row
     """The rule between one kernel around a decoded token's state and the three that it stands for takes the faster way of measured steps."""
     from gibbs_amd.ops.lib import library
     assert library().gibbs_rule_token_kernel(time_mix, rows, H, D, D) == (one < three)
+
+
+@pytest.mark.parametrize("page", [16, 32, 64])
+@pytest.mark.parametrize("hd,group", [(64, 1), (64, 4), (64, 8), (64, 3), (128, 4), (96, 2)])
+def test_a_slice_of_the_decode_attention_is_never_longer_than_its_page_ids_have_room(hd, group, page):
+    """Slices of the rule's number, each rounded up to whole tiles of every wave (256 keys at most), hold at most the 512 page ids that
+    the matrix-core walk keeps: a bias on the scores has no other kernel, and a call whose slices are longer is refused."""
+    import ctypes
+    from gibbs_amd.ops.lib import library
+    n_splits, waves = ctypes.c_int(0), ctypes.c_int(0)
+    for kind in (0, 2):
+        for rows in (1, 2, 7, 8, 16, 31, 32, 64, 100, 256):
+            for nkv in (1, 2, 4, 8, 32):
+                for keys in (1, 500, 4096, 7904, 7905, 8192, 10368, 16384, 40000, 131072):
+                    library().gibbs_rule_decode_splits(rows, nkv, group, keys, hd, page, kind, ctypes.byref(n_splits), ctypes.byref(waves))
+                    assert (-(-keys // n_splits.value) + 256) // page + 2 <= 512, (rows, nkv, keys, n_splits.value)
