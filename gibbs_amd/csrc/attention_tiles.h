@@ -216,7 +216,7 @@ __global__ __launch_bounds__(NW * WAVE, HD == 64 ? 4 : 2) void attention_tiles_k
 #pragma unroll
         for (int i = 0; i < EPL; ++i) {
           const float other = lane_xor<LPK / 2>(v[i]);
-          v[i] = low ? v[i] * c8[i] - other * s8[i] : other * s8[i] + v[i] * c8[i];
+          v[i] = fmaf(v[i], c8[i], low ? -(other * s8[i]) : other * s8[i]);   // (the product that is rounded is the one the compiler rounds in norm_rope8)
         }
       }
       ready[j] = pack8(v);                             // bfloat16, as the pages hold keys and other kernels queries

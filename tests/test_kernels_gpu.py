@@ -1308,6 +1308,34 @@ def test_tiles_give_the_bits_of_the_general_decode_kernel(nh, nkv, hd, page, n_s
         close(got[0][r].view(nh, hd), want, bf, f"row of {l} keys", bf16=8e-3)
 
 
+@pytest.mark.parametrize("gained", [False, True])
+@pytest.mark.parametrize("nh,nkv,hd", [(32, 8, 64), (16, 8, 64), (8, 1, 64), (4, 4, 128), (16, 2, 128)])
+def test_tiles_rotate_to_the_bit_as_the_general_decode_kernel(nh, nkv, hd, gained):
+    """Enough rotated queries and keys that another rounding inside a rotation (which of its two products is rounded before the sum) shows in
+    the bfloat16 keys in the pages and in the outputs: it moves one value in some 10,000."""
+    from gibbs_amd import ops
+    from gibbs_amd.ops.lib import call, ptr, stream
+    from gibbs_amd.parts.rope import rope_inv_freq
+    bf, rows, page, keys = torch.bfloat16, 512, 16, 48
+    inv = torch.from_numpy(rope_inv_freq(hd, 10000.0, "f32")).to(DEV)
+    gains = (rnd(hd, seed=1) * 0.1 + 1, rnd(hd, seed=2) * 0.1 + 1) if gained else (None, None)
+    factors = ops.rope_table(inv, keys)
+    pages = rows * keys // page
+    kp, vp = rnd(pages, nkv, page, hd, dtype=bf, seed=3), rnd(pages, nkv, page, hd, dtype=bf, seed=4)
+    table = torch.arange(pages, dtype=torch.int32, device=DEV).view(rows, -1)
+    pos = i32([5 + r % (keys - 5) for r in range(rows)])
+    qkv = rnd(rows, (nh + 2 * nkv) * hd, dtype=bf, seed=5)
+
+    def run(ldo):
+        out, k, v = torch.zeros(rows, ldo, dtype=bf, device=DEV), kp.clone(), vp.clone()
+        call("gibbs_attention_decode_fused", ptr(qkv), ptr(k), ptr(v), ptr(out), None, ptr(gains[0]), ptr(gains[1]), 1e-6, ptr(inv), hd, 0, ptr(factors), keys,
+             ptr(pos), None, ptr(table), table.shape[1], page, pages, rows, nh, nkv, hd, qkv.shape[1], ldo, hd ** -0.5, 0, 1, 4, 0, keys, stream())
+        return out[:, :nh * hd], k, v
+
+    for a, b in zip(run(nh * hd), run(nh * hd + 1)):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("rows,nh,nkv,max_seq,kind", [(32, 32, 8, 8192, "auto"), (64, 16, 4, 10368, "auto"), (16, 8, 8, 16384, "auto"), (64, 8, 8, 16384, "mfma")])
 def test_decode_attention_of_many_rows_under_a_far_bound(rows, nh, nkv, max_seq, kind):
     """Rows that fill the chip, under a bound on their keys beyond the page ids that one slice has room for: a bias on the scores, and the matrix
