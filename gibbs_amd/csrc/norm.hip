@@ -376,7 +376,10 @@ __global__ void rows_add_norm_vec_kernel(float* __restrict__ x, const void* __re
           }
         }
       }
-      ss += v[c].x * v[c].x + v[c].y * v[c].y + v[c].z * v[c].z + v[c].w * v[c].w;
+      // (whole rows: which of the squares is rounded before the others are added is stated.  Left to the compiler it was the second here, and
+      // the first once the partial sums' loads stood in front: a root mean square in some ten a bit apart)
+      if constexpr (FROM == FROM_ROWS) ss += fmaf(v[c].w, v[c].w, fmaf(v[c].z, v[c].z, fmaf(v[c].x, v[c].x, v[c].y * v[c].y)));
+      else ss += v[c].x * v[c].x + v[c].y * v[c].y + v[c].z * v[c].z + v[c].w * v[c].w;
     }
   }
   ss = block_sum(ss, scratch);

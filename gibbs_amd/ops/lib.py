@@ -97,6 +97,7 @@ _SIGNATURES = {
     "gibbs_embed_norm": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_float, c_int, c_int, c_int, c_void_p],
     "gibbs_stream_rows": [c_void_p, c_void_p, c_int, c_long, c_void_p],
     "gibbs_stream_shift": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
+    "gibbs_rmsnorm_rows_add_norm": [c_void_p, c_void_p, c_int, c_long, c_void_p, c_float, c_void_p, c_float, c_void_p, c_int, c_int, c_int, c_void_p],
     "gibbs_rmsnorm_rows_add_read": [c_void_p, c_void_p, c_int, c_long, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_float, c_int,
                                     c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
     "gibbs_diff_prepare": [c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_float, c_void_p, c_int, c_int, c_void_p,

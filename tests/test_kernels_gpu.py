@@ -1193,6 +1193,49 @@ def test_few_rows_experts_without_grouping(n, top, experts, identity, width, inn
         close(direct[i], F.silu(g) * u, bf, f"pair {i}", bf16=8e-3)
 
 
+@pytest.mark.parametrize("parts", [1, 3, 9])
+@pytest.mark.parametrize("hidden", [100, 1024, 2048, 5000])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_a_sublayers_norm_sums_its_squares_in_one_order(dtype, hidden, parts):
+    """x += norm(rows): of four squares the second is rounded and the others are added to it, then come a thread's stretches, lanes by
+    halves of a wave, waves in turn.  The same in float32 here, to the bit, so that a row does not depend on how its kernel was compiled; one
+    stretch a thread and several, whole rows and partial sums, what follows normed or read as it is."""
+    from gibbs_amd.ops.lib import call, dtype_code, ptr, stream
+    n, eps = 64, 1e-6
+    rows = rnd(n, hidden, dtype=dtype, seed=1) if parts == 1 else rnd(parts, n, hidden, seed=1)
+    x0, gain, gain_n = rnd(n, hidden, seed=2), rnd(hidden, seed=3), rnd(hidden, seed=4)
+    f32, f64 = np.float32, np.float64
+    fused = lambda a, b, c: (a.astype(f64) * b.astype(f64) + c.astype(f64)).astype(f32)
+    v = np.zeros((n, hidden), f32)
+    for part in (rows.float().view(-1, n, hidden).cpu().numpy()):
+        v = v + part
+    threads = 1024 if hidden >= 4096 else 512 if hidden >= 2048 else 256 if hidden >= 512 else 64
+    stretches = -(-hidden // (4 * threads))
+    four = np.zeros((n, stretches * threads * 4), f32)
+    four[:, :hidden] = v
+    a, b, c, d = np.moveaxis(four.reshape(n, stretches, threads, 4), 3, 0)
+    squares = fused(d, d, fused(c, c, fused(a, a, b * b)))
+    lanes = np.zeros((n, threads), f32)
+    for s in range(stretches):
+        lanes = lanes + squares[:, s]
+    lanes = lanes.reshape(n, -1, 64)
+    for half in (32, 16, 8, 4, 2, 1):
+        lanes = lanes + lanes[:, :, np.arange(64) ^ half]
+    total = np.zeros(n, f32)
+    for w in range(lanes.shape[1]):
+        total = total + lanes[:, w, 0]
+    scale = (f32(1) / np.sqrt(total / f32(hidden) + f32(eps)))[:, None]
+    want = torch.from_numpy(fused(v * scale, gain.cpu().numpy()[None], x0.cpu().numpy()))
+    x, out = x0.clone(), torch.empty(n, hidden, dtype=dtype, device=DEV)
+    call("gibbs_rmsnorm_rows_add_norm", ptr(x), ptr(rows), parts, n * hidden, ptr(gain), eps, ptr(gain_n), eps, ptr(out), dtype_code(dtype), n, hidden, stream())
+    assert torch.equal(x.cpu(), want)
+    x = x0.clone()
+    call("gibbs_rmsnorm_rows_add_read", ptr(x), ptr(rows), parts, n * hidden, None, None, 0, None, None, ptr(gain), eps, 1, None, None, 0, None, ptr(out),
+         dtype_code(dtype), n, hidden, stream())
+    assert torch.equal(x.cpu(), want)
+    assert torch.equal(out.cpu(), want.to(dtype))
+
+
 @pytest.mark.parametrize("parts", [0, 1, 3])
 @pytest.mark.parametrize("hidden", [4, 516, 2048, 5000])
 def test_norm_that_leaves_a_mirror(hidden, parts):
