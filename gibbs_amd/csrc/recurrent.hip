@@ -597,7 +597,11 @@ __global__ __launch_bounds__(STEP_THREADS) void delta_step_kernel(DeltaStepArgs 
     }
   }
   const float out = leave(x);
-  const float inv = 1.0f / sqrtf(block_sum(out * out, scratch) / (float)V + a.eps);
+  // (the first of the wave's exchanges fuses a lane's own square with the rounded one of the lane 32 on: the order is part of the result's bits.  Moves between
+  // lanes are no operands of a sum to the compiler, which fused the two by itself where they were exchanged through LDS)
+  const float square = lane_xor_float<32>(out * out);
+  const float squares = block_sum(lane < 32 ? fmaf(out, out, square) : 0.f, scratch);
+  const float inv = 1.0f / sqrtf(squares / (float)V + a.eps);
   if (j < V) ((T*)a.y)[((size_t)n * a.H + h) * V + j] = from_float<T>(out * inv * gain * gate);
 }
 // lanes across a state's columns; 0: the kernel does not take the sizes (a head's state has to fit the workgroup's registers)

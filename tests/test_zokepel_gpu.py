@@ -613,6 +613,36 @@ def test_delta_step_equals_its_parts(n, H, G, D, V, per_channel, dtype):
     assert far(y, want) <= 32 * 2.0 ** -24 + (2.0 ** -8 if kind else 0), far(y, want)
 
 
+@pytest.mark.parametrize("V", [4, 32, 36, 64, 100, 128, 256, 512])
+def test_delta_step_sums_a_heads_squares_in_one_order(V):
+    """Empty states, keys and queries of one channel and a full write leave the values themselves as the read-out, so that what comes out is their norm
+    alone: a lane's own square fused with the rounded one 32 lanes on, lanes by halves, waves in turn, to the bit."""
+    from gibbs_amd.ops.lib import call, ptr, stream
+    n, D, eps = 200, 4, 1e-6
+    g = torch.Generator().manual_seed(V)
+    v = torch.randn(n, V, generator=g)
+    one = torch.zeros(n, D)
+    one[:, 0] = 1.0
+    qkv, sure = torch.cat([one, one, v], 1).cuda(), torch.full((n, 1), 200.0, device="cuda")      # (a sigmoid of 1: beta and the gate)
+    zero, gain, gate = torch.zeros(1, device="cuda"), torch.ones(V, device="cuda"), torch.full((n, V), 200.0, device="cuda")
+    state, slot = torch.zeros(n, 1, D, V, device="cuda"), torch.arange(n, dtype=torch.int32, device="cuda")
+    y = torch.empty(n, V, device="cuda")
+    call("gibbs_delta_step", ptr(qkv), 2 * D + V, ptr(sure), ptr(sure), 1, 0, None, ptr(zero), ptr(zero), ptr(gate), V, 1, ptr(gain), eps, ptr(state),
+         state.stride(0), ptr(slot), ptr(y), n, 1, 1, D, V, 1.0, 0.0, stream())
+    f32, f64 = np.float32, np.float64
+    x = np.zeros((n, 8, 64), f32)
+    x.reshape(n, 512)[:, :V] = v.numpy()
+    far = np.roll(x, 32, axis=2)
+    lanes = (x.astype(f64) ** 2 + (far * far).astype(f64)).astype(f32)[:, :, :32]
+    for half in (16, 8, 4, 2, 1):
+        lanes = lanes + lanes[:, :, np.arange(32) ^ half]
+    total = np.zeros(n, f32)
+    for w in range(8):
+        total = total + lanes[:, w, 0]
+    scale = f32(1) / np.sqrt(total / f32(V) + f32(eps))
+    assert np.array_equal(y.cpu().numpy(), v.numpy() * scale[:, None])
+
+
 @pytest.mark.parametrize("how", ["chunks", "rows"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("lens,H,D,shift", [([1], 2, 16, 0), ([1, 1, 1], 2, 64, -3), ([64], 3, 64, -3), ([65, 1, 17], 2, 64, -3), ([130, 63], 2, 24, 1), ([200], 2, 32, 4),
