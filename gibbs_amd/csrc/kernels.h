@@ -166,6 +166,7 @@ int gibbs_rmsnorm_rows_sum_add_read(float* x, const void* in, int parts, long pa
 int gibbs_rows_terms(const void* in, int parts, const float* bias, float scale, const void* in2, int parts2, float scale2, float* out,
                      int dtype, int n, int hidden, hipStream_t stream);
 // ---- moe.hip: mixture of experts
+int gibbs_moe_gated_features(int tiles, int F);
 int gibbs_moe_direct_takes(int n, int top, int E, int W, int F);
 int gibbs_moe_route_placed(const void* h, long ldh, int dtype, const float* router, const float* router_bias, const float* shared_gate, int* chosen,
                            float* weight, float* sgate, int* place, int matrices, int n, int W, int E, int top, int mode, float weight_scale, hipStream_t stream);

@@ -469,21 +469,21 @@ typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 
-// Few pairs: a tile is 16 places, a workgroup takes 32 features of it (GLU: 16, of both matrices) and its four waves a
+// Few pairs: a tile is 16 places, a workgroup takes 16 NF features of it (GLU: of both matrices) and its four waves a
 // quarter of k each, so that the experts' matrices, which are read once, are spread over many workgroups; the waves'
 // sums meet in LDS and are added in wave order.  W is the first operand of the 16 x 16 x 32 product (the
 // tile is Y^T = W X^T): lane l holds 8 values along k of feature or place l % 16, and its four results are four
 // neighbouring features of place l % 16.  Operands come straight from memory.  Measured (16 experts of 1,024 at width 2,048, 4 chosen; us, gated and
 // back): 1 row 13.7 and 6.7 with loads under conditions, 32 features and one wave's tail, 10.1 and 5.6 now; 8 rows (126 and 63 MB) 34.8 and
-// 13.7, now 29.7 and 13.1; 16 gated features a workgroup or 32: 1 row 10.1 / 11.7, 8 rows 29.7 / 31.4, 32 rows 33.6 / 34.3; back, 8 rows 13.7 / 13.1.
+// 13.7, now 29.7 and 13.1; back with 16 features a workgroup or 32, 8 rows 13.7 / 13.1 (gated: gibbs_moe_gated_features).
 // DIRECT (at most 64 pairs, an expert at most 16 of them): no grouping in front: blockIdx.y is the expert, `sorted_pair` holds each pair's choice, and
 // places are the pairs' own numbers.
-template <bool GLU, bool DIRECT>
+template <bool GLU, bool DIRECT, int NF>
 __global__ __launch_bounds__(256) void moe_gemm_few_kernel(const bf16* __restrict__ X, const int* __restrict__ sorted_pair,
                                                            const int* __restrict__ tile_expert, const bf16* __restrict__ Wa,
                                                            const bf16* __restrict__ Wb, int top, int I, long ldx, long expert_stride, bf16* __restrict__ Y,
                                                            long ldy, int O, int act, const float* __restrict__ in_weight, int pairs) {
-  constexpr int NF = GLU ? 1 : 2, NA = GLU ? 2 * NF : NF;    // feature tiles of 16 a workgroup; accumulators a wave
+  constexpr int NA = GLU ? 2 * NF : NF;    // accumulators a wave
   __shared__ __attribute__((aligned(16))) floatx4 part[4][NA][WAVE];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, lr = lane % 16, lg = lane / 16;
   int e, pair, place;
@@ -1012,6 +1012,13 @@ GIBBS_EXPORT long gibbs_moe_capacity(int n_pairs, int E, int bm) {
 // Tiles of pairs: 16 while the matrices are streamed for few pairs each (at most 64 an expert on average), 128 beyond.
 GIBBS_EXPORT int gibbs_moe_tile(int n_pairs, int E) { return (long)n_pairs <= 64L * E ? 16 : 128; }
 
+// Features of a workgroup of the gated product of few pairs, in `tiles` tiles at most (those that no expert takes among them): 16 while they give the chip no more than
+// ten workgroups a compute unit, 32 beyond, where the rows of X and the features that several tiles share come from the L2s and are read less often so.
+// 32 / 16, us: 16 experts of 1,024 at width 2,048, 4 chosen, 32 rows (1,472 workgroups of 16) 30.6 / 28.7, 96 (2,496) 44.5 / 45.1, 128 (3,008) 50.3 / 55.2, 256 90.2 / 98.9;
+// of 512 at 1,024 192 rows (2,016) 24.1 / 22.9, 256 (2,528) 28.5 / 29.1; 8 of 1,024 at 1,024, 2 chosen, 256 rows (2,528) 28.3 / 27.8; 64 of 512 at 2,048, 8 chosen, 96 rows
+// (3,456) 59.9 / 54.5, 128 65.4 / 66.6, 235 (5,664) 88 / 98, 512 167 / 191.
+GIBBS_EXPORT int gibbs_moe_gated_features(int tiles, int F) { return (long)tiles * ceil_div(F, 16) <= 2560 ? 16 : 32; }
+
 // Few rows, whose products need no grouping (gibbs_moe_gemm_direct): at most 16, so that an expert has at most one of each row's pairs, a tile, and
 // 64 pairs, one for each lane of a wave.
 GIBBS_EXPORT int gibbs_moe_direct_takes(int n, int top, int E, int W, int F) {
@@ -1121,10 +1128,14 @@ GIBBS_EXPORT int gibbs_moe_gemm_weighted(const void* X, long ldx, int top, const
               : launch_tiled<false>((const bf16*)X, ldx, top, sorted_pair, tile_expert, tiles, (const bf16*)w_a, nullptr, stride, (bf16*)Y, ldy, O, I, act, nullptr, stream))
         return 1;
     } else if (w_b) {
-      moe_gemm_few_kernel<true, false><<<dim3(ceil_div(O, 16), tiles), 256, 0, stream>>>((const bf16*)X, sorted_pair, tile_expert, (const bf16*)w_a, (const bf16*)w_b,
-                                                                                        top, I, ldx, stride, (bf16*)Y, ldy, O, act, in_weight, 0);
+      const auto queue = [&](auto kernel, int features) {
+        kernel<<<dim3(ceil_div(O, features), tiles), 256, 0, stream>>>((const bf16*)X, sorted_pair, tile_expert, (const bf16*)w_a, (const bf16*)w_b, top, I, ldx, stride, (bf16*)Y,
+                                                                       ldy, O, act, in_weight, 0);
+      };
+      if (gibbs_moe_gated_features(tiles, O) == 16) queue(moe_gemm_few_kernel<true, false, 1>, 16);
+      else queue(moe_gemm_few_kernel<true, false, 2>, 32);
     } else {
-      moe_gemm_few_kernel<false, false><<<dim3(ceil_div(O, 32), tiles), 256, 0, stream>>>((const bf16*)X, sorted_pair, tile_expert, (const bf16*)w_a, nullptr, top, I,
+      moe_gemm_few_kernel<false, false, 2><<<dim3(ceil_div(O, 32), tiles), 256, 0, stream>>>((const bf16*)X, sorted_pair, tile_expert, (const bf16*)w_a, nullptr, top, I,
                                                                                          ldx, stride, (bf16*)Y, ldy, O, act, nullptr, 0);
     }
   } else {
@@ -1145,10 +1156,10 @@ GIBBS_EXPORT int gibbs_moe_gemm_direct(const void* X, long ldx, int top, const i
   GIBBS_REQUIRE(I % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)X % 16) == 0 && ((uintptr_t)w_a % 16) == 0 && ((uintptr_t)w_b % 16) == 0, "moe_gemm: rows of whole 16 bytes");
   const long stride = (long)O * I;
   if (w_b)
-    moe_gemm_few_kernel<true, true><<<dim3(ceil_div(O, 16), E), 256, 0, stream>>>((const bf16*)X, chosen, nullptr, (const bf16*)w_a, (const bf16*)w_b, top, I, ldx, stride,
+    moe_gemm_few_kernel<true, true, 1><<<dim3(ceil_div(O, 16), E), 256, 0, stream>>>((const bf16*)X, chosen, nullptr, (const bf16*)w_a, (const bf16*)w_b, top, I, ldx, stride,
                                                                                  (bf16*)Y, ldy, O, act, in_weight, pairs);
   else
-    moe_gemm_few_kernel<false, true><<<dim3(ceil_div(O, 32), E), 256, 0, stream>>>((const bf16*)X, chosen, nullptr, (const bf16*)w_a, nullptr, 0, I, ldx, stride, (bf16*)Y,
+    moe_gemm_few_kernel<false, true, 2><<<dim3(ceil_div(O, 32), E), 256, 0, stream>>>((const bf16*)X, chosen, nullptr, (const bf16*)w_a, nullptr, 0, I, ldx, stride, (bf16*)Y,
                                                                                   ldy, O, act, nullptr, pairs);
   GIBBS_LAUNCH_STATUS("moe_gemm");
 }

@@ -217,6 +217,7 @@ _SIGNATURES = {
 _VALUE_SIGNATURES = {
     "gibbs_moe_capacity": ([c_int, c_int, c_int], c_long),
     "gibbs_moe_tile": ([c_int, c_int], c_int),
+    "gibbs_moe_gated_features": ([c_int, c_int], c_int),
     "gibbs_pair_layout_below_tiles": ([], c_int),
     "gibbs_rule_skinny_splits": ([c_int, c_int, c_int, c_int, c_int], c_int),
     "gibbs_rule_decode_splits": ([c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p], None),

@@ -1193,6 +1193,32 @@ def test_few_rows_experts_without_grouping(n, top, experts, identity, width, inn
         close(direct[i], F.silu(g) * u, bf, f"pair {i}", bf16=8e-3)
 
 
+@pytest.mark.parametrize("n,top,experts,width,inner", [(240, 2, 8, 72, 1160), (240, 2, 8, 264, 1304), (96, 8, 64, 64, 520), (17, 4, 300, 8, 152)])
+def test_gated_experts_of_many_workgroups(n, top, experts, width, inner):
+    """From the line on a workgroup takes 32 features: each pair's row has the bits that 16 give it (the product without grouping of 8 rows at a time), the last
+    tile of features whole or not, experts of several tiles and of none."""
+    from gibbs_amd.ops.lib import call, dtype_code, library, ptr, stream
+    bf, pairs, tile = torch.bfloat16, n * top, 16
+    h, wa, wb = rnd(n, width, dtype=bf, seed=1), rnd(experts, inner, width, dtype=bf, seed=2), rnd(experts, inner, width, dtype=bf, seed=3)
+    chosen = torch.stack([torch.randperm(max(top, experts - 1), generator=torch.Generator().manual_seed(r))[:top] for r in range(n)]).int().to(DEV)
+    cap = int(library().gibbs_moe_capacity(pairs, experts, tile))
+    assert int(library().gibbs_moe_gated_features(cap // tile, inner)) == 32
+    new = lambda *shape, dtype=torch.int32: torch.full(shape, 77, dtype=dtype, device=DEV)
+    order, at, tiles = new(cap), new(pairs), new(cap // tile)
+    call("gibbs_moe_group", ptr(chosen), pairs, experts, tile, ptr(order), ptr(at), ptr(tiles), cap, stream())
+    grouped = new(cap, inner, dtype=bf)
+    call("gibbs_moe_gemm_weighted", ptr(h), width, top, ptr(order), ptr(tiles), cap, tile, ptr(wa), ptr(wb), None, ptr(grouped), inner, dtype_code(bf), inner, width, 0, stream())
+    for r in range(0, n, 8):
+        few = min(8, n - r)
+        direct = new(few * top, inner, dtype=bf)
+        call("gibbs_moe_gemm_direct", ptr(h[r:]), width, top, ptr(chosen[r:]), few * top, experts, ptr(wa), ptr(wb), None, ptr(direct), inner, inner, width, 0, stream())
+        assert torch.equal(direct, grouped[at[r * top:(r + few) * top].long()]), r
+    # (against float64: sums of bfloat16 products in float32, a rounding to bfloat16 at the end)
+    for i in (0, pairs // 2, pairs - 1):
+        e, x = int(chosen.view(-1)[i]), h[i // top].double()
+        close(grouped[int(at[i])], F.silu(wa[e].double() @ x) * (wb[e].double() @ x), bf, f"pair {i}", bf16=8e-3)
+
+
 @pytest.mark.parametrize("parts", [1, 3, 9])
 @pytest.mark.parametrize("hidden", [100, 1024, 2048, 5000])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

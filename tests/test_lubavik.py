@@ -226,3 +226,13 @@ def test_plain_forward_runs_every_configuration(tmp_path):
         assert np.allclose(LH.plain_logits(d, ids[:17]), logits[:17], atol=1e-9)
         settled = LH.settle_choices(d, str(tmp_path))
         assert LH.plain_margins(settled, ids).min() > 0.05
+
+
+@pytest.mark.parametrize("rows,top,experts,ff,narrow,wide", [(32, 4, 16, 1024, 28.7, 30.6), (128, 4, 16, 1024, 55.2, 50.3), (256, 4, 16, 1024, 98.9, 90.2), (192, 4, 16, 512, 22.9, 24.1),
+                                                             (256, 2, 8, 1024, 27.8, 28.3), (128, 8, 64, 512, 66.6, 65.4), (235, 8, 64, 512, 97.7, 88.3),
+                                                             (512, 8, 64, 512, 191.0, 167.4)])
+def test_gated_experts_take_the_faster_number_of_features(rows, top, experts, ff, narrow, wide):
+    """The rule between 16 and 32 features a workgroup takes the faster way of measured calls (us)."""
+    from gibbs_amd.ops.lib import library
+    tiles = library().gibbs_moe_capacity(rows * top, experts, 16) // 16
+    assert library().gibbs_moe_gated_features(tiles, ff) == (16 if narrow < wide else 32)
