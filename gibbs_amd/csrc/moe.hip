@@ -1020,7 +1020,9 @@ GIBBS_EXPORT int gibbs_moe_tile(int n_pairs, int E) { return (long)n_pairs <= 64
 GIBBS_EXPORT int gibbs_moe_gated_features(int tiles, int F) { return (long)tiles * ceil_div(F, 16) <= 2560 ? 16 : 32; }
 
 // Few rows, whose products need no grouping (gibbs_moe_gemm_direct): at most 16, so that an expert has at most one of each row's pairs, a tile, and
-// 64 pairs, one for each lane of a wave.
+// 64 pairs, one for each lane of a wave.  Any number of experts: a grid of grouped products has a workgroup for the tile that each may begin, as this one has for each.
+// Route, group and products grouped / without grouping, us, width 2,048, F 1,024, 4 chosen, 8 rows: 16 experts 48 / 50, 64 87 / 86, 256 133 / 135, 512 177 / 165, 1,024
+// 304 / 272; 1 row: 64 31 / 32, 256 66 / 59, 1,024 215 / 169; width 1,024, F 512, 8 rows: 16 22 / 19, 256 58 / 51, 1,024 153 / 110.
 GIBBS_EXPORT int gibbs_moe_direct_takes(int n, int top, int E, int W, int F) {
   return n > 0 && n <= 16 && n * top <= WAVE && E <= 65535 && W % 8 == 0 && F % 8 == 0;
 }
