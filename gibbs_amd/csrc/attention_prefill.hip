@@ -1,5 +1,6 @@
 // Paged causal attention for prompt portions on the gfx950 matrix cores (bfloat16 in, float32
-// scores, maxima, sums and accumulators).
+// scores, maxima, sums and accumulators): the entry points, and the kernel for what attention_prompt.hip does not take
+// (head sizes other than 64 and 128, pages of fewer than 8 keys or of a size that is no power of two).
 //
 // A workgroup takes 64 consecutive query rows of one request and HPW query heads that share a kv head
 // (1, 2 or 4 of the group's); 4 waves per head, each owning 16 of the rows.  One K and one V tile in LDS
@@ -24,6 +25,7 @@
 // workgroups of their own (grid z) and leave (max, sum, weighted values) for the merge kernel.
 #include "common.h"
 #include "attention_merge.h"
+#include "attention_prompt.h"
 
 namespace {
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
@@ -58,27 +60,6 @@ __device__ __forceinline__ short4v lds_read_transposed(const bf16* p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4v __attribute__((address_space(3)))*)p);
 }
 
-struct PrefillArgs {
-  const int* cu;
-  const int* ctx;
-  const int* table;
-  int n_req, max_pages, page_size, num_pages;
-  int page_shift;  // log2(page_size) if it is a power of two, else -1
-  int nh, nkv, hd;
-  long ldq, ldo;
-  float scale;
-  int window;
-  int n_splits;    // slices of the key tiles (1: the workgroup writes the finished rows)
-  // a bias on the scores by distance, or null: [nh, bias_len], row h entry d for keys d positions back (the last
-  // entry for all farther ones), divided by `scale` already (it is added to the raw scores, which are scaled later)
-  const float* bias;
-  int bias_len;
-  // a sink per head, or null: [nh]; the softmax's denominator also holds exp(sink[h]) (natural units, not scaled)
-  const float* sink;
-  int chunk;       // > 0: a row sees the keys of its own stretch of `chunk` positions (counted from 0) instead of a window
-  float softcap;   // > 0: scaled scores are capped as softcap * tanh(s / softcap)
-};
-
 // DT: head size = 16 * DT.  POW2: the page size is a power of two (shifts instead of divisions: an
 // integer division costs dozens of instructions, several times per thread and tile).
 // Five waves a SIMD are asked for: the walk over the keys is a chain of short waits (two barriers a tile, LDS, the
@@ -91,7 +72,6 @@ struct PrefillArgs {
 // 1,500 keys: 37.0 us with all in one kernel, 27.4 without; 16,384 rows: 2,287 and 2,161).  The bias comes through LDS, 127
 // values a tile and head: read from memory by every lane for each of its 16 scores it took a third of the time (2,048 rows, 32 heads
 // in groups of 4: 107 us, now 70).
-enum { SCORES_PLAIN = 0, SCORES_BIASED = 1, SCORES_CAPPED = 2 };
 template <int DT, bool POW2, int HPW, int SCORES>
 __global__ __launch_bounds__(256 * HPW) __attribute__((amdgpu_waves_per_eu(DT <= 4 ? (HPW == 1 ? 5 : 4) : 1))) void attention_prefill_kernel(const bf16* __restrict__ q,
                                                                 const bf16* __restrict__ kpages,
@@ -435,10 +415,16 @@ template <int DT, int HPW>
 void launch_prefill_heads(dim3 grid, hipStream_t stream, const bf16* q, const bf16* k, const bf16* v, bf16* out, float* partial,
                           const PrefillArgs& a) {
   grid.y = a.nh / HPW;
+  // (head sizes 64 and 128 come here with pages of other sizes only)
 #define PREFILL(SCORES)                                                                                                              \
   do {                                                                                                                               \
-    if (a.page_shift >= 0) attention_prefill_kernel<DT, true, HPW, SCORES><<<grid, 256 * HPW, 0, stream>>>(q, k, v, out, partial, a); \
-    else attention_prefill_kernel<DT, false, HPW, SCORES><<<grid, 256 * HPW, 0, stream>>>(q, k, v, out, partial, a);                  \
+    if constexpr (DT != 4 && DT != 8) {                                                                                              \
+      if (a.page_shift >= 0) {                                                                                                       \
+        attention_prefill_kernel<DT, true, HPW, SCORES><<<grid, 256 * HPW, 0, stream>>>(q, k, v, out, partial, a);                   \
+        break;                                                                                                                       \
+      }                                                                                                                              \
+    }                                                                                                                                \
+    attention_prefill_kernel<DT, false, HPW, SCORES><<<grid, 256 * HPW, 0, stream>>>(q, k, v, out, partial, a);                      \
   } while (0)
   if (a.softcap > 0.f) PREFILL(SCORES_CAPPED);
   else if (a.bias) PREFILL(SCORES_BIASED);
@@ -463,7 +449,7 @@ void launch_prefill(dim3 grid, int heads_per_wg, hipStream_t stream, const bf16*
 // workspace of (first_row + n_rows) * nh * n_splits * (hd + 2) floats.  cu may start above 0 (the requests
 // of a step from some request on): first_row = cu[0] then, and n_rows counts the rows from there.
 // heads_per_wg: query heads of a kv head's group that a workgroup takes (1, 2 or 4; 0 counts as 1; the step's
-// rule for it is gibbs_rule_prefill_heads).
+// rule for it is gibbs_rule_prefill_heads; attention_prompt.hip takes as many as the group has, with the same bits).
 // bias (or null): float32 [nh, bias_len], the score of a key d positions back gets bias[h][min(d, bias_len - 1)] * scale added.
 // sink (or null): float32 [nh], a term exp(sink[h]) in the softmax's denominator that has no key and no value.
 // chunk > 0: a row sees the keys of its own stretch of `chunk` positions, counted from position 0 (no window then).
@@ -491,18 +477,22 @@ GIBBS_EXPORT int gibbs_attention_prefill_masked(const void* q, const void* kpage
   if (n_rows == 0 || n_req == 0) return 0;
   const int page_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1;
   PrefillArgs a{cu, ctx, table, n_req, max_pages, page_size, num_pages, page_shift, nh, nkv, hd, ldq, ldo, scale, window, n_splits, bias, bias_len, sink, chunk, softcap};
-  dim3 grid(ceil_div(n_rows, BM) + n_req, nh, n_splits);
   const bf16 *qq = (const bf16*)q, *kk = (const bf16*)kpages, *vv = (const bf16*)vpages;
   bf16* oo = (bf16*)out;
-  switch (hd / 16) {
-    case 1: launch_prefill<1>(grid, heads_per_wg, stream, qq, kk, vv, oo, partial, a); break;
-    case 2: launch_prefill<2>(grid, heads_per_wg, stream, qq, kk, vv, oo, partial, a); break;
-    case 3: launch_prefill<3>(grid, heads_per_wg, stream, qq, kk, vv, oo, partial, a); break;
-    case 4: launch_prefill<4>(grid, heads_per_wg, stream, qq, kk, vv, oo, partial, a); break;
-    case 5: launch_prefill<5>(grid, heads_per_wg, stream, qq, kk, vv, oo, partial, a); break;
-    case 6: launch_prefill<6>(grid, heads_per_wg, stream, qq, kk, vv, oo, partial, a); break;
-    case 7: launch_prefill<7>(grid, heads_per_wg, stream, qq, kk, vv, oo, partial, a); break;
-    default: launch_prefill<8>(grid, heads_per_wg, stream, qq, kk, vv, oo, partial, a); break;
+  if (prompt_attention_takes(hd, page_size, kpages, vpages)) {
+    launch_prompt_attention(qq, kk, vv, oo, partial, a, n_rows, stream);
+  } else {
+    dim3 grid(ceil_div(n_rows, BM) + n_req, nh, n_splits);
+    switch (hd / 16) {
+      case 1: launch_prefill<1>(grid, heads_per_wg, stream, qq, kk, vv, oo, partial, a); break;
+      case 2: launch_prefill<2>(grid, heads_per_wg, stream, qq, kk, vv, oo, partial, a); break;
+      case 3: launch_prefill<3>(grid, heads_per_wg, stream, qq, kk, vv, oo, partial, a); break;
+      case 4: launch_prefill<4>(grid, heads_per_wg, stream, qq, kk, vv, oo, partial, a); break;
+      case 5: launch_prefill<5>(grid, heads_per_wg, stream, qq, kk, vv, oo, partial, a); break;
+      case 6: launch_prefill<6>(grid, heads_per_wg, stream, qq, kk, vv, oo, partial, a); break;
+      case 7: launch_prefill<7>(grid, heads_per_wg, stream, qq, kk, vv, oo, partial, a); break;
+      default: launch_prefill<8>(grid, heads_per_wg, stream, qq, kk, vv, oo, partial, a); break;
+    }
   }
   if (n_splits > 1) {
     hipError_t e = hipGetLastError();

@@ -27,6 +27,7 @@
 // reports the bytes a step needs, so the caller can size the workspace before the real run.  Buffers are
 // taken and given back in the order of the code below; kernels run in stream order, so a buffer that
 // was given back can be handed out again at once.
+#include "attention_prompt.h"
 #include "common.h"
 #include "step_plan_api.h"
 #include <algorithm>
@@ -100,13 +101,25 @@ int prefill_splits(long n_tiles, int nh, int max_seq, int window) {
   return (int)std::max<long>(1, std::min<long>(std::min<long>(ceil_div_l(2048, blocks), keys / 256), 16));
 }
 
+// The same for attention_prompt.hip, whose workgroups are 32 rows of four heads (64 of two, 128 of one): two workgroups a compute unit, with at
+// least 512 keys to a slice on average, as a slice more costs every row its partial result and the merge's kernel.  Measured, us a call in
+// 1 / 2 / 4 / 8 slices, 32 heads of 64 in groups of 4: 512 rows behind 1,536 keys (128 workgroups) 31 / 31 / 28 / 36; behind 7,680 - / 84 / 57 / 64;
+// 128 rows behind 1,000 20 / 17 / 17; 1,024 rows behind none (256 workgroups) 19 / 30; 512 behind none 13 / 18 / 20.
+int prompt_splits(int rows, int reqs, int nh, int nkv, int max_seq, int window) {
+  const int group = nh / std::max(nkv, 1), heads = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1), tile = 128 / heads;
+  const long blocks = std::max<long>(1, (ceil_div_l(rows, tile) + reqs / 2) * (nh / heads));
+  long seen = max_seq - rows / (2 * std::max(reqs, 1));
+  if (window > 0) seen = std::min<long>(seen, window);
+  return (int)std::max<long>(1, std::min<long>(std::min<long>((512 + blocks / 2) / blocks, seen / 512), 16));
+}
+
 // Query heads of a kv head's group that a workgroup of the prompt attention takes (they share its K and V
 // tiles).  With one head a workgroup re-reads all keys and values of its rows' past for 64 x 64 scores at a
 // time, and from about 4,000 keys a row that traffic, not the arithmetic, bounds the kernel (537 TFLOP/s at
 // 8.4 TB/s through L2 and the L1s); more heads a workgroup are fewer, longer workgroups.  Measured at 32 heads
 // in groups of 4, head size 64 (us, with 1 / 2 / 4 heads): 2,048 rows 68 / 63 / 63; 4,096 rows 196 / 209 / 203;
 // 8,192 rows 577 / 562 / 584; 32,768 rows 8,086 / 7,147 / 6,626; 2,048 rows behind 6,144 keys 281 / 220 / 205;
-// 512 rows behind 7,680 keys in 8 slices 80 / 84 / 92.
+// 512 rows behind 7,680 keys in 8 slices 80 / 84 / 92.  (Heads of 64 in pages of a power of two take attention_prompt.hip now.)
 int prefill_heads(int rows, int reqs, int nh, int nkv, int hd, int max_seq, int n_splits) {
   const int group = nh / std::max(nkv, 1);
   if (hd > 64 || group % 2 || n_splits > 1) return 1;
@@ -735,7 +748,11 @@ void* attend_prepared(Exec& e, const PagedAttention& t, void* raw, long ldq, lon
     const int lead = a.lead_single >= 2 ? a.lead_single : 0;
     if (lead) decode_attention(e, t, raw, ldq, lead, a.pos, a.row_req, att);
     const int rows = N - lead, reqs = a.n_req - lead;
-    const int n_splits = a.max_seq > 0 ? prefill_splits(prefill_tiles(rows, reqs), t.nh, a.max_seq, t.chunk > 0 ? t.chunk : t.window) : 1;
+    const int bound = t.chunk > 0 ? t.chunk : t.window;
+    const int n_splits = a.max_seq <= 0 ? 1
+                         : prompt_attention_takes(t.hd, t.page_size, t.kpages, t.vpages)
+                             ? prompt_splits(rows, reqs, t.nh, t.nkv, a.max_seq, bound)
+                             : prefill_splits(prefill_tiles(rows, reqs), t.nh, a.max_seq, bound);
     float* partial = n_splits > 1 ? (float*)e.take(gibbs_attention_decode_workspace(N, t.nh, t.hd, n_splits) * 4) : nullptr;
     RUN(e, gibbs_attention_prefill_masked(raw, t.kpages, t.vpages, att, partial, a.cu + lead, a.ctx + lead, table + (long)lead * width, reqs,
                                           width, t.page_size, t.num_pages, rows, t.nh, t.nkv, t.hd, ldq, ldo, t.scale, t.window, n_splits, lead,
@@ -2649,6 +2666,10 @@ GIBBS_EXPORT void gibbs_rule_decode_splits(int n_rows, int nkv, int group, int m
 }
 GIBBS_EXPORT int gibbs_rule_prefill_splits(long n_tiles, int nh, int max_seq, int window) {
   return prefill_splits(n_tiles, nh, max_seq, window);
+}
+GIBBS_EXPORT int gibbs_rule_prompt_splits(int rows, int reqs, int nh, int nkv, int hd, int page_size, int max_seq, int window) {
+  return prompt_attention_takes(hd, page_size, nullptr, nullptr) ? prompt_splits(rows, reqs, nh, nkv, max_seq, window)
+                                                                 : prefill_splits(prefill_tiles(rows, reqs), nh, max_seq, window);
 }
 GIBBS_EXPORT long gibbs_rule_prefill_tiles(int rows, int reqs) { return prefill_tiles(rows, reqs); }
 GIBBS_EXPORT int gibbs_rule_prefill_heads(int rows, int reqs, int nh, int nkv, int hd, int max_seq, int n_splits) {

@@ -707,7 +707,8 @@ def attention_prefill(q: torch.Tensor, n_rows: int, nh: int, nkv: int, hd: int, 
     assert out.shape == (n_rows, nh * hd) and out.dtype == q.dtype and out.is_contiguous()
     rows, reqs = n_rows - first_row, n_req - first_req
     if n_splits is None:
-        n_splits = prefill_splits(int(library().gibbs_rule_prefill_tiles(rows, reqs)), nh, max_seq, window) if max_seq > 0 else 1
+        n_splits = (int(library().gibbs_rule_prompt_splits(rows, reqs, nh, nkv, hd, page_size, int(max_seq), int(chunk or window or 0)))
+                    if max_seq > 0 else 1)
     if heads_per_wg is None:
         heads_per_wg = int(library().gibbs_rule_prefill_heads(rows, reqs, nh, nkv, hd, int(max_seq), int(n_splits)))
     partial = None

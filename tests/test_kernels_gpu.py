@@ -664,6 +664,36 @@ def test_attention_float32_many_requests():
     assert whole.isfinite().all() and (whole.abs().sum(1) > 0).all()
 
 
+@pytest.mark.parametrize("nh,nkv,hd,page,how", [
+    (8, 2, 64, 16, {}), (4, 2, 64, 8, {"window": 70}), (3, 1, 64, 64, {"chunk": 100}), (4, 1, 128, 16, {"softcap": 3.0}),
+    (2, 1, 128, 8, {"window": 1}), (3, 3, 128, 32, {"sink": True}), (2, 1, 64, 128, {"splits": 3})])
+def test_attention_prompt_edges(nh, nkv, hd, page, how):
+    """Rows around the edges of a wave's 32 and keys around those of a tile's 64, one tile and more than 64 of them (page ids are
+    taken anew), unused keys of the last page that are no numbers, against the kernel with a wave a row."""
+    from gibbs_amd import ops
+    q_lens = [1, 31, 32, 33, 64, 65, 129, 3, 40]
+    seq_lens = [1, 63, 64, 65, 128, 193, 129, 2050, 4330]
+    kp, vp, table, _, _ = paged_setup(torch.bfloat16, nkv, hd, page, seq_lens, sum(-(-s // page) for s in seq_lens) + 3, seed=17)
+    for r, s in enumerate(seq_lens):
+        if s % page:
+            kp[table[r, s // page].item(), :, s % page:] = math.nan
+            vp[table[r, s // page].item(), :, s % page:] = math.nan
+    ctx = [s - n for s, n in zip(seq_lens, q_lens)]
+    cu = np.concatenate([[0], np.cumsum(q_lens)])
+    n = int(cu[-1])
+    q = rnd(n, nh * hd, dtype=torch.bfloat16, seed=4)
+    scale, window, chunk, softcap = 1 / math.sqrt(hd), how.get("window"), how.get("chunk", 0), how.get("softcap", 0.0)
+    sink = rnd(nh, seed=6) if how.get("sink") else None
+    out = ops.attention_prefill(q, n, nh, nkv, hd, kp, vp, table, len(q_lens), i32(cu), i32(ctx), scale, window, sink=sink, chunk=chunk,
+                                softcap=softcap, n_splits=how.get("splits", 1))
+    pos = i32([c + t for c, m in zip(ctx, q_lens) for t in range(m)])
+    row_req = i32([r for r, m in enumerate(q_lens) for _ in range(m)])
+    plain = ops.attention_plain(q, n, nh, nkv, hd, kp, vp, table, len(q_lens), pos, row_req, scale, window, sink=sink, chunk=chunk,
+                                softcap=softcap)
+    assert out.isfinite().all()
+    close(out, plain, torch.bfloat16, "prompt attention", bf16=1e-2)
+
+
 def test_prefill_splits_choice():
     from gibbs_amd.ops import prefill_splits
     assert prefill_splits(32, 32, 2048) == 1                 # a whole 2,048-token prompt fills the chip
