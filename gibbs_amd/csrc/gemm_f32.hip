@@ -22,6 +22,7 @@
 // The plain kernel (vector units, ascending k) takes what these refuse: rows that are no whole number of 16 bytes, and
 // bfloat16 operands (float32 accumulation) of any size and stride.
 #include "f32_parts.h"
+#include <algorithm>
 #include <utility>
 
 namespace {
@@ -39,21 +40,41 @@ __device__ __forceinline__ void each(F&& f) { each(f, std::make_integer_sequence
 // the stretch after the next.  Three stretches in LDS let the reads for the first products of a stretch stand in front of its barrier.
 // Workgroup ids go round the 8 chips' L2 caches; the remapping gives each of them whole panels of features, whose rows of W
 // then come from memory once.
-template <int WO, int WN, int FO, int FN, int OCC>
+// SHARED: tiles too few to fill the chip.  The tiles' stretches of k stand in one line, and a workgroup takes `run` of them in a row, so that
+// every compute unit gets as much whatever the number of tiles: the end of one tile and the beginning of the next (a run is shorter than
+// a tile).  They leave the stretches' sums in `sums` (those from a tile's first on added up) and the rows with lost digits in `marks`, and
+// gemm_f32_join_kernel adds the sums in the same order as ever.  1,194 rows, 1,024 features, inner size 4,608: 152 tiles on as many of
+// the 256 units 128 us, shared 98; 700 rows 61 (102 in tiles of 32 x 64).
+struct SharedSums {
+  f32x4* sums;      // [tiles][stretches][FO FN][threads]
+  int* marks;       // [tiles][SHARED_PARTS][BO + BN]
+  int run;
+};
+constexpr int SHARED_PARTS = 6;      // workgroups of a tile at most: runs of two and more of at most 8 stretches, and one that they begin within
+template <int WO, int WN, int FO, int FN, int OCC, bool SHARED = false>
 __global__ __launch_bounds__(64 * WO * WN, OCC) void gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                             float* __restrict__ C, int N, int O, int I, long lda, long ldw,
-                                                            long ldc, int row_tiles, int tiles, int wide) {
+                                                            long ldc, int row_tiles, int tiles, int wide, SharedSums shared) {
   constexpr int T = 64 * WO * WN, BO = 16 * FO * WO, BN = 16 * FN * WN, ROWS = T / 8, NW = BO / ROWS, NX = BN / ROWS, NP = NW + NX;
   constexpr int PART = (BO + BN) * F32_BK, BUF = 3 * PART;      // a part of both operands (W's rows first), a stretch
   static_assert(NW * ROWS == BO && NX * ROWS == BN && ROWS % 16 == 0, "whole passes, a thread's rows in the same order");
   __shared__ __attribute__((aligned(16))) __bf16 s_p[3 * BUF];
-  const int per = (tiles + 7) / 8, tile = (blockIdx.x % 8) * per + blockIdx.x / 8;
-  if (tile >= tiles) return;
-  const int o0 = tile / row_tiles * BO, n0 = tile % row_tiles * BN;
+  const int segment = f32_segment(I), stretches = (I + segment - 1) / segment;
+  const int groups = SHARED ? (tiles * stretches + shared.run - 1) / shared.run : tiles;
+  const int per = (groups + 7) / 8, group = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  if (group >= groups) return;
   const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, g = lane / 16, c = lane % 16;
   const int wo = wave / WN * 16 * FO, wn = wave % WN * 16 * FN;
   const int r0 = threadIdx.x / 8, quad = threadIdx.x % 8 * 4;      // this thread's row (of ROWS at a time) and four k of a stretch
   const int at = r0 * F32_BK + ((quad / 8) ^ (r0 / 4 % 4)) * 8 + quad % 8, from = c * F32_BK + (g ^ (c / 4)) * 8;
+  // (one tile's stretches from `s_from` on; without SHARED the only one, all of them)
+  int line = SHARED ? group * shared.run : group * stretches;
+  const int line_end = SHARED ? min(line + shared.run, tiles * stretches) : line + stretches;
+  while (true) {
+  const int tile = SHARED ? line / stretches : group, s_from = SHARED ? line % stretches : 0;
+  const int s_to = SHARED ? min(stretches, s_from + line_end - line) : stretches;
+  const int k_from = s_from * segment, k_to = min(s_to * segment, I);
+  const int o0 = tile / row_tiles * BO, n0 = tile % row_tiles * BN;
   const float* src[NP];
 #pragma unroll
   for (int i = 0; i < NP; ++i)
@@ -101,19 +122,18 @@ __global__ __launch_bounds__(64 * WO * WN, OCC) void gemm_f32_tile_kernel(const 
   };
   auto read = [&](int buf, int q, int row) { return *(const bf16x8*)&s_p[buf + q * PART + row * F32_BK + from]; };
   f32x4 total[FO][FN] = {};
-  const int segment = f32_segment(I);
   bf16x8 fw[3][FO], fx[3][FN], ahead[FN];      // `ahead`: the next stretch's high parts of A
 #pragma unroll
-  for (int i = 0; i < NP; ++i) ask(i, 0);
-  each<NP * STEPS>([&](auto x) __attribute__((always_inline)) { step(x, 0, 0, F32_BK); });
-  each<NP * STEPS>([&](auto x) __attribute__((always_inline)) { step(x, BUF, F32_BK, 2 * F32_BK); });
+  for (int i = 0; i < NP; ++i) ask(i, k_from);
+  each<NP * STEPS>([&](auto x) __attribute__((always_inline)) { step(x, 0, k_from, k_from + F32_BK); });
+  each<NP * STEPS>([&](auto x) __attribute__((always_inline)) { step(x, BUF, k_from + F32_BK, k_from + 2 * F32_BK); });
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < FO; ++i) fw[2][i] = read(0, 2, wo + 16 * i);
 #pragma unroll
   for (int i = 0; i < FN; ++i) fx[0][i] = read(0, 0, BO + wn + 16 * i);
   int now = 0, then = BUF, free = 2 * BUF;      // the stretch at hand, the next one, and the one that is filled
-  for (int begin = 0; begin < I; begin += segment) {
+  for (int begin = k_from; begin < k_to; begin += segment) {
     const int end = min(begin + segment, I);
     f32x4 acc[FO][FN] = {};
     for (int k0 = begin; k0 < end; k0 += F32_BK) {
@@ -147,7 +167,25 @@ __global__ __launch_bounds__(64 * WO * WN, OCC) void gemm_f32_tile_kernel(const 
 #pragma unroll
     for (int i = 0; i < FO; ++i)
 #pragma unroll
-      for (int h = 0; h < FN; ++h) total[i][h] += acc[i][h];
+      for (int h = 0; h < FN; ++h) {
+        total[i][h] += acc[i][h];
+        if (SHARED && s_from > 0) shared.sums[(((size_t)tile * stretches + begin / segment) * (FO * FN) + i * FN + h) * T + threadIdx.x] = acc[i][h];
+      }
+  }
+  if constexpr (SHARED) {
+#pragma unroll
+    for (int i = 0; i < FO * FN; ++i)
+      if (s_from == 0) shared.sums[(((size_t)tile * stretches + s_to - 1) * (FO * FN) + i) * T + threadIdx.x] = total[i / FN][i % FN];
+    int* marks = shared.marks + ((size_t)tile * SHARED_PARTS + group - tile * stretches / shared.run) * (BO + BN);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {      // (a row's eight threads are neighbours)
+      const uint64_t row = __builtin_amdgcn_ballot_w64(digits_lost(left[i])) >> (lane & ~7) & 0xff;
+      if (lane % 8 == 0) marks[ROWS * i + r0] = row != 0;
+    }
+    line += s_to - s_from;
+    if (line >= line_end) return;
+    __syncthreads();      // (everyone is done with this tile's operands in LDS)
+    continue;
   }
   // which of the tile's rows have lost digits: hardly ever one
   uint32_t any = 0;
@@ -177,7 +215,7 @@ __global__ __launch_bounds__(64 * WO * WN, OCC) void gemm_f32_tile_kernel(const 
       want |= wants_again(total[i][h], lost && s_lost[BO + wn + 16 * h + c], w_lost) << (4 * (i * FN + h));
       store_f32x4(C, ldc, n0 + wn + 16 * h + c, o0 + wo + 16 * i + 4 * g, N, O, wide, total[i][h]);
     }
-  if (__builtin_expect(__builtin_amdgcn_ballot_w64(want != 0) == 0, 1)) return;
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(want != 0) != 0, 0))
 #pragma unroll 1
   for (int b = 0; b < FO * FN; ++b) {
     const uint32_t mine = want >> (4 * b) & 15;
@@ -188,6 +226,48 @@ __global__ __launch_bounds__(64 * WO * WN, OCC) void gemm_f32_tile_kernel(const 
     for (int j = 0; j < 4; ++j)
       if ((mine >> j & 1) && row < N && col + 4 * g + j < O) C[(size_t)row * ldc + col + 4 * g + j] = y[j];
   }
+  return;
+  }
+}
+
+// What several workgroups have left of a tile: a block of 16 x 16 a wave has, added in the stretches' order, and the rows that want to be taken again.
+template <int WO, int WN, int FO, int FN>
+__global__ __launch_bounds__(64 * WO * WN) void gemm_f32_join_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int N,
+                                                                     int O, int I, long lda, long ldw, long ldc, int row_tiles, int wide, SharedSums shared) {
+  constexpr int T = 64 * WO * WN, BO = 16 * FO * WO, BN = 16 * FN * WN;
+  const int segment = f32_segment(I), stretches = (I + segment - 1) / segment;
+  const int tile = blockIdx.x, block = blockIdx.y, line = tile * stretches;
+  const int first = min(shared.run - line % shared.run, stretches);      // stretches that the first of the tile's workgroups has added up
+  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, g = lane / 16, c = lane % 16;
+  const int wo = wave / WN * 16 * FO + 16 * (block / FN), wn = wave % WN * 16 * FN + 16 * (block % FN);
+  const f32x4* sums = shared.sums + ((size_t)line * (FO * FN) + block) * T + threadIdx.x;
+  f32x4 sum[F32_SEGMENTS];
+#pragma unroll
+  for (int s = 0; s < F32_SEGMENTS; ++s) sum[s] = sums[(size_t)min(max(s, first - 1), stretches - 1) * (FO * FN) * T];
+  const int parts = (line + stretches - 1) / shared.run - line / shared.run + 1;
+  const int* marks = shared.marks + (size_t)tile * SHARED_PARTS * (BO + BN);
+  int x_lost = 0;
+  uint32_t w_lost = 0;
+  for (int p = 0; p < parts; ++p) {
+    const int* m = marks + p * (BO + BN);
+    x_lost |= m[BO + wn + c];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w_lost |= (uint32_t)m[wo + 4 * g + j] << j;
+  }
+  f32x4 total = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < F32_SEGMENTS; ++s)
+    if (s == first - 1) total = sum[s];
+    else if (s >= first && s < stretches) total += sum[s];
+  const int row = tile % row_tiles * BN + wn + c, col = tile / row_tiles * BO + wo;
+  const uint32_t want = wants_again(total, x_lost != 0, w_lost);
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(want != 0) != 0, 0)) {
+    const f32x4 y = again(W + (size_t)min(col + c, O - 1) * ldw, A + (size_t)min(row, N - 1) * lda, I, g, want);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (want >> j & 1) total[j] = y[j];
+  }
+  store_f32x4(C, ldc, row, col + 4 * g, N, O, wide, total);
 }
 
 // Few rows or few tiles: a workgroup takes 16 FO features x 16 FN rows and its eight waves a stretch of k each (f32_stretch; no barrier before
@@ -280,7 +360,35 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const T* __restrict__ A
 template <int WO, int WN, int FO, int FN, int OCC>
 void launch_tile(const float* A, const float* W, float* C, int N, int O, int I, long lda, long ldw, long ldc, bool wide, hipStream_t stream) {
   const int row_tiles = ceil_div(N, 16 * FN * WN), tiles = row_tiles * ceil_div(O, 16 * FO * WO);
-  gemm_f32_tile_kernel<WO, WN, FO, FN, OCC><<<(tiles + 7) / 8 * 8, 64 * WO * WN, 0, stream>>>(A, W, C, N, O, I, lda, ldw, ldc, row_tiles, tiles, wide);
+  gemm_f32_tile_kernel<WO, WN, FO, FN, OCC><<<(tiles + 7) / 8 * 8, 64 * WO * WN, 0, stream>>>(A, W, C, N, O, I, lda, ldw, ldc, row_tiles, tiles, wide, SharedSums{});
+}
+// Tiles of 128 features x 64 rows whose stretches workgroups share: 31 us a tile at an inner size of 1,024 as without, and SHARED_JOIN us for the
+// sums' way through memory and the second kernel, whatever the inner size.  (us, without / with, 1,024 features: inner size 4,608 150 rows 36.3 / 37.3, 333
+// 69 / 40, 700 102 / 61, 1,194 128 / 98; 4,096 700 rows 92 / 57; 1,024 333 rows 20.2 / 20.0, 1,194 34.5 / 36.0, 700 rows of 2,048 features 33.4 / 36.9.)
+constexpr int SHARED_FEATURES = 128, SHARED_ROWS = 64, SHARED_TILES = 256;
+constexpr float SHARED_TILE = 31.f, SHARED_JOIN = 12.f;
+struct SharedShape {
+  int tiles, stretches, run, groups;
+  float cost;      // as the variants' below; 0: does not take the shape
+};
+SharedShape shared_shape(int N, int O, int I) {
+  const int segment = f32_segment(I), stretches = (I + segment - 1) / segment;
+  const long tiles = (long)ceil_div(N, SHARED_ROWS) * ceil_div(O, SHARED_FEATURES);
+  SharedShape s{(int)tiles, stretches, 0, 0, 0.f};
+  if (tiles > SHARED_TILES || I < 2048) return s;      // (256 tiles' sums are 64 MB)
+  s.run = std::max(2, (int)ceil_div(tiles * stretches, 256));
+  s.groups = ceil_div(tiles * stretches, s.run);
+  if (s.run < stretches) s.cost = SHARED_TILE * s.run / stretches + SHARED_JOIN * 1024.f / I;
+  return s;
+}
+size_t shared_sums_bytes(const SharedShape& s) { return (size_t)s.tiles * s.stretches * SHARED_FEATURES * SHARED_ROWS * 4; }
+size_t shared_marks_bytes(const SharedShape& s) { return (size_t)s.tiles * SHARED_PARTS * (SHARED_FEATURES + SHARED_ROWS) * 4; }
+void launch_shared(const SharedShape& s, void* work, const float* A, const float* W, float* C, int N, int O, int I, long lda, long ldw, long ldc, bool wide,
+                   hipStream_t stream) {
+  const SharedSums shared{(f32x4*)work, (int*)((char*)work + shared_sums_bytes(s)), s.run};
+  const int row_tiles = ceil_div(N, SHARED_ROWS);
+  gemm_f32_tile_kernel<4, 2, 2, 2, 2, true><<<(s.groups + 7) / 8 * 8, 512, 0, stream>>>(A, W, C, N, O, I, lda, ldw, ldc, row_tiles, s.tiles, wide, shared);
+  gemm_f32_join_kernel<4, 2, 2, 2><<<dim3(s.tiles, 4), 512, 0, stream>>>(A, W, C, N, O, I, lda, ldw, ldc, row_tiles, wide, shared);
 }
 template <int FO, int FN>
 void launch_split(const float* A, const float* W, float* C, int N, int O, int I, long lda, long ldw, long ldc, bool wide, hipStream_t stream) {
@@ -308,10 +416,9 @@ const F32Variant F32_VARIANTS[] = {
     {64, 64, 26.f, 18.f, launch_tile<2, 2, 2, 2, 2>, false}, {32, 64, 20.f, 13.5f, launch_tile<2, 2, 1, 2, 3>, false},
     {32, 32, 10.f, 9.6f, launch_split<2, 2>, true}, {16, 32, 7.f, 7.f, launch_split<1, 2>, true}, {16, 16, 6.f, 4.2f, launch_split<1, 1>, true}};
 
-bool launch_f32(const float* A, const float* W, float* C, int N, int O, int I, long lda, long ldw, long ldc, hipStream_t stream) {
-  if (I % 4 || lda % 4 || ldw % 4 || (uintptr_t)A % 16 || (uintptr_t)W % 16) return false;
+// The variant of least cost, which is left in `least`.
+const F32Variant* best_variant(int N, int O, int I, float& least) {
   const F32Variant* best = nullptr;
-  float least = 0.f;
   for (const F32Variant& v : F32_VARIANTS) {
     if (v.split && ceil_div(N, v.rows) > 65535) continue;
     const long tiles = (long)ceil_div(N, v.rows) * ceil_div(O, v.features);
@@ -321,22 +428,48 @@ bool launch_f32(const float* A, const float* W, float* C, int N, int O, int I, l
       least = cost;
     }
   }
-  best->launch(A, W, C, N, O, I, lda, ldw, ldc, O % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % 16 == 0, stream);
+  return best;
+}
+// Whether the stretches are shared where a workspace is there for it.
+bool shares(const SharedShape& s, int N, int O, int I) {
+  if (s.cost == 0.f) return false;
+  float least;
+  best_variant(N, O, I, least);
+  return s.cost < least;
+}
+bool launch_f32(const float* A, const float* W, float* C, int N, int O, int I, long lda, long ldw, long ldc, void* work, hipStream_t stream) {
+  if (I % 4 || lda % 4 || ldw % 4 || (uintptr_t)A % 16 || (uintptr_t)W % 16) return false;
+  const bool wide = O % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % 16 == 0;
+  const SharedShape s = shared_shape(N, O, I);
+  float least;
+  if (work && shares(s, N, O, I)) launch_shared(s, work, A, W, C, N, O, I, lda, ldw, ldc, wide, stream);
+  else best_variant(N, O, I, least)->launch(A, W, C, N, O, I, lda, ldw, ldc, wide, stream);
   return true;
 }
 }  // namespace
 
-// A: [N, I] (row stride lda), W: [O, I] (row stride ldw), C: [N, O] (row stride ldc), all float32.
-GIBBS_EXPORT int gibbs_gemm_f32(const float* A, const float* W, float* C, int N, int O, int I, long lda,
-                                long ldw, long ldc, hipStream_t stream) {
+// Bytes of workspace that gibbs_gemm_f32_in can use (0: none).  The results are the same to the bit with and without.
+GIBBS_EXPORT long gibbs_gemm_f32_workspace(int N, int O, int I) {
+  if (N <= 0 || O <= 0 || I <= 0) return 0;
+  const SharedShape s = shared_shape(N, O, I);
+  return shares(s, N, O, I) ? (long)(shared_sums_bytes(s) + shared_marks_bytes(s)) : 0;
+}
+// A: [N, I] (row stride lda), W: [O, I] (row stride ldw), C: [N, O] (row stride ldc), all float32; work: null or a workspace of
+// gibbs_gemm_f32_workspace bytes, aligned to 16.
+GIBBS_EXPORT int gibbs_gemm_f32_in(const float* A, const float* W, float* C, int N, int O, int I, long lda, long ldw, long ldc, void* work,
+                                   hipStream_t stream) {
   GIBBS_REQUIRE(N >= 0 && O > 0 && I > 0, "gemm_f32: bad sizes N=%d O=%d I=%d", N, O, I);
   GIBBS_REQUIRE(lda >= I && ldw >= I && ldc >= O, "gemm_f32: row strides shorter than rows");
+  GIBBS_REQUIRE((uintptr_t)work % 16 == 0, "gemm_f32: the workspace must be 16-byte aligned");
   if (N == 0) return 0;
   dim3 grid(ceil_div(O, TN), ceil_div(N, TM));
   GIBBS_REQUIRE(grid.y <= 65535, "gemm_f32: too many rows (%d)", N);
-  if (launch_f32(A, W, C, N, O, I, lda, ldw, ldc, stream)) GIBBS_LAUNCH_STATUS("gemm_f32");
+  if (launch_f32(A, W, C, N, O, I, lda, ldw, ldc, work, stream)) GIBBS_LAUNCH_STATUS("gemm_f32");
   gemm_plain_kernel<float, float><<<grid, 256, 0, stream>>>(A, W, C, N, O, I, lda, ldw, ldc);
   GIBBS_LAUNCH_STATUS("gemm_f32");
+}
+GIBBS_EXPORT int gibbs_gemm_f32(const float* A, const float* W, float* C, int N, int O, int I, long lda, long ldw, long ldc, hipStream_t stream) {
+  return gibbs_gemm_f32_in(A, W, C, N, O, I, lda, ldw, ldc, nullptr, stream);
 }
 
 // A: [N, I], W: [O, I] bfloat16 with any sizes and strides; C: [N, O] bfloat16 (out_dtype 1) or float32 (0).

@@ -268,6 +268,8 @@ int gibbs_residual_add(float* x, const void* delta, int dtype, int n_partials, l
                        long count, hipStream_t stream);
 int gibbs_gemm_f32(const float* A, const float* W, float* C, int N, int O, int I, long lda, long ldw, long ldc,
                    hipStream_t stream);
+long gibbs_gemm_f32_workspace(int N, int O, int I);
+int gibbs_gemm_f32_in(const float* A, const float* W, float* C, int N, int O, int I, long lda, long ldw, long ldc, void* work, hipStream_t stream);
 int gibbs_gemm_bf16_plain(const void* A, const void* W, void* C, int out_dtype, int N, int O, int I, long lda, long ldw,
                           long ldc, hipStream_t stream);
 int gibbs_gemm_bf16(const void* A, const void* W, void* C, int out_dtype, int N, int O, int I, long lda, long ldw,

@@ -326,6 +326,7 @@ struct Exec {
   // buffer ([N, O], or [parts, N, O] float32 with *parts >= 2).
   void* linear(const void* x, const Matrix& m, int n, bool out_f32, bool partial_ok, bool use_packed, int* parts, long ldx = 0);
   void linear_into(const void* x, const Matrix& m, int n, bool out_f32, bool use_packed, void* y);
+  void run_product(const LinearChoice& c, const void* x, long ldx, const Matrix& m, bool use_packed, void* y, int n, bool out_f32);
   // takes a delta's open sum: two float32 partial sums
   void plain(Pending& d);
   // adds what is pending and makes sure the bfloat16 mirror of x exists
@@ -458,13 +459,23 @@ void* Exec::linear(const void* x, const Matrix& m, int n, bool out_f32, bool par
   const LinearChoice c = choose_linear(bf16_run, n, m.O, m.I, aligned_for_matrix_cores(x, ldx, m.w, m.I), out_f32, partial_ok, p.own_gemm);
   const long elem = !bf16_run || out_f32 || c.splits > 1 ? 4 : 2;
   void* y = take((long)c.splits * n * m.O * elem);
-  RUN(*this, run_linear(c, x, ldx, m, use_packed, y, n, out_f32, a.stream));
+  run_product(c, x, ldx, m, use_packed, y, n, out_f32);
   if (parts) *parts = c.splits;
   return y;
 }
+void Exec::run_product(const LinearChoice& c, const void* x, long ldx, const Matrix& m, bool use_packed, void* y, int n, bool out_f32) {
+  const long bytes = c.kernel == LIN_F32 ? gibbs_gemm_f32_workspace(n, m.O, m.I) : 0;
+  if (bytes == 0) {
+    RUN(*this, run_linear(c, x, ldx, m, use_packed, y, n, out_f32, a.stream));
+    return;
+  }
+  void* work = take(bytes);
+  RUN(*this, gibbs_gemm_f32_in((const float*)x, (const float*)m.w, (float*)y, n, m.O, m.I, ldx, m.I, m.O, work, a.stream));
+  give(work);
+}
 void Exec::linear_into(const void* x, const Matrix& m, int n, bool out_f32, bool use_packed, void* y) {
   const LinearChoice c = choose_linear(bf16_run, n, m.O, m.I, aligned_for_matrix_cores(x, m.I, m.w, m.I), out_f32, false, p.own_gemm);
-  RUN(*this, run_linear(c, x, m.I, m, use_packed, y, n, out_f32, a.stream));
+  run_product(c, x, m.I, m, use_packed, y, n, out_f32);
 }
 void Exec::with_mirror(float* x, Pending& pending, void** mirror) {
   if (pending.parts == 0 && *mirror) return;

@@ -86,8 +86,9 @@ def residual_add(x: torch.Tensor, delta: Optional[torch.Tensor], mirror: Optiona
          x.numel(), ptr(mirror), x.numel(), stream())
 
 
-def gemm_f32(a: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """out[n, o] = sum_k a[n, k] * w[o, k], all float32 (32-bit operands, products and sums)."""
+def gemm_f32(a: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, workspace: bool = True) -> torch.Tensor:
+    """out[n, o] = sum_k a[n, k] * w[o, k], all float32 (32-bit operands, products and sums).  `workspace`: few tiles of a long
+    inner size may share the chip through one, as in a step (the same bits)."""
     require_cuda(a, w)
     assert a.dtype == torch.float32 and w.dtype == torch.float32
     assert a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1], (a.shape, w.shape)
@@ -97,8 +98,10 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = Non
     if out is None:
         out = torch.empty((n, o), dtype=torch.float32, device=a.device)
     assert out.shape == (n, o) and out.dtype == torch.float32 and out.stride(1) == 1
-    call("gibbs_gemm_f32", ptr(a), ptr(w), ptr(out), n, o, i, a.stride(0) if n > 1 else i,
-         w.stride(0), out.stride(0) if n > 1 else o, stream())
+    size = int(library().gibbs_gemm_f32_workspace(n, o, i)) if workspace else 0
+    work = torch.empty(size, dtype=torch.uint8, device=a.device) if size else None
+    call("gibbs_gemm_f32_in", ptr(a), ptr(w), ptr(out), n, o, i, a.stride(0) if n > 1 else i,
+         w.stride(0), out.stride(0) if n > 1 else o, ptr(work), stream())
     return out
 
 

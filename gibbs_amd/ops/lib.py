@@ -28,6 +28,7 @@ _SIGNATURES = {
     "gibbs_embed": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
     "gibbs_add_rmsnorm": [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p],
     "gibbs_residual_add": [c_void_p, c_void_p, c_int, c_int, c_long, c_void_p, c_long, c_void_p],
+    "gibbs_gemm_f32_in": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p, c_void_p],
     "gibbs_gemm_f32": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p],
     "gibbs_gemm_bf16_plain": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p],
     "gibbs_gemm_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p],
@@ -219,6 +220,7 @@ _VALUE_SIGNATURES = {
     "gibbs_moe_tile": ([c_int, c_int], c_int),
     "gibbs_moe_gated_features": ([c_int, c_int], c_int),
     "gibbs_pair_layout_below_tiles": ([], c_int),
+    "gibbs_gemm_f32_workspace": ([c_int] * 3, c_long),
     "gibbs_rule_skinny_splits": ([c_int, c_int, c_int, c_int, c_int], c_int),
     "gibbs_rule_decode_splits": ([c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p], None),
     "gibbs_rule_prefill_splits": ([c_long, c_int, c_int, c_int], c_int),

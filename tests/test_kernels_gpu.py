@@ -151,6 +151,25 @@ def test_gemm_f32_keeps_the_digits_of_small_operands(shape):
     check(a, w, "small values that count")
 
 
+@pytest.mark.parametrize("shape", [(333, 1000, 2052), (270, 1024, 4608), (450, 640, 3000), (700, 500, 2080)])
+def test_gemm_f32_stretches_shared_between_workgroups(shape):
+    """Few tiles of a long inner size share the chip through a workspace: the bits of the product without one, for ordinary values and for
+    rows whose results are taken again (infinities, NaN, digits that three bfloat16 do not hold, in a stretch of any of a tile's workgroups)."""
+    from gibbs_amd import ops
+    from gibbs_amd.ops.lib import library
+    n, o, i = shape
+    assert library().gibbs_gemm_f32_workspace(n, o, i) > 0
+    a, w = rnd(n, i, seed=1), rnd(o, i, seed=2)
+    want = ops.gemm_f32(a, w, workspace=False)
+    assert torch.equal(ops.gemm_f32(a, w), want)
+    a[0, 7], a[n // 2, i - 1], a[n - 1, i // 2], w[o // 3, 5] = float("inf"), float("nan"), 3.4e38, -float("inf")
+    a[1, i - 2], a[70, 3], w[o - 1, i // 3] = 2.0 ** -124, 2.0 ** -130, 2.0 ** -120
+    a[5] *= 2.0 ** -118
+    bits = [ops.gemm_f32(a, w, workspace=k).view(torch.int32) for k in (False, True)]
+    assert torch.equal(*bits)
+    assert not torch.equal(bits[0].view(torch.float32), want)
+
+
 def test_gemm_f32_as_many_rows_as_the_plain_kernel_takes():
     """4,194,240 rows, which is where the plain kernel's grid ends, of few features: the tiles that cut k over their waves have no grid for them."""
     from gibbs_amd import ops
