@@ -475,26 +475,39 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 // tile is Y^T = W X^T): lane l holds 8 values along k of feature or place l % 16, and its four results are four
 // neighbouring features of place l % 16.  Operands come straight from memory.  Measured (16 experts of 1,024 at width 2,048, 4 chosen; us, gated and
 // back): 1 row 13.7 and 6.7 with loads under conditions, 32 features and one wave's tail, 10.1 and 5.6 now; 8 rows (126 and 63 MB) 34.8 and
-// 13.7, now 29.7 and 13.1; back with 16 features a workgroup or 32, 8 rows 13.7 / 13.1 (gated: gibbs_moe_gated_features).
-// DIRECT (at most 64 pairs, an expert at most 16 of them): no grouping in front: blockIdx.y is the expert, `sorted_pair` holds each pair's choice, and
-// places are the pairs' own numbers.
+// 13.7, now 27.0 and 12.9; back with 16 features a workgroup or 32, 8 rows 13.7 / 13.1 (gated: gibbs_moe_gated_features).
+// DIRECT (at most 64 pairs, an expert at most 16 of them): no grouping in front: `sorted_pair` holds each pair's choice, places are the pairs' own
+// numbers, and the workgroups are laid out over the experts that are chosen, not over all: with a grid of all of them the chosen ones' could meet on
+// the same compute units (16 experts, 2 rows, 7 of them chosen: gated 21.6 us and back 11.1, now 13.3 and 7.5).
 template <bool GLU, bool DIRECT, int NF>
 __global__ __launch_bounds__(256) void moe_gemm_few_kernel(const bf16* __restrict__ X, const int* __restrict__ sorted_pair,
                                                            const int* __restrict__ tile_expert, const bf16* __restrict__ Wa,
                                                            const bf16* __restrict__ Wb, int top, int I, long ldx, long expert_stride, bf16* __restrict__ Y,
-                                                           long ldy, int O, int act, const float* __restrict__ in_weight, int pairs) {
+                                                           long ldy, int O, int act, const float* __restrict__ in_weight, int pairs, int experts) {
   constexpr int NA = GLU ? 2 * NF : NF;    // accumulators a wave
   __shared__ __attribute__((aligned(16))) floatx4 part[4][NA][WAVE];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, lr = lane % 16, lg = lane / 16;
-  int e, pair, place;
+  int e, pair, place, block = blockIdx.x;
   if constexpr (DIRECT) {
-    e = blockIdx.y;
-    const bool mine = lane < pairs && sorted_pair[min(lane, pairs - 1)] == e;
-    const uint64_t all = __builtin_amdgcn_ballot_w64(mine);
-    if (all == 0) return;
+    const int columns = (O + 16 * NF - 1) / (16 * NF), nth = blockIdx.x / columns;
+    block = blockIdx.x - nth * columns;
+    const int choice = sorted_pair[min(lane, pairs - 1)];
+    // the pairs with a lane's own choice, by the choices' bits; the `nth` expert of those chosen is the one whose first pair is the nth such
+    const bool live = lane < pairs && choice < experts;
+    uint64_t same = __builtin_amdgcn_ballot_w64(live);
+    for (int b = 0; (experts - 1) >> b; ++b) {
+      const bool bit = choice >> b & 1;
+      const uint64_t with = __builtin_amdgcn_ballot_w64(bit);
+      same &= bit ? with : ~with;
+    }
+    const bool first = live && __builtin_ctzll(same) == lane;
+    const uint64_t firsts = __builtin_amdgcn_ballot_w64(first), found = __builtin_amdgcn_ballot_w64(first && __popcll(firsts & ((1ull << lane) - 1)) == nth);
+    if (found == 0) return;
+    e = __builtin_amdgcn_readlane(choice, __builtin_ctzll(found));
+    const uint64_t all = __builtin_amdgcn_ballot_w64(live && choice == e);
     // the expert's pairs, in ascending order, to lanes 0, 1, ...; every lane then takes its place's
     const int rank = __popcll(all & ((1ull << lane) - 1));
-    const int sent = __builtin_amdgcn_ds_permute((mine ? rank : WAVE - 1) * 4, lane);
+    const int sent = __builtin_amdgcn_ds_permute((all >> lane & 1 ? rank : WAVE - 1) * 4, lane);
     pair = __builtin_amdgcn_ds_bpermute(lr * 4, sent);
     if (lr >= __popcll(all)) pair = -1;
     place = pair < 0 ? 0 : pair;
@@ -504,7 +517,7 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(const bf16* __restric
     pair = sorted_pair[place];
     if (e < 0) return;
   }
-  const int col0 = blockIdx.x * (16 * NF);
+  const int col0 = block * (16 * NF);
   const int src = pair < 0 ? 0 : (top > 0 ? pair / top : place);      // (a place without a pair: some row, its results are not stored)
   const bf16* xr = X + (size_t)src * ldx;
   const bf16* w[NA];
@@ -537,19 +550,23 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(const bf16* __restric
     }
   };
   if (n > 0) {
-    ask(0, 0);
-    ask(1, min(1, n - 1));
+    // The workgroups begin at different k: rows of 4 KB and more, all read at one k at a time, are a few of the memory's channels (8 and 32 rows, gated,
+    // 32.1 and 35.5 us without, 27.0 and 30.4; rows of 2 KB, back, 13.1 / 13.4).  By the feature, so that a result's sum does not depend on the grid.
+    const int turn = I >= 2048 ? col0 / 32 % n : 0;
+    auto nth = [&](int it) { return it + turn < n ? it + turn : it + turn - n; };
+    ask(0, nth(0));
+    ask(1, nth(min(1, n - 1)));
     int it = 0;
     for (; it + 2 < n; it += 2) {
-      use(0, it);
-      ask(0, it + 2);
+      use(0, nth(it));
+      ask(0, nth(it + 2));
       __builtin_amdgcn_sched_barrier(0x7 | 0x8 | 0x380);
-      use(1, it + 1);
-      ask(1, min(it + 3, n - 1));
+      use(1, nth(it + 1));
+      ask(1, nth(min(it + 3, n - 1)));
       __builtin_amdgcn_sched_barrier(0x7 | 0x8 | 0x380);
     }
-    use(0, it);
-    if (it + 1 < n) use(1, it + 1);
+    use(0, nth(it));
+    if (it + 1 < n) use(1, nth(it + 1));
   }
 #pragma unroll
   for (int t = 0; t < NA; ++t) part[wave][t][lane] = acc[t];
@@ -1132,13 +1149,13 @@ GIBBS_EXPORT int gibbs_moe_gemm_weighted(const void* X, long ldx, int top, const
     } else if (w_b) {
       const auto queue = [&](auto kernel, int features) {
         kernel<<<dim3(ceil_div(O, features), tiles), 256, 0, stream>>>((const bf16*)X, sorted_pair, tile_expert, (const bf16*)w_a, (const bf16*)w_b, top, I, ldx, stride, (bf16*)Y,
-                                                                       ldy, O, act, in_weight, 0);
+                                                                       ldy, O, act, in_weight, 0, 0);
       };
       if (gibbs_moe_gated_features(tiles, O) == 16) queue(moe_gemm_few_kernel<true, false, 1>, 16);
       else queue(moe_gemm_few_kernel<true, false, 2>, 32);
     } else {
       moe_gemm_few_kernel<false, false, 2><<<dim3(ceil_div(O, 32), tiles), 256, 0, stream>>>((const bf16*)X, sorted_pair, tile_expert, (const bf16*)w_a, nullptr, top, I,
-                                                                                         ldx, stride, (bf16*)Y, ldy, O, act, nullptr, 0);
+                                                                                         ldx, stride, (bf16*)Y, ldy, O, act, nullptr, 0, 0);
     }
   } else {
     return gibbs_fail("moe_gemm: unknown dtype %d", dtype);
@@ -1158,11 +1175,11 @@ GIBBS_EXPORT int gibbs_moe_gemm_direct(const void* X, long ldx, int top, const i
   GIBBS_REQUIRE(I % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)X % 16) == 0 && ((uintptr_t)w_a % 16) == 0 && ((uintptr_t)w_b % 16) == 0, "moe_gemm: rows of whole 16 bytes");
   const long stride = (long)O * I;
   if (w_b)
-    moe_gemm_few_kernel<true, true, 1><<<dim3(ceil_div(O, 16), E), 256, 0, stream>>>((const bf16*)X, chosen, nullptr, (const bf16*)w_a, (const bf16*)w_b, top, I, ldx, stride,
-                                                                                 (bf16*)Y, ldy, O, act, in_weight, pairs);
+    moe_gemm_few_kernel<true, true, 1><<<ceil_div(O, 16) * std::min(E, pairs), 256, 0, stream>>>((const bf16*)X, chosen, nullptr, (const bf16*)w_a, (const bf16*)w_b, top, I, ldx, stride,
+                                                                                 (bf16*)Y, ldy, O, act, in_weight, pairs, E);
   else
-    moe_gemm_few_kernel<false, true, 2><<<dim3(ceil_div(O, 32), E), 256, 0, stream>>>((const bf16*)X, chosen, nullptr, (const bf16*)w_a, nullptr, 0, I, ldx, stride, (bf16*)Y,
-                                                                                  ldy, O, act, nullptr, pairs);
+    moe_gemm_few_kernel<false, true, 2><<<ceil_div(O, 32) * std::min(E, pairs), 256, 0, stream>>>((const bf16*)X, chosen, nullptr, (const bf16*)w_a, nullptr, 0, I, ldx, stride, (bf16*)Y,
+                                                                                  ldy, O, act, nullptr, pairs, E);
   GIBBS_LAUNCH_STATUS("moe_gemm");
 }
 
