@@ -493,7 +493,7 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(const bf16* __restric
     block = blockIdx.x - nth * columns;
     const int choice = sorted_pair[min(lane, pairs - 1)];
     // the pairs with a lane's own choice, by the choices' bits; the `nth` expert of those chosen is the one whose first pair is the nth such
-    const bool live = lane < pairs && choice < experts;
+    const bool live = lane < pairs && (unsigned)choice < (unsigned)experts;
     uint64_t same = __builtin_amdgcn_ballot_w64(live);
     for (int b = 0; (experts - 1) >> b; ++b) {
       const bool bit = choice >> b & 1;

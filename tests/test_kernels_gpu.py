@@ -1242,6 +1242,30 @@ def test_few_rows_experts_without_grouping(n, top, experts, identity, width, inn
         close(direct[i], F.silu(g) * u, bf, f"pair {i}", bf16=8e-3)
 
 
+@pytest.mark.parametrize("n,top,experts,width,inner", [(2, 3, 5, 2048, 40), (16, 4, 16, 2312, 72), (7, 2, 3, 4104, 33)])
+def test_few_rows_experts_begin_at_different_k(n, top, experts, width, inner):
+    """Rows of 2,048 values and more, whose blocks of features begin at k of their own: against float64, and choices below 0 and beyond the
+    last expert have no result."""
+    from gibbs_amd.ops.lib import call, ptr, stream
+    bf, pairs = torch.bfloat16, n * top
+    h, wa, wb = rnd(n, width, dtype=bf, seed=1), rnd(experts, inner, width, dtype=bf, seed=2) * 0.05, rnd(experts, inner, width, dtype=bf, seed=3) * 0.05
+    chosen = torch.stack([torch.randperm(experts + 1, generator=torch.Generator().manual_seed(r))[:top] for r in range(n)]).int().view(-1)
+    chosen[1::5] = torch.where(chosen[1::5] < 2, torch.full_like(chosen[1::5], -1), chosen[1::5])
+    chosen = chosen.to(DEV)
+    gated, back = torch.full((pairs, inner), 77, dtype=bf, device=DEV), torch.full((pairs, inner), 77, dtype=bf, device=DEV)
+    own = rnd(pairs, width, dtype=bf, seed=4)
+    call("gibbs_moe_gemm_direct", ptr(h), width, top, ptr(chosen), pairs, experts, ptr(wa), ptr(wb), None, ptr(gated), inner, inner, width, 0, stream())
+    call("gibbs_moe_gemm_direct", ptr(own), width, top, ptr(chosen), pairs, experts, ptr(wa), None, None, ptr(back), inner, inner, width, 0, stream())
+    for i, e in enumerate(chosen.tolist()):
+        if not 0 <= e < experts:
+            assert (gated[i] == 77).all() and (back[i] == 77).all()
+            continue
+        x = h[i // top].double()
+        # (sums of bfloat16 products in float32, a rounding to bfloat16 at the end)
+        close(gated[i], F.silu(wa[e].double() @ x) * (wb[e].double() @ x), bf, f"pair {i}", bf16=8e-3)
+        close(back[i], wa[e].double() @ own[i].double(), bf, f"pair {i} back", bf16=8e-3)
+
+
 @pytest.mark.parametrize("n,top,experts,width,inner", [(240, 2, 8, 72, 1160), (240, 2, 8, 264, 1304), (96, 8, 64, 64, 520), (17, 4, 300, 8, 152)])
 def test_gated_experts_of_many_workgroups(n, top, experts, width, inner):
     """From the line on a workgroup takes 32 features: each pair's row has the bits that 16 give it (the product without grouping of 8 rows at a time), the last
