@@ -1080,6 +1080,37 @@ def test_few_row_products_add_waves_in_order_and_a_waves_halves_one_after_the_ot
     assert torch.equal(state[:, 1], b * d) and torch.equal(y, (c * (b * d)).to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("f", [8, 520, 2056])
+@pytest.mark.parametrize("clamped", [False, True])
+def test_gates_of_every_size(f, clamped):
+    """Gates around 80, beyond which the exponential is taken in full for a wave's elements, signed zeros, infinities and NaN among them, against
+    float64, and each row the same beside any other."""
+    from gibbs_amd import ops
+    from gibbs_amd.ops.lib import call, dtype_code, ptr, stream
+    bf = torch.bfloat16
+    gu = rnd(9, 2 * f, dtype=bf, scale=4.0, seed=f)
+    odd = torch.tensor([80.0, -80.0, 80.5, -80.5, -100.0, -0.0, 0.0, 1e37], dtype=bf, device=DEV)      # (1e37 times an up value is still a bfloat16)
+    gu[1, :8], gu[2, f - 8:f], gu[3, :2], gu[4, f - 1] = odd, odd, torch.tensor([math.inf, -math.inf], dtype=bf, device=DEV), math.nan
+    def run(t):
+        if not clamped:
+            return ops.glu(t)
+        o = torch.empty((t.shape[0], f), dtype=bf, device=DEV)
+        call("gibbs_glu_clamped", ptr(t), ptr(o), dtype_code(bf), t.shape[0], f, 1.702, 7.0, stream())
+        return o
+    out, x, u = run(gu), gu[:, :f].double(), gu[:, f:].double()
+    if clamped:
+        g = torch.fmin(x, torch.full_like(x, 7.0))      # (a gate that is no number counts as the cap)
+        want = g * torch.sigmoid(1.702 * g) * (1 + u.clamp(-7.0, 7.0))
+    else:
+        want = x * torch.sigmoid(x) * u
+    rows = [0, 1, 2, 5, 8]
+    # (half a unit of bfloat16, and some 1e-7 of float32 arithmetic in front of it)
+    assert ((out[rows].double() - want[rows]).abs() <= 2.0 ** -8 * 1.001 * want[rows].abs() + 1e-33).all()
+    assert torch.equal(out[3:5].isnan(), want[3:5].to(bf).isnan())
+    for r in rows:
+        assert torch.equal(run(gu[r:r + 1].contiguous())[0], out[r])
+
+
 @pytest.mark.parametrize("n,f,i", [(1, 8192, 2048), (8, 200, 512), (40, 128, 72), (64, 256, 1024), (64, 6200, 256),
                                    (36, 8192, 2048),                        # two tiles a workgroup
                                    (5, 4100, 104), (8, 52, 40), (11, 4090, 72), (14, 2200, 104), (9, 60, 136)])
