@@ -1111,6 +1111,23 @@ def test_gates_of_every_size(f, clamped):
         assert torch.equal(run(gu[r:r + 1].contiguous())[0], out[r])
 
 
+@pytest.mark.parametrize("hidden", [2044, 2052, 3072, 4096, 4100])
+@pytest.mark.parametrize("parts", [0, 1, 3])
+def test_add_rmsnorm_of_rows_two_threads_share(hidden, parts):
+    """Around the widths whose rows 256 threads take twice: the stream, the normed rows and their bits in other company, against float64."""
+    from gibbs_amd import ops
+    bf = torch.bfloat16
+    x, gain = rnd(5, hidden, scale=2.0), 1 + 0.1 * rnd(hidden, seed=2)
+    delta = None if parts == 0 else (rnd(5, hidden, dtype=bf, seed=3) if parts == 1 else rnd(parts, 5, hidden, seed=3))
+    v = x.double() + (0 if parts == 0 else delta.double() if parts == 1 else delta.double().sum(0))
+    y, alone = x.clone(), x[2:3].clone()
+    out = ops.add_rmsnorm(y, delta, gain, 1e-5, bf)
+    close(y, v, torch.float32, "stream")
+    close(out, v * torch.rsqrt(v.pow(2).mean(1, keepdim=True) + 1e-5) * gain.double(), bf, "normed", bf16=4e-3)
+    one = None if parts == 0 else delta[2:3].contiguous() if parts == 1 else delta[:, 2:3].contiguous()
+    assert torch.equal(ops.add_rmsnorm(alone, one, gain, 1e-5, bf)[0], out[2]) and torch.equal(alone[0], y[2])
+
+
 @pytest.mark.parametrize("n,f,i", [(1, 8192, 2048), (8, 200, 512), (40, 128, 72), (64, 256, 1024), (64, 6200, 256),
                                    (36, 8192, 2048),                        # two tiles a workgroup
                                    (5, 4100, 104), (8, 52, 40), (11, 4090, 72), (14, 2200, 104), (9, 60, 136)])
