@@ -10,10 +10,12 @@
 // the weights of tile t, the scores of tile t + 1 and the values of tile t - 1, sixteen slices (head size 64) of one matrix instruction
 // with the vector instructions that fit its 32 cycles, the order pinned.  Left to the compiler each kind came in a block of its own, and three
 // waves a SIMD side by side did no better (16,384 rows of 32 heads: 1,373 us against 1,277).  Against 16 rows a wave, twice the products
-// per byte read from LDS; K and V go from memory to LDS without registers (global_load_lds), 16-byte chunks of a row swapped by its number so that
+// per byte read from LDS; K and V go from memory to LDS without registers (buffer_to_lds), 16-byte chunks of a row swapped by its number so that
 // no read has a bank conflict.  The longest workgroup's chain of tiles bounds short prompts, so workgroups are 32 rows rather than 64.
 // Measured, us a call, 32 heads of 64 in groups of 4, the kernel of 16 rows a wave and this one: 1,024 rows 30 and 19; 2,048 58 and 38; 4,096
-// 193 and 104; 16,384 1,764 and 1,280 (860 TFLOP/s); 3 x 700 rows 28 and 19, and 16 heads of 128 31 and 24.
+// 193 and 104; 16,384 1,764 and 1,280 (860 TFLOP/s); 3 x 700 rows 28 and 19, and 16 heads of 128 31 and 24.  With the loads to LDS as buffer loads,
+// beside which the compiler waits for the reads of LDS that a product needs and not for those of the next three: 2,048 rows 38.1 -> 36.7, 4,096
+// 107 -> 103, 16,384 1,253 -> 1,230.
 // Tiles in flight for longer (four of each in LDS): the same.
 #include "attention_prompt.h"
 
@@ -157,8 +159,7 @@ __global__ __launch_bounds__(64 * HW * RW) __attribute__((amdgpu_waves_per_eu(2)
       const bf16* at = pages + (size_t)page * page_stride + head_off + (size_t)((unsigned)(key & (a.page_size - 1)) / RPL * RPL * HD);
       const int chunk = lslot ^ (values ? value_swizzle<HD>(row + lrow) : key_swizzle<HD>(row + lrow));
       const unsigned lane_at = (unsigned)(lrow * HD + chunk * 8) * 2;
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)((const char*)at + lane_at),
-                                       (__attribute__((address_space(3))) void*)(dst + row * HD), 16, 0, 0);
+      buffer_to_lds(at, RPL * HD * 2, 0, lane_at, dst + row * HD);
     }
   };
   // values beyond the last key: whatever the page held there, a weight of zero must not meet a NaN
@@ -366,8 +367,7 @@ __global__ __launch_bounds__(64 * HW * RW) __attribute__((amdgpu_waves_per_eu(2)
         for (int i = 0; i < 16; ++i) o[t][i] *= keep;
     }
     // this wave's part of the next step's tiles has landed and its reads of LDS are through (the barrier covers the other waves')
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
+    barrier_behind_loads<0>();
   };
   if (kt_first == kt_last) {
     // one tile: nothing to run side by side (45 rows of 16 heads 5.9 us a call, through the steps below 6.8)

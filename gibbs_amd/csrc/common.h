@@ -82,6 +82,24 @@ __device__ __forceinline__ float wave_max(float v) {
   return wave_fold(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
+// 16 bytes a lane from memory to LDS without registers: from base + at (the same in all lanes) + lane_at, to lds + 16 x lane.  `bytes` from base are there;
+// beyond, zeros come.  A buffer load, not a global one: beside a global load to LDS the compiler waits for all LDS reads wherever it waits for one.
+__device__ __forceinline__ void buffer_to_lds(const void* base, uint32_t bytes, uint32_t at, uint32_t lane_at, void* lds) {
+#if defined(__HIP_DEVICE_COMPILE__)      // (the host's pass does not know the builtin)
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)bytes, 0x00020000),
+                                           (__attribute__((address_space(3))) void*)lds, 16, (int)lane_at, (int)at, 0, 0);
+#endif
+}
+// A barrier behind which the wave's LDS reads and all but the last LEFT of its loads are through.  Known to the compiler (waits in assembler are not, and it
+// waits once more), and without the wait for every load that __syncthreads() is.
+template <int LEFT>
+__device__ __forceinline__ void barrier_behind_loads() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((LEFT & 15) | LEFT >> 4 << 14 | 7 << 4);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // Sum over a block of up to 1024 threads; every thread gets the result.  `scratch` holds
 // one float per wave.  The order of additions is fixed by the thread layout alone.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {

@@ -768,13 +768,12 @@ int launch_tiled_as(const bf16* X, long ldx, int top, const int* sorted_pair, co
 // position c ^ ((r >> 1) & 7), so that the operand reads (32 rows x one chunk an instruction) are free of bank conflicts; the lane
 // that fills a position asks memory for the chunk that belongs there.  The product is computed transposed (features x places): a
 // lane's results are 4 neighbouring features of one place.
-// A tile of k takes 1.0 us where its matrix instructions take 0.45 and LDS accepts its 48 KB in 0.33: what is left is what
-// comes from behind the L2s, 24 KB of it at the 6.3 TB/s that all units get together.  8,412 pairs of 16 experts, width 2,048, 1,024
-// features: gated 114 us, down 76 (the kernel above 164 and 93); 16,384 pairs, width 4,096, 2,048 features 660 and 335 (799 and
-// 400; 830 TFLOP/s); 1,400 pairs of 8 experts, width 2,048, 512 features 41 and 20 (70 and 23).  Slower: a workgroup an item (122 us
-// in the first of these), tiles of 32 k with two workgroups a compute unit (133: requests of 64 bytes), 128 rows of W (148), and an
-// XCD's units on neighbouring items (129; 127 against 149 at a width of 2,112, but 750 against 654 at 4,096).
-constexpr int ASYNC_BK = 64, ASYNC_BN = 256, ASYNC_STAGES = 3, ASYNC_UNITS = 256;   // (units: one workgroup a compute unit)
+// A tile of k takes 1.0 us; alone its loads take 0.79, its matrix instructions 0.58 and its LDS reads 0.41 (128 bytes a cycle; products and reads together
+// 0.81), and neither the order of the items over the XCDs nor where in k an item begins changes that.  The loads are buffer loads: with global
+// ones the compiler waited for the reads of the next products in front of these (8,412 pairs of 16 experts, width 2,048, 1,024 features: gated
+// 104 us, down 60, now 101 and 58; 16,384 pairs, width 4,096, 2,048 features 575 and 312, now 553 and 300, 1.0 PFLOP/s; 1,400 pairs of 8 experts,
+// width 2,048, 512 features 30 and 14, now 28 and 13).  The kernel above takes 164 and 93, 799 and 400, 70 and 23.  Slower: a workgroup an item (122 us
+// where this took 114 in the first of these), tiles of 32 k with two workgroups a compute unit (133: requests of 64 bytes), and 128 rows of W (148).
 // v <- activate(w * v): the activation is chosen once, not for each of the 16
 __device__ __forceinline__ void activate_all(floatx16& v, float w, int act) {
   auto all = [&](auto f) {
@@ -800,27 +799,33 @@ __global__ __launch_bounds__(512) void moe_gemm_async_kernel(const bf16* __restr
   constexpr int A_ELEMS = TBM * BK, STAGE_ELEMS = (TBM + BN) * BK;
   extern __shared__ __attribute__((aligned(16))) char moe_lds[];
   bf16* tiles = (bf16*)moe_lds;                                            // [STAGES][places, then rows of W][BK]
-  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
   auto swz = [](int row) { return (row >> 1) & 7; };
   // An item is a tile of places and a block of columns; tiles without an expert stand behind all others.
   auto there = [&](int item) { return item < items && tile_expert[item / columns] >= 0; };
   // What this thread brings of an item's tile of k: chunk (tid % CPR) ^ swz(r) of row r = tid / CPR + i * THREADS / CPR.  A place
   // without a pair repeats row 0 and a row of W past the last one the last: their results are not stored.
-  const bf16 *from[LOADS], *from_next[LOADS];
-  auto rows_of = [&](int item, const bf16* (&f)[LOADS]) {
+  // (Bytes from X's, the tile's or the matrix's beginning.)
+  struct Source {
+    const bf16* x;
+    uint32_t at[LOADS];
+    int expert;
+  } from, from_next;
+  auto rows_of = [&](int item, Source& f) {
     const int tile = item / columns, col0 = item % columns * COLS;
-    const size_t e = tile_expert[tile];
+    f.expert = tile_expert[tile];
+    f.x = top > 0 ? X : X + (size_t)tile * TBM * ldx;
 #pragma unroll
     for (int i = 0; i < CA; ++i) {
       const int r = (tid + i * THREADS) / CPR, pair = sorted_pair[tile * TBM + r];
-      const int src = pair < 0 ? 0 : (top > 0 ? pair / top : tile * TBM + r);
-      f[i] = X + (size_t)src * ldx + ((tid % CPR) ^ swz(r)) * 8;
+      const int src = pair < 0 ? 0 : (top > 0 ? pair / top : r);
+      f.at[i] = ((uint32_t)src * (uint32_t)ldx + ((tid % CPR) ^ swz(r)) * 8) * 2;
     }
 #pragma unroll
     for (int i = 0; i < CW; ++i) {
       const int r = (tid + i * THREADS) / CPR;
       const int col = min(col0 + (GLU ? r % COLS : r), O - 1);
-      f[CA + i] = ((GLU && r >= COLS) ? Wb : Wa) + e * expert_stride + (size_t)col * I + ((tid % CPR) ^ swz(r)) * 8;
+      f.at[CA + i] = ((uint32_t)col * (uint32_t)I + ((tid % CPR) ^ swz(r)) * 8) * 2;
     }
   };
   int item = blockIdx.x;
@@ -828,14 +833,17 @@ __global__ __launch_bounds__(512) void moe_gemm_async_kernel(const bf16* __restr
   rows_of(item, from);
   const int n_tiles = I / BK;                                              // (at least two)
   // (W's rows follow the places in a stage, and the lanes' slots follow each other: load i fills chunks i * THREADS on)
-  auto load_one = [&](const bf16* at, int buf, int i) {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)at,
-                                     (__attribute__((address_space(3))) void*)(tiles + buf * STAGE_ELEMS + (wave * WAVE + i * THREADS) * 8), 16, 0, 0);
+  // (buffer loads: a scalar base and step along k and one 32-bit offset a lane, so no vector instructions for addresses; and the compiler counts LDS reads beside
+  // them, where beside the global ones it waits for all of them)
+  static_assert(COLS % (THREADS / CPR) == 0, "a load's rows belong to one matrix");
+  auto load_one = [&](const Source& f, int k, int buf, int i) {
+    const bf16* base = i < CA ? f.x : ((GLU && (i - CA) * (THREADS / CPR) >= COLS) ? Wb : Wa) + (size_t)f.expert * expert_stride;
+    buffer_to_lds(base, ~0u, k * 2, f.at[i], tiles + buf * STAGE_ELEMS + (wave * WAVE + i * THREADS) * 8);
   };
 #pragma unroll
   for (int t = 0; t < STAGES - 1; ++t)
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) load_one(from[i] + t * BK, t, i);
+    for (int i = 0; i < LOADS; ++i) load_one(from, t * BK, t, i);
   const int wr = (wave / WN) * 64, r32 = lane % 32, h = lane / 32;
   // the wave's blocks of 32 rows of W: neighbours, or the same features of gate (first half of its blocks) and up (second half)
   int wc[NB];
@@ -864,11 +872,9 @@ __global__ __launch_bounds__(512) void moe_gemm_async_kernel(const bf16* __restr
 #pragma unroll
         for (int m = 0; m < 2; ++m) acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[n], a[m], acc[n][m], 0, 0, 0);
     };
-    auto tile_of_k = [&](const bf16* const (&ahead)[LOADS], int k_ahead) {
-      // this thread's part of the tile has landed (the barrier covers the others'); the next tile's may be on their way.  The bare
-      // barrier: with a fence the compiler would wait for all of them.
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 2) * LOADS) : "memory");
-      __builtin_amdgcn_s_barrier();
+    auto tile_of_k = [&](const Source& ahead, int k_ahead) {
+      // this thread's part of the tile has landed (the barrier covers the others'); the next tile's may be on their way
+      barrier_behind_loads<(STAGES - 2) * LOADS>();
       const int fill = buf == 0 ? STAGES - 1 : buf - 1;  // the buffer of the tile before, which everyone has left
       const bf16* cA = tiles + buf * STAGE_ELEMS;
       const bf16* cW = cA + A_ELEMS;
@@ -890,7 +896,7 @@ __global__ __launch_bounds__(512) void moe_gemm_async_kernel(const bf16* __restr
         __builtin_amdgcn_sched_barrier(0);
         products(fa[now], fw[now]);
 #pragma unroll
-        for (int i = kk * LOADS / STEPS; i < (kk + 1) * LOADS / STEPS; ++i) load_one(ahead[i] + k_ahead, fill, i);
+        for (int i = kk * LOADS / STEPS; i < (kk + 1) * LOADS / STEPS; ++i) load_one(ahead, k_ahead, fill, i);
         __builtin_amdgcn_sched_barrier(0);
       }
       buf = buf == STAGES - 1 ? 0 : buf + 1;
@@ -931,8 +937,7 @@ __global__ __launch_bounds__(512) void moe_gemm_async_kernel(const bf16* __restr
     }
     if (!more) break;
     item = following;
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) from[i] = from_next[i];
+    from = from_next;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // nothing may still be writing LDS when the workgroup ends
 }
@@ -961,7 +966,9 @@ int launch_tiled(const bf16* X, long ldx, int top, const int* sorted_pair, const
   // 14.5 and 17.1, 256 19.3 and 21.5, 512 28.2 and 27.1; 2,048 features, 128 23.6 and 26.3).
   const long items = (long)ceil_div(O, GLU ? ASYNC_BN / 2 : ASYNC_BN) * tiles, last = items % ASYNC_UNITS;
   const bool idle = !GLU && I < 512 && items > ASYNC_UNITS && items <= 3 * ASYNC_UNITS && last > 0 && last <= ASYNC_UNITS * 5 / 8;
-  if (I % ASYNC_BK == 0 && I >= 2 * ASYNC_BK && !idle)
+  // (its loads have 32-bit offsets within X, the rows of a step, and within a matrix)
+  const bool near = (top > 0 ? (long)tiles * TBM / top + 1 : TBM) * ldx < (1L << 31) && (long)O * I < (1L << 31);
+  if (I % ASYNC_BK == 0 && I >= 2 * ASYNC_BK && !idle && near)
     return launch_async<GLU>(X, ldx, top, sorted_pair, tile_expert, tiles, wa, wb, stride, Y, ldy, O, I, act, in_weight, stream);
   // what is left: wide results with a long inner size 256 rows of W a workgroup and 8 waves (the tile of X is read by half as many
   // workgroups: 8,320 pairs, 2,048 features, inner size 2,056 gated 264 us, with 128 rows 306); otherwise 128 rows and 4 waves, which leaves
