@@ -762,7 +762,7 @@ int launch_tiled_as(const bf16* X, long ldx, int top, const int* sorted_pair, co
   return 0;
 }
 // Many pairs and whole tiles of k (an inner size that is a multiple of 64, two tiles or more): the same product with loads that go
-// from memory to LDS without passing through registers (global_load_lds, 16 bytes a lane), three tiles deep.  An item is 128 places
+// from memory to LDS without passing through registers (buffer_to_lds), three tiles deep.  An item is 128 places
 // x 256 rows of W, a wave of the 8 takes 64 x 64 of it; a compute unit has one workgroup, which goes on from item to item and has
 // the next one's first tiles under way while it finishes this one.  A tile in LDS is [row][64] with the 16-byte chunk c of row r at
 // position c ^ ((r >> 1) & 7), so that the operand reads (32 rows x one chunk an instruction) are free of bank conflicts; the lane
@@ -774,6 +774,8 @@ int launch_tiled_as(const bf16* X, long ldx, int top, const int* sorted_pair, co
 // 104 us, down 60, now 101 and 58; 16,384 pairs, width 4,096, 2,048 features 575 and 312, now 553 and 300, 1.0 PFLOP/s; 1,400 pairs of 8 experts,
 // width 2,048, 512 features 30 and 14, now 28 and 13).  The kernel above takes 164 and 93, 799 and 400, 70 and 23.  Slower: a workgroup an item (122 us
 // where this took 114 in the first of these), tiles of 32 k with two workgroups a compute unit (133: requests of 64 bytes), and 128 rows of W (148).
+constexpr int ASYNC_BK = 64, ASYNC_BN = 256, ASYNC_STAGES = 3, ASYNC_UNITS = 256;   // (units: one workgroup a compute unit)
+
 // v <- activate(w * v): the activation is chosen once, not for each of the 16
 __device__ __forceinline__ void activate_all(floatx16& v, float w, int act) {
   auto all = [&](auto f) {
