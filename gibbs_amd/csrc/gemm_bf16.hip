@@ -7,7 +7,7 @@
 // staged through LDS (rows padded by 16 bytes against bank conflicts), double-buffered so that
 // the next tile's global loads are in flight while the matrix cores work on the current one.
 // Rows beyond N or O and k beyond I are read as zero.  I and the row strides must be multiples
-// of 8 elements (16-byte loads).  Large aligned shapes take a 256 x 256 kernel (below).
+// of 8 elements (16-byte loads).  Large aligned shapes take a 256 x 256 kernel, at most 64 rows one of 64 x 128 (below).
 #include "common.h"
 
 namespace {
@@ -226,7 +226,102 @@ int launch_256(const bf16* A, const bf16* W, OutT* C, int N, int O, int I, long 
   GIBBS_LAUNCH_STATUS("gemm_bf16");
 }
 
-// Large aligned shapes that fill the chip with 256 x 256 tiles take the kernel above.
+// The same product for at most 64 rows (I a multiple of 64, 128 at least), whose time is that of reading W once: a workgroup of 4 waves takes 64 rows x 128
+// features, each wave 32 of the features, two workgroups a compute unit.  Tiles of 64 k go from memory to LDS without registers, three deep, so that
+// 72 KB a compute unit are on their way; the 128 x 128 kernel has the next tile alone in flight, and half of its rows are none here.  Tiles in LDS
+// and results lie as in the 256 x 256 kernel.  Rows beyond N and features beyond O repeat the last: their results are not stored.
+// Measured, us, 128 x 128 and this: 64 rows, 65,536 features, inner size 2,048 71.6 and 59.1 (64.7 with all from k 0), 1,024 33.9 and 30.2; 2,048 features
+// 30.2 and 14.2; 512 of inner size 1,024 17.1 and 8.4.
+constexpr int FEW_ROWS = 64, FEW_FEATURES = 128, FEW_STAGES = 3;
+template <typename OutT>
+__global__ __launch_bounds__(256) void gemm_bf16_few_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W, OutT* __restrict__ C, int N, int O, int I,
+                                                            long lda, long ldw, long ldc, int wide) {
+  constexpr int THREADS = 256, ROWS = THREADS / 8, CA = FEW_ROWS / ROWS, CW = FEW_FEATURES / ROWS, LOADS = CA + CW, STAGE = (FEW_ROWS + FEW_FEATURES) * TK;
+  extern __shared__ __attribute__((aligned(16))) bf16 few_tiles[];      // [FEW_STAGES][rows of A, then of W][TK]
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE, r32 = lane % 32, h = lane / 32;
+  const int col0 = blockIdx.x * FEW_FEATURES, nt = I / TK;
+  const bf16* w = W + (size_t)col0 * ldw;
+  uint32_t from[LOADS];      // bytes from A's beginning, or the first feature's
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int r = tid / 8 + i * ROWS, c = (tid % 8) ^ ((r >> 1) & 7);
+    from[i] = i < CA ? ((uint32_t)min(r, N - 1) * (uint32_t)lda + c * 8) * 2 : ((uint32_t)min(r - FEW_ROWS, O - 1 - col0) * (uint32_t)ldw + c * 8) * 2;
+  }
+  // The workgroups begin at different k: rows of 4 KB, all read at one k at a time, are a few of the memory's channels.
+  const int turn = blockIdx.x % nt;
+  auto bring = [&](int t, int buf, int i) {      // (a tile beyond the last: the last once more)
+    const int at = min(t, nt - 1) + turn;
+    buffer_to_lds(i < CA ? A : w, ~0u, (at < nt ? at : at - nt) * TK * 2, from[i], few_tiles + buf * STAGE + (wave * WAVE + i * THREADS) * 8);
+  };
+#pragma unroll
+  for (int t = 0; t < FEW_STAGES - 1; ++t)
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) bring(t, t, i);
+  floatx16 acc[2];      // [block of 32 rows]
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[m][i] = 0.f;
+  int buf = 0;
+  for (int t = 0; t < nt; ++t) {
+    barrier_behind_loads<(FEW_STAGES - 2) * LOADS>();
+    const int fill = buf == 0 ? FEW_STAGES - 1 : buf - 1;      // the buffer of the tile before, which everyone has left
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) bring(t + FEW_STAGES - 1, fill, i);
+    const bf16* cA = few_tiles + buf * STAGE;
+    const bf16* cW = cA + FEW_ROWS * TK;
+#pragma unroll
+    for (int kk = 0; kk < TK / 16; ++kk) {
+      const int chunk = kk * 2 + h;
+      const bf16x8 fw = *(const bf16x8*)(cW + swizzled(wave * 32 + r32, chunk));
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        const bf16x8 fa = *(const bf16x8*)(cA + swizzled(m * 32 + r32, chunk));
+        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw, fa, acc[m], 0, 0, 0);
+      }
+    }
+    buf = buf == FEW_STAGES - 1 ? 0 : buf + 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // nothing may still be writing LDS when the workgroup ends
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const int row = m * 32 + r32;
+    if (row >= N) continue;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int col = col0 + wave * 32 + q * 8 + h * 4;
+      OutT* out = C + (size_t)row * ldc + col;
+      typedef OutT out4 __attribute__((ext_vector_type(4)));
+      if (wide && col < O) {
+        out4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = from_float<OutT>(acc[m][q * 4 + e]);
+        *(out4*)out = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (col + e < O) out[e] = from_float<OutT>(acc[m][q * 4 + e]);
+      }
+    }
+  }
+}
+template <typename OutT>
+int launch_few(const bf16* A, const bf16* W, OutT* C, int N, int O, int I, long lda, long ldw, long ldc, hipStream_t stream) {
+  constexpr int LDS_BYTES = FEW_STAGES * (FEW_ROWS + FEW_FEATURES) * TK * (int)sizeof(bf16);
+  static bool prepared = false;    // (per output type: the template makes one flag each)
+  if (!prepared) {
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_bf16_few_kernel<OutT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
+    if (e != hipSuccess) return gibbs_fail("gemm_bf16: %s", hipGetErrorString(e));
+    prepared = true;
+  }
+  const int wide = O % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % (4 * sizeof(OutT)) == 0;
+  gemm_bf16_few_kernel<OutT><<<ceil_div(O, FEW_FEATURES), 256, LDS_BYTES, stream>>>(A, W, C, N, O, I, lda, ldw, ldc, wide);
+  GIBBS_LAUNCH_STATUS("gemm_bf16");
+}
+// (offsets of 32 bits within 64 rows of A and 128 of W)
+bool takes_few(int N, int I, long lda, long ldw) { return N <= FEW_ROWS && I % TK == 0 && I >= 2 * TK && lda < (1L << 24) && ldw < (1L << 24); }
+
+// Large aligned shapes that fill the chip with 256 x 256 tiles take their kernel.
 bool takes_256(int N, int O, int I, long ldc) {
   return N % TM == 0 && O % TN == 0 && I % TK == 0 && ldc % 4 == 0 && (long)(N / TM) * (O / TN) >= 192;
 }
@@ -243,6 +338,10 @@ GIBBS_EXPORT int gibbs_gemm_bf16(const void* A, const void* W, void* C, int out_
   if (takes_256(N, O, I, ldc)) {
     if (out_dtype == GIBBS_BF16) return launch_256((const bf16*)A, (const bf16*)W, (bf16*)C, N, O, I, lda, ldw, ldc, stream);
     if (out_dtype == GIBBS_F32) return launch_256((const bf16*)A, (const bf16*)W, (float*)C, N, O, I, lda, ldw, ldc, stream);
+  }
+  if (takes_few(N, I, lda, ldw)) {
+    if (out_dtype == GIBBS_BF16) return launch_few((const bf16*)A, (const bf16*)W, (bf16*)C, N, O, I, lda, ldw, ldc, stream);
+    if (out_dtype == GIBBS_F32) return launch_few((const bf16*)A, (const bf16*)W, (float*)C, N, O, I, lda, ldw, ldc, stream);
   }
   dim3 grid(ceil_div(O, BN), ceil_div(N, BM));
   GIBBS_REQUIRE(grid.y <= 65535, "gemm_bf16: too many rows (%d)", N);

@@ -1128,6 +1128,22 @@ def test_add_rmsnorm_of_rows_two_threads_share(hidden, parts):
     assert torch.equal(ops.add_rmsnorm(alone, one, gain, 1e-5, bf)[0], out[2]) and torch.equal(alone[0], y[2])
 
 
+@pytest.mark.parametrize("n,o,i", [(1, 1, 128), (31, 129, 192), (33, 127, 128), (64, 4100, 2048), (49, 130, 320), (64, 128, 4160)])
+@pytest.mark.parametrize("out_dtype", DT)
+def test_gemm_bf16_of_few_rows(n, o, i, out_dtype):
+    """Around the edges of 32 and 64 rows and of 128 features, two tiles of k and many, rows of the results that are no whole 16 bytes, and nothing
+    written beside them."""
+    from gibbs_amd import ops
+    x, w = rnd(n, i, dtype=torch.bfloat16), rnd(o, i, dtype=torch.bfloat16, seed=1)
+    room = torch.full((n + 1, o + 3), 77, dtype=out_dtype, device=DEV)
+    got = ops.gemm_bf16(x, w, out_dtype, out=room[:n, :o])
+    close(got, x.double() @ w.double().t(), out_dtype, "few rows", f32=2e-5, bf16=4e-3)
+    assert (room[n] == 77).all() and (room[:, o:] == 77).all()
+    whole = ops.gemm_bf16(x, w, out_dtype)
+    assert torch.equal(whole, got)
+    assert torch.equal(ops.gemm_bf16(x[:1].contiguous(), w, out_dtype)[0], whole[0])
+
+
 @pytest.mark.parametrize("n,f,i", [(1, 8192, 2048), (8, 200, 512), (40, 128, 72), (64, 256, 1024), (64, 6200, 256),
                                    (36, 8192, 2048),                        # two tiles a workgroup
                                    (5, 4100, 104), (8, 52, 40), (11, 4090, 72), (14, 2200, 104), (9, 60, 136)])
