@@ -105,12 +105,14 @@ int prefill_splits(long n_tiles, int nh, int max_seq, int window) {
 // least 512 keys to a slice on average, as a slice more costs every row its partial result and the merge's kernel.  Measured, us a call in
 // 1 / 2 / 4 / 8 slices, 32 heads of 64 in groups of 4: 512 rows behind 1,536 keys (128 workgroups) 31 / 31 / 28 / 36; behind 7,680 - / 84 / 57 / 64;
 // 128 rows behind 1,000 20 / 17 / 17; 1,024 rows behind none (256 workgroups) 19 / 30; 512 behind none 13 / 18 / 20.
+// Up to 64 workgroups, where the chain of tiles is all there is to wait for, at least 256 keys: 79 rows of 16 heads behind 621 keys 14.5 -> 11.9 us, 128 rows of
+// 32 heads behind 1,000 16.5 -> 13.2, 40 rows and one behind 900 17.1 -> 11.3, 64 rows of 16 heads of 128 behind 700 22.9 -> 17.6.
 int prompt_splits(int rows, int reqs, int nh, int nkv, int max_seq, int window) {
   const int group = nh / std::max(nkv, 1), heads = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1), tile = 128 / heads;
   const long blocks = std::max<long>(1, (ceil_div_l(rows, tile) + reqs / 2) * (nh / heads));
   long seen = max_seq - rows / (2 * std::max(reqs, 1));
   if (window > 0) seen = std::min<long>(seen, window);
-  return (int)std::max<long>(1, std::min<long>(std::min<long>((512 + blocks / 2) / blocks, seen / 512), 16));
+  return (int)std::max<long>(1, std::min<long>(std::min<long>((512 + blocks / 2) / blocks, seen / (blocks <= 64 ? 256 : 512)), 16));
 }
 
 // Query heads of a kv head's group that a workgroup of the prompt attention takes (they share its K and V
