@@ -420,6 +420,54 @@ __global__ __launch_bounds__(64 * HW * RW) __attribute__((amdgpu_waves_per_eu(2)
     }
   }
 
+  // A weight of zero makes a value that is not finite a NaN, in rows of the wave that do not see its key too.  Rows that come out
+  // so are taken again, a row at a time over its own keys: scores with a key a lane, sums with a place or two of the head a lane.
+  // (The look at the results, us: 2,048 rows of 32 heads of 64 36.0 -> 36.2, calls of 5 us 0.1 more.)
+  float probe = 0.f;
+#pragma unroll
+  for (int t = 0; t < ND; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) probe = fmaf(o[t][i], 0.f, probe);
+  const uint64_t spoilt = __builtin_amdgcn_ballot_w64(row0 + lr < rows_here && !(probe == 0.f) && l < INFINITY);   // (a sum that is none: every place is)
+  if (__builtin_expect(spoilt != 0, 0)) {
+    auto offset_of = [&](int key) {
+      const int page = table[key >> a.page_shift];
+      return (size_t)min(max(page, 0), a.num_pages - 1) * page_stride + head_off + (size_t)(key & (a.page_size - 1)) * HD;
+    };
+#pragma unroll 1
+    for (uint32_t rows = (uint32_t)spoilt | (uint32_t)(spoilt >> 32); rows != 0; rows &= rows - 1) {
+      const int n = __builtin_ctz(rows), upto = __builtin_amdgcn_readlane(pos_row, n), from = __builtin_amdgcn_readlane(lo_row, n);
+      const float shift = -__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(m), n)) * scale2;
+      const bf16* qr = q + (size_t)(n0 + row0 + n) * a.ldq + (size_t)head * HD;
+      float sum[HD / WAVE] = {};
+#pragma unroll 1
+      for (int key0 = max(kt_first, (from + 1) / BN) * BN; key0 <= min(upto, kt_stop * BN - 1); key0 += BN) {
+        const int key = min(key0 + lane, last_pos);
+        const bf16* kr = kpages + offset_of(key);
+        float s = 0.f;
+#pragma unroll 1
+        for (int d = 0; d < HD; ++d) s = fmaf(to_float(kr[d]), to_float(qr[d]), s);
+        if constexpr (CAP) s = cap_raw * tanhf(s * cap_inv);
+        if (biased) s += a.bias[(size_t)head * a.bias_len + min(max(upto - key, 0), a.bias_len - 1)];
+        const float p = to_float((bf16)__builtin_amdgcn_exp2f(fmaf(s, scale2, shift)));
+#pragma unroll 1
+        for (int j = max(0, from + 1 - key0); j < BN && key0 + j <= upto; ++j) {
+          const bf16* vr = vpages + offset_of(key0 + j);
+          const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(p), j));
+#pragma unroll
+          for (int t = 0; t < HD / WAVE; ++t) sum[t] = fmaf(w, to_float(vr[t * WAVE + lane]), sum[t]);
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < ND; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const float v = __shfl(sum[t * 32 / WAVE], (t * 32 + (i / 4) * 8 + h * 4 + i % 4) % WAVE, WAVE);
+          if (lr == n) o[t][i] = v;
+        }
+    }
+  }
+
   l = halves_sum(l);
   const int row = row0 + lr;
   if (row >= rows_here) return;

@@ -713,6 +713,44 @@ def test_attention_prompt_edges(nh, nkv, hd, page, how):
     close(out, plain, torch.bfloat16, "prompt attention", bf16=1e-2)
 
 
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("nh,nkv,hd,page,how", [
+    (4, 1, 64, 16, {}), (4, 2, 64, 8, {"window": 40}), (3, 3, 64, 16, {}), (2, 2, 64, 32, {"chunk": 90}), (4, 1, 128, 16, {"window": 70}),
+    (3, 3, 128, 8, {"softcap": 4.0}), (2, 1, 128, 16, {})])
+def test_attention_prompt_values_that_are_not_finite(nh, nkv, hd, page, how, splits):
+    """A value that is not finite reaches the rows that see its key and no other, whatever rows a wave and a workgroup have: in one tile and
+    in several, on and beside the diagonal, behind rows that no longer see it.  The rest is what it is without those values."""
+    from gibbs_amd import ops
+    q_lens, ctx = [64, 150, 300], [0, 70, 3]
+    seq_lens = [a + b for a, b in zip(q_lens, ctx)]
+    cu = np.concatenate([[0], np.cumsum(q_lens)])
+    n, scale, window, chunk = int(cu[-1]), 1 / math.sqrt(hd), how.get("window"), how.get("chunk", 0)
+    kp, vp, table, _, _ = paged_setup(torch.bfloat16, nkv, hd, page, seq_lens, sum(-(-s // page) for s in seq_lens), seed=3)
+    q = rnd(n, nh * hd, dtype=torch.bfloat16, seed=4)
+    pos = i32([c + t for c, m in zip(ctx, q_lens) for t in range(m)])
+    row_req = i32([r for r, m in enumerate(q_lens) for _ in range(m)])
+
+    def run():
+        return ops.attention_prefill(q, n, nh, nkv, hd, kp, vp, table, 3, i32(cu), i32(ctx), scale, window, chunk=chunk, n_splits=splits,
+                                     softcap=how.get("softcap", 0.0), heads_per_wg=0).view(n, nh, hd)
+    clean = run()
+    seen = torch.zeros(n, nh, hd, dtype=torch.bool, device=DEV)
+    for r, key, kvh, d, bad in ((0, 63, 0, 5, math.nan), (1, 100, nkv - 1, hd - 1, math.inf), (1, 219, 0, 33, math.nan), (2, 17, 0, 8, -math.inf),
+                                (2, 130, nkv - 1, 0, math.nan), (2, 302, 0, 31, math.inf)):
+        vp[table[r, key // page].item(), kvh, key % page, d] = bad
+        sees = (row_req == r) & (pos >= key)
+        if window:
+            sees &= pos - key < window
+        if chunk:
+            sees &= pos // chunk == key // chunk
+        heads = slice(kvh * (nh // nkv), (kvh + 1) * (nh // nkv))
+        seen[:, heads, d] |= sees[:, None]
+    got = run()
+    assert torch.equal(~got.isfinite(), seen)
+    # (rows that are taken again: other roundings of float32 sums, and a weight's bfloat16 may round the other way)
+    close(got[~seen], clean[~seen], torch.bfloat16, "beside values that are not finite", bf16=4e-3)
+
+
 def test_prefill_splits_choice():
     from gibbs_amd.ops import prefill_splits
     assert prefill_splits(32, 32, 2048) == 1                 # a whole 2,048-token prompt fills the chip
