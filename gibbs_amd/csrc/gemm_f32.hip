@@ -448,9 +448,10 @@ bool launch_f32(const float* A, const float* W, float* C, int N, int O, int I, l
 }
 }  // namespace
 
-// Bytes of workspace that gibbs_gemm_f32_in can use (0: none).  The results are the same to the bit with and without.
+// Bytes of workspace that gibbs_gemm_f32_in can use (0: none; rows that are no whole 16 bytes take the plain kernel).  The results are the same to
+// the bit with and without.
 GIBBS_EXPORT long gibbs_gemm_f32_workspace(int N, int O, int I) {
-  if (N <= 0 || O <= 0 || I <= 0) return 0;
+  if (N <= 0 || O <= 0 || I <= 0 || I % 4) return 0;
   const SharedShape s = shared_shape(N, O, I);
   return shares(s, N, O, I) ? (long)(shared_sums_bytes(s) + shared_marks_bytes(s)) : 0;
 }

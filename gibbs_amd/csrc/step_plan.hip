@@ -466,7 +466,7 @@ void* Exec::linear(const void* x, const Matrix& m, int n, bool out_f32, bool par
   return y;
 }
 void Exec::run_product(const LinearChoice& c, const void* x, long ldx, const Matrix& m, bool use_packed, void* y, int n, bool out_f32) {
-  const long bytes = c.kernel == LIN_F32 ? gibbs_gemm_f32_workspace(n, m.O, m.I) : 0;
+  const long bytes = c.kernel == LIN_F32 && ldx % 4 == 0 ? gibbs_gemm_f32_workspace(n, m.O, m.I) : 0;
   if (bytes == 0) {
     RUN(*this, run_linear(c, x, ldx, m, use_packed, y, n, out_f32, a.stream));
     return;
