@@ -362,11 +362,13 @@ void launch_tile(const float* A, const float* W, float* C, int N, int O, int I, 
   const int row_tiles = ceil_div(N, 16 * FN * WN), tiles = row_tiles * ceil_div(O, 16 * FO * WO);
   gemm_f32_tile_kernel<WO, WN, FO, FN, OCC><<<(tiles + 7) / 8 * 8, 64 * WO * WN, 0, stream>>>(A, W, C, N, O, I, lda, ldw, ldc, row_tiles, tiles, wide, SharedSums{});
 }
-// Tiles of 128 features x 64 rows whose stretches workgroups share: 31 us a tile at an inner size of 1,024 as without, and SHARED_JOIN us for the
-// sums' way through memory and the second kernel, whatever the inner size.  (us, without / with, 1,024 features: inner size 4,608 150 rows 36.3 / 37.3, 333
-// 69 / 40, 700 102 / 61, 1,194 128 / 98; 4,096 700 rows 92 / 57; 1,024 333 rows 20.2 / 20.0, 1,194 34.5 / 36.0, 700 rows of 2,048 features 33.4 / 36.9.)
+// Tiles of 128 features x 64 rows whose stretches workgroups share: 31 us a tile at an inner size of 1,024 as without, and for the second kernel and the
+// sums' way through memory 12 us or, of many tiles, 9 and a sixteenth a tile, whatever the inner size.  (us, without / with, 1,024 features: inner size 4,608
+// 150 rows 36.3 / 37.3, 333 69 / 40, 700 102 / 61, 1,194 128 / 98, 1,600 119.1 / 116.5; 4,096 700 rows 92 / 57; 3,072 1,600 rows 82.2 / 84.1; 2,048 1,500 rows
+// 58.0 / 55.9, 1,700 59.0 / 64.6; 1,024 333 rows 20.2 / 20.0, 1,194 34.5 / 36.0, 700 rows of 2,048 features 33.4 / 36.9; 4,096 features of inner size 2,048
+// 333 rows 61.1 / 58.9, 400 61.5 / 67.4, of 4,096 400 rows 110.7 / 110.9.)
 constexpr int SHARED_FEATURES = 128, SHARED_ROWS = 64, SHARED_TILES = 256;
-constexpr float SHARED_TILE = 31.f, SHARED_JOIN = 12.f;
+constexpr float SHARED_TILE = 31.f;
 struct SharedShape {
   int tiles, stretches, run, groups;
   float cost;      // as the variants' below; 0: does not take the shape
@@ -378,7 +380,8 @@ SharedShape shared_shape(int N, int O, int I) {
   if (tiles > SHARED_TILES || I < 2048) return s;      // (256 tiles' sums are 64 MB)
   s.run = std::max(2, (int)ceil_div(tiles * stretches, 256));
   s.groups = ceil_div(tiles * stretches, s.run);
-  if (s.run < stretches) s.cost = SHARED_TILE * s.run / stretches + SHARED_JOIN * 1024.f / I;
+  const float join = fmaxf(12.f, 9.f + tiles / 16.f);
+  if (s.run < stretches) s.cost = SHARED_TILE * s.run / stretches + join * 1024.f / I;
   return s;
 }
 size_t shared_sums_bytes(const SharedShape& s) { return (size_t)s.tiles * s.stretches * SHARED_FEATURES * SHARED_ROWS * 4; }
