@@ -68,15 +68,12 @@ __device__ __forceinline__ void store4(bf16* p, float4 v) {
 // is float32 partial sums, `apart` values from one to the next, added in ascending order (8 rows of 2,048, two parts: 8.2 us with a value
 // at a time and a second pass, 4.7 here).
 // What bounds it: a trip to memory in front of the sum and the stores behind it while rows are few, the rate of a copy from a few thousand on.
-// So everything is asked for at once, the gains too (behind the sum they were one more trip), and nothing is stored before the sum.
-// TWO: a thread has the elements of two of twice as many threads and keeps their sums apart, so that the sum is the same to the bit as with 512
-// threads; rows of 2,048 with 256 threads, us: 544 rows 4.6 -> 4.2, 1,024 6.4 -> 5.7, 2,048 10.2 -> 8.9, 4,096 17.3 -> 16.1 (512 threads
-// and the rest as here 4.2, 5.8, 9.4, 16.5), 45 rows 2.3 both.
-template <typename T, int CHUNKS, bool TWO, typename D = T>
+// EARLY: everything is asked for at once, the gains too (behind the sum they are one more trip), and nothing is stored before the sum.  Which
+// of the two a call takes: launch_vec.
+template <typename T, int CHUNKS, bool EARLY, typename D = T>
 __global__ void add_rmsnorm_vec_kernel(float* __restrict__ x, const D* __restrict__ delta,
                                        const float* __restrict__ gain, float eps, T* __restrict__ out,
                                        const int* __restrict__ rows, int hidden, int write_x, int parts = 0, long apart = 0, bf16* __restrict__ mirror = nullptr) {
-  constexpr bool EARLY = CHUNKS <= 4;      // (more are registers that cost more than the trip)
   __shared__ float scratch[16];
   const int m = blockIdx.x;
   const int r = rows ? rows[m] : m;
@@ -84,68 +81,81 @@ __global__ void add_rmsnorm_vec_kernel(float* __restrict__ x, const D* __restric
   const D* dr = delta ? delta + (size_t)r * hidden : nullptr;
   auto at = [&](int c) { return (int)(c * blockDim.x + threadIdx.x) * 4; };
   auto gains = [&](int i) { return gain ? *(const float4*)(gain + i) : make_float4(1.f, 1.f, 1.f, 1.f); };
-  float4 v[CHUNKS], d[CHUNKS], g[EARLY ? CHUNKS : 1];
+  // (which of the squares is rounded before the others are added is stated, so that both kinds have the same sum)
+  auto squares = [](float4 v) {
+    const float two = std::is_same_v<D, float> && CHUNKS == 1 ? fmaf(v.y, v.y, v.x * v.x) : fmaf(v.x, v.x, v.y * v.y);
+    return fmaf(v.w, v.w, fmaf(v.z, v.z, two));
+  };
+  float4 v[CHUNKS], g[CHUNKS];
+  float ss = 0.f;
+  if constexpr (EARLY) {
+    float4 d[CHUNKS];
 #pragma unroll
-  for (int c = 0; c < CHUNKS; ++c) {
-    const int i = min(at(c), hidden - 4);
-    v[c] = *(const float4*)(xr + i);
-    if (dr) d[c] = load4(dr + i);
-    if (EARLY) g[c] = gains(i);
-  }
-  float ss[2] = {0.f, 0.f};
+    for (int c = 0; c < CHUNKS; ++c) {
+      const int i = min(at(c), hidden - 4);
+      v[c] = *(const float4*)(xr + i);
+      d[c] = load4(dr + i);
+      g[c] = gains(i);
+    }
 #pragma unroll
-  for (int c = 0; c < CHUNKS; ++c) {
-    if (dr) {
+    for (int c = 0; c < CHUNKS; ++c) {
       add_parts4(d[c], dr + min(at(c), hidden - 4), 1, parts, apart);
       v[c].x += d[c].x; v[c].y += d[c].y; v[c].z += d[c].z; v[c].w += d[c].w;
+      if (at(c) < hidden) ss += squares(v[c]);
     }
-    // (which of the squares is rounded before the others are added is stated, so that the sum is what it was: the first where one float32 delta's
-    // elements are four a thread of 512, the second elsewhere)
-    const float two = std::is_same_v<D, float> && CHUNKS == (TWO ? 2 : 1) ? fmaf(v[c].y, v[c].y, v[c].x * v[c].x) : fmaf(v[c].x, v[c].x, v[c].y * v[c].y);
-    if (at(c) < hidden) ss[TWO ? c % 2 : 0] += fmaf(v[c].w, v[c].w, fmaf(v[c].z, v[c].z, two));
-  }
-  float sum;
-  if constexpr (TWO) {      // (of 256 threads: 8 sums, those of the first halves in front)
-    const float first = wave_sum(ss[0]), second = wave_sum(ss[1]);
-    const int wave = threadIdx.x / WAVE;
-    if (threadIdx.x % WAVE == 0) {
-      scratch[wave] = first;
-      scratch[4 + wave] = second;
-    }
-    __syncthreads();
-    sum = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) sum += scratch[i];
   } else {
-    sum = block_sum(ss[0], scratch);
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      const int i = at(c);
+      v[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (i < hidden) {
+        v[c] = *(const float4*)(xr + i);
+        if (dr) {
+          float4 d = load4(dr + i);
+          add_parts4(d, dr + i, 1, parts, apart);
+          v[c].x += d.x; v[c].y += d.y; v[c].z += d.z; v[c].w += d.w;
+          if (write_x) *(float4*)(xr + i) = v[c];
+        }
+        if (mirror) store4(mirror + (size_t)r * hidden + i, v[c]);
+        ss += squares(v[c]);
+      }
+    }
   }
-  const float scale = 1.0f / sqrtf(sum / (float)hidden + eps);
+  ss = block_sum(ss, scratch);
+  const float scale = 1.0f / sqrtf(ss / (float)hidden + eps);
   T* o = out + (size_t)m * hidden;
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
     const int i = at(c);
     if (i < hidden) {
-      if (dr && write_x) *(float4*)(xr + i) = v[c];
-      if (mirror) store4(mirror + (size_t)r * hidden + i, v[c]);
-      const float4 f = EARLY ? g[EARLY ? c : 0] : gains(i);
-      store4(o + i, make_float4(v[c].x * scale * f.x, v[c].y * scale * f.y, v[c].z * scale * f.z, v[c].w * scale * f.w));
+      if constexpr (EARLY) {
+        if (write_x) *(float4*)(xr + i) = v[c];
+        if (mirror) store4(mirror + (size_t)r * hidden + i, v[c]);
+      } else {
+        g[c] = gains(i);
+      }
+      store4(o + i, make_float4(v[c].x * scale * g[c].x, v[c].y * scale * g[c].y, v[c].z * scale * g[c].z, v[c].w * scale * g[c].w));
     }
   }
 }
 
+// Asking for everything at once pays where there is a delta to wait for beside the stream and few registers to hold it in: whole threads of
+// four elements, or up to two such chunks of partial sums.  us, otherwise / at once, behind other kernels: with a bfloat16 delta 544 rows of 2,048 4.94 /
+// 4.64, 2,048 13.31 / 12.52, 45 3.04 / 2.97, 2,048 of 1,024 6.98 / 6.62; two partial sums, 45 rows of 2,048 3.60 / 3.35, of 4,096 4.62 / 4.08.  Where it
+// does not: no delta, 1,024 rows of 2,048 4.54 / 4.63; half of the threads' elements, 45 rows of 512 2.77 / 2.90; two chunks, 544 rows of 3,072
+// 6.19 / 6.40, and as partial sums 10.2 / 10.7; three, 544 of 5,120 10.56 / 13.48.  (A row of 2,048 in 256 threads instead of 512: 544 rows 5.11, 45 3.55.)
 template <typename T, typename D = T>
 bool launch_vec(float* x, const D* delta, const float* gain, float eps, T* out, const int* rows, int n_out, int hidden,
                 int write_x, hipStream_t stream, int parts = 0, long apart = 0, bf16* mirror = nullptr) {
   if (hidden % 4 || ((uintptr_t)x % 16) || (gain && ((uintptr_t)gain % 16)) || ((uintptr_t)out % (4 * sizeof(T))) ||
       (delta && ((uintptr_t)delta % (4 * sizeof(D)))) || apart % 4 || ((uintptr_t)mirror % 8))
     return false;
-  const bool two = hidden >= 2048 && hidden <= 4096;
-  const int threads = hidden >= 2048 && !two ? 512 : (hidden >= 512 ? 256 : 64);
+  const int threads = hidden >= 2048 ? 512 : (hidden >= 512 ? 256 : 64);
   const int chunks = ceil_div(hidden, 4 * threads);
-#define ADD_RMSNORM(C, TWO) add_rmsnorm_vec_kernel<T, C, TWO, D><<<n_out, threads, 0, stream>>>(x, delta, gain, eps, out, rows, hidden, write_x, parts, apart, mirror)
-  if (two && chunks == 2) ADD_RMSNORM(2, true);
-  else if (two) ADD_RMSNORM(4, true);
+#define ADD_RMSNORM(C, EARLY) add_rmsnorm_vec_kernel<T, C, EARLY, D><<<n_out, threads, 0, stream>>>(x, delta, gain, eps, out, rows, hidden, write_x, parts, apart, mirror)
+  if (delta && chunks == 1 && (parts >= 2 || hidden == 4 * threads)) ADD_RMSNORM(1, true);
   else if (chunks == 1) ADD_RMSNORM(1, false);
+  else if (delta && chunks == 2 && parts >= 2 && n_out <= 512) ADD_RMSNORM(2, true);
   else if (chunks == 2) ADD_RMSNORM(2, false);
   else if (chunks <= 4) ADD_RMSNORM(4, false);
   else if (chunks <= 8) ADD_RMSNORM(8, false);

@@ -1149,14 +1149,16 @@ def test_gates_of_every_size(f, clamped):
         assert torch.equal(run(gu[r:r + 1].contiguous())[0], out[r])
 
 
-@pytest.mark.parametrize("hidden", [2044, 2052, 3072, 4096, 4100])
+@pytest.mark.parametrize("hidden", [512, 1020, 1024, 1028, 2044, 2048, 2052, 3072, 4096, 4100])
 @pytest.mark.parametrize("parts", [0, 1, 3])
-def test_add_rmsnorm_of_rows_two_threads_share(hidden, parts):
-    """Around the widths whose rows 256 threads take twice: the stream, the normed rows and their bits in other company, against float64."""
+@pytest.mark.parametrize("n", [5, 520])
+def test_add_rmsnorm_whether_or_not_everything_is_asked_for_at_once(n, hidden, parts):
+    """Around the widths that are whole threads of four elements, and the rows up to which two chunks of partial sums are asked for at once:
+    the stream, the normed rows and their bits in other company, against float64."""
     from gibbs_amd import ops
     bf = torch.bfloat16
-    x, gain = rnd(5, hidden, scale=2.0), 1 + 0.1 * rnd(hidden, seed=2)
-    delta = None if parts == 0 else (rnd(5, hidden, dtype=bf, seed=3) if parts == 1 else rnd(parts, 5, hidden, seed=3))
+    x, gain = rnd(n, hidden, scale=2.0), 1 + 0.1 * rnd(hidden, seed=2)
+    delta = None if parts == 0 else (rnd(n, hidden, dtype=bf, seed=3) if parts == 1 else rnd(parts, n, hidden, seed=3))
     v = x.double() + (0 if parts == 0 else delta.double() if parts == 1 else delta.double().sum(0))
     y, alone = x.clone(), x[2:3].clone()
     out = ops.add_rmsnorm(y, delta, gain, 1e-5, bf)
