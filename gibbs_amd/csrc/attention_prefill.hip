@@ -415,16 +415,10 @@ template <int DT, int HPW>
 void launch_prefill_heads(dim3 grid, hipStream_t stream, const bf16* q, const bf16* k, const bf16* v, bf16* out, float* partial,
                           const PrefillArgs& a) {
   grid.y = a.nh / HPW;
-  // (head sizes 64 and 128 come here with pages of other sizes only)
 #define PREFILL(SCORES)                                                                                                              \
   do {                                                                                                                               \
-    if constexpr (DT != 4 && DT != 8) {                                                                                              \
-      if (a.page_shift >= 0) {                                                                                                       \
-        attention_prefill_kernel<DT, true, HPW, SCORES><<<grid, 256 * HPW, 0, stream>>>(q, k, v, out, partial, a);                   \
-        break;                                                                                                                       \
-      }                                                                                                                              \
-    }                                                                                                                                \
-    attention_prefill_kernel<DT, false, HPW, SCORES><<<grid, 256 * HPW, 0, stream>>>(q, k, v, out, partial, a);                      \
+    if (a.page_shift >= 0) attention_prefill_kernel<DT, true, HPW, SCORES><<<grid, 256 * HPW, 0, stream>>>(q, k, v, out, partial, a); \
+    else attention_prefill_kernel<DT, false, HPW, SCORES><<<grid, 256 * HPW, 0, stream>>>(q, k, v, out, partial, a);                  \
   } while (0)
   if (a.softcap > 0.f) PREFILL(SCORES_CAPPED);
   else if (a.bias) PREFILL(SCORES_BIASED);

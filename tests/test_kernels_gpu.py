@@ -530,7 +530,9 @@ def test_attention_decode_rows_as_requests_and_rows_beyond_the_bound(bound, n_sp
 @pytest.mark.parametrize("n_splits", [1, 3, 7])
 @pytest.mark.parametrize("nh,nkv,hd,page,window", [(4, 2, 16, 16, None), (6, 1, 48, 8, None), (5, 5, 80, 32, 37),
                                                    (32, 8, 64, 16, None), (4, 2, 128, 16, None), (2, 2, 96, 64, 100),
-                                                   (3, 1, 32, 16, 5), (8, 2, 48, 16, None), (12, 2, 32, 8, 90)])
+                                                   (3, 1, 32, 16, 5), (8, 2, 48, 16, None), (12, 2, 32, 8, 90),
+                                                   (4, 1, 64, 4, None), (4, 2, 64, 5, 60), (2, 1, 64, 24, None), (4, 2, 128, 2, None),
+                                                   (2, 1, 128, 24, 70), (4, 2, 32, 12, None), (2, 2, 64, 1, None)])
 def test_attention_prefill_matrix_cores(nh, nkv, hd, page, window, n_splits):
     """Prompt portions on the matrix cores: a long portion after a cached context that ends off a
     tile edge, a whole short prompt, a 2-token portion, a single decoded row and a 65-row portion
@@ -540,7 +542,7 @@ def test_attention_prefill_matrix_cores(nh, nkv, hd, page, window, n_splits):
     dtype = torch.bfloat16
     seq_lens = [333, 9, 130, 77, 65]
     q_lens = [150, 9, 2, 1, 65]
-    kp, vp, table, ks, vs = paged_setup(dtype, nkv, hd, page, seq_lens, 120, seed=11)
+    kp, vp, table, ks, vs = paged_setup(dtype, nkv, hd, page, seq_lens, max(120, sum(-(-s // page) for s in seq_lens) + 3), seed=11)
     ctx = [s - q for s, q in zip(seq_lens, q_lens)]
     cu = np.concatenate([[0], np.cumsum(q_lens)])
     n = int(cu[-1])
