@@ -1,6 +1,7 @@
 // Paged causal attention for prompt portions on the gfx950 matrix cores (bfloat16 in, float32
-// scores, maxima, sums and accumulators): the entry points, and the kernel for what attention_prompt.hip does not take
-// (head sizes other than 64 and 128, pages of fewer than 8 keys or of a size that is no power of two).
+// scores, maxima, sums and accumulators): the entry points, and the general kernel, for what attention_prompt.hip does not take
+// (head sizes other than 64 and 128, pages of fewer than 8 keys or of a size that is no power of two) and for short portions
+// of what it does (gibbs_rule_prefill).
 //
 // A workgroup takes 64 consecutive query rows of one request and HPW query heads that share a kv head
 // (1, 2 or 4 of the group's); 4 waves per head, each owning 16 of the rows.  One K and one V tile in LDS
@@ -442,8 +443,8 @@ void launch_prefill(dim3 grid, int heads_per_wg, hipStream_t stream, const bf16*
 // n_splits > 1: the key tiles of every workgroup's rows are cut into that many slices; partial is a
 // workspace of (first_row + n_rows) * nh * n_splits * (hd + 2) floats.  cu may start above 0 (the requests
 // of a step from some request on): first_row = cu[0] then, and n_rows counts the rows from there.
-// heads_per_wg: query heads of a kv head's group that a workgroup takes (1, 2 or 4; 0 counts as 1; the step's
-// rule for it is gibbs_rule_prefill_heads; attention_prompt.hip takes as many as the group has, with the same bits).
+// heads_per_wg: query heads of a kv head's group that a workgroup of the general kernel takes (1, 2 or 4); 0: attention_prompt.hip where it
+// takes the heads and pages, one head elsewhere.  (The step's rule is gibbs_rule_prefill.)
 // bias (or null): float32 [nh, bias_len], the score of a key d positions back gets bias[h][min(d, bias_len - 1)] * scale added.
 // sink (or null): float32 [nh], a term exp(sink[h]) in the softmax's denominator that has no key and no value.
 // chunk > 0: a row sees the keys of its own stretch of `chunk` positions, counted from position 0 (no window then).
@@ -473,7 +474,7 @@ GIBBS_EXPORT int gibbs_attention_prefill_masked(const void* q, const void* kpage
   PrefillArgs a{cu, ctx, table, n_req, max_pages, page_size, num_pages, page_shift, nh, nkv, hd, ldq, ldo, scale, window, n_splits, bias, bias_len, sink, chunk, softcap};
   const bf16 *qq = (const bf16*)q, *kk = (const bf16*)kpages, *vv = (const bf16*)vpages;
   bf16* oo = (bf16*)out;
-  if (prompt_attention_takes(hd, page_size, kpages, vpages)) {
+  if (heads_per_wg == 0 && prompt_attention_takes(hd, page_size, kpages, vpages)) {
     launch_prompt_attention(qq, kk, vv, oo, partial, a, n_rows, stream);
   } else {
     dim3 grid(ceil_div(n_rows, BM) + n_req, nh, n_splits);

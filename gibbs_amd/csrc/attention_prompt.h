@@ -27,7 +27,7 @@ struct PrefillArgs {
 enum { SCORES_PLAIN = 0, SCORES_BIASED = 1, SCORES_CAPPED = 2 };
 
 // Head sizes 64 and 128, pages of 8 keys or a larger power of two (a load of a wave covers 8 or 4 whole keys of one page), pools that start
-// at 16 bytes.
+// at 16 bytes.  (Which calls of those take it in a step: gibbs_rule_prefill.)
 static inline bool prompt_attention_takes(int hd, int page_size, const void* kpages, const void* vpages) {
   return (hd == 64 || hd == 128) && page_size >= 8 && (page_size & (page_size - 1)) == 0 && ((uintptr_t)kpages | (uintptr_t)vpages) % 16 == 0;
 }

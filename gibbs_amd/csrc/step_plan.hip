@@ -101,32 +101,65 @@ int prefill_splits(long n_tiles, int nh, int max_seq, int window) {
   return (int)std::max<long>(1, std::min<long>(std::min<long>(ceil_div_l(2048, blocks), keys / 256), 16));
 }
 
-// The same for attention_prompt.hip, whose workgroups are 32 rows of four heads (64 of two, 128 of one): two workgroups a compute unit, with at
-// least 512 keys to a slice on average, as a slice more costs every row its partial result and the merge's kernel.  Measured, us a call in
+// The same for attention_prompt.hip, whose workgroups are 32 rows of four heads (64 of two, 128 of one): a power of two that gives at most two workgroups
+// a compute unit, with at least 512 keys to a slice on average, as a slice more costs every row its partial result and the merge's kernel.  Measured, us a call in
 // 1 / 2 / 4 / 8 slices, 32 heads of 64 in groups of 4: 512 rows behind 1,536 keys (128 workgroups) 31 / 31 / 28 / 36; behind 7,680 - / 84 / 57 / 64;
-// 128 rows behind 1,000 20 / 17 / 17; 1,024 rows behind none (256 workgroups) 19 / 30; 512 behind none 13 / 18 / 20.
-// Up to 64 workgroups, where the chain of tiles is all there is to wait for, at least 256 keys: 79 rows of 16 heads behind 621 keys 14.5 -> 11.9 us, 128 rows of
-// 32 heads behind 1,000 16.5 -> 13.2, 40 rows and one behind 900 17.1 -> 11.3, 64 rows of 16 heads of 128 behind 700 22.9 -> 17.6.
+// 128 rows behind 1,000 20 / 17 / 17; 512 behind none 13 / 18 / 20; 200 rows behind 4,000 (56) in 4 / 8 / 9 slices 25.2 / 26.9 / 34.3; 400 behind 4,000 (104) in 4 / 5
+// 36.3 / 44.0.  A workgroup for every compute unit is not cut below 3,000 keys: 1,024 rows behind none (256) 19 / 30, behind 700 29 / 37, behind 2,000 45 / 49.
+// Up to 64 workgroups, where the chain of tiles is all there is to wait for, at least 256 keys: 16 rows behind 4,000 in 8 / 15 slices 14.0 / 11.9.
 int prompt_splits(int rows, int reqs, int nh, int nkv, int max_seq, int window) {
   const int group = nh / std::max(nkv, 1), heads = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1), tile = 128 / heads;
   const long blocks = std::max<long>(1, (ceil_div_l(rows, tile) + reqs / 2) * (nh / heads));
-  long seen = max_seq - rows / (2 * std::max(reqs, 1));
+  long seen = max_seq - rows / (2 * std::max(reqs, 1)), fill = 1;
   if (window > 0) seen = std::min<long>(seen, window);
-  return (int)std::max<long>(1, std::min<long>(std::min<long>((512 + blocks / 2) / blocks, seen / (blocks <= 64 ? 256 : 512)), 16));
+  if (blocks >= 256 && seen < 3000) return 1;
+  while (fill < 16 && fill * 2 * blocks <= 512) fill *= 2;
+  return (int)std::max<long>(1, std::min<long>(fill, seen / (blocks <= 64 ? 256 : 512)));
 }
 
-// Query heads of a kv head's group that a workgroup of the prompt attention takes (they share its K and V
+// Query heads of a kv head's group that a workgroup of the general prompt attention takes (they share its K and V
 // tiles).  With one head a workgroup re-reads all keys and values of its rows' past for 64 x 64 scores at a
 // time, and from about 4,000 keys a row that traffic, not the arithmetic, bounds the kernel (537 TFLOP/s at
 // 8.4 TB/s through L2 and the L1s); more heads a workgroup are fewer, longer workgroups.  Measured at 32 heads
 // in groups of 4, head size 64 (us, with 1 / 2 / 4 heads): 2,048 rows 68 / 63 / 63; 4,096 rows 196 / 209 / 203;
 // 8,192 rows 577 / 562 / 584; 32,768 rows 8,086 / 7,147 / 6,626; 2,048 rows behind 6,144 keys 281 / 220 / 205;
-// 512 rows behind 7,680 keys in 8 slices 80 / 84 / 92.  (Heads of 64 in pages of a power of two take attention_prompt.hip now.)
+// 512 rows behind 7,680 keys in 8 slices 80 / 84 / 92.  (The longer ones of these take attention_prompt.hip, but in pages of fewer than 8 keys or
+// of a size that is no power of two.)
 int prefill_heads(int rows, int reqs, int nh, int nkv, int hd, int max_seq, int n_splits) {
   const int group = nh / std::max(nkv, 1);
   if (hd > 64 || group % 2 || n_splits > 1) return 1;
   const long seen = (long)max_seq - rows / (2 * std::max(reqs, 1));   // keys a row sees on average, if one request has them all
   return (group % 4 == 0 && seen >= 6000) ? 4 : 2;
+}
+
+// Which kernel the prompt attention of a step takes, in how many slices of the keys, and how many heads a workgroup of the general kernel has (0:
+// attention_prompt.hip, where it takes the heads and pages).  The latter's workgroups are fewer and their chains of tiles longer, so it pays where there is work
+// for the chip: where the general kernel's workgroups (64 rows of a head), without slices, are one a compute unit; or, of fewer and for a single request, where
+// their keys make up for it, or a tile of rows has a long cache and heads that share it (of several requests the longest says little about the others).  A cap
+// on the scores stands between its products, not beside them: from 1,024 workgroups on.  Keys that a window hides are taken out tile by tile: twice the
+// workgroups, or no slices.  With a kv head for every head its workgroups are 128 rows: not for requests of a few rows.
+// Measured over 1,935 calls of one request (heads of 64 and 128 in groups of 1, 2 and 4, 2 to 4,096 rows behind 0 to 8,000 keys): 0.88 of the general kernel's
+// time in the mean, 1.02 at most.  us, general / attention_prompt.hip, 32 heads of 64 in groups of 4: 128 rows behind 700 keys 13.1 / 13.7,
+// 512 behind none 17.0 / 11.5, 16 behind 4,000 15.2 / 11.9; 16 heads of 128 in groups of 4: 45 rows 5.3 / 7.0, 128 behind 100 10.2 / 12.2, 128 behind 700 15.6 / 18.6,
+// 1,024 31.2 / 27.2, 2,048 74 / 53; 16 heads of 64: 79 rows 5.0 / 6.6, 512 under a window of 256 behind 1,500 10.9 / 13.4, 64 requests of 8 rows behind 300
+// 21.9 / 24.3; 200 rows of 32 heads of 64 behind 2,000 21.9 / 22.4, 400 of 16 heads of 128 behind 2,000 47.7 / 29.8; portions of 100, 300 and 5 rows behind 500, 0 and 2,000, 32 heads 23.2 / 25.3; capped, 512 rows of 16 heads 17.0 / 22.8, 2,048 56.6 / 64.0, of 32 88 / 81.
+struct PrefillChoice {
+  int splits, heads;
+};
+PrefillChoice prefill_choice(int rows, int reqs, int nh, int nkv, int hd, int max_seq, int window, bool capped, bool prompt_takes) {
+  const long tiles = prefill_tiles(rows, reqs), blocks = tiles * nh;
+  if (prompt_takes && max_seq > 0) {
+    const int group = nh / std::max(nkv, 1), splits = prompt_splits(rows, reqs, nh, nkv, max_seq, window);
+    long seen = max_seq - rows / (2 * std::max(reqs, 1));
+    if (window > 0) seen = std::min<long>(seen, window);
+    const bool pays = capped       ? blocks >= 1024
+                      : window > 0 ? blocks >= 512 || (blocks >= 256 && splits == 1)
+                      : reqs > 1   ? blocks >= 320
+                                   : blocks >= 256 || blocks * seen >= (hd == 64 ? 280000 : 160000) || (tiles == 1 && group % 2 == 0 && blocks * seen >= 60000);
+    if (pays && (group % 2 == 0 || rows >= 16 * reqs)) return {splits, 0};
+  }
+  const int splits = max_seq > 0 ? prefill_splits(tiles, nh, max_seq, window) : 1;
+  return {splits, prefill_heads(rows, reqs, nh, nkv, hd, max_seq, splits)};
 }
 
 // Which product runs y = x W^T, and in how many float32 partial sums it leaves its result.
@@ -761,16 +794,12 @@ void* attend_prepared(Exec& e, const PagedAttention& t, void* raw, long ldq, lon
     const int lead = a.lead_single >= 2 ? a.lead_single : 0;
     if (lead) decode_attention(e, t, raw, ldq, lead, a.pos, a.row_req, att);
     const int rows = N - lead, reqs = a.n_req - lead;
-    const int bound = t.chunk > 0 ? t.chunk : t.window;
-    const int n_splits = a.max_seq <= 0 ? 1
-                         : prompt_attention_takes(t.hd, t.page_size, t.kpages, t.vpages)
-                             ? prompt_splits(rows, reqs, t.nh, t.nkv, a.max_seq, bound)
-                             : prefill_splits(prefill_tiles(rows, reqs), t.nh, a.max_seq, bound);
-    float* partial = n_splits > 1 ? (float*)e.take(gibbs_attention_decode_workspace(N, t.nh, t.hd, n_splits) * 4) : nullptr;
+    const PrefillChoice c = prefill_choice(rows, reqs, t.nh, t.nkv, t.hd, a.max_seq, t.chunk > 0 ? t.chunk : t.window, t.softcap > 0.f,
+                                           prompt_attention_takes(t.hd, t.page_size, t.kpages, t.vpages));
+    float* partial = c.splits > 1 ? (float*)e.take(gibbs_attention_decode_workspace(N, t.nh, t.hd, c.splits) * 4) : nullptr;
     RUN(e, gibbs_attention_prefill_masked(raw, t.kpages, t.vpages, att, partial, a.cu + lead, a.ctx + lead, table + (long)lead * width, reqs,
-                                          width, t.page_size, t.num_pages, rows, t.nh, t.nkv, t.hd, ldq, ldo, t.scale, t.window, n_splits, lead,
-                                          prefill_heads(rows, reqs, t.nh, t.nkv, t.hd, a.max_seq, n_splits), t.bias_t, t.bias_len, t.sink,
-                                          t.chunk, t.softcap, a.stream));
+                                          width, t.page_size, t.num_pages, rows, t.nh, t.nkv, t.hd, ldq, ldo, t.scale, t.window, c.splits, lead, c.heads,
+                                          t.bias_t, t.bias_len, t.sink, t.chunk, t.softcap, a.stream));
     e.give(partial);
   } else if (fast_bf16 && a.max_q == 1 && t.hd % 8 == 0 && t.hd <= 256 && (!t.bias || matrix_sizes)) {
     decode_attention(e, t, raw, ldq, N, a.pos, a.row_req, att);
@@ -2680,9 +2709,11 @@ GIBBS_EXPORT void gibbs_rule_decode_splits(int n_rows, int nkv, int group, int m
 GIBBS_EXPORT int gibbs_rule_prefill_splits(long n_tiles, int nh, int max_seq, int window) {
   return prefill_splits(n_tiles, nh, max_seq, window);
 }
-GIBBS_EXPORT int gibbs_rule_prompt_splits(int rows, int reqs, int nh, int nkv, int hd, int page_size, int max_seq, int window) {
-  return prompt_attention_takes(hd, page_size, nullptr, nullptr) ? prompt_splits(rows, reqs, nh, nkv, max_seq, window)
-                                                                 : prefill_splits(prefill_tiles(rows, reqs), nh, max_seq, window);
+GIBBS_EXPORT void gibbs_rule_prefill(int rows, int reqs, int nh, int nkv, int hd, int page_size, int max_seq, int window, int capped, int* n_splits,
+                                     int* heads) {
+  const PrefillChoice c = prefill_choice(rows, reqs, nh, nkv, hd, max_seq, window, capped != 0, prompt_attention_takes(hd, page_size, nullptr, nullptr));
+  *n_splits = c.splits;
+  *heads = c.heads;
 }
 GIBBS_EXPORT long gibbs_rule_prefill_tiles(int rows, int reqs) { return prefill_tiles(rows, reqs); }
 GIBBS_EXPORT int gibbs_rule_prefill_heads(int rows, int reqs, int nh, int nkv, int hd, int max_seq, int n_splits) {

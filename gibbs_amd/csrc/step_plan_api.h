@@ -306,7 +306,8 @@ void gibbs_rule_decode_splits(int n_rows, int nkv, int group, int max_seq, int h
                               int* waves);
 long gibbs_rule_prefill_tiles(int rows, int reqs);            // query tiles that the rows of a ragged batch make
 int gibbs_rule_prefill_splits(long n_tiles, int nh, int max_seq, int window);
-int gibbs_rule_prompt_splits(int rows, int reqs, int nh, int nkv, int hd, int page_size, int max_seq, int window);   // of whichever kernel takes them
+// the prompt attention of a step: slices of its keys, and the heads a workgroup of the general kernel has (0: attention_prompt.hip)
+void gibbs_rule_prefill(int rows, int reqs, int nh, int nkv, int hd, int page_size, int max_seq, int window, int capped, int* n_splits, int* heads);
 int gibbs_rule_prefill_heads(int rows, int reqs, int nh, int nkv, int hd, int max_seq, int n_splits);   // query heads a workgroup
 int gibbs_rule_chunked(int time_mix, int rows, int reqs, int max_q, int H, int D, int V);   // delta rule or time mixing: in chunks or a walk
 int gibbs_rule_token_kernel(int time_mix, int rows, int H, int D, int V);     // theirs for requests of one row: one kernel or three

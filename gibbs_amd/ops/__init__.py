@@ -682,6 +682,15 @@ def prefill_splits(n_tiles: int, nh: int, max_seq: int, window: Optional[int] = 
     return int(library().gibbs_rule_prefill_splits(n_tiles, nh, max_seq, int(window or 0)))
 
 
+def prefill_rule(rows: int, reqs: int, nh: int, nkv: int, hd: int, page_size: int, max_seq: int, window: int = 0,
+                 capped: bool = False) -> tuple[int, int]:
+    """(slices, heads a workgroup) of the prompt attention of a step; heads 0: the kernel with 32 rows a wave."""
+    import ctypes
+    n_splits, heads = ctypes.c_int(0), ctypes.c_int(0)
+    library().gibbs_rule_prefill(rows, reqs, nh, nkv, hd, page_size, int(max_seq), int(window), int(capped), ctypes.byref(n_splits), ctypes.byref(heads))
+    return n_splits.value, heads.value
+
+
 def attention_prefill(q: torch.Tensor, n_rows: int, nh: int, nkv: int, hd: int, kpages: torch.Tensor,
                       vpages: torch.Tensor, table: torch.Tensor, n_req: int, cu: torch.Tensor, ctx: torch.Tensor,
                       scale: float, window: Optional[int] = None, out: Optional[torch.Tensor] = None,
@@ -693,7 +702,8 @@ def attention_prefill(q: torch.Tensor, n_rows: int, nh: int, nkv: int, hd: int, 
     of 16 up to 128.  `max_seq`: a bound on the keys of any row, from which the number of key slices
     is chosen (or `n_splits`).  `first_req`, `first_row`: only the requests from `first_req` on are
     attended to (their rows start at `first_row`); the rows before are left as they are in `out`.
-    `heads_per_wg`: query heads of a kv head's group per workgroup (1, 2 or 4; default: the native step's rule)."""
+    `heads_per_wg`: query heads of a kv head's group per workgroup of the general kernel (1, 2 or 4), or 0: the kernel with 32 rows a
+    wave where it takes the heads and pages (default: the native step's rule)."""
     require_cuda(q, kpages, vpages, table, cu, ctx)
     if q.dtype != torch.bfloat16:
         raise KernelError("attention_prefill is the bfloat16 kernel; the float32 path uses attention_plain")
@@ -709,11 +719,11 @@ def attention_prefill(q: torch.Tensor, n_rows: int, nh: int, nkv: int, hd: int, 
         out = torch.empty((n_rows, nh * hd), dtype=q.dtype, device=q.device)
     assert out.shape == (n_rows, nh * hd) and out.dtype == q.dtype and out.is_contiguous()
     rows, reqs = n_rows - first_row, n_req - first_req
-    if n_splits is None:
-        n_splits = (int(library().gibbs_rule_prompt_splits(rows, reqs, nh, nkv, hd, page_size, int(max_seq), int(chunk or window or 0)))
-                    if max_seq > 0 else 1)
-    if heads_per_wg is None:
-        heads_per_wg = int(library().gibbs_rule_prefill_heads(rows, reqs, nh, nkv, hd, int(max_seq), int(n_splits)))
+    if n_splits is None or heads_per_wg is None:
+        splits, heads = prefill_rule(rows, reqs, nh, nkv, hd, page_size, max_seq, chunk or window or 0, softcap > 0)
+        n_splits = splits if n_splits is None else n_splits
+        if heads_per_wg is None:
+            heads_per_wg = heads if n_splits == splits else int(library().gibbs_rule_prefill_heads(rows, reqs, nh, nkv, hd, int(max_seq), int(n_splits)))
     partial = None
     if n_splits > 1:
         partial = torch.empty(slices_workspace(n_rows, nh, hd, n_splits), dtype=torch.float32, device=q.device)

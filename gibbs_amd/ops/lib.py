@@ -225,7 +225,7 @@ _VALUE_SIGNATURES = {
     "gibbs_rule_skinny_splits": ([c_int, c_int, c_int, c_int, c_int], c_int),
     "gibbs_rule_decode_splits": ([c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p], None),
     "gibbs_rule_prefill_splits": ([c_long, c_int, c_int, c_int], c_int),
-    "gibbs_rule_prompt_splits": ([c_int] * 8, c_int),
+    "gibbs_rule_prefill": ([c_int] * 9 + [c_void_p] * 2, None),
     "gibbs_rule_prefill_tiles": ([c_int, c_int], c_long),
     "gibbs_rule_prefill_heads": ([c_int, c_int, c_int, c_int, c_int, c_int, c_int], c_int),
     "gibbs_rule_chunked": ([c_int] * 7, c_int),

@@ -706,7 +706,7 @@ def test_attention_prompt_edges(nh, nkv, hd, page, how):
     scale, window, chunk, softcap = 1 / math.sqrt(hd), how.get("window"), how.get("chunk", 0), how.get("softcap", 0.0)
     sink = rnd(nh, seed=6) if how.get("sink") else None
     out = ops.attention_prefill(q, n, nh, nkv, hd, kp, vp, table, len(q_lens), i32(cu), i32(ctx), scale, window, sink=sink, chunk=chunk,
-                                softcap=softcap, n_splits=how.get("splits", 1))
+                                softcap=softcap, n_splits=how.get("splits", 1), heads_per_wg=0)
     pos = i32([c + t for c, m in zip(ctx, q_lens) for t in range(m)])
     row_req = i32([r for r, m in enumerate(q_lens) for _ in range(m)])
     plain = ops.attention_plain(q, n, nh, nkv, hd, kp, vp, table, len(q_lens), pos, row_req, scale, window, sink=sink, chunk=chunk,
