@@ -478,8 +478,10 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 // 13.7, now 27.0 and 12.9; back with 16 features a workgroup or 32, 8 rows 13.7 / 13.1 (gated: gibbs_moe_gated_features).
 // DIRECT (at most 64 pairs, an expert at most 16 of them): no grouping in front: `sorted_pair` holds each pair's choice, places are the pairs' own
 // numbers, and the workgroups are laid out over the experts that are chosen, not over all: with a grid of all of them the chosen ones' could meet on
-// the same compute units (16 experts, 2 rows, 7 of them chosen: gated 21.6 us and back 11.1, now 13.3 and 7.5).
-template <bool GLU, bool DIRECT, int NF>
+// the same compute units (16 experts, 2 rows, 7 of them chosen: gated 20.4 us and back 11.8, now 12.7 and 8.2).  Finding its expert costs a workgroup 0.1 to 0.2
+// us, which one row's products back feel (5.6 -> 5.8 us).
+// TURN: workgroups begin at different k (few_turns).
+template <bool GLU, bool DIRECT, int NF, bool TURN>
 __global__ __launch_bounds__(256) void moe_gemm_few_kernel(const bf16* __restrict__ X, const int* __restrict__ sorted_pair,
                                                            const int* __restrict__ tile_expert, const bf16* __restrict__ Wa,
                                                            const bf16* __restrict__ Wb, int top, int I, long ldx, long expert_stride, bf16* __restrict__ Y,
@@ -487,21 +489,21 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(const bf16* __restric
   constexpr int NA = GLU ? 2 * NF : NF;    // accumulators a wave
   __shared__ __attribute__((aligned(16))) floatx4 part[4][NA][WAVE];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, lr = lane % 16, lg = lane / 16;
-  int e, pair, place, block = blockIdx.x;
+  int e, pair, place;
   if constexpr (DIRECT) {
-    const int columns = (O + 16 * NF - 1) / (16 * NF), nth = blockIdx.x / columns;
-    block = blockIdx.x - nth * columns;
     const int choice = sorted_pair[min(lane, pairs - 1)];
     // the pairs with a lane's own choice, by the choices' bits; the `nth` expert of those chosen is the one whose first pair is the nth such
     const bool live = lane < pairs && (unsigned)choice < (unsigned)experts;
     uint64_t same = __builtin_amdgcn_ballot_w64(live);
-    for (int b = 0; (experts - 1) >> b; ++b) {
-      const bool bit = choice >> b & 1;
-      const uint64_t with = __builtin_amdgcn_ballot_w64(bit);
-      same &= bit ? with : ~with;
-    }
+    for (int b = 0; (experts - 1) >> b; b += 4)      // (bits that no choice has change nothing)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const bool bit = choice >> (b + u) & 1;
+        const uint64_t with = __builtin_amdgcn_ballot_w64(bit);
+        same &= bit ? with : ~with;
+      }
     const bool first = live && __builtin_ctzll(same) == lane;
-    const uint64_t firsts = __builtin_amdgcn_ballot_w64(first), found = __builtin_amdgcn_ballot_w64(first && __popcll(firsts & ((1ull << lane) - 1)) == nth);
+    const uint64_t firsts = __builtin_amdgcn_ballot_w64(first), found = __builtin_amdgcn_ballot_w64(first && __popcll(firsts & ((1ull << lane) - 1)) == (int)blockIdx.y);
     if (found == 0) return;
     e = __builtin_amdgcn_readlane(choice, __builtin_ctzll(found));
     const uint64_t all = __builtin_amdgcn_ballot_w64(live && choice == e);
@@ -517,7 +519,7 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(const bf16* __restric
     pair = sorted_pair[place];
     if (e < 0) return;
   }
-  const int col0 = block * (16 * NF);
+  const int col0 = blockIdx.x * (16 * NF);
   const int src = pair < 0 ? 0 : (top > 0 ? pair / top : place);      // (a place without a pair: some row, its results are not stored)
   const bf16* xr = X + (size_t)src * ldx;
   const bf16* w[NA];
@@ -552,8 +554,8 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(const bf16* __restric
   if (n > 0) {
     // The workgroups begin at different k: rows of 4 KB and more, all read at one k at a time, are a few of the memory's channels (8 and 32 rows, gated,
     // 32.1 and 35.5 us without, 27.0 and 30.4; rows of 2 KB, back, 13.1 / 13.4).  By the feature, so that a result's sum does not depend on the grid.
-    const int turn = I >= 2048 ? col0 / 32 % n : 0;
-    auto nth = [&](int it) { return it + turn < n ? it + turn : it + turn - n; };
+    const int turn = TURN ? col0 / 32 % n : 0;
+    auto nth = [&](int it) { return !TURN || it + turn < n ? it + turn : it + turn - n; };
     ask(0, nth(0));
     ask(1, nth(min(1, n - 1)));
     int it = 0;
@@ -1118,6 +1120,10 @@ GIBBS_EXPORT int gibbs_moe_group(const int* chosen, int n_pairs, int E, int bm, 
   GIBBS_LAUNCH_STATUS("moe_group");
 }
 
+// Rows of 4 KB and more are read from a k of the features' own on; a loop that can turn costs shorter ones more than it gives (8 rows of 16 experts of 512 at width
+// 1,024, gated, us: 8.74, 9.12 with a turn of none).
+static bool few_turns(int I) { return I >= 2048; }
+
 // Y[m] = W_a,e X[src(m)] (w_b null), or act(W_a,e X[src(m)]) * (W_b,e X[src(m)]), for every place m of the sorted pairs; e the
 // expert of m's tile; src(m) = pair / top (top > 0: rows of the step, gathered) or m itself (top 0: X is in sorted order).
 // W_a, W_b: [experts, O, I].
@@ -1160,11 +1166,13 @@ GIBBS_EXPORT int gibbs_moe_gemm_weighted(const void* X, long ldx, int top, const
         kernel<<<dim3(ceil_div(O, features), tiles), 256, 0, stream>>>((const bf16*)X, sorted_pair, tile_expert, (const bf16*)w_a, (const bf16*)w_b, top, I, ldx, stride, (bf16*)Y,
                                                                        ldy, O, act, in_weight, 0, 0);
       };
-      if (gibbs_moe_gated_features(tiles, O) == 16) queue(moe_gemm_few_kernel<true, false, 1>, 16);
-      else queue(moe_gemm_few_kernel<true, false, 2>, 32);
+      const bool narrow = gibbs_moe_gated_features(tiles, O) == 16;
+      if (few_turns(I)) narrow ? queue(moe_gemm_few_kernel<true, false, 1, true>, 16) : queue(moe_gemm_few_kernel<true, false, 2, true>, 32);
+      else narrow ? queue(moe_gemm_few_kernel<true, false, 1, false>, 16) : queue(moe_gemm_few_kernel<true, false, 2, false>, 32);
     } else {
-      moe_gemm_few_kernel<false, false, 2><<<dim3(ceil_div(O, 32), tiles), 256, 0, stream>>>((const bf16*)X, sorted_pair, tile_expert, (const bf16*)w_a, nullptr, top, I,
-                                                                                         ldx, stride, (bf16*)Y, ldy, O, act, nullptr, 0, 0);
+      const auto kernel = few_turns(I) ? moe_gemm_few_kernel<false, false, 2, true> : moe_gemm_few_kernel<false, false, 2, false>;
+      kernel<<<dim3(ceil_div(O, 32), tiles), 256, 0, stream>>>((const bf16*)X, sorted_pair, tile_expert, (const bf16*)w_a, nullptr, top, I, ldx, stride, (bf16*)Y, ldy, O, act,
+                                                               nullptr, 0, 0);
     }
   } else {
     return gibbs_fail("moe_gemm: unknown dtype %d", dtype);
@@ -1183,12 +1191,16 @@ GIBBS_EXPORT int gibbs_moe_gemm_direct(const void* X, long ldx, int top, const i
   GIBBS_REQUIRE(act >= 0 && act < ACT_COUNT && (!in_weight || w_b), "moe_gemm: bad activation, or weights on the inputs of an ungated product");
   GIBBS_REQUIRE(I % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)X % 16) == 0 && ((uintptr_t)w_a % 16) == 0 && ((uintptr_t)w_b % 16) == 0, "moe_gemm: rows of whole 16 bytes");
   const long stride = (long)O * I;
-  if (w_b)
-    moe_gemm_few_kernel<true, true, 1><<<ceil_div(O, 16) * std::min(E, pairs), 256, 0, stream>>>((const bf16*)X, chosen, nullptr, (const bf16*)w_a, (const bf16*)w_b, top, I, ldx, stride,
-                                                                                 (bf16*)Y, ldy, O, act, in_weight, pairs, E);
-  else
-    moe_gemm_few_kernel<false, true, 2><<<ceil_div(O, 32) * std::min(E, pairs), 256, 0, stream>>>((const bf16*)X, chosen, nullptr, (const bf16*)w_a, nullptr, 0, I, ldx, stride, (bf16*)Y,
-                                                                                  ldy, O, act, nullptr, pairs, E);
+  const int chosen_experts = std::min(E, pairs);      // (at most)
+  if (w_b) {
+    const auto kernel = few_turns(I) ? moe_gemm_few_kernel<true, true, 1, true> : moe_gemm_few_kernel<true, true, 1, false>;
+    kernel<<<dim3(ceil_div(O, 16), chosen_experts), 256, 0, stream>>>((const bf16*)X, chosen, nullptr, (const bf16*)w_a, (const bf16*)w_b, top, I, ldx, stride, (bf16*)Y, ldy, O, act,
+                                                                      in_weight, pairs, E);
+  } else {
+    const auto kernel = few_turns(I) ? moe_gemm_few_kernel<false, true, 2, true> : moe_gemm_few_kernel<false, true, 2, false>;
+    kernel<<<dim3(ceil_div(O, 32), chosen_experts), 256, 0, stream>>>((const bf16*)X, chosen, nullptr, (const bf16*)w_a, nullptr, 0, I, ldx, stride, (bf16*)Y, ldy, O, act, nullptr,
+                                                                      pairs, E);
+  }
   GIBBS_LAUNCH_STATUS("moe_gemm");
 }
 
