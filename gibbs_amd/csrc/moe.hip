@@ -774,7 +774,7 @@ int launch_tiled_as(const bf16* X, long ldx, int top, const int* sorted_pair, co
 // 0.81), and neither the order of the items over the XCDs nor where in k an item begins changes that.  The loads are buffer loads: with global
 // ones the compiler waited for the reads of the next products in front of these (8,412 pairs of 16 experts, width 2,048, 1,024 features: gated
 // 104 us, down 60, now 101 and 58; 16,384 pairs, width 4,096, 2,048 features 575 and 312, now 553 and 300, 1.0 PFLOP/s; 1,400 pairs of 8 experts,
-// width 2,048, 512 features 30 and 14, now 28 and 13).  The kernel above takes 164 and 93, 799 and 400, 70 and 23.  Slower: a workgroup an item (122 us
+// width 2,048, 512 features 30 and 14, now 28 and 13; 2,400 pairs of 16 experts, 1,024 features, are the other way round, gated 43.6 and down 25.7, now 43.4 and 27.1).  The kernel above takes 164 and 93, 799 and 400, 70 and 23.  Slower: a workgroup an item (122 us
 // where this took 114 in the first of these), tiles of 32 k with two workgroups a compute unit (133: requests of 64 bytes), and 128 rows of W (148).
 constexpr int ASYNC_BK = 64, ASYNC_BN = 256, ASYNC_STAGES = 3, ASYNC_UNITS = 256;   // (units: one workgroup a compute unit)
 

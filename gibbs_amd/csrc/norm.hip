@@ -255,8 +255,8 @@ GIBBS_EXPORT int gibbs_add_partials_rmsnorm(float* x, const float* partials, int
 // x[r] += delta[r] alone (the last residual add of a model whose tail norms only some rows
 // still has to leave x whole for callers that read it).  float32 delta may be `n_partials` partial
 // sums, `partial_stride` elements apart, added in ascending order.
-// The sums of three parts and more are asked for 8 at a time before the first is added (beyond the last: the last again, not added): one after
-// the other each is a trip to memory.  64 rows of 2,048, us: 4 parts 3.0 -> 2.5, 8 3.7 -> 2.6; 64 of 1,024 in 12 parts 5.1 -> 3.1.  (Two or four elements a
+// The sums of four parts and more are asked for 8 at a time before the first is added (beyond the last: the last again, not added): one after
+// the other each is a trip to memory.  64 rows of 2,048, us: 4 parts 3.0 -> 2.5, 8 3.7 -> 2.6; 64 of 1,024 in 12 parts 5.1 -> 3.1; 64 of 4,096 in 3 parts 3.36, and 3.53 so.  (Two or four elements a
 // thread: the same.)
 template <typename T>
 __global__ void residual_add_kernel(float* __restrict__ x, const T* __restrict__ delta, int n_partials,
@@ -264,7 +264,7 @@ __global__ void residual_add_kernel(float* __restrict__ x, const T* __restrict__
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < count) {
     float v = x[i];
-    if (delta && n_partials <= 2) {
+    if (delta && n_partials <= 3) {
       for (int s = 0; s < n_partials; ++s) v += to_float(delta[s * partial_stride + i]);
     } else if (delta) {
       for (int s = 0; s < n_partials; s += 8) {
