@@ -84,7 +84,7 @@ __global__ void glu_clamped_bf16x8_kernel(const bf16* __restrict__ gu, bf16* __r
   const uint4 ur = *(const uint4*)(gu + (size_t)n * 2 * F + F + f);
   const uint32_t gw[4] = {gr.x, gr.y, gr.z, gr.w}, uw[4] = {ur.x, ur.y, ur.z, ur.w};
   uint32_t ow[4];
-  bool far = false;      // (infinities and NaN among them)
+  bool far = false;      // (of the gates as they are capped)
   auto all = [&](auto f) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -97,7 +97,7 @@ __global__ void glu_clamped_bf16x8_kernel(const bf16* __restrict__ gu, bf16* __r
   };
 #pragma unroll
   for (int i = 0; i < 4; ++i)
-    far |= !(fabsf(alpha * __uint_as_float(gw[i] << 16)) <= NEAR) | !(fabsf(alpha * __uint_as_float(gw[i] & 0xffff0000u)) <= NEAR);
+    far |= !(fabsf(alpha * fminf(__uint_as_float(gw[i] << 16), limit)) <= NEAR) | !(fabsf(alpha * fminf(__uint_as_float(gw[i] & 0xffff0000u), limit)) <= NEAR);
   if (__builtin_expect(__builtin_amdgcn_ballot_w64(far) == 0, 1)) all([&](float g, float u) { return clamped_swish_product_near(g, u, alpha, limit); });
   else all([&](float g, float u) { return clamped_swish_product(g, u, alpha, limit); });
   *(uint4*)(out + (size_t)n * F + f) = make_uint4(ow[0], ow[1], ow[2], ow[3]);

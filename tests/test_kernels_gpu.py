@@ -1151,6 +1151,26 @@ def test_gates_of_every_size(f, clamped):
         assert torch.equal(run(gu[r:r + 1].contiguous())[0], out[r])
 
 
+@pytest.mark.parametrize("limit", [-100.0, -60.0, -3.0, 7.0, 60.0, 100.0, math.inf])
+@pytest.mark.parametrize("f", [520, 521])
+def test_clamped_gates_whatever_the_limit(f, limit):
+    """The cap is part of the gate that the exponential is taken of: caps on both sides of where it is taken in full, for rows of whole 16 bytes and
+    for others, against float64."""
+    from gibbs_amd.ops.lib import call, dtype_code, ptr, stream
+    bf = torch.bfloat16
+    gu = rnd(3, 2 * f, dtype=bf, scale=30.0, seed=5)
+    gu[1, 3], gu[1, 70], gu[2, 9] = math.nan, math.inf, -math.inf
+    out = torch.empty((3, f), dtype=bf, device=DEV)
+    call("gibbs_glu_clamped", ptr(gu), ptr(out), dtype_code(bf), 3, f, 1.702, limit, stream())
+    cap = torch.full((), limit, dtype=torch.float64, device=DEV)
+    g = torch.fmin(gu[:, :f].double(), cap)
+    want = g * torch.sigmoid(1.702 * g) * (1 + torch.minimum(torch.maximum(gu[:, f:].double(), -cap), cap))
+    ok = want.isfinite()
+    # (half a unit of bfloat16, some 1e-7 of float32 arithmetic in front of it, and products under the smallest float32)
+    assert ((out[ok].double() - want[ok]).abs() <= 2.0 ** -8 * 1.001 * want[ok].abs() + 1e-33).all()
+    assert not out[~ok].isfinite().any()
+
+
 @pytest.mark.parametrize("hidden", [512, 1020, 1024, 1028, 2044, 2048, 2052, 3072, 4096, 4100])
 @pytest.mark.parametrize("parts", [0, 1, 3])
 @pytest.mark.parametrize("n", [5, 520])
