@@ -237,7 +237,7 @@ template <typename OutT>
 __global__ __launch_bounds__(256) void gemm_bf16_few_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W, OutT* __restrict__ C, int N, int O, int I,
                                                             long lda, long ldw, long ldc, int wide) {
   constexpr int THREADS = 256, ROWS = THREADS / 8, CA = FEW_ROWS / ROWS, CW = FEW_FEATURES / ROWS, LOADS = CA + CW, STAGE = (FEW_ROWS + FEW_FEATURES) * TK;
-  extern __shared__ __attribute__((aligned(16))) bf16 few_tiles[];      // [FEW_STAGES][rows of A, then of W][TK]
+  __shared__ __attribute__((aligned(16))) bf16 few_tiles[FEW_STAGES * STAGE];      // [FEW_STAGES][rows of A, then of W][TK]
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE, r32 = lane % 32, h = lane / 32;
   const int col0 = blockIdx.x * FEW_FEATURES, nt = I / TK;
   const bf16* w = W + (size_t)col0 * ldw;
@@ -307,15 +307,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_few_kernel(const bf16* __restri
 }
 template <typename OutT>
 int launch_few(const bf16* A, const bf16* W, OutT* C, int N, int O, int I, long lda, long ldw, long ldc, hipStream_t stream) {
-  constexpr int LDS_BYTES = FEW_STAGES * (FEW_ROWS + FEW_FEATURES) * TK * (int)sizeof(bf16);
-  static bool prepared = false;    // (per output type: the template makes one flag each)
-  if (!prepared) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_bf16_few_kernel<OutT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
-    if (e != hipSuccess) return gibbs_fail("gemm_bf16: %s", hipGetErrorString(e));
-    prepared = true;
-  }
   const int wide = O % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % (4 * sizeof(OutT)) == 0;
-  gemm_bf16_few_kernel<OutT><<<ceil_div(O, FEW_FEATURES), 256, LDS_BYTES, stream>>>(A, W, C, N, O, I, lda, ldw, ldc, wide);
+  gemm_bf16_few_kernel<OutT><<<ceil_div(O, FEW_FEATURES), 256, 0, stream>>>(A, W, C, N, O, I, lda, ldw, ldc, wide);
   GIBBS_LAUNCH_STATUS("gemm_bf16");
 }
 // (offsets of 32 bits within 64 rows of A and 128 of W)
