@@ -696,15 +696,17 @@ def attention_prefill(q: torch.Tensor, n_rows: int, nh: int, nkv: int, hd: int, 
                       scale: float, window: Optional[int] = None, out: Optional[torch.Tensor] = None,
                       max_seq: int = 0, n_splits: Optional[int] = None, first_req: int = 0,
                       first_row: int = 0, heads_per_wg: Optional[int] = None,
-                      sink: Optional[torch.Tensor] = None, chunk: int = 0, softcap: float = 0.0) -> torch.Tensor:
+                      sink: Optional[torch.Tensor] = None, chunk: int = 0, softcap: float = 0.0,
+                      bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """bfloat16 paged causal attention for prompt portions on the matrix cores: rows cu[r] .. cu[r+1]
     of request r sit at positions ctx[r] ..; same result as `attention_plain`.  Head sizes: multiples
     of 16 up to 128.  `max_seq`: a bound on the keys of any row, from which the number of key slices
     is chosen (or `n_splits`).  `first_req`, `first_row`: only the requests from `first_req` on are
     attended to (their rows start at `first_row`); the rows before are left as they are in `out`.
     `heads_per_wg`: query heads of a kv head's group per workgroup of the general kernel (1, 2 or 4), or 0: the kernel with 32 rows a
-    wave where it takes the heads and pages (default: the native step's rule)."""
-    require_cuda(q, kpages, vpages, table, cu, ctx)
+    wave where it takes the heads and pages (default: the native step's rule).  `sink`, `chunk`, `softcap` and `bias` (float32
+    [distances, nh]) as in `attention_plain`."""
+    require_cuda(q, kpages, vpages, table, cu, ctx, bias)
     if q.dtype != torch.bfloat16:
         raise KernelError("attention_prefill is the bfloat16 kernel; the float32 path uses attention_plain")
     if hd % 16 or not 16 <= hd <= 128:
@@ -728,10 +730,12 @@ def attention_prefill(q: torch.Tensor, n_rows: int, nh: int, nkv: int, hd: int, 
     if n_splits > 1:
         partial = torch.empty(slices_workspace(n_rows, nh, hd, n_splits), dtype=torch.float32, device=q.device)
     assert sink is None or (sink.is_cuda and sink.dtype == torch.float32 and sink.shape == (nh,) and sink.is_contiguous())
+    assert bias is None or (bias.dtype == torch.float32 and bias.dim() == 2 and bias.shape[0] > 0 and bias.shape[1] == nh and scale > 0)
+    by_head = None if bias is None else (bias.t() / scale).contiguous()      # (held until the kernel is queued)
     call("gibbs_attention_prefill_masked", ptr(q), ptr(kpages), ptr(vpages), ptr(out), ptr(partial), ptr(cu[first_req:]),
          ptr(ctx[first_req:]), ptr(table[first_req:]), reqs, table.shape[1], page_size, num_pages, rows, nh, nkv, hd,
          q.stride(0) if n_rows > 1 else q.shape[1], nh * hd, float(scale), int(window or 0), int(n_splits), int(first_row),
-         int(heads_per_wg), None, 0, ptr(sink), int(chunk), float(softcap), stream())
+         int(heads_per_wg), ptr(by_head), 0 if bias is None else bias.shape[0], ptr(sink), int(chunk), float(softcap), stream())
     return out
 
 

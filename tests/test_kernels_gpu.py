@@ -170,6 +170,36 @@ def test_gemm_f32_stretches_shared_between_workgroups(shape):
     assert not torch.equal(bits[0].view(torch.float32), want)
 
 
+# (stretches of a workgroup: 3 to 7, which no tile's 8 are a multiple of)
+@pytest.mark.parametrize("shape,run", [((700, 1000, 4608), 3), ((1000, 1040, 2052), 5), ((1194, 1000, 2052), 5), ((1500, 1000, 2080), 6), ((1590, 1000, 4608), 7)])
+def test_gemm_f32_workgroups_that_go_on_to_the_next_tile(shape, run):
+    """A workgroup's run of stretches that ends one tile and begins the next: the bits of a workgroup a tile, for ordinary values and with
+    infinities, NaN and lost digits in rows of every tile, in stretches on both sides of wherever a tile is cut."""
+    from gibbs_amd import ops
+    from gibbs_amd.ops.lib import library
+    n, o, i = shape
+    assert library().gibbs_gemm_f32_workspace(n, o, i) > 0
+    rows, cols = -(-n // 64), -(-o // 128)
+    assert run == max(2, -(-rows * cols * 8 // 256)) and 8 % run
+    a, w = rnd(n, i, seed=1), rnd(o, i, seed=2)
+    want = ops.gemm_f32(a, w, workspace=False)
+    assert torch.equal(ops.gemm_f32(a, w), want)
+    segment = -(-(-(-i // 8)) // 32) * 32
+    for t in range(rows):      # (tile t of rows: its special values in other stretches than its neighbours')
+        def put(row, stretch, v):
+            a[min(64 * t + row, n - 1), min(stretch % 8 * segment + 5 + row, i - 1)] = v
+        put(3, t, 2.0 ** -124)
+        put(17, t + 7, float("inf"))
+        put(40, t + 4, float("nan"))
+        put(63, 3 * t + 1, 2.0 ** -130)
+    for t in range(cols):
+        w[min(128 * t + 9, o - 1), t % 8 * segment + 3] = 2.0 ** -121
+        w[min(128 * t + 100, o - 1), (t + 5) % 8 * segment + 1] = -float("inf")
+    bits = [ops.gemm_f32(a, w, workspace=k).view(torch.int32) for k in (False, True)]
+    assert torch.equal(*bits)
+    assert not torch.equal(bits[0].view(torch.float32), want)
+
+
 def test_gemm_f32_as_many_rows_as_the_plain_kernel_takes():
     """4,194,240 rows, which is where the plain kernel's grid ends, of few features: the tiles that cut k over their waves have no grid for them."""
     from gibbs_amd import ops
@@ -713,6 +743,30 @@ def test_attention_prompt_edges(nh, nkv, hd, page, how):
                                 softcap=softcap)
     assert out.isfinite().all()
     close(out, plain, torch.bfloat16, "prompt attention", bf16=1e-2)
+
+
+@pytest.mark.parametrize("heads", [0, 1])
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("softcap", [0.0, 6.0])
+@pytest.mark.parametrize("nh,nkv,hd,page", [(4, 1, 64, 16), (2, 1, 64, 8), (3, 3, 64, 64), (4, 1, 128, 16), (2, 1, 128, 32), (2, 2, 128, 8)])
+def test_attention_prompt_bias_by_distance(nh, nkv, hd, page, softcap, splits, heads):
+    """A bias on the scores by distance, with heads that look at one distance each: a table that lies one key or one row off gives other
+    rows altogether.  One, two and four heads a workgroup, capped scores too, slices that begin at any tile, more than 64 tiles; both kernels against
+    the one with a wave a row."""
+    from gibbs_amd import ops
+    q_lens, seq_lens = [1, 33, 64, 129, 70, 200], [1, 65, 64, 193, 4300, 333]
+    kp, vp, table, _, _ = paged_setup(torch.bfloat16, nkv, hd, page, seq_lens, sum(-(-s // page) for s in seq_lens) + 3, seed=17)
+    ctx = [s - n for s, n in zip(seq_lens, q_lens)]
+    cu, n, scale = np.concatenate([[0], np.cumsum(q_lens)]), sum(q_lens), 1 / math.sqrt(hd)
+    q, bias = rnd(n, nh * hd, dtype=torch.bfloat16, seed=4), rnd(300, nh, seed=5)
+    for h in range(nh):
+        bias[[63, 64, 1, 130][h], h] += 12.0
+    pos = i32([c + t for c, m in zip(ctx, q_lens) for t in range(m)])
+    row_req = i32([r for r, m in enumerate(q_lens) for _ in range(m)])
+    out = ops.attention_prefill(q, n, nh, nkv, hd, kp, vp, table, len(q_lens), i32(cu), i32(ctx), scale, n_splits=splits, heads_per_wg=heads,
+                                softcap=softcap, bias=bias)
+    plain = ops.attention_plain(q, n, nh, nkv, hd, kp, vp, table, len(q_lens), pos, row_req, scale, bias=bias, softcap=softcap)
+    close(out, plain, torch.bfloat16, "biased prompt attention", bf16=1e-2)
 
 
 @pytest.mark.parametrize("splits", [1, 3])
