@@ -8,8 +8,8 @@
 // serve all of the workgroup's heads: with one head a workgroup re-reads every key and value of its rows'
 // past for 64 x 64 scores, and at 8,192 rows and more that traffic through L2 and the compute units' L1s,
 // not the arithmetic, bounds the kernel (32,768 rows: 69 GB a call, 8.4 TB/s).  Keys are walked in tiles of
-// 64 aligned to absolute key index (so a row's sequence of operations does not depend on how the prompt
-// was cut).  Per tile:
+// 64 aligned to absolute key index (so in a call of one slice a row's sequence of operations does not depend on how the
+// prompt was cut).  Per tile:
 //   K and V tiles -> LDS as stored ([key][d]);
 //   scores transposed, S^T (64 keys x 16 rows per wave) = K Q^T by v_mfma_f32_16x16x32_bf16 over d:
 //   a lane then holds 16 scores of ONE query row (lane % 16), so that the online softmax needs no

@@ -1,8 +1,8 @@
 // Paged causal attention for prompt portions, head sizes 64 and 128: matrix instructions of 32 x 32, scores, weights and values side by side.
 //
 // A workgroup of 4 waves takes 32 RW consecutive query rows of one request and HW query heads that share a kv head (as many of the group's as
-// divide 4); a wave owns 32 rows of one head.  Keys are walked in tiles of 64 aligned to absolute key index, so that a row's sequence of
-// operations depends neither on how the prompt was cut nor on HW.  As in attention_prefill.hip the scores are made transposed, S^T = K Q^T, and
+// divide 4); a wave owns 32 rows of one head.  Keys are walked in tiles of 64 aligned to absolute key index, so that in a call of one slice a row's
+// sequence of operations depends neither on how the prompt was cut nor on HW (slices begin and end by the workgroup's rows).  As in attention_prefill.hip the scores are made transposed, S^T = K Q^T, and
 // exp(S - m) is, as it lies in the registers, the B operand of O^T += V^T P^T, V^T by the transposing LDS read.
 //
 // What bounds it: the vector instructions of the softmax (per 64 keys and 32 rows some 135, 33 of them exponentials of 8 cycles: 800 cycles),

@@ -21,9 +21,10 @@ __device__ __forceinline__ float one_and_exp_near(float z) {
   const float t = -z * LOG2E, rest = fmaf(-z, LOG2E_REST, fmaf(-z, LOG2E, -t)), power = __builtin_amdgcn_exp2f(t);
   return 1.0f + fmaf(power, rest * LN2, power);
 }
-// g / (1 + exp(-g)) in 12 instructions where `activate` takes 25, no further from the exact value: the quotient by the hardware's reciprocal with one correction
-// from its remainder.  Relative errors against float64, root mean square and largest, `activate` / here: normal values 4.8e-8, 1.8e-7 /
-// 4.2e-8, 1.7e-7; evenly from -80 to 80 3.5e-8, 2.0e-7 / 3.4e-8, 2.3e-7; rounded to bfloat16 6.1e-4, 3.9e-3 both.
+// g / (1 + exp(-g)) in 12 instructions where `activate` takes 25: the quotient by the hardware's reciprocal with one correction from its remainder.  Relative
+// errors against float64, root mean square and largest, `activate` / here: normal values 4.8e-8, 1.8e-7 / 4.2e-8, 1.7e-7; evenly from -80 to 80 3.5e-8,
+// 2.0e-7 / 3.4e-8, 2.3e-7 (the largest a little more, the mean less); rounded to bfloat16 the same for every gate, 6.1e-4, 3.9e-3, and of products with up
+// values the same within 1e-9 of the error, clamped ones too (2,048 rows of 8,192: 6 of 16.8 million values differ, 1.66e-3 both).
 __device__ __forceinline__ float silu_near(float g) {
   const float d = one_and_exp_near(g), r = __builtin_amdgcn_rcpf(d), q = g * r;
   return copysignf(fmaf(fmaf(-d, q, g), r, q), g);

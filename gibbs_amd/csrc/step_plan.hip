@@ -47,7 +47,10 @@ long ceil_div_l(long a, long b) { return (a + b - 1) / b; }
 // ------------------------------------------------------------------------------------------------- rules
 constexpr int FUSED_ROWS = 64;            // rows that the few-row products (and so the fused decode kernels) take
 constexpr int SKINNY_ROWS = 64;           // rows up to which a plain product takes the weight-streaming kernel
-constexpr int SKINNY_ROWS_F32_OUT = 48;   // the same for float32 output (the head: it streams faster than the tiled product)
+// The same for float32 output (the head).  The line was drawn against tiles of 128 x 128; those of 64 x 128, which take what is beyond it, are faster on its near
+// side too: 65,536 features of inner size 2,048, row-major, us, streaming / tiles: 40 rows 72.8 / 57.4, 48 74.6 / 57.8.  Where the two cross, and how matrices in
+// tile order stand, is not measured.
+constexpr int SKINNY_ROWS_F32_OUT = 48;
 constexpr int ACT_TANGENT = 6;            // (activation.h: ACT_TANH)
 constexpr int ACT_CLAMPED = 4;            // the gated feed-forward's clamped activation (activation.h: ACT_CLAMPED_SWISH)
 constexpr int SSD_CHUNKED_ROWS = 256;     // rows of one request from which the state-space rule runs in chunks
